@@ -1,0 +1,77 @@
+"""FP32 near field (matrix-core squared distances and the pass by differences).
+
+The FP32 modes and the FP64 mode of one input share tree, lists and order, and
+the points lie on a grid that FP32 positions relative to the root centre hold
+exactly, so the modes differ by the rounding of FP32 sums and products alone.
+Its bound: a source tile that is taken by the expansion
+|x_j|^2 - 2 x_i x_j + |x_i|^2 lies at least R / 8 from the targets' box of
+radius R, where the squared distance loses at most 2 (9/8 R)^2 / (R / 8)^2 ~ 160
+roundings of 2^-24, 1e-5, and the pair force 1.5 times that; sums over pairs of
+both signs of error stay below the single worst pair, and the FP32 expansions
+add 1e-6: 5e-5 of the force in the 2-norm leaves a factor of 3."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+BOUND = 5e-5
+
+
+@pytest.fixture(scope="module")
+def vg():
+    import vipp_gravity
+    return vipp_gravity
+
+
+def _points(n, kind, seed):
+    rng = np.random.default_rng(seed)
+    if kind == "uniform":
+        x = rng.random((n, 3)) * np.array([1.0, 0.6, 1.7])
+    else:  # a dense core inside a sparse halo: leaves of a few points beside cells of thousands
+        k = n // 2
+        x = np.concatenate([0.01 * rng.standard_normal((k, 3)) + 0.3, np.clip(rng.standard_normal((n - k, 3)), -3.9, 3.9)])
+    return np.round(x * 2 ** 18) / 2 ** 18
+
+
+# leaf thresholds floor(sqrt(8) s) around the 16-target tiles, the 96 targets of
+# one pass and beyond several passes; particle counts around the 64-source groups
+@pytest.mark.parametrize("n,s,kind", [(3, 1, "uniform"), (700, 1, "core"), (1025, 6, "uniform"), (4100, 12, "core"), (9001, 34, "uniform"),
+                                      (20011, 35, "core"), (30000, 130, "core"), (12000, 1500, "uniform")])
+@pytest.mark.parametrize("eps,masses", [(0.0, False), (1e-3, True)])
+def test_p2p_f32_against_f64_mode(vg, n, s, kind, eps, masses):
+    x = _points(n, kind, n)
+    m = np.random.default_rng(1).uniform(0.5, 1.5, n) / n if masses else None
+    r = {}
+    for mode in ("f64", "f32"):
+        with vg.Gravity(n, s, 8, mode, eps=eps, G=1.3) as g:
+            g.upload(x, None, m)
+            r[mode] = g.accelerations(), g.energy()[1]
+    a, b = r["f64"][0], r["f32"][0]
+    assert np.linalg.norm(b - a) <= BOUND * np.linalg.norm(a)
+    assert abs(r["f32"][1] - r["f64"][1]) <= 5e-6 * abs(r["f64"][1])
+
+
+def test_p2p_f32_same_twice(vg):
+    """Leaves whose sources are cut into many items: partial sums in a fixed order."""
+    x = _points(40000, "core", 5)
+    with vg.Gravity(len(x), 40, 4, "f32", eps=1e-3) as g:
+        g.upload(x)
+        a = g.accelerations()
+        assert np.array_equal(a, g.accelerations())
+
+
+def test_p2p_f32_beyond_the_range_of_squared_distances(vg):
+    """A cluster at the root centre and 20 points at each of two corners 1e19
+    away: those tiles' squared distances leave the range in which FP32 pairs
+    still pull, and the cluster feels itself alone, as an FP64 direct sum over
+    its own members gives it."""
+    c = np.random.default_rng(3).uniform(-0.5, 0.5, (40, 3))
+    far = np.full((20, 3), 6e18)
+    x = np.concatenate([far, -far, c])
+    with vg.Gravity(80, 16, 4, "f32", eps=1e-2, mass=1.0) as g:
+        g.upload(x)
+        a = g.accelerations()[40:]
+    d = c[None] - c[:, None]
+    w = ((d ** 2).sum(2) + 1e-4) ** -1.5
+    ref = (w[..., None] * d).sum(1)
+    assert np.isfinite(a).all()
+    assert np.linalg.norm(a - ref) <= BOUND * np.linalg.norm(ref)

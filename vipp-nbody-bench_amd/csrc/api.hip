@@ -99,7 +99,7 @@ static void evaluate_overlapped(Ctx &c, bool potential) {
         VG_HIP(hipEventRecord(c.ev_lists, c.stream2));
         {
             Swap on_stream2(c);
-            fmm_p2p_plan(c);
+            fmm_p2p_plan(c, potential);
         }
         operators_build(c);
         fmm_upward(c);  // enqueued while the P2P plan's item counts come back

@@ -101,7 +101,6 @@ struct Ctx {
     hipStream_t stream2 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_lists = nullptr;
     hipEvent_t ev_plan = nullptr;  // the P2P plan scalars are in the pinned words
-    uint32_t p2p_chunk = 0;        // sources per P2P work item of the current plan
     bool p2p_pending = false;
     // pinned host words for the scalars read back during an evaluation (tree
     // level sizes, root box, P2P plan): a pinned copy returns sooner
@@ -159,9 +158,9 @@ struct Ctx {
     DevBuf<uint32_t> rval[2];
 
     // P2P work items
-    DevBuf<uint32_t> p2p_scal, p2p_nchunk, p2p_item_off, p2p_local, p2p_pre, p2p_btot;
+    DevBuf<uint32_t> p2p_scal, p2p_nchunk, p2p_cls, p2p_src, p2p_item_off, p2p_local, p2p_pre, p2p_btot;
     DevBuf<uint32_t> p2p_ticket;  // per leaf: work items of a split leaf that have finished
-    DevBuf<int64_t> p2p_items;  // int2 (leaf index, chunk)
+    DevBuf<int64_t> p2p_items;  // int2 (leaf index, chunk) or, in FP32, 32-byte records
     DevBuf<float> p2p_part32;
     DevBuf<double> p2p_part64;
 
@@ -178,7 +177,7 @@ void operators_build(Ctx &c);            // M2M / L2L / M2L operators for the cu
 void fmm_upward(Ctx &c);                 // P2M + M2M
 void fmm_m2l(Ctx &c);                    // M2L (plain VALU or split MFMA by mode)
 void fmm_p2p(Ctx &c, bool potential);    // near field into the sorted accelerations (plan, then run)
-void fmm_p2p_plan(Ctx &c);               // P2P work items; the item counts are read back without waiting
+void fmm_p2p_plan(Ctx &c, bool potential);  // P2P work items; the item counts are read back without waiting
 void fmm_p2p_run(Ctx &c, bool potential);  // waits for the item counts, then the P2P kernels
 void fmm_downward(Ctx &c, bool potential);  // L2L + L2P
 void join_p2p(Ctx &c);                       // ctx.stream waits for a P2P launched on ctx.stream2

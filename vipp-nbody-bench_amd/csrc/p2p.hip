@@ -8,18 +8,19 @@
 // entries of its ancestors and itself.  Every subtree is one contiguous range
 // of the sorted particles, so each entry is a (start, count) range.
 //
-// Work items: a plan kernel counts each non-empty leaf's sources; every leaf
-// is cut into chunks of at most P2P_CHUNK sources (fewer when the leaves are
-// too few to fill the device) and each (leaf, chunk) pair is one 256-thread
-// block, so leaves with long inherited lists spread over many blocks.  A
-// block flattens its ranges in LDS, streams the chunk's sources through LDS
-// tiles and gives each lane T = 1..6 targets, in groups of 8 to 64 lanes, by
-// leaf-size class (the fewest idle lanes).
+// Work items: a plan kernel counts each non-empty leaf's sources and cuts them
+// into even chunks, so leaves with long inherited lists spread over many
+// wavefronts or blocks; each (leaf, chunk) is one item.
+//  * FP64 (k_p2p): one 256-thread block per item, which flattens its ranges in
+//    LDS, streams the chunk's sources through LDS tiles and gives each lane
+//    T = 1..6 targets, in groups of 8 to 64 lanes, by leaf-size class (the
+//    fewest idle lanes).
+//  * FP32 (k_p2p_mc): one wavefront per item, squared distances on the matrix
+//    cores.
 // A leaf with one chunk writes its result; split leaves write partial sums,
-// and the work item that finishes last adds them in chunk order
-// (deterministic).  With a nonzero
-// softening the i == j term is exactly zero (dx = dy = dz = 0), so it needs no
-// branch; without softening a select removes it.
+// which are added in chunk order (deterministic).  With a nonzero softening the
+// i == j term is exactly zero (dx = dy = dz = 0), so it needs no branch;
+// without softening a select removes it.
 #include "gravity.hpp"
 
 namespace vg {
@@ -37,6 +38,9 @@ __host__ __device__ inline int tpw_for(uint32_t nt, int T) {
     return 0;
 }
 constexpr int TMAX = 6;  // targets per lane of the largest regular class
+
+// Sources per work item of a leaf cut into nch: even, in whole groups of 64.
+__host__ __device__ inline uint32_t chunk_len(uint32_t total, uint32_t nch) { return ((total + nch - 1) / nch + 63) / 64 * 64; }
 
 template <class R>
 struct Vec4;
@@ -183,8 +187,7 @@ __global__ __launch_bounds__(P2P_THREADS) void k_p2p(const int2 *__restrict__ it
                                                      const uint32_t *__restrict__ start, const uint32_t *__restrict__ count, const int32_t *__restrict__ anc,
                                                      const int32_t *__restrict__ ni, const int32_t *__restrict__ ni_cnt,
                                                      const typename Vec4<R>::T *__restrict__ xs, R eps2, R G, R mu, typename Vec4<R>::T *__restrict__ acc,
-                                                     typename Vec4<R>::T *__restrict__ partial, uint32_t pstride, uint32_t *__restrict__ ticket,
-                                                     uint32_t chunk) {
+                                                     typename Vec4<R>::T *__restrict__ partial, uint32_t pstride, uint32_t *__restrict__ ticket) {
     using V4 = typename Vec4<R>::T;
     constexpr int CH = sizeof(R) == 4 ? 1024 : 512;
     constexpr int TR = T <= TMAX ? T : 4;  // T = TMAX + 1: leaves in batches of 256 targets, 4 per lane
@@ -240,7 +243,8 @@ __global__ __launch_bounds__(P2P_THREADS) void k_p2p(const int2 *__restrict__ it
     }
     __syncthreads();
     const uint32_t total = ent_off[E];
-    const uint32_t src0 = static_cast<uint32_t>(item.y) * chunk, src1 = min(total, src0 + chunk);
+    const uint32_t per = chunk_len(total, nchunk[item.x]);
+    const uint32_t src0 = min(total, item.y * per), src1 = min(total, src0 + per);
     V4 *out = nchunk[item.x] > 1 ? partial + static_cast<size_t>(item_off[item.x] + item.y) * pstride : nullptr;
     if constexpr (T <= TMAX) {
         p2p_leaf<R, SELF_GUARD, POT, UM, T>(tile, red, ent_start, ent_off, E, src0, src1, nt, pt0, xs, eps2, G, mu, acc, out);
@@ -279,6 +283,474 @@ __global__ __launch_bounds__(P2P_THREADS) void k_p2p(const int2 *__restrict__ it
     }
 }
 
+
+// ---- FP32: squared distances on the matrix cores -------------------------
+//
+// What bounds it: VALU issue.  Measured per wavefront instruction on gfx950
+// with 4 or more wavefronts per SIMD: FP32 add / mul / fma 2.4-2.9 cycles,
+// v_rsq_f32 8.4, other VALU 4.3, v_mfma_f32_4x4x1 8.8; FP32 matrix
+// instructions run in the VALU's own FMA units (their times add up), bf16 ones
+// beside it.  Differences, squared distance, rsq, cube and three sums cost 11
+// FP32 instructions and one rsq for 64 pairs, and the kernel that did so ran
+// at that bound: 5.97 ms for the 1.66e10 pairs of the 4M Plummer input.  Here
+//   r^2 = |x_j|^2 - 2 x_i x_j + (|x_i|^2 + eps^2)
+// is one v_mfma_f32_16x16x32_bf16 per 16 sources x 16 targets: every operand
+// is split into three bf16 values that add up to it exactly, and 8 of the 9
+// products of the parts (the last is below 2^-32) of the three coordinates and
+// the two norms fill 30 of the 32 products of a row.  Then rsq, two products,
+// and sum w (x_j - x_i) = sum w x_j - x_i sum w by v_mfma_f32_4x4x1, whose rows
+// are (x, y, z, 1) times the source's mass and whose columns are the lanes'
+// own w: 2 products and one rsq for 64 pairs beside the 8.8 cycles.  4.26 ms on
+// that input; one wavefront per item, without block barriers, and all leaf
+// sizes in one launch: 0.85 -> 0.34 ms on a 100k Plummer sphere, 0.30 -> 0.10 ms
+// on 8,000 particles.
+//
+// Error: positions are taken relative to the centre of the targets' box (radius
+// R), so at distance d from the box the expansion loses (R + d)^2 / d^2 in the
+// relative accuracy of r^2.  Tiles of 16 sources that come nearer than R / 8 are
+// left to a second pass by differences, which also has the pairs of a particle
+// with itself: 15 % of the tiles on the 4M Plummer input (R / 16: 7 %, 3 % less
+// time, but 1 % larger median errors).  Against the FP64 mode at order 12 (2^18
+// particles) RMS and median force errors are what differences alone gave:
+// 4.27e-5 and 3.9e-7 (uniform), 1.63e-6 and 3.3e-7 (Plummer), 4.98e-5 and 5.3e-7
+// (mixture), most of it the rounding of positions relative to the root centre.
+constexpr float MC_NEAR = 1.0f / 8;
+// 16-target tiles of an item at most: 8 registers a tile and 4 more in flight;
+// the potential's mass products take the registers of one (6 there: 0.71
+// against 0.66 ms at 2^18 particles)
+constexpr int mc_tiles(bool pot) { return pot ? 5 : 6; }
+// An item's cost is its target tiles times its 64-source groups: at most 512
+// (256 and 1024: +4 % and +0 % on the 4M Plummer input, -10 % and +20 % at 100k
+// particles), less with few leaves, and at most 64 groups, one per lane of the
+// entry table.
+constexpr uint32_t MC_COST = 512, MC_MINCOST = 16;
+constexpr uint32_t MC_CHUNK = 64 * 64;
+// A leaf's targets go to items of at most mt tiles, evenly.
+__host__ __device__ inline uint32_t mc_batches(uint32_t nt, int mt) { return ((nt + 15) / 16 + mt - 1) / mt; }
+__host__ __device__ inline uint32_t mc_batch_tiles(uint32_t nt, int mt) { return ((nt + 15) / 16 + mc_batches(nt, mt) - 1) / mc_batches(nt, mt); }
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+
+// [upper 16 bits of lo, upper 16 bits of hi]: two bf16 values cut off (not rounded)
+__device__ __forceinline__ uint32_t pk_bf16(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
+__device__ __forceinline__ float cut_bf16(float x) { return __uint_as_float(__float_as_uint(x) & 0xffff0000u); }
+// x = h + m + l with three bf16 values, exactly (3 x 8 of the 24 bits): h, m
+// and l are the upper halves of x, r1 and r2.
+struct Split3 {
+    float x, r1, r2;
+    __device__ __forceinline__ explicit Split3(float v) : x(v), r1(v - cut_bf16(v)), r2(r1 - cut_bf16(r1)) {}
+    __device__ __forceinline__ uint32_t hm() const { return pk_bf16(x, r1); }
+    __device__ __forceinline__ uint32_t hh() const { return pk_bf16(x, x); }
+    __device__ __forceinline__ uint32_t mm() const { return pk_bf16(r1, r1); }
+    __device__ __forceinline__ uint32_t ll() const { return pk_bf16(r2, r2); }
+};
+constexpr uint32_t BF16_ONES = 0x3f803f80u;
+
+struct McLds {
+    uint4 P[4][64];        // 64 staged sources: bf16 operand, one 16-byte group per 16 lanes of the product
+    float4 Q[64];          // m (x, y, z, 1) of the staged sources; (x, y, z, m) in the near pass; while the entries are laid out, their masks
+    int32_t delta[MAXE];   // per entry of the item: particle index minus position in the item
+    uint16_t near[64 * 4]; // 16-source tiles left to the near pass
+    float4 M[16];          // masses of the staged sources (for the potential)
+};
+
+// A work item as the plan leaves it.
+struct alignas(32) McWork {
+    int32_t cell, level;  // the leaf
+    uint32_t pt0, nt;     // its targets: particles pt0 .. pt0 + nt - 1, of the leaf's from t0 on
+    uint32_t src0, len;   // its share of the leaf's sources
+    uint32_t out;         // row of partial sums of this share, ~0: the only share
+    uint32_t t0;
+};
+
+// What a wavefront knows of its work item.
+struct McItem {
+    const float4 *xs;     // sorted particles (x, y, z relative to the root centre, m)
+    uint32_t len;         // sources
+    uint32_t mlo, mhi;    // lane g: where entries begin in group g (from its second source on)
+    int rank;             // lane g: entry of group g's first source
+    uint32_t pt0;         // first target
+    int nt;               // targets
+    float cell;           // half diagonal of the leaf
+    float eps2;
+    bool um;              // one mass: left out here, the sums are scaled once
+    bool big;             // squared distances may leave the FP32 range
+};
+
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The item's T tiles of 16 targets against its sources; emit(t, v) gets target
+// t's sums (force xyz, potential), in one lane.
+template <int T, bool POT, class F>
+__device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
+    const int lane = threadIdx.x, col = lane & 15, quad = lane >> 4;
+    const int ng = static_cast<int>((I.len + 63) / 64);
+    const float4 first = I.xs[I.pt0];
+    float cx = first.x, cy = first.y, cz = first.z;
+    auto target = [&](int t) {  // columns past the last target repeat it and are dropped
+        const float4 v = I.xs[I.pt0 + min(16 * t + col, I.nt - 1)];
+        return float3{v.x - cx, v.y - cy, v.z - cz};
+    };
+    // box of the targets, relative to the first one; its centre is the origin from here on
+    float hx, hy, hz, ns;
+    {
+        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const float3 x = target(t);
+            lo[0] = fminf(lo[0], x.x), hi[0] = fmaxf(hi[0], x.x);
+            lo[1] = fminf(lo[1], x.y), hi[1] = fmaxf(hi[1], x.y);
+            lo[2] = fminf(lo[2], x.z), hi[2] = fmaxf(hi[2], x.z);
+        }
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            for (int d = 1; d < 16; d <<= 1) {
+                lo[a] = fminf(lo[a], __shfl_xor(lo[a], d, 64));
+                hi[a] = fmaxf(hi[a], __shfl_xor(hi[a], d, 64));
+            }
+        cx += 0.5f * (lo[0] + hi[0]), cy += 0.5f * (lo[1] + hi[1]), cz += 0.5f * (lo[2] + hi[2]);
+        hx = 0.5f * (hi[0] - lo[0]), hy = 0.5f * (hi[1] - lo[1]), hz = 0.5f * (hi[2] - lo[2]);
+        // sources up to near from the box are near; ns = 1 / (2 near), 0 where all are
+        const float r = sqrtf(hx * hx + hy * hy + hz * hz);
+        const float nearest = fmaxf(r * MC_NEAR, I.cell * 0.0078125f);
+        ns = r < 1e18f ? 0.5f / nearest : 0.0f;
+        hx = -ns * (hx + I.cell * 1e-5f), hy = -ns * (hy + I.cell * 1e-5f), hz = -ns * (hz + I.cell * 1e-5f);
+    }
+    asm volatile("" ::: "memory");  // the targets are read again, not kept in registers
+    bf8 b[T];
+    f4 acc[T];
+    float pot[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const float3 x = target(t);
+        const Split3 v(quad == 0 ? -2.0f * x.x : quad == 1 ? -2.0f * x.y : quad == 2 ? -2.0f * x.z : x.x * x.x + x.y * x.y + x.z * x.z + I.eps2);
+        const uint4 w = quad < 3 ? uint4{v.hh(), v.mm(), v.ll(), v.hm()} : uint4{BF16_ONES, pk_bf16(1.0f, v.x), pk_bf16(v.r1, v.r2), 0u};
+        b[t] = __builtin_bit_cast(bf8, w);
+        acc[t] = f4{0, 0, 0, 0};
+        pot[t] = 0;
+    }
+    const float *Qw = reinterpret_cast<const float *>(S.Q);
+    const f4 zero = {0, 0, 0, 0};
+    // far pass: groups of 64 sources, near tiles put aside
+    auto source = [&](int g) {  // this lane's source of group g
+        const uint32_t lo = __builtin_amdgcn_readlane(I.mlo, g), hi = __builtin_amdgcn_readlane(I.mhi, g);
+        const int e = __builtin_amdgcn_readlane(I.rank, g) + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+        return I.xs[S.delta[e] + static_cast<int32_t>(min(64u * g + lane, I.len - 1))];
+    };
+    uint32_t mynear = 0;  // lane g: near tiles of group g
+    float4 nx = source(0);
+    for (int g = 0; g < ng; ++g) {
+        float x = nx.x - cx, y = nx.y - cy, z = nx.z - cz;
+        float m = I.um ? 1.0f : nx.w;
+        if (g + 1 < ng)
+            nx = source(g + 1);
+        else if (64u * g + lane >= I.len)  // the last source again, without mass
+            m = 0.0f;
+        auto out01 = [&](float v, float h) { return __builtin_amdgcn_fmed3f(fmaf(fabsf(v), ns, h), 0.0f, 1.0f); };
+        const float ex = out01(x, hx), ey = out01(y, hy), ez = out01(z, hz);
+        const uint64_t near = __ballot(ex * ex + ey * ey + ez * ez <= 0.25f);
+        uint32_t nib = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) nib |= ((near >> (16 * k)) & 0xffff) ? 1u << k : 0u;
+        if (nib) {
+            mynear = lane == g ? nib : mynear;
+            if (nib == 15) continue;
+        }
+        float n2 = x * x + y * y + z * z;
+        if (I.big && !(n2 < 1e37f)) x = y = z = m = 0.0f, n2 = 1e37f;  // a source that far away pulls with 0 in FP32
+        __builtin_amdgcn_wave_barrier();  // the last group's reads come before these writes (one wavefront's LDS accesses keep their order)
+        const Split3 sx(x), sy(y), sz(z), sn(n2);
+        S.P[0][lane] = uint4{sx.hm(), sx.hm(), sx.hm(), sx.ll()};
+        S.P[1][lane] = uint4{sy.hm(), sy.hm(), sy.hm(), sy.ll()};
+        S.P[2][lane] = uint4{sz.hm(), sz.hm(), sz.hm(), sz.ll()};
+        S.P[3][lane] = uint4{sn.hm(), pk_bf16(sn.r2, 1.0f), BF16_ONES, 0u};
+        S.Q[lane] = float4{m * x, m * y, m * z, m};
+        if (POT) reinterpret_cast<float *>(S.M)[lane] = m;
+        wave_lds_sync();
+        auto distances = [&](int k, f4 *r) {
+            const bf8 a = __builtin_bit_cast(bf8, S.P[quad][16 * k + col]);
+#pragma unroll
+            for (int t = 0; t < T; ++t) r[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[t], zero, 0, 0, 0);
+        };
+        auto sums = [&](int k, float q, f4 *r) {
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r[t][i] = rsq(r[t][i]);
+            if (POT) {
+                const float4 m4 = S.M[4 * k + quad];
+#pragma unroll
+                for (int t = 0; t < T; ++t) pot[t] += m4.x * r[t][0] + m4.y * r[t][1] + m4.z * r[t][2] + m4.w * r[t][3];
+            }
+#pragma unroll
+            for (int t = 0; t < T; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r[t][i] = r[t][i] * r[t][i] * r[t][i];
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(q, r[t][0], acc[t], 2, 0, 0);
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(q, r[t][1], acc[t], 2, 1, 0);
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(q, r[t][2], acc[t], 2, 2, 0);
+#pragma unroll
+            for (int t = 0; t < T; ++t) acc[t] = __builtin_amdgcn_mfma_f32_4x4x1f32(q, r[t][3], acc[t], 2, 3, 0);
+        };
+#pragma unroll 1
+        for (int k = 0; k < 4; ++k) {
+            if (nib >> k & 1) continue;
+            f4 r[T];
+            const float q = Qw[64 * k + lane];
+            distances(k, r);
+            sums(k, q, r);
+            // all rsq, then the products, then the sums: 4.69 -> 4.52 ms on the 4M Plummer input against the compiler's order
+            __builtin_amdgcn_sched_group_barrier(0x400, 4 * T, 0);
+            __builtin_amdgcn_sched_group_barrier(0x2, (POT ? 12 : 8) * T, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 4 * T, 0);
+        }
+    }
+    asm volatile("" ::: "memory");
+    // sum m w (x_j - x_i) = sum m w x_j - x_i sum m w; from here on positions are as stored
+    float xt[T], yt[T], zt[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const float3 x = target(t);
+        acc[t][0] -= x.x * acc[t][3];
+        acc[t][1] -= x.y * acc[t][3];
+        acc[t][2] -= x.z * acc[t][3];
+        acc[t][3] = pot[t];
+    }
+    cx = cy = cz = 0.0f;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const float3 x = target(t);
+        xt[t] = x.x, yt[t] = x.y, zt[t] = x.z;
+    }
+    // near pass: four 16-source tiles at a time, by differences
+    int nn;
+    {
+        int incl = __builtin_popcount(mynear);
+        const int own = incl;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        nn = __builtin_amdgcn_readlane(incl, 63);
+        int at = incl - own;
+        for (int k = 0; k < 4; ++k)
+            if (mynear >> k & 1) S.near[at++] = static_cast<uint16_t>(4 * lane + k);
+        wave_lds_sync();
+    }
+    auto near_source = [&](int j) {  // this lane's source of the near tiles 4 j .. 4 j + 3
+        const int n = 4 * j + quad;
+        const int tl = S.near[min(n, nn - 1)], g = tl >> 2, pos = 16 * (tl & 3) + col;
+        const uint64_t m = static_cast<uint64_t>(static_cast<uint32_t>(__shfl(static_cast<int>(I.mhi), g, 64))) << 32 | static_cast<uint32_t>(__shfl(static_cast<int>(I.mlo), g, 64));
+        const int e = __shfl(I.rank, g, 64) + __popcll(m & ((1ull << pos) - 1));
+        const uint32_t f = 64u * g + pos;
+        float4 v = I.xs[S.delta[e] + static_cast<int32_t>(min(f, I.len - 1))];
+        if (I.um) v.w = 1.0f;
+        if (n >= nn || f >= I.len) v.w = 0.0f;
+        return v;
+    };
+    if (nn > 0) nx = near_source(0);
+    for (int j = 0; 4 * j < nn; ++j) {
+        __builtin_amdgcn_wave_barrier();
+        S.Q[lane] = nx;
+        if (4 * j + 4 < nn) nx = near_source(j + 1);
+        wave_lds_sync();
+        const int kn = min(4, nn - 4 * j);
+        auto pairs = [&](auto soft) {
+#pragma unroll 1
+            for (int k = 0; k < kn; ++k) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float4 s = S.Q[16 * k + 4 * quad + i];
+#pragma unroll
+                    for (int t = 0; t < T; ++t) {
+                        const float dx = s.x - xt[t], dy = s.y - yt[t], dz = s.z - zt[t];
+                        const float r2 = I.eps2 + dx * dx + dy * dy + dz * dz;
+                        float ri = rsq(r2);
+                        if (!decltype(soft)::value) ri = r2 > 0.0f ? ri : 0.0f;  // a particle and itself
+                        const float mr = s.w * ri, w = mr * ri * ri;
+                        acc[t][0] += w * dx;
+                        acc[t][1] += w * dy;
+                        acc[t][2] += w * dz;
+                        if (POT) acc[t][3] += mr;
+                    }
+                }
+            }
+        };
+        if (I.eps2 > 0.0f)
+            pairs(std::true_type{});
+        else
+            pairs(std::false_type{});
+    }
+    // the four lane groups hold the sums over their own source rows
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+#pragma unroll
+        for (int j = 0; j < (POT ? 4 : 3); ++j) {
+            acc[t][j] += __shfl_xor(acc[t][j], 16, 64);
+            acc[t][j] += __shfl_xor(acc[t][j], 32, 64);
+        }
+        if (quad == 0 && 16 * t + col < I.nt) emit(16 * t + col, acc[t]);
+    }
+}
+
+// One wavefront per work item.
+template <bool POT>
+__global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ items, const uint32_t *__restrict__ start,
+                                                       const uint32_t *__restrict__ count, const int32_t *__restrict__ anc,
+                                                       const int32_t *__restrict__ ni, const int32_t *__restrict__ ni_cnt,
+                                                       const double *__restrict__ bmin, const double *__restrict__ bmax, const float4 *__restrict__ xs,
+                                                       float eps2, float G, bool um, bool big, float mu, float4 *__restrict__ acc,
+                                                       float4 *__restrict__ partial, uint32_t pstride) {
+    __shared__ McLds S;
+    const McWork wk = items[blockIdx.x];
+    const int32_t c = wk.cell;
+    const int lev = wk.level, lane = threadIdx.x;
+    McItem I;
+    I.nt = static_cast<int>(wk.nt);
+    I.pt0 = wk.pt0;
+    I.len = wk.len;
+    uint64_t *mask = reinterpret_cast<uint64_t *>(S.Q);
+    mask[lane] = 0;
+    // the leaf's NI list: its ancestors' own entries, root first; lane l has ancestor l
+    const int32_t an = lane <= lev ? anc[static_cast<int64_t>(c) * (MAXD + 1) + lane] : 0;
+    const int an_cnt = lane <= lev ? ni_cnt[an] : 0;
+    int an_end = an_cnt;
+    for (int d = 1; d < 32; d <<= 1) {
+        const int o = __shfl_up(an_end, d, 64);
+        if (lane >= d) an_end += o;
+    }
+    const int E = __builtin_amdgcn_readlane(an_end, lev);
+    const uint64_t live = __ballot(an_cnt > 0);
+    auto entry = [&](int e, uint32_t &st, uint32_t &cn) {  // particle range of entry e
+        int l = 0;
+        for (uint64_t w = live; w; w &= w - 1) {  // the last ancestor with entries whose first one is <= e
+            const int k = __builtin_ctzll(w);
+            if (__builtin_amdgcn_readlane(an_end - an_cnt, k) <= e) l = k;
+        }
+        const int32_t a = __shfl(an, l, 64);
+        const int o = e - __shfl(an_end - an_cnt, l, 64);
+        st = cn = 0;
+        if (e < E) {
+            const int32_t cell = ni[27 * static_cast<int64_t>(a) + o];
+            st = start[cell];
+            cn = count[cell];
+        }
+    };
+    // the entries that reach into [src0, src1), empty ones dropped, and where they begin in it
+    const uint32_t src0 = wk.src0, src1 = src0 + wk.len;
+    wave_lds_sync();
+    uint32_t carry = 0, st, cn;
+    int kept = 0;
+    entry(lane, st, cn);
+    for (int e0 = 0; e0 < E && carry < src1; e0 += 64) {
+        uint32_t nst = 0, ncn = 0;
+        if (e0 + 64 < E) entry(e0 + 64 + lane, nst, ncn);  // on its way while this run is laid out
+        uint32_t incl = cn;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        const uint32_t off = carry + incl - cn;
+        const bool in = cn > 0 && off + cn > src0 && off < src1;
+        const uint64_t bal = __ballot(in);
+        if (in) {
+            S.delta[kept + __popcll(bal & ((1ull << lane) - 1))] = static_cast<int32_t>(st - (off - src0));
+            const uint32_t o = max(off, src0) - src0;
+            atomicOr(reinterpret_cast<unsigned long long *>(&mask[o >> 6]), 1ull << (o & 63));
+        }
+        kept += __popcll(bal);
+        carry += __builtin_amdgcn_readlane(incl, 63);
+        st = nst, cn = ncn;
+    }
+    wave_lds_sync();
+    {  // lane g: the entry of group g's first source, and the later begins shifted so that mbcnt counts them
+        const uint64_t m = mask[lane];
+        const int own = __popcll(m);
+        int incl = own;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        I.rank = incl - own + static_cast<int>(m & 1) - 1;
+        I.mlo = static_cast<uint32_t>(m >> 1);
+        I.mhi = static_cast<uint32_t>(m >> 33);
+    }
+    wave_lds_sync();
+    I.xs = xs;
+    const double lx = bmin[3ll * c], ly = bmin[3ll * c + 1], lz = bmin[3ll * c + 2], ux = bmax[3ll * c], uy = bmax[3ll * c + 1], uz = bmax[3ll * c + 2];
+    const float wx = static_cast<float>(ux - lx), wy = static_cast<float>(uy - ly), wz = static_cast<float>(uz - lz);
+    I.cell = 0.5f * sqrtf(wx * wx + wy * wy + wz * wz);
+    I.eps2 = eps2;
+    I.um = um;
+    I.big = big;
+    const float sc = um ? mu : 1.0f;
+    float4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * pstride : nullptr;
+    auto emit = [&](int t, const f4 &v) {
+        const float sx = v[0] * sc, sy = v[1] * sc, sz = v[2] * sc;
+        float sp = v[3] * sc;
+        if (out) {
+            out[wk.t0 + t] = float4{sx, sy, sz, sp};
+        } else {
+            if (POT && eps2 > 0.0f) sp -= xs[I.pt0 + t].w * rsq(eps2);  // drop the m_i / eps self term
+            acc[I.pt0 + t] = float4{G * sx, G * sy, G * sz, sp};
+        }
+    };
+    if (I.len == 0) {  // a last chunk that the even lengths left empty
+        for (int t = lane; t < I.nt; t += 64) emit(t, f4{0, 0, 0, 0});
+        return;
+    }
+    constexpr int MT = mc_tiles(POT);
+    const int T = (I.nt + 15) / 16;  // at most MT
+    if (T == 1)
+        mc_pass<1, POT>(I, S, emit);
+    else if (T == 2)
+        mc_pass<2, POT>(I, S, emit);
+    else if (T == 3)
+        mc_pass<3, POT>(I, S, emit);
+    else if (T == 4)
+        mc_pass<4, POT>(I, S, emit);
+    else if (T == 5)
+        mc_pass<5, POT>(I, S, emit);
+    else
+        mc_pass<MT, POT>(I, S, emit);
+}
+
+// Leaves split over several work items: partial sums added in chunk order
+// (the same order every run), a wavefront per leaf.
+template <bool POT>
+__global__ __launch_bounds__(256) void k_p2p_sum(const int32_t *__restrict__ leaves, int nleaves, const uint32_t *__restrict__ nchunk,
+                                                 const uint32_t *__restrict__ item_off, const uint32_t *__restrict__ start, const uint32_t *__restrict__ count,
+                                                 const float4 *__restrict__ xs, float eps2, float G, float4 *__restrict__ acc,
+                                                 const float4 *__restrict__ partial, uint32_t pstride) {
+    const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (k >= nleaves) return;
+    const uint32_t nch = nchunk[k];
+    if (nch < 2) return;
+    const int32_t c = leaves[k];
+    const uint32_t nt = count[c], pt0 = start[c];
+    const float4 *pk = partial + static_cast<size_t>(item_off[k]) * pstride;
+    for (uint32_t t = threadIdx.x & 63; t < nt; t += 64) {
+        float sx = 0, sy = 0, sz = 0, sp = 0;
+#pragma unroll 8
+        for (uint32_t q = 0; q < nch; ++q) {
+            const float4 v = pk[static_cast<size_t>(q) * pstride + t];
+            sx += v.x;
+            sy += v.y;
+            sz += v.z;
+            sp += v.w;
+        }
+        if (POT && eps2 > 0.0f) sp -= xs[pt0 + t].w * rsq(eps2);
+        acc[pt0 + t] = float4{G * sx, G * sy, G * sz, sp};
+    }
+}
+
 // Per leaf: number of sources in its NI chain, split into chunks of at most
 // chunk sources (bounded work per block), and its class by targets per lane.
 // Sources of each cell's own NI entries (the leaf's full list is its
@@ -297,9 +769,15 @@ __global__ __launch_bounds__(256) void k_ni_local(int64_t ncells, const uint32_t
 // of tpw_for(nt, T) lanes, T chosen for the fewest lane slots TPW T >= nt
 // (ties: fewer targets per lane); class TMAX: more than 64 TMAX targets, in
 // batches of 256.
+// FP32 items (mt > 0: at most mt target tiles) differ only in cost (16-target
+// tiles times 64-source groups): class j costs at least 2^(8 - j), so the largest start first.
 constexpr int NCLS = TMAX + 1;
 constexpr int NSC = NCLS + 2;  // scanned per leaf: chunks, chunks of each class, split flag
-__device__ inline int leaf_class(uint32_t nt) {
+__device__ inline int leaf_class(uint32_t nt, uint32_t src, uint32_t nch, int mt) {
+    if (mt) {
+        const uint32_t cost = mc_batch_tiles(nt, mt) * (chunk_len(src, nch) / 64);
+        return max(0, min(TMAX, 8 - (31 - __builtin_clz(max(cost, 1u)))));
+    }
     if (nt > 64u * TMAX) return TMAX;
     int best = 0;
     uint32_t slots = ~0u;
@@ -313,12 +791,13 @@ __device__ inline int leaf_class(uint32_t nt) {
     return best;
 }
 
-// Per leaf: source count -> chunks and class; block-local exclusive scans of
+// Per leaf: source count -> chunks (of at most chunk sources or, for mc, of at
+// most chunk target tiles times source groups) and class; block-local exclusive scans of
 // the NSC components (one leaf per thread, 256 per block) and block totals.
 __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ leaves, int nleaves, const int8_t *__restrict__ level,
                                                   const uint32_t *__restrict__ count, const int32_t *__restrict__ anc, const uint32_t *__restrict__ local,
-                                                  uint32_t *__restrict__ nchunk, uint32_t *__restrict__ pre, uint32_t *__restrict__ btot,
-                                                  uint32_t chunk) {
+                                                  uint32_t *__restrict__ nchunk, uint32_t *__restrict__ cls, uint32_t *__restrict__ nsrc, uint32_t *__restrict__ pre,
+                                                  uint32_t *__restrict__ btot, uint32_t chunk, int mt, uint32_t minrow) {
     __shared__ uint32_t wtot[4][NSC];
     const int k = blockIdx.x * 256 + threadIdx.x;
     const unsigned lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -327,10 +806,18 @@ __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ le
         const int32_t c = leaves[k];
         uint32_t src = 0;
         for (int l = 0; l <= level[c]; ++l) src += local[anc[static_cast<int64_t>(c) * (MAXD + 1) + l]];
-        const uint32_t nch = max(1u, (src + chunk - 1) / chunk);
+        const uint32_t nt = count[c];
+        // mt: as many groups as the cost allows, but no fewer than minrow eighths of the tiles (the rows of partial sums of a large leaf stay few)
+        const uint32_t lim = mt ? 64 * min(MC_CHUNK / 64, max(1 + (nt + 15) / 16 * minrow / 8, chunk / mc_batch_tiles(nt, mt))) : chunk;
+        const uint32_t nch = max(1u, (src + lim - 1) / lim);
         nchunk[k] = nch;
-        v[0] = nch;
-        v[1 + leaf_class(count[c])] = nch;
+        nsrc[k] = src;
+        const uint32_t nit = mt ? nch * mc_batches(nt, mt) : nch;
+        v[0] = nch > 1 ? nch : 0u;
+        const int cl = leaf_class(nt, src, nch, mt);
+        cls[k] = cl;
+#pragma unroll
+        for (int q = 0; q < NCLS; ++q) v[1 + q] = q == cl ? nit : 0u;
         v[NSC - 1] = nch > 1 ? 1u : 0u;
     }
     uint32_t inc[NSC];
@@ -357,7 +844,7 @@ __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ le
 // One block: exclusive scan of the block totals; writes the class counts and
 // bases, the item total and the split-leaf total into scal:
 //   scal[0..NCLS) items per class, scal[NCLS..2 NCLS) class bases,
-//   scal[2 NCLS] items, scal[2 NCLS + 1] split leaves.
+//   scal[2 NCLS] rows of partial sums, scal[2 NCLS + 1] split leaves.
 __global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ btot, int nblocks, uint32_t *__restrict__ scal) {
     // exclusive scan of each component over the plan blocks, one wavefront per
     // component (wavefront-wide inclusive scans, carried across runs of 64)
@@ -379,7 +866,7 @@ __global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ 
         if (lane == 0) tot[q] = carry;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {  // scal: [class items] [class bases] total items, split leaves
+    if (threadIdx.x == 0) {  // scal: [class items] [class bases] rows, split leaves
         scal[2 * NCLS] = tot[0];
         scal[2 * NCLS + 1] = tot[NSC - 1];
         uint32_t base = 0;
@@ -393,7 +880,7 @@ __global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ 
 
 // Item offsets, items (leaf, chunk) bucketed by class in leaf order, and the
 // list of leaves whose sources span several chunks.
-__global__ __launch_bounds__(256) void k_p2p_items(const int32_t *__restrict__ leaves, int nleaves, const uint32_t *__restrict__ count,
+__global__ __launch_bounds__(256) void k_p2p_items(int nleaves, const uint32_t *__restrict__ lcls,
                                                    const uint32_t *__restrict__ nchunk, const uint32_t *__restrict__ pre,
                                                    const uint32_t *__restrict__ boff, const uint32_t *__restrict__ scal,
                                                    uint32_t *__restrict__ item_off, int2 *__restrict__ items) {
@@ -403,22 +890,48 @@ __global__ __launch_bounds__(256) void k_p2p_items(const int32_t *__restrict__ l
     const uint32_t *bk = boff + blockIdx.x * NSC;
     const uint32_t nch = nchunk[k];
     item_off[k] = bk[0] + pk[0];
-    const int cls = leaf_class(count[leaves[k]]);
+    const int cls = lcls[k];
     const uint32_t pos = scal[NCLS + cls] + bk[1 + cls] + pk[1 + cls];
     for (uint32_t q = 0; q < nch; ++q) items[pos + q] = make_int2(k, static_cast<int>(q));
+}
+
+// The FP32 kernel's items, each with what its wavefront needs to start.
+__global__ __launch_bounds__(256) void k_p2p_items_mc(const int32_t *__restrict__ leaves, int nleaves, const int8_t *__restrict__ level,
+                                                      const uint32_t *__restrict__ start, const uint32_t *__restrict__ count,
+                                                      const uint32_t *__restrict__ lcls, const uint32_t *__restrict__ nchunk,
+                                                      const uint32_t *__restrict__ nsrc, const uint32_t *__restrict__ pre,
+                                                      const uint32_t *__restrict__ boff, const uint32_t *__restrict__ scal,
+                                                      uint32_t *__restrict__ item_off, McWork *__restrict__ items, int mt) {
+    const int k = blockIdx.x * 256 + threadIdx.x;
+    if (k >= nleaves) return;
+    const uint32_t *pk = pre + static_cast<int64_t>(k) * NSC;
+    const uint32_t *bk = boff + blockIdx.x * NSC;
+    const uint32_t nch = nchunk[k], off = bk[0] + pk[0], src = nsrc[k], per = chunk_len(src, nch);
+    item_off[k] = off;
+    const int cls = lcls[k];
+    const int32_t c = leaves[k];
+    const uint32_t nt = count[c], pt0 = start[c], bt = 16 * mc_batch_tiles(nt, mt);
+    McWork *it = items + scal[NCLS + cls] + bk[1 + cls] + pk[1 + cls];
+    for (uint32_t t0 = 0; t0 < nt; t0 += bt)
+        for (uint32_t q = 0; q < nch; ++q) {
+            const uint32_t s0 = min(src, q * per);
+            *it++ = McWork{c, level[c], pt0 + t0, min(bt, nt - t0), s0, min(src, s0 + per) - s0, nch > 1 ? off + q : ~0u, t0};
+        }
 }
 
 // Work items of the P2P: counts per leaf, then the plan scalars (items per
 // class) copied back to pinned host words, with ev_plan recorded after the
 // copy.  Nothing here waits, so the caller can enqueue other work before
 // p2p_run needs the scalars.
-void p2p_plan(Ctx &c) {
+void p2p_plan(Ctx &c, bool potential) {
     TreeDev &t = c.t;
     if (!t.nleaves) return;
     const int nl = static_cast<int>(t.nleaves);
     const int nb = static_cast<int>(ceil_div(nl, 256));
     c.p2p_scal.ensure(16);
     c.p2p_nchunk.ensure(nl);
+    c.p2p_cls.ensure(nl);
+    c.p2p_src.ensure(nl);
     c.p2p_item_off.ensure(nl);
     c.p2p_local.ensure(t.ncells);
     c.p2p_pre.ensure(static_cast<size_t>(nl) * NSC);
@@ -426,13 +939,14 @@ void p2p_plan(Ctx &c) {
     c.p2p_ticket.ensure(nl);
     k_ni_local<<<ceil_div(t.ncells, 256), 256, 0, c.stream>>>(t.ncells, t.count, t.ni, t.ni_cnt, c.p2p_local);
     // under 8 leaves per CU (the 16k Plummer sphere has 430): chunks of 8192
-    // sources scaled down by the leaf shortfall (at least 1024), so that the
-    // work items still give every CU several blocks
-    uint32_t chunk = P2P_CHUNK;
+    // sources, or items of MC_COST, scaled down by the leaf shortfall, so that
+    // the work items still give every CU several blocks
+    uint32_t chunk = c.prec == 0 ? P2P_CHUNK : MC_COST;
     if (c.ncu > 0 && nl < 8 * c.ncu)
-        chunk = std::max<uint32_t>(1024, static_cast<uint32_t>(8192ull * nl / (8 * c.ncu)) / 256 * 256);
-    c.p2p_chunk = chunk;
-    k_p2p_plan<<<nb, 256, 0, c.stream>>>(t.leaf_ids, nl, t.level, t.count, t.anc, c.p2p_local, c.p2p_nchunk, c.p2p_pre, c.p2p_btot, chunk);
+        chunk = c.prec == 0 ? std::max<uint32_t>(1024, static_cast<uint32_t>(8192ull * nl / (8 * c.ncu)) / 256 * 256)
+                            : std::max<uint32_t>(MC_MINCOST, static_cast<uint32_t>(1ull * MC_COST * nl / (8 * c.ncu)));
+    k_p2p_plan<<<nb, 256, 0, c.stream>>>(t.leaf_ids, nl, t.level, t.count, t.anc, c.p2p_local, c.p2p_nchunk, c.p2p_cls, c.p2p_src, c.p2p_pre, c.p2p_btot, chunk,
+                                        c.prec == 0 ? 0 : mc_tiles(potential), nl < 8 * c.ncu ? 1 : 8);
     k_p2p_plan_blocks<<<1, 256, 0, c.stream>>>(c.p2p_btot, nb, c.p2p_scal);
     VG_LAUNCH_CHECK();
     static_assert(2 * NCLS + 2 <= 16, "plan scalars");
@@ -441,59 +955,78 @@ void p2p_plan(Ctx &c) {
     VG_HIP(hipEventRecord(c.ev_plan, c.stream));
 }
 
-// The P2P itself, on the stream p2p_plan used: waits on the host for the plan
-// scalars, then launches one kernel per leaf class.
-template <class R>
-void p2p_run(Ctx &c, bool potential) {
+// The plan's scalars, waited for on the host: items per class, class bases,
+// rows of partial sums, split leaves.
+static const uint32_t *p2p_scalars(Ctx &c) {
+    VG_HIP(hipEventSynchronize(c.ev_plan));
+    return reinterpret_cast<const uint32_t *>(static_cast<const char *>(c.pinned) + 128);
+}
+
+// FP32 P2P: one launch over all items, on the stream p2p_plan used.
+void p2p_run_f32(Ctx &c, bool potential) {
     TreeDev &t = c.t;
     if (!t.nleaves) return;
-    using V4 = typename Vec4<R>::T;
-    const V4 *xs = reinterpret_cast<const V4 *>(sizeof(R) == 4 ? static_cast<const void *>(c.xs32.p) : static_cast<const void *>(c.xs64.p));
-    V4 *acc;
-    if (sizeof(R) == 4) {
-        c.as32.ensure(4 * std::max<int64_t>(1, c.n));
-        acc = reinterpret_cast<V4 *>(c.as32.p);
-    } else {
-        c.as64.ensure(4 * std::max<int64_t>(1, c.n));
-        acc = reinterpret_cast<V4 *>(c.as64.p);
-    }
-    const R eps2 = static_cast<R>(c.eps * c.eps);
+    const uint32_t *hs = p2p_scalars(c);
+    const uint32_t nitems = hs[2 * NCLS - 1] + hs[NCLS - 1], nrows = hs[2 * NCLS], pstride = c.thr;
+    const bool split = hs[2 * NCLS + 1] > 0;
+    const int nl = static_cast<int>(t.nleaves);
+    c.p2p_items.ensure(sizeof(McWork) / 8 * static_cast<size_t>(std::max<uint32_t>(1, nitems)));
+    McWork *items = reinterpret_cast<McWork *>(c.p2p_items.p);
+    k_p2p_items_mc<<<ceil_div(nl, 256), 256, 0, c.stream>>>(t.leaf_ids, nl, t.level, t.start, t.count, c.p2p_cls, c.p2p_nchunk, c.p2p_src, c.p2p_pre,
+                                                            c.p2p_btot, c.p2p_scal, c.p2p_item_off, items, mc_tiles(potential));
+    VG_LAUNCH_CHECK();
+    c.as32.ensure(4 * std::max<int64_t>(1, c.n));
+    if (split) c.p2p_part32.ensure(4 * static_cast<size_t>(nrows) * pstride);
+    const float eps2 = static_cast<float>(c.eps * c.eps);
+    const float4 *xs = reinterpret_cast<const float4 *>(c.xs32.p);
+    float4 *acc = reinterpret_cast<float4 *>(c.as32.p), *part = reinterpret_cast<float4 *>(c.p2p_part32.p);
+    const float G = static_cast<float>(c.G);
+    bool big = false;  // a root box so wide that squared distances may leave the FP32 range
+    for (int a = 0; a < 3; ++a) big |= !(t.box[3 + a] - t.box[a] < 1e18);
+    auto run = [&](auto kernel, auto sum) {
+        kernel<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs, eps2, G, !c.has_masses, big, static_cast<float>(c.mass), acc, part, pstride);
+        if (split) sum<<<ceil_div(nl, 4), 256, 0, c.stream>>>(t.leaf_ids, nl, c.p2p_nchunk, c.p2p_item_off, t.start, t.count, xs, eps2, G, acc, part, pstride);
+    };
+    if (potential)
+        run(k_p2p_mc<true>, k_p2p_sum<true>);
+    else
+        run(k_p2p_mc<false>, k_p2p_sum<false>);
+    VG_LAUNCH_CHECK();
+}
+
+// FP64 P2P: one kernel per leaf class.
+void p2p_run_f64(Ctx &c, bool potential) {
+    TreeDev &t = c.t;
+    if (!t.nleaves) return;
+    using R = double;
+    using V4 = double4;
+    const V4 *xs = reinterpret_cast<const V4 *>(c.xs64.p);
+    c.as64.ensure(4 * std::max<int64_t>(1, c.n));
+    V4 *acc = reinterpret_cast<V4 *>(c.as64.p);
+    const R eps2 = c.eps * c.eps;
     const bool guard = !(eps2 > 0);
     // one mass for every particle (no per-particle masses uploaded): force
     // kernels take it out of the pair terms (the potential keeps the general path)
     const bool um = !c.has_masses;
-    const R mu = static_cast<R>(c.mass);
+    const R mu = c.mass;
+    const uint32_t *hs = p2p_scalars(c), *hbase = hs + NCLS;
     const int nl = static_cast<int>(t.nleaves);
-    const int nb = static_cast<int>(ceil_div(nl, 256));
-    const uint32_t *hs = reinterpret_cast<const uint32_t *>(static_cast<const char *>(c.pinned) + 128);
-    VG_HIP(hipEventSynchronize(c.ev_plan));
-    const uint32_t nitems = hs[2 * NCLS], nsplit = hs[2 * NCLS + 1];
-    const uint32_t *hbase = hs + NCLS;
-    c.p2p_items.ensure(std::max<uint32_t>(1, nitems));
+    c.p2p_items.ensure(std::max<uint32_t>(1, hs[2 * NCLS - 1] + hs[NCLS - 1]));
     int2 *items = reinterpret_cast<int2 *>(c.p2p_items.p);
-    k_p2p_items<<<nb, 256, 0, c.stream>>>(t.leaf_ids, nl, t.count, c.p2p_nchunk, c.p2p_pre, c.p2p_btot, c.p2p_scal, c.p2p_item_off, items);
+    k_p2p_items<<<ceil_div(nl, 256), 256, 0, c.stream>>>(nl, c.p2p_cls, c.p2p_nchunk, c.p2p_pre, c.p2p_btot, c.p2p_scal, c.p2p_item_off, items);
     VG_LAUNCH_CHECK();
-    const bool split = nsplit > 0;
+    const bool split = hs[2 * NCLS + 1] > 0;
     const uint32_t pstride = c.thr;
-    V4 *partial = nullptr;
-    if (split) {
-        VG_HIP(hipMemsetAsync(c.p2p_ticket.p, 0, static_cast<size_t>(nl) * sizeof(uint32_t), c.stream));
-        if (sizeof(R) == 4) {
-            c.p2p_part32.ensure(4 * static_cast<size_t>(nitems) * pstride);
-            partial = reinterpret_cast<V4 *>(c.p2p_part32.p);
-        } else {
-            c.p2p_part64.ensure(4 * static_cast<size_t>(nitems) * pstride);
-            partial = reinterpret_cast<V4 *>(c.p2p_part64.p);
-        }
-    }
+    if (split) VG_HIP(hipMemsetAsync(c.p2p_ticket.p, 0, static_cast<size_t>(t.nleaves) * sizeof(uint32_t), c.stream));
+    if (split) c.p2p_part64.ensure(4 * static_cast<size_t>(hs[2 * NCLS]) * pstride);
+    V4 *partial = reinterpret_cast<V4 *>(c.p2p_part64.p);
     for (int cls = 0; cls < NCLS; ++cls) {
         if (!hs[cls]) continue;
         const dim3 grid(hs[cls]);
         const int2 *it = items + hbase[cls];
 #define VG_P2P_T(G_, P_, U_, T_)                                                                                                                \
     k_p2p<R, G_, P_, U_, T_><<<grid, P2P_THREADS, 0, c.stream>>>(it, t.leaf_ids, c.p2p_nchunk, c.p2p_item_off, t.level, t.start, t.count, t.anc, \
-                                                                 t.ni, t.ni_cnt, xs, eps2, static_cast<R>(c.G), mu, acc, partial, pstride, c.p2p_ticket, \
-                                                                 c.p2p_chunk)
+                                                                 t.ni, t.ni_cnt, xs, eps2, c.G, mu, acc, partial, pstride, c.p2p_ticket)
 #define VG_P2P(G_, P_, U_)           \
     do {                             \
         if (cls == 0)                \
@@ -534,17 +1067,17 @@ void p2p_run(Ctx &c, bool potential) {
 
 }  // namespace
 
-void fmm_p2p_plan(Ctx &c) { p2p_plan(c); }
+void fmm_p2p_plan(Ctx &c, bool potential) { p2p_plan(c, potential); }
 
 void fmm_p2p_run(Ctx &c, bool potential) {
     if (c.prec == 0)
-        p2p_run<double>(c, potential);
+        p2p_run_f64(c, potential);
     else
-        p2p_run<float>(c, potential);
+        p2p_run_f32(c, potential);
 }
 
 void fmm_p2p(Ctx &c, bool potential) {
-    fmm_p2p_plan(c);
+    fmm_p2p_plan(c, potential);
     fmm_p2p_run(c, potential);
 }
 
