@@ -35,6 +35,7 @@ void swap_expansions(Ctx &c, ExpSet &e) {
     c.harm.swap(e.harm);
     c.op64.swap(e.op64);
     c.op32.swap(e.op32);
+    c.opfrag.swap(e.opfrag);
     c.M32.swap(e.M32);
     c.L32.swap(e.L32);
     c.opsplit.swap(e.opsplit);
@@ -388,7 +389,7 @@ int vipp_grav_create(const vipp_grav_config *cfg, vipp_grav_ctx **out) {
             c.p = static_cast<int>(cfg->p);
             c.K = (c.p + 1) * (c.p + 1);
             c.prec = static_cast<int>(cfg->precision);
-            c.ldk = c.prec == 2 ? (c.K + 15) / 16 * 16 : c.K;  // the MFMA path reads whole 16-coefficient k-steps
+            c.ldk = vg::coeff_stride(c.prec, c.K);
             c.eps = cfg->epsilon;
             c.G = cfg->G;
             c.mass = cfg->mass;

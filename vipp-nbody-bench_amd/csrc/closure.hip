@@ -191,7 +191,7 @@ bool closure_fallback_prepare(Ctx &c) {
     ExpSet &hi = cl.hi;
     hi.p = cl.p_hi;
     hi.K = (cl.p_hi + 1) * (cl.p_hi + 1);
-    hi.ldk = c.prec == 2 ? (hi.K + 15) / 16 * 16 : hi.K;
+    hi.ldk = coeff_stride(c.prec, hi.K);
     swap_expansions(c, hi);
     try {
         operators_build(c);

@@ -17,7 +17,7 @@ constexpr int MAXD = 21;
 constexpr int MAXP = 12;
 constexpr int MAXK = (MAXP + 1) * (MAXP + 1);
 // Operators built per evaluation: 8 M2M, 8 L2L and the 189 M2L offsets of
-// octant 0's walk (m2l_walk below; the other octants reuse them mirrored).
+// octant 0's walk (m2l_step below; the other octants reuse them mirrored).
 constexpr int NOPS_USED = 16 + 189;
 
 struct Error : std::runtime_error {
@@ -101,23 +101,58 @@ __device__ inline void aabb_block_store(const double *lo, const double *hi, doub
 // octant q) pairs of a target of octant 0 are walked in one fixed order; for a
 // target of octant qt the geometry is octant 0's mirrored in the axes where qt
 // has a bit set (d -> mirror(d), q -> q ^ qt), so the cell offset, and with it
-// the operator T_e, is octant 0's.  m2l_walk fills, per step of that order,
-// the operator index o (offset + (3,3,3) in base 7), the parent-neighbour slot
-// dn (0..26) of the mirrored neighbour and the mirrored source octant qs.
-__host__ __device__ inline void m2l_walk(int qt, int16_t *o, int16_t *dn, int16_t *qs) {
+// the operator T_e, is octant 0's.  m2l_step gives, per step of that order, the
+// operator index o (offset + (3,3,3) in base 7), the parent-neighbour slot dn
+// (0..26) of the mirrored neighbour and the mirrored source octant qs.
+struct M2lSteps {
+    int8_t d[189], q[189];
+};
+constexpr M2lSteps m2l_steps() {
+    M2lSteps t{};
     int st = 0;
     for (int d = 0; d < 27; ++d) {
         const int dx = d % 3 - 1, dy = (d / 3) % 3 - 1, dz = d / 9 - 1;
         for (int q = 0; q < 8; ++q) {
             const int ex = 2 * dx - (q & 1), ey = 2 * dy - ((q >> 1) & 1), ez = 2 * dz - ((q >> 2) & 1);
             if (ex >= -1 && ex <= 1 && ey >= -1 && ey <= 1 && ez >= -1 && ez <= 1) continue;  // adjacent: near field
-            const int mx = (qt & 1) ? -dx : dx, my = (qt & 2) ? -dy : dy, mz = (qt & 4) ? -dz : dz;
-            o[st] = static_cast<int16_t>((ex + 3) + 7 * (ey + 3) + 49 * (ez + 3));
-            dn[st] = static_cast<int16_t>((mx + 1) + 3 * (my + 1) + 9 * (mz + 1));
-            qs[st] = static_cast<int16_t>(q ^ qt);
+            t.d[st] = static_cast<int8_t>(d);
+            t.q[st] = static_cast<int8_t>(q);
             ++st;
         }
     }
+    return t;
+}
+static __constant__ const M2lSteps c_m2l_steps = m2l_steps();
+struct M2lStep {
+    int o, dn, qs;
+};
+__host__ __device__ inline M2lStep m2l_step(int d, int q, int qt) {
+    const int dx = d % 3 - 1, dy = (d / 3) % 3 - 1, dz = d / 9 - 1;
+    const int ex = 2 * dx - (q & 1), ey = 2 * dy - ((q >> 1) & 1), ez = 2 * dz - ((q >> 2) & 1);
+    const int mx = (qt & 1) ? -dx : dx, my = (qt & 2) ? -dy : dy, mz = (qt & 4) ? -dz : dz;
+    return {(ex + 3) + 7 * (ey + 3) + 49 * (ez + 3), (mx + 1) + 3 * (my + 1) + 9 * (mz + 1), q ^ qt};
+}
+// The steps of octant qt into o, dn, qs by a block of nth threads.
+__device__ inline void m2l_walk(int tid, int nth, int qt, int16_t *o, int16_t *dn, int16_t *qs) {
+    for (int st = tid; st < 189; st += nth) {
+        const M2lStep s = m2l_step(c_m2l_steps.d[st], c_m2l_steps.q[st], qt);
+        o[st] = static_cast<int16_t>(s.o);
+        dn[st] = static_cast<int16_t>(s.dn);
+        qs[st] = static_cast<int16_t>(s.qs);
+    }
+}
+// The steps st whose live(st) holds, in order, into list, their number into
+// *n: called by every thread of a block of at least 192; list, n and the 3 words
+// of count in LDS.  Ends with a barrier.
+template <class F>
+__device__ inline void m2l_live_steps(int tid, int16_t *list, int *n, int *count, F &&live) {
+    const bool on = tid < 189 && live(tid);
+    const uint64_t b = __ballot(on);
+    if (tid < 192 && (tid & 63) == 0) count[tid >> 6] = __popcll(b);
+    __syncthreads();
+    if (on) list[(tid > 63 ? count[0] : 0) + (tid > 127 ? count[1] : 0) + __popcll(b & ((1ull << (tid & 63)) - 1))] = static_cast<int16_t>(tid);
+    if (tid == 0) *n = count[0] + count[1] + count[2];
+    __syncthreads();
 }
 
 // The mirrored operator is D_qt T_e D_qt with D_qt diagonal +-1; its entry for

@@ -136,22 +136,42 @@ __device__ inline void row_of(int r, int &j, int &k, int &part) {
     }
 }
 
+// FP32 M2L operators are kept in the order in which k_m2l_f32's lanes read
+// them: per operator RT x NJ fragments (16 rows, 16 columns) of 64 lanes x 4
+// columns.  Lane 16 q + row holds columns 4 q .. 4 q + 3 of the fragment, so
+// that its four words are the operands of four products v_mfma_f32_16x16x4;
+// the last column group has only the nks = ceil(rest / 4) products it needs,
+// lane 16 q + row then holds columns nks q .. nks q + nks - 1.
+struct OpFrag {
+    int nt, nks;  // 16-row tiles (and 16-column groups), products of the last group
+    __host__ __device__ explicit OpFrag(int K) : nt((K + 15) / 16), nks((K - 16 * ((K + 15) / 16 - 1) + 3) / 4) {}
+    __host__ __device__ size_t size() const { return static_cast<size_t>(nt) * nt * 256; }
+    __host__ __device__ size_t at(int r, int c) const {
+        const int j = c >> 4, w = j + 1 < nt ? 4 : nks;
+        return (static_cast<size_t>((r >> 4) * nt + j) * 64 + (c & 15) / w * 16 + (r & 15)) * 4 + (c & 15) % w;
+    }
+};
+
 // op block layout: [M2M 0..7][L2L 8..15][M2L 16..16+342], each K*K; M2L
-// blocks row-major [row][col], M2M and L2L blocks column-major [col][row] (their
-// kernels give each lane one output row, so lanes then read consecutive words).
+// blocks row-major [row][col] (or, with frag, OpFrag's order there), M2M and
+// L2L blocks column-major [col][row] (their kernels give each lane one output
+// row, so lanes then read consecutive words).
 // One block per (operator, OPS_ROWS rows), 128 threads per row r; thread t of
 // a row takes the column pair (n, m >= 0) number t, i.e. the real-packed
 // columns of degree n, order m.
 constexpr int OPS_ROWS = 4;
 template <class R>
-__global__ __launch_bounds__(128 * OPS_ROWS) void k_ops(const int16_t *__restrict__ sel, const double *__restrict__ harm, int p, int K, R *__restrict__ op) {
+__global__ __launch_bounds__(128 * OPS_ROWS) void k_ops(const int16_t *__restrict__ sel, const double *__restrict__ harm, int p, int K, R *__restrict__ op,
+                                                         R *__restrict__ frag) {
     const int blk = sel[blockIdx.x];  // operator index
     const int r = blockIdx.y * OPS_ROWS + static_cast<int>(threadIdx.x >> 7);
     const int t = threadIdx.x & 127;
     const bool cmaj = blk < 16;
+    const OpFrag fr(K);
+    const bool fragment = frag && !cmaj;  // every column is written below, the padding stays zero
     R *dst = cmaj ? op + static_cast<size_t>(blk) * K * K + r : op + (static_cast<size_t>(blk) * K + r) * K;
     const size_t cs = cmaj ? static_cast<size_t>(K) : 1;  // column stride
-    if (r < K)
+    if (r < K && !fragment)
         for (int c = t; c < K; c += 128) dst[c * cs] = R(0);
     __syncthreads();
     if (r >= K) return;
@@ -204,12 +224,18 @@ __global__ __launch_bounds__(128 * OPS_ROWS) void k_ops(const int16_t *__restric
         }
     }
     // the pair's real-packed columns (each written by this thread only)
+    auto put = [&](int c, double v) {
+        if (fragment)
+            frag[(blk - 16) * fr.size() + fr.at(r, c)] = static_cast<R>(v);
+        else
+            dst[c * cs] = static_cast<R>(v);
+    };
     if (mp == 0) {
-        dst[kidx_re(n, 0) * cs] = static_cast<R>(part == 0 ? tpm[0].re : tpm[0].im);
+        put(kidx_re(n, 0), part == 0 ? tpm[0].re : tpm[0].im);
     } else {
         const dc sum = cadd(tpm[0], tpm[1]), dif = csub(tpm[0], tpm[1]);
-        dst[kidx_re(n, mp) * cs] = static_cast<R>(part == 0 ? sum.re : sum.im);
-        dst[kidx_im(n, mp) * cs] = static_cast<R>(part == 0 ? -dif.im : dif.re);
+        put(kidx_re(n, mp), part == 0 ? sum.re : sum.im);
+        put(kidx_im(n, mp), part == 0 ? -dif.im : dif.re);
     }
 }
 
@@ -430,11 +456,11 @@ __global__ __launch_bounds__(256) void k_l2l(const int32_t *__restrict__ ids, in
 
 
 // ---------------------------------------------------------------------------
-// Plain M2L: targets are the children of octant qt of a chunk of TB internal
+// FP64 M2L: targets are the children of octant qt of a chunk of TB internal
 // parents; for each well-separated (parent neighbour, source octant) pair the
 // (static) cell offset selects one operator, applied as a K x K by K x TB
 // product with the gathered source multipoles (offset-grouped GEMM on VALU).
-// As on the matrix cores, every block walks octant 0's 189 offsets (m2l_walk)
+// As on the matrix cores, every block walks octant 0's 189 offsets (m2l_step)
 // and the mirror signs D_qt go on the gathered multipoles and on the result,
 // so all blocks share 189 operators.  Blocks are placed XCD-aware: the eight
 // octant blocks of a parent chunk run side by side on one XCD and share its
@@ -443,26 +469,25 @@ __global__ __launch_bounds__(256) void k_l2l(const int32_t *__restrict__ ids, in
 // hold any source; only those are walked.  With nsplit > 1 the walked offsets
 // are cut into nsplit consecutive parts, one block each, which write partial
 // sums per target slot (parent index * 8 + octant) to part; k_m2l_sum adds
-// them in part order.  A block has RG groups of 256
-// threads; a thread owns the rows tr + 32 (rg + RG i), i < RPT / RG, and CPT
+// them in part order.  A thread owns the rows tr + 32 i, i < RPT, and CPT
 // consecutive targets; the operator streams through LDS in chunks of KC
 // columns, double-buffered through registers (one barrier per chunk), and the
 // next offset's first chunk is fetched during the last.
 // ---------------------------------------------------------------------------
-template <class R, int TB, int RPT, int RG>
-__global__ __launch_bounds__(256 * RG) void k_m2l_plain(const int32_t *__restrict__ parents, int nparents, const int32_t *__restrict__ child,
-                                                   const uint32_t *__restrict__ count, const int32_t *__restrict__ nbr27, const R *__restrict__ Mx,
-                                                   R *__restrict__ Lx, const R *__restrict__ op, int K, int ldk, int nsplit,
-                                                   R *__restrict__ part) {
-    constexpr int KC = sizeof(R) == 4 ? 16 : 8;     // operator columns per chunk
+template <int TB, int RPT>
+__global__ __launch_bounds__(256) void k_m2l_plain(const int32_t *__restrict__ parents, int nparents, const int32_t *__restrict__ child,
+                                                   const uint32_t *__restrict__ count, const int32_t *__restrict__ nbr27, const double *__restrict__ Mx,
+                                                   double *__restrict__ Lx, const double *__restrict__ op, int K, int ldk, int nsplit,
+                                                   double *__restrict__ part) {
+    using R = double;
+    constexpr int KC = 8;                            // operator columns per chunk
     constexpr int CPT = TB / 8;                      // targets per thread
     constexpr int VW = 16 / sizeof(R);               // elements per 16-byte LDS read
     constexpr int SMS = TB + VW;                     // multipole column stride (16-byte rows)
     constexpr int SOS = 32 * RPT + 1;                // operator column stride (odd: no bank conflicts)
-    constexpr int NTH = 256 * RG;                    // threads
-    constexpr int RPL = RPT / RG;                    // rows per thread
+    constexpr int NTH = 256;                         // threads
     constexpr int NPF = KC * 32 * RPT / NTH;         // prefetched operator words per thread
-    static_assert(CPT % VW == 0 && (KC * 32 * RPT) % NTH == 0 && RPT % RG == 0, "tile shape");
+    static_assert(CPT % VW == 0 && (KC * 32 * RPT) % NTH == 0, "tile shape");
     extern __shared__ __align__(16) unsigned char m2l_smem[];
     R *sM = reinterpret_cast<R *>(m2l_smem);         // K x SMS: column k of the gathered, signed multipoles
     R *sOp = sM + K * SMS;                           // 2 x KC x SOS: operator columns, transposed
@@ -471,15 +496,15 @@ __global__ __launch_bounds__(256 * RG) void k_m2l_plain(const int32_t *__restric
     __shared__ uint8_t s_nm[27 * TB];                // its non-empty children
     __shared__ int32_t tgt[TB];
     __shared__ int16_t s_o[189], s_dn[189], s_qs[189], s_live[189];
-    __shared__ int s_nlive;
+    __shared__ int s_nlive, s_cnt[3];
     const int nchunks = (nparents + TB - 1) / TB;
     const int per = nchunks * nsplit;                          // work items per XCD
     const int wi = (blockIdx.x & 7) * per + (blockIdx.x >> 3);  // XCD x takes work items [x W / 8, (x + 1) W / 8)
     if (wi >= 8 * per) return;
     const int sp = wi % nsplit, w = wi / nsplit;  // the parts of one (chunk, octant) are neighbours
     const int chunk = w >> 3, qt = w & 7;
-    const int tid = threadIdx.x, tr = tid & 31, tc = (tid >> 5) & 7, rg = tid >> 8;
-    if (tid == 0) m2l_walk(qt, s_o, s_dn, s_qs);
+    const int tid = threadIdx.x, tr = tid & 31, tc = tid >> 5;
+    m2l_walk(tid, 256, qt, s_o, s_dn, s_qs);
     for (int k = tid; k < 32 * RPT; k += NTH) sg[k] = static_cast<R>(k < K ? m2l_mirror_sign(qt, k) : 0);
     if (tid < TB) {
         const int pi = chunk * TB + tid;
@@ -504,25 +529,17 @@ __global__ __launch_bounds__(256 * RG) void k_m2l_plain(const int32_t *__restric
         s_nm[i] = static_cast<uint8_t>(msk);
     }
     __syncthreads();
-    if (tid < 189) {
-        const int dn = s_dn[tid], qs = s_qs[tid];
-        int live = 0;
-        for (int t = 0; t < TB; ++t) live |= (s_nm[dn * TB + t] >> qs) & 1;
-        s_live[tid] = static_cast<int16_t>(live);
-    }
-    __syncthreads();
-    if (tid == 0) {
-        int nl = 0;
-        for (int st = 0; st < 189; ++st)
-            if (s_live[st]) s_live[nl++] = static_cast<int16_t>(st);
-        s_nlive = nl;
-    }
-    __syncthreads();
+    m2l_live_steps(tid, s_live, &s_nlive, s_cnt, [&](int st) {
+        const int dn = s_dn[st], qs = s_qs[st];
+        int any = 0;
+        for (int t = 0; t < TB; ++t) any |= s_nm[dn * TB + t] >> qs;
+        return (any & 1) != 0;
+    });
     const int nlive = s_nlive;
     const int lo = sp * nlive / nsplit, hi = (sp + 1) * nlive / nsplit;  // this block's walked offsets
-    R acc[RPL][CPT];
+    R acc[RPT][CPT];
 #pragma unroll
-    for (int i = 0; i < RPL; ++i)
+    for (int i = 0; i < RPT; ++i)
 #pragma unroll
         for (int jj = 0; jj < CPT; ++jj) acc[i][jj] = 0;
     const int nkc = (K + KC - 1) / KC;
@@ -556,8 +573,8 @@ __global__ __launch_bounds__(256 * RG) void k_m2l_plain(const int32_t *__restric
             for (int e = 0; e < VW; ++e) mv[v * VW + e] = x[e];
         }
 #pragma unroll
-        for (int i = 0; i < RPL; ++i) {
-            const R ov = S[tr + 32 * (rg + RG * i)];
+        for (int i = 0; i < RPT; ++i) {
+            const R ov = S[tr + 32 * i];
 #pragma unroll
             for (int jj = 0; jj < CPT; ++jj) acc[i][jj] += ov * mv[jj];
         }
@@ -566,8 +583,8 @@ __global__ __launch_bounds__(256 * RG) void k_m2l_plain(const int32_t *__restric
     const int wv = tid >> 6, lane = tid & 63;
     for (int li = lo; li < hi; ++li) {
         const int st = s_live[li], dn = s_dn[st], qs = s_qs[st];
-        // gather: wave wv takes targets wv, wv + 4 RG, ..., lanes the columns
-        for (int t = wv; t < TB; t += 4 * RG) {
+        // gather: wave wv takes targets wv, wv + 4, ..., lanes the columns
+        for (int t = wv; t < TB; t += 4) {
             const int32_t cb = s_nc[dn * TB + t];
             const bool has = (s_nm[dn * TB + t] >> qs) & 1;
             const R *src = Mx + static_cast<size_t>(has ? cb + qs : 0) * ldk;
@@ -601,11 +618,209 @@ __global__ __launch_bounds__(256 * RG) void k_m2l_plain(const int32_t *__restric
         R *dst = nsplit == 1 ? Lx + static_cast<size_t>(t) * ldk
                              : part + (static_cast<size_t>(sp) * 8 * nparents + static_cast<size_t>(chunk * TB + tc * CPT + jj) * 8 + qt) * ldk;
 #pragma unroll
-        for (int i = 0; i < RPL; ++i) {
-            const int r = tr + 32 * (rg + RG * i);
+        for (int i = 0; i < RPT; ++i) {
+            const int r = tr + 32 * i;
             if (r < K) dst[r] = sg[r] * acc[i][jj];
         }
     }
+}
+
+// ---------------------------------------------------------------------------
+// FP32 M2L on v_mfma_f32_16x16x4: the same offset-grouped product as
+// k_m2l_plain, a block of 4 wavefronts per (chunk of TB parents, child octant).
+// A wavefront (wr, wc) owns half of the 16-row tiles and half of the 16-target
+// tiles (an odd middle row tile is split by target tiles), so operator
+// fragments come straight from L2 in 16-byte words that feed 4 x TB / 32
+// products each, one column group ahead, and only the gathered, mirrored
+// multipoles go through LDS, in rows of the targets (16-byte copies of the
+// expansions; the row stride is an odd number of 16-byte words, so reads have
+// no bank conflicts).  The matrix pipe is what bounds it: a product takes 32
+// cycles and VALU work adds to it (both use the FP32 units), so the layout
+// keeps that work small: operator addresses are uniform, a lane gathers the
+// same word of every target, so its mirror signs are four registers, and the
+// next offset's multipoles are on their way during the products.  FP32 FMAs
+// from LDS (k_m2l_plain's form, 64 targets) ran at 58 % of the one-FMA-a-cycle
+// rate; M2L per evaluation, then and now: 4M Plummer p = 12 19.1 -> 9.4 ms
+// (91 TFLOP/s, 60 % of a large FP32 matrix product), 10^6 Plummer p = 12 6.1 ->
+// 2.4, 2^20 uniform p = 8 2.67 -> 1.14, p = 5 1.40 -> 0.33, p = 3 0.59 -> 0.09,
+// 16,384 Plummer p = 8 0.099 -> 0.070.  Blocks of 32 targets were slower at every size.
+// ---------------------------------------------------------------------------
+typedef float f4 __attribute__((ext_vector_type(4)));
+template <int P>
+struct M2lShape {
+    static constexpr int K = (P + 1) * (P + 1), NT = (K + 15) / 16, NKS = (K - 16 * (NT - 1) + 3) / 4, LD = (K + 3) / 4 * 4, LD4 = LD / 4;
+    static constexpr int SK = (LD4 | 1) * 4;  // LDS row stride
+    static constexpr int H = NT / 2;          // whole row tiles per wavefront
+    static constexpr int TPI = 64 / LD4;      // targets a wavefront gathers with one load
+};
+template <int P>
+__global__ __launch_bounds__(256, 2) void k_m2l_f32(const int32_t *__restrict__ parents, int nparents, const int32_t *__restrict__ child,
+                                                    const uint32_t *__restrict__ count, const int32_t *__restrict__ nbr27,
+                                                    const f4 *__restrict__ Mx, float *__restrict__ Lx, const f4 *__restrict__ op, int nsplit,
+                                                    float *__restrict__ part) {
+    using S = M2lShape<P>;
+    constexpr int TB = 64;                          // targets
+    constexpr int NC = TB / 32;                     // 16-target tiles per wavefront
+    constexpr int HX = S::H + (S::NT & 1);          // row tiles it loads
+    constexpr int NG = (TB + 4 * S::TPI - 1) / (4 * S::TPI);  // 16-byte words a thread gathers
+    __shared__ __align__(16) float sM[TB * S::SK];
+    __shared__ int32_t s_nc[27 * TB];  // first child of parent neighbour d of target t, or -1
+    __shared__ uint8_t s_nm[27 * TB];  // its non-empty children
+    __shared__ int32_t tgt[TB];
+    __shared__ int16_t s_o[189], s_dn[189], s_qs[189], s_live[189];
+    __shared__ int s_nlive, s_cnt[3];
+    const int nchunks = (nparents + TB - 1) / TB;
+    const int per = nchunks * nsplit;                           // work items per XCD
+    const int wi = (blockIdx.x & 7) * per + (blockIdx.x >> 3);  // XCD x takes work items [x W / 8, (x + 1) W / 8)
+    if (wi >= 8 * per) return;
+    const int sp = wi % nsplit, w = wi / nsplit;  // the parts of one (chunk, octant) are neighbours
+    const int chunk = w >> 3, qt = w & 7;
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, quad = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wr = wv & 1, wc = wv >> 1;
+    m2l_walk(tid, 256, qt, s_o, s_dn, s_qs);
+    if (tid < TB) {
+        const int pi = chunk * TB + tid;
+        const int32_t p = pi < nparents ? parents[pi] : -1;
+        int32_t t = p >= 0 ? child[p] + qt : -1;
+        if (t >= 0 && count[t] == 0) t = -1;
+        tgt[tid] = t;
+    }
+    __syncthreads();
+    for (int i = tid; i < 27 * TB; i += 256) {
+        const int d = i / TB, t = i % TB;
+        int32_t cb = -1;
+        uint32_t msk = 0;
+        if (tgt[t] >= 0) {
+            const int32_t p = nbr27[27 * static_cast<int64_t>(parents[chunk * TB + t]) + d];
+            cb = p >= 0 ? child[p] : -1;
+            if (cb >= 0)
+                for (int q = 0; q < 8; ++q) msk |= (count[cb + q] != 0 ? 1u : 0u) << q;
+        }
+        s_nc[i] = cb;
+        s_nm[i] = static_cast<uint8_t>(msk);
+    }
+    __syncthreads();
+    m2l_live_steps(tid, s_live, &s_nlive, s_cnt, [&](int st) {
+        const int dn = s_dn[st], qs = s_qs[st];
+        int any = 0;
+        for (int t = 0; t < TB; ++t) any |= s_nm[dn * TB + t] >> qs;
+        return (any & 1) != 0;
+    });
+    // this lane gathers word ch of the targets (wv + 4 u) TPI + sub
+    const int sub = lane / S::LD4, ch = lane % S::LD4;
+    uint32_t sg[4];  // its mirror signs
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sg[e] = 4 * ch + e < S::K && m2l_mirror_sign(qt, 4 * ch + e) < 0 ? 0x80000000u : 0u;
+    __syncthreads();
+    const int nlive = s_nlive;
+    const int lo = sp * nlive / nsplit, hi = (sp + 1) * nlive / nsplit;  // this block's walked offsets
+    f4 acc[HX][NC], sum[HX][NC];  // the current offset's products, and the sum of the offsets before it
+#pragma unroll
+    for (int h = 0; h < HX; ++h)
+#pragma unroll
+        for (int n = 0; n < NC; ++n) sum[h][n] = f4{0, 0, 0, 0};
+    // row tile h of this wavefront: wr H .. wr H + H - 1, and the last one (of an odd number) for half of the targets
+    auto row_tile = [&](int h) { return h < S::H ? wr * S::H + h : S::NT - 1; };
+    auto load_a = [&](int li, int j, f4 *a) {  // (uniform base, lane offset)
+        const f4 *O = op + static_cast<size_t>(__builtin_amdgcn_readfirstlane(s_o[s_live[li]])) * (S::NT * S::NT * 64) + j * 64;
+#pragma unroll
+        for (int h = 0; h < HX; ++h) a[h] = (O + row_tile(h) * (S::NT * 64))[static_cast<unsigned>(lane)];
+    };
+    const float *Brow = sM + (wc * 16 * NC + col) * S::SK;
+    f4 an[HX], v[NG];
+    auto gather = [&](int li) {  // this thread's words of the multipoles of walked offset li
+        const int st = s_live[li], dn = __builtin_amdgcn_readfirstlane(s_dn[st]) * TB, qs = __builtin_amdgcn_readfirstlane(s_qs[st]);
+#pragma unroll
+        for (int u = 0; u < NG; ++u) {
+            v[u] = f4{0, 0, 0, 0};
+            if constexpr (S::TPI == 1) {  // one target: its lookups are uniform
+                const int t = dn + wv + 4 * u;
+                const int cell = __builtin_amdgcn_readfirstlane(s_nc[t]) + qs;
+                if ((__builtin_amdgcn_readfirstlane(s_nm[t]) >> qs) & 1)
+                    if (lane < S::LD4) v[u] = (Mx + static_cast<size_t>(cell) * S::LD4)[static_cast<unsigned>(lane)];
+            } else {
+                const int t = (wv + 4 * u) * S::TPI + sub;
+                if (sub < S::TPI && t < TB && ((s_nm[dn + t] >> qs) & 1)) v[u] = Mx[static_cast<size_t>(s_nc[dn + t] + qs) * S::LD4 + ch];
+            }
+        }
+    };
+    if (hi > lo) {
+        load_a(lo, 0, an);
+        gather(lo);
+    }
+    for (int li = lo; li < hi; ++li) {
+#pragma unroll
+        for (int u = 0; u < NG; ++u) {
+            const int t = (wv + 4 * u) * S::TPI + sub;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[u][e] = __uint_as_float(__float_as_uint(v[u][e]) ^ sg[e]);
+            if (sub < S::TPI && t < TB) *reinterpret_cast<f4 *>(sM + t * S::SK + 4 * ch) = v[u];
+        }
+        if (li + 1 < hi) gather(li + 1);  // on its way during the products
+        __syncthreads();  // the multipoles of this offset are in LDS
+        // the products of one column group; the offset's first ones start its sums
+        auto group = [&](const f4 *a, const f4 *b, int nk, auto first) {
+            const f4 zero = {0, 0, 0, 0};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (i >= nk) break;
+                const bool start = decltype(first)::value && i == 0;
+#pragma unroll
+                for (int h = 0; h < S::H; ++h)
+#pragma unroll
+                    for (int n = 0; n < NC; ++n) acc[h][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h][i], b[n][i], start ? zero : acc[h][n], 0, 0, 0);
+                if constexpr (S::NT & 1)
+                    acc[S::H][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[S::H][i], wr ? b[1][i] : b[0][i], start ? zero : acc[S::H][0], 0, 0, 0);
+            }
+        };
+        auto full = [&](int j, auto first) {
+            f4 a[HX], b[NC];
+#pragma unroll
+            for (int h = 0; h < HX; ++h) a[h] = an[h];
+            load_a(li, j + 1, an);
+#pragma unroll
+            for (int n = 0; n < NC; ++n) b[n] = *reinterpret_cast<const f4 *>(Brow + 16 * n * S::SK + 16 * j + 4 * quad);
+            group(a, b, 4, first);
+        };
+        if constexpr (S::NT > 1) full(0, std::true_type{});
+#pragma unroll 2
+        for (int j = 1; j + 1 < S::NT; ++j) full(j, std::false_type{});
+        {  // the last column group
+            f4 a[HX], b[NC];
+#pragma unroll
+            for (int h = 0; h < HX; ++h) a[h] = an[h];
+            if (li + 1 < hi) load_a(li + 1, 0, an);
+#pragma unroll
+            for (int n = 0; n < NC; ++n)
+#pragma unroll
+                for (int i = 0; i < S::NKS; ++i) b[n][i] = Brow[16 * n * S::SK + 16 * (S::NT - 1) + S::NKS * quad + i];
+            group(a, b, S::NKS, std::bool_constant<S::NT == 1>{});
+        }
+        // offset by offset: shorter sums, so less rounding (RMS error of the locals against FP64 at p = 3 and 5:
+        // 1.1e-7 and 1.6e-7 in one sum, as in k_m2l_plain's form, 0.8e-7 and 1.0e-7 here)
+#pragma unroll
+        for (int h = 0; h < HX; ++h)
+#pragma unroll
+            for (int n = 0; n < NC; ++n) sum[h][n] += acc[h][n];
+        __syncthreads();  // every wavefront has read the multipoles
+    }
+    // D: lane holds rows 4 quad .. 4 quad + 3 of a tile for target col
+    auto put = [&](int tile, int n, f4 v) {
+        const int ti = (wc * NC + n) * 16 + col, r0 = 16 * tile + 4 * quad;
+        const int32_t t = tgt[ti];
+        if (t < 0 || r0 >= S::LD) return;
+        float *dst = nsplit == 1 ? Lx + static_cast<size_t>(t) * S::LD
+                                 : part + (static_cast<size_t>(sp) * 8 * nparents + static_cast<size_t>(chunk * TB + ti) * 8 + qt) * S::LD;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (r0 + e < S::K && m2l_mirror_sign(qt, r0 + e) < 0) v[e] = -v[e];
+        *reinterpret_cast<f4 *>(dst + r0) = v;
+    };
+#pragma unroll
+    for (int h = 0; h < S::H; ++h)
+#pragma unroll
+        for (int n = 0; n < NC; ++n) put(wr * S::H + h, n, sum[h][n]);
+    if constexpr (S::NT & 1) put(S::NT - 1, wr, sum[S::H][0]);
 }
 
 // The nsplit partial sums of each non-empty M2L target into its local
@@ -880,10 +1095,10 @@ void upward_t(Ctx &c) {
     VG_LAUNCH_CHECK();
 }
 
-template <class R, int TB, int RPT, int RG = 1>
-void m2l_plain_launch(Ctx &c, const int32_t *parents, int np, unsigned grid, int nsplit, R *part) {
-    constexpr int KC = sizeof(R) == 4 ? 16 : 8;
-    const size_t lds = (static_cast<size_t>(c.K) * (TB + 16 / sizeof(R)) + 2 * KC * (32 * RPT + 1)) * sizeof(R);
+template <int TB, int RPT>
+void m2l_plain_launch(Ctx &c, const int32_t *parents, int np, unsigned grid, int nsplit, double *part) {
+    constexpr int KC = 8;
+    const size_t lds = (static_cast<size_t>(c.K) * (TB + 2) + 2 * KC * (32 * RPT + 1)) * sizeof(double);
     // dynamic LDS above 64 KiB is allowed per kernel and device, here for the
     // largest K of this RPT (set once per device, under a lock: contexts of
     // different host threads may launch concurrently)
@@ -893,80 +1108,107 @@ void m2l_plain_launch(Ctx &c, const int32_t *parents, int np, unsigned grid, int
         std::lock_guard<std::mutex> lock(mu);
         const uint64_t bit = c.device < 64 ? (1ull << c.device) : 0;
         if (!bit || !(done & bit)) {
-            const size_t cap = (static_cast<size_t>(32 * RPT) * (TB + 16 / sizeof(R)) + 2 * KC * (32 * RPT + 1)) * sizeof(R);
-            VG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_m2l_plain<R, TB, RPT, RG>), hipFuncAttributeMaxDynamicSharedMemorySize,
+            const size_t cap = (static_cast<size_t>(32 * RPT) * (TB + 2) + 2 * KC * (32 * RPT + 1)) * sizeof(double);
+            VG_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_m2l_plain<TB, RPT>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        static_cast<int>(cap)));
             done |= bit;
         }
     }
     const TreeDev &t = c.t;
-    k_m2l_plain<R, TB, RPT, RG><<<grid * nsplit, 256 * RG, lds, c.stream>>>(parents, np, t.child, t.count, t.nbr27, Bufs<R>::M(c), Bufs<R>::L(c),
-                                                                           Bufs<R>::op(c), c.K, c.ldk, nsplit, part);
+    k_m2l_plain<TB, RPT><<<grid * nsplit, 256, lds, c.stream>>>(parents, np, t.child, t.count, t.nbr27, c.M64, c.L64, c.op64, c.K, c.ldk, nsplit, part);
     if (nsplit > 1)
-        k_m2l_sum<R><<<ceil_div(static_cast<size_t>(8) * np * c.K, 256), 256, 0, c.stream>>>(parents, np, t.child, t.count, nsplit, part,
-                                                                                          Bufs<R>::L(c), c.K, c.ldk);
+        k_m2l_sum<double><<<ceil_div(static_cast<size_t>(8) * np * c.K, 256), 256, 0, c.stream>>>(parents, np, t.child, t.count, nsplit, part, c.L64,
+                                                                                               c.K, c.ldk);
     VG_LAUNCH_CHECK();
 }
 
-template <class R, int TB>
+template <int TB>
 void m2l_plain_rows(Ctx &c, const int32_t *parents, int np) {
-    // FP32 with an even number of 32-row groups: two thread groups split the
-    // rows (512 threads, twice the wavefronts per CU within the same LDS)
-    constexpr int RG2 = sizeof(R) == 4 ? 2 : 1;
     const int rpt = ceil_div(c.K, 32);
     const unsigned grid = 8 * ceil_div(np, TB);  // one block per (parent chunk, child octant)
-    // still under four blocks per CU: the walked offsets of a (chunk, octant)
-    // are cut into parts, one block each (at most 32 parts, so a part keeps
-    // about six of the at most 189 offsets), and a second kernel adds the
-    // partial sums (the 16k Plummer sphere at p = 4: 40 blocks, 26 parts,
-    // FP64 M2L 0.46 -> 0.05 ms; cutting grids of up to eight blocks per CU
-    // as well gained nothing on the 2^20 cube or the 4M sphere)
+    // under four blocks per CU: the walked offsets of a (chunk, octant) are cut
+    // into parts, one block each (at most 32 parts, so a part keeps about six of
+    // the at most 189 offsets), and a second kernel adds the partial sums (the
+    // 16k Plummer sphere at p = 4: 40 blocks, 26 parts, 0.46 -> 0.05 ms)
     int nsplit = 1;
     if (c.ncu > 0 && grid < 4u * static_cast<unsigned>(c.ncu)) nsplit = std::min<int>(32, static_cast<int>(ceil_div(4 * c.ncu, grid)));
-    R *part = nullptr;
+    double *part = nullptr;
     if (nsplit > 1) {
-        c.m2l_part.ensure(static_cast<size_t>(nsplit) * 8 * np * c.ldk * sizeof(R));
-        part = reinterpret_cast<R *>(c.m2l_part.p);
+        c.m2l_part.ensure(static_cast<size_t>(nsplit) * 8 * np * c.ldk * sizeof(double));
+        part = reinterpret_cast<double *>(c.m2l_part.p);
     }
     switch (rpt) {
-    case 1: m2l_plain_launch<R, TB, 1>(c, parents, np, grid, nsplit, part); break;
-    case 2: m2l_plain_launch<R, TB, 2, RG2>(c, parents, np, grid, nsplit, part); break;
-    case 3: m2l_plain_launch<R, TB, 3>(c, parents, np, grid, nsplit, part); break;
-    case 4: m2l_plain_launch<R, TB, 4, RG2>(c, parents, np, grid, nsplit, part); break;
-    case 5:  // FP32: padded to 6 row groups on two thread groups (p = 11 on the 4M Plummer input: 19.9 -> 16.7 ms;
-             // padding 3 to 4 at p = 8 was slower, 3.0 -> 4.1 ms)
-        if (sizeof(R) == 4)
-            m2l_plain_launch<R, TB, 6, RG2>(c, parents, np, grid, nsplit, part);
-        else
-            m2l_plain_launch<R, TB, 5>(c, parents, np, grid, nsplit, part);
-        break;
-    case 6: m2l_plain_launch<R, TB, 6, RG2>(c, parents, np, grid, nsplit, part); break;
+    case 1: m2l_plain_launch<TB, 1>(c, parents, np, grid, nsplit, part); break;
+    case 2: m2l_plain_launch<TB, 2>(c, parents, np, grid, nsplit, part); break;
+    case 3: m2l_plain_launch<TB, 3>(c, parents, np, grid, nsplit, part); break;
+    case 4: m2l_plain_launch<TB, 4>(c, parents, np, grid, nsplit, part); break;
+    case 5: m2l_plain_launch<TB, 5>(c, parents, np, grid, nsplit, part); break;
+    case 6: m2l_plain_launch<TB, 6>(c, parents, np, grid, nsplit, part); break;
     default: throw std::runtime_error("plain M2L: expansion order out of range");
     }
 }
 
-template <class R>
-void m2l_plain_list_t(Ctx &c, const int32_t *parents, int np) {
-    if (np <= 0) return;
-    constexpr int TB = sizeof(R) == 4 ? 64 : 32;
-    // Fewer than four blocks per CU at TB targets (2^20 uniform points have
-    // 4,680 parents: 592 blocks): half the targets per block, twice the
-    // blocks, which keeps more wavefronts in flight per CU (FP32 p = 8 on that
-    // input: 2.97 against 3.35 ms).
-    if (8 * static_cast<int64_t>(ceil_div(np, TB)) < 4 * static_cast<int64_t>(c.ncu))
-        m2l_plain_rows<R, TB / 2>(c, parents, np);
-    else
-        m2l_plain_rows<R, TB>(c, parents, np);
+// Parts of the walked offsets of a grid of `grid` equal blocks: a CU's blocks
+// share its matrix pipes, so the time goes with the fullest CU's share of the
+// work, ceil(grid n / ncu) / n, and each part costs about 1 % (prologue, partial
+// sums).  Grids of 8 and more blocks per CU are not cut.
+int m2l_f32_parts(unsigned grid, int ncu) {
+    int best = 1;
+    if (ncu <= 0 || grid >= 8u * static_cast<unsigned>(ncu)) return best;
+    double t = 1e300;
+    for (int n = 1; n <= 32; ++n) {
+        const double x = static_cast<double>(ceil_div(static_cast<size_t>(grid) * n, ncu)) / n * (1 + 0.01 * n);
+        if (x < t) t = x, best = n;
+    }
+    return best;
 }
 
-template <class R>
-void m2l_plain_t(Ctx &c) {
-    TreeDev &t = c.t;
-    // parents: internal cells of levels >= 1 (their children are the targets at level >= 2)
-    if (t.depth < 1) return;
-    const int64_t a = t.int_off[1], b = t.int_off.back();
-    if (b <= a) return;
-    m2l_plain_list_t<R>(c, t.int_ids.p + a, static_cast<int>(b - a));
+template <int P>
+void m2l_f32_launch(Ctx &c, const int32_t *parents, int np) {
+    const unsigned grid = 8 * ceil_div(np, 64);
+    const int nsplit = m2l_f32_parts(grid, c.ncu);
+    float *part = nullptr;
+    if (nsplit > 1) {
+        c.m2l_part.ensure(static_cast<size_t>(nsplit) * 8 * np * c.ldk * sizeof(float));
+        part = reinterpret_cast<float *>(c.m2l_part.p);
+    }
+    if (c.ldk != M2lShape<P>::LD) throw Error(1, "FP32 M2L: the coefficient stride must be K rounded up to 4");
+    const TreeDev &t = c.t;
+    k_m2l_f32<P><<<grid * nsplit, 256, 0, c.stream>>>(parents, np, t.child, t.count, t.nbr27, reinterpret_cast<const f4 *>(c.M32.p), c.L32.p,
+                                                          reinterpret_cast<const f4 *>(c.opfrag.p), nsplit, part);
+    if (nsplit > 1)
+        k_m2l_sum<float><<<ceil_div(static_cast<size_t>(8) * np * c.K, 256), 256, 0, c.stream>>>(parents, np, t.child, t.count, nsplit, part, c.L32, c.K,
+                                                                                              c.ldk);
+    VG_LAUNCH_CHECK();
+}
+
+void m2l_f32_list(Ctx &c, const int32_t *parents, int np) {
+    if (np <= 0) return;
+    switch (c.p) {
+    case 1: m2l_f32_launch<1>(c, parents, np); break;
+    case 2: m2l_f32_launch<2>(c, parents, np); break;
+    case 3: m2l_f32_launch<3>(c, parents, np); break;
+    case 4: m2l_f32_launch<4>(c, parents, np); break;
+    case 5: m2l_f32_launch<5>(c, parents, np); break;
+    case 6: m2l_f32_launch<6>(c, parents, np); break;
+    case 7: m2l_f32_launch<7>(c, parents, np); break;
+    case 8: m2l_f32_launch<8>(c, parents, np); break;
+    case 9: m2l_f32_launch<9>(c, parents, np); break;
+    case 10: m2l_f32_launch<10>(c, parents, np); break;
+    case 11: m2l_f32_launch<11>(c, parents, np); break;
+    case 12: m2l_f32_launch<12>(c, parents, np); break;
+    default: throw Error(1, "M2L supports 1 <= p <= 12");
+    }
+}
+
+// FP64: 32 targets per block, half of that when this leaves fewer than four
+// blocks per CU (twice the blocks keep more wavefronts in flight per CU).
+void m2l_f64_list(Ctx &c, const int32_t *parents, int np) {
+    if (np <= 0) return;
+    if (8 * static_cast<int64_t>(ceil_div(np, 32)) < 4 * static_cast<int64_t>(c.ncu))
+        m2l_plain_rows<16>(c, parents, np);
+    else
+        m2l_plain_rows<32>(c, parents, np);
 }
 
 template <class R>
@@ -1075,11 +1317,10 @@ void fmm_constants_init() {
 // walk.  A device table, written once per context.
 void ops_selection(Ctx &c) {
     if (c.ops_sel.p) return;
-    int16_t o[189], dn[189], qs[189];
-    m2l_walk(0, o, dn, qs);
+    constexpr M2lSteps steps = m2l_steps();
     std::vector<int16_t> h(NOPS_USED);
     for (int i = 0; i < 16; ++i) h[static_cast<size_t>(i)] = static_cast<int16_t>(i);
-    for (int i = 0; i < 189; ++i) h[static_cast<size_t>(16 + i)] = static_cast<int16_t>(16 + o[i]);
+    for (int i = 0; i < 189; ++i) h[static_cast<size_t>(16 + i)] = static_cast<int16_t>(16 + m2l_step(steps.d[i], steps.q[i], 0).o);
     c.ops_sel.ensure(NOPS_USED);
     VG_HIP(hipMemcpy(c.ops_sel.p, h.data(), NOPS_USED * sizeof(int16_t), hipMemcpyHostToDevice));
 }
@@ -1101,15 +1342,20 @@ void operators_build(Ctx &c) {
     dim3 grid(NOPS_USED, ceil_div(c.K, OPS_ROWS));
     if (c.prec == 0) {
         c.op64.ensure(static_cast<size_t>(nvec) * c.K * c.K);
-        k_ops<double><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op64);
+        k_ops<double><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op64, nullptr);
     } else if (c.prec == 2) {
         c.op64.ensure(static_cast<size_t>(nvec) * c.K * c.K);
-        k_ops<double><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op64);
+        k_ops<double><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op64, nullptr);
         c.op32.ensure(static_cast<size_t>(nvec) * c.K * c.K);
         m2l_split_operators(c, nvec);
     } else {
-        c.op32.ensure(static_cast<size_t>(nvec) * c.K * c.K);
-        k_ops<float><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op32);
+        c.op32.ensure(static_cast<size_t>(16) * c.K * c.K);
+        if (!c.opfrag.p) {
+            const size_t words = 343 * OpFrag(c.K).size();
+            c.opfrag.ensure(words);
+            VG_HIP(hipMemsetAsync(c.opfrag.p, 0, words * sizeof(float), c.stream));  // the padding, once
+        }
+        k_ops<float><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op32, c.opfrag);
     }
     VG_LAUNCH_CHECK();
 }
@@ -1121,18 +1367,19 @@ void fmm_upward(Ctx &c) {
         upward_t<float>(c);
 }
 
-void fmm_m2l_plain(Ctx &c) {
-    if (c.prec == 0)
-        m2l_plain_t<double>(c);
-    else
-        m2l_plain_t<float>(c);
-}
-
 void fmm_m2l_plain_list(Ctx &c, const int32_t *parents, int np) {
     if (c.prec == 0)
-        m2l_plain_list_t<double>(c, parents, np);
+        m2l_f64_list(c, parents, np);
     else
-        m2l_plain_list_t<float>(c, parents, np);
+        m2l_f32_list(c, parents, np);
+}
+
+void fmm_m2l_plain(Ctx &c) {
+    const TreeDev &t = c.t;
+    // parents: internal cells of levels >= 1 (their children are the targets at level >= 2)
+    if (t.depth < 1) return;
+    const int64_t a = t.int_off[1], b = t.int_off.back();
+    if (b > a) fmm_m2l_plain_list(c, t.int_ids.p + a, static_cast<int>(b - a));
 }
 
 void l2l_list(Ctx &c, const int32_t *parents, int64_t np) {

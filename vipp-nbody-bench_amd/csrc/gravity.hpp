@@ -11,6 +11,10 @@
 
 namespace vg {
 
+// Row stride of the expansion arrays: K in FP64; rounded up to 4 in FP32 (16-byte
+// rows) and to 16 for the split path, which reads whole 16-coefficient steps.
+inline int coeff_stride(int prec, int K) { return prec == 0 ? K : prec == 1 ? (K + 3) / 4 * 4 : (K + 15) / 16 * 16; }
+
 enum Phase { PH_TREE = 0, PH_LISTS, PH_UP, PH_M2L, PH_P2P, PH_DOWN, PH_RK4, PH_OPS, PH_COUNT };
 
 struct TreeDev {
@@ -50,7 +54,7 @@ struct TreeDev {
 struct ExpSet {
     int p = 0, K = 0, ldk = 0;
     DevBuf<double> harm, op64;
-    DevBuf<float> op32, M32, L32;
+    DevBuf<float> op32, opfrag, M32, L32;
     DevBuf<uint16_t> opsplit, opsplit_ml, msplit;
 };
 
@@ -83,7 +87,7 @@ struct Ctx {
     uint32_t thr = 0;  // floor(sqrt(8) s)
     int p = 4;
     int K = 25;        // (p+1)^2 real coefficients
-    int ldk = 25;      // row stride of the expansion arrays (K, or K rounded up to 16 for the MFMA path)
+    int ldk = 25;      // row stride of the expansion arrays (coeff_stride)
     int prec = 1;
     double eps = 0, G = 1, mass = 0;
     uint32_t flags = 0;
@@ -144,6 +148,7 @@ struct Ctx {
     DevBuf<double> harm;        // harmonic tables of the operator offsets
     DevBuf<double> op64;        // M2M (8), L2L (8), M2L (343) blocks of K*K
     DevBuf<float> op32;
+    DevBuf<float> opfrag;       // FP32 mode: M2L operators in the order the matrix cores' lanes read them
     DevBuf<uint16_t> opsplit;   // M2L operators as BF16 hi/lo MFMA fragments
     DevBuf<uint16_t> opsplit_ml;  // the 8 M2M and 8 L2L operators, the same way
     DevBuf<float> ml_part;      // split M2M: the 8 octant products of one level before their sum

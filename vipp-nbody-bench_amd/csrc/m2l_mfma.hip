@@ -127,7 +127,7 @@ __global__ __launch_bounds__(64 * NG * mt_m2l((P + 1) * (P + 1))) void k_m2l_spl
     // (-1)^m on cosine, -(-1)^m on sine coefficients; y -> -y: -1 on sine;
     // z -> -z: (-1)^(n+m)).  So L = D_qt sum_e T_e (D_qt M): the signs go on the
     // gathered multipoles and on the result, and all blocks share 189 operators.
-    if (tid == 0) m2l_walk(qt, s_o, s_dn, s_qs);
+    m2l_walk(tid, NTH, qt, s_o, s_dn, s_qs);
     for (int k = tid; k < 16 * NKS; k += NTH) s_sgn[k] = static_cast<float>(m2l_mirror_sign(qt, k));
     __syncthreads();
     for (int k8 = tid; k8 < 2 * NKS; k8 += NTH) {
