@@ -1148,38 +1148,17 @@ void m2l_plain_rows(Ctx &c, const int32_t *parents, int np) {
     }
 }
 
-// Parts of the walked offsets of a grid of `grid` equal blocks: a CU's blocks
-// share its matrix pipes, so the time goes with the fullest CU's share of the
-// work, ceil(grid n / ncu) / n, and each part costs about 1 % (prologue, partial
-// sums).  Grids of 8 and more blocks per CU are not cut.
-int m2l_f32_parts(unsigned grid, int ncu) {
-    int best = 1;
-    if (ncu <= 0 || grid >= 8u * static_cast<unsigned>(ncu)) return best;
-    double t = 1e300;
-    for (int n = 1; n <= 32; ++n) {
-        const double x = static_cast<double>(ceil_div(static_cast<size_t>(grid) * n, ncu)) / n * (1 + 0.01 * n);
-        if (x < t) t = x, best = n;
-    }
-    return best;
-}
-
 template <int P>
 void m2l_f32_launch(Ctx &c, const int32_t *parents, int np) {
     const unsigned grid = 8 * ceil_div(np, 64);
-    const int nsplit = m2l_f32_parts(grid, c.ncu);
-    float *part = nullptr;
-    if (nsplit > 1) {
-        c.m2l_part.ensure(static_cast<size_t>(nsplit) * 8 * np * c.ldk * sizeof(float));
-        part = reinterpret_cast<float *>(c.m2l_part.p);
-    }
+    const int nsplit = m2l_parts(grid, c.ncu);
+    float *part = m2l_part_sums(c, np, nsplit);
     if (c.ldk != M2lShape<P>::LD) throw Error(1, "FP32 M2L: the coefficient stride must be K rounded up to 4");
     const TreeDev &t = c.t;
     k_m2l_f32<P><<<grid * nsplit, 256, 0, c.stream>>>(parents, np, t.child, t.count, t.nbr27, reinterpret_cast<const f4 *>(c.M32.p), c.L32.p,
                                                           reinterpret_cast<const f4 *>(c.opfrag.p), nsplit, part);
-    if (nsplit > 1)
-        k_m2l_sum<float><<<ceil_div(static_cast<size_t>(8) * np * c.K, 256), 256, 0, c.stream>>>(parents, np, t.child, t.count, nsplit, part, c.L32, c.K,
-                                                                                              c.ldk);
     VG_LAUNCH_CHECK();
+    m2l_add_parts(c, parents, np, nsplit, part);
 }
 
 void m2l_f32_list(Ctx &c, const int32_t *parents, int np) {
@@ -1365,6 +1344,35 @@ void fmm_upward(Ctx &c) {
         upward_t<double>(c);
     else
         upward_t<float>(c);
+}
+
+// Parts of the walked offsets of a grid of `grid` equal blocks: a CU's blocks
+// share its matrix pipes, so the time goes with the fullest CU's share of the
+// work, ceil(grid n / ncu) / n, and each part costs about 1 % (prologue, partial
+// sums).  Grids of 8 and more blocks per CU are not cut.
+int m2l_parts(unsigned grid, int ncu) {
+    int best = 1;
+    if (ncu <= 0 || grid >= 8u * static_cast<unsigned>(ncu)) return best;
+    double t = 1e300;
+    for (int n = 1; n <= 32; ++n) {
+        const double x = static_cast<double>(ceil_div(static_cast<size_t>(grid) * n, ncu)) / n * (1 + 0.01 * n);
+        if (x < t) t = x, best = n;
+    }
+    return best;
+}
+
+// Room for the partial sums of nsplit parts (nullptr for one), and their sum
+// into the local expansions.
+float *m2l_part_sums(Ctx &c, int np, int nsplit) {
+    if (nsplit < 2) return nullptr;
+    c.m2l_part.ensure(static_cast<size_t>(nsplit) * 8 * np * c.ldk * sizeof(float));
+    return reinterpret_cast<float *>(c.m2l_part.p);
+}
+void m2l_add_parts(Ctx &c, const int32_t *parents, int np, int nsplit, const float *part) {
+    if (nsplit < 2) return;
+    k_m2l_sum<float><<<ceil_div(static_cast<size_t>(8) * np * c.K, 256), 256, 0, c.stream>>>(parents, np, c.t.child, c.t.count, nsplit, part, c.L32, c.K,
+                                                                                          c.ldk);
+    VG_LAUNCH_CHECK();
 }
 
 void fmm_m2l_plain_list(Ctx &c, const int32_t *parents, int np) {

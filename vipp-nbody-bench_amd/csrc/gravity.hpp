@@ -198,6 +198,9 @@ bool closure_fallback_prepare(Ctx &c);        // order-p_hi locals of the flagge
 void closure_fallback_l2p(Ctx &c);            // order-p_hi L2P of the flagged leaves
 void swap_expansions(Ctx &c, ExpSet &e);      // exchange the context's expansion set with e
 void m2l_list(Ctx &c, const int32_t *parents, int np);      // M2L of the children of the given internal cells
+int m2l_parts(unsigned grid, int ncu);        // parts of the walked offsets of an M2L grid
+float *m2l_part_sums(Ctx &c, int np, int nsplit);  // their partial sums (FP32), and the sums into the locals
+void m2l_add_parts(Ctx &c, const int32_t *parents, int np, int nsplit, const float *part);
 void l2l_list(Ctx &c, const int32_t *parents, int64_t np);  // L2L into the children of the given internal cells (FP32)
 void ml_split_level(Ctx &c, const int32_t *ids, int64_t n, bool m2m);  // M2M (m2m) or L2L of one level on the matrix cores
 void l2p_list(Ctx &c, const int32_t *leaves, int64_t n, const uint8_t *skip);  // L2P of the given leaves (FP32)

@@ -3,13 +3,13 @@
 //
 // The M2L of one target is L~(t) = sum_o T_o M~(s(t, o)) over its (at most
 // 189) source offsets o (fmm.hpp:277-304 in the scaled real basis of
-// fmm.hip).  A block owns 32 NT targets of one child octant qt, so that every
+// fmm.hip).  A block owns 64 targets of one child octant qt, so that every
 // target sees the same 189 offsets in the same order (offsets follow from
 // (parent-neighbour offset, source octant, qt) alone).  Per offset the block
-// forms T_o (K x K) times the targets' source multipoles (K x 32 NT) on
-// v_mfma_f32_32x32x16_bf16, two wavefronts per 32 output rows, accumulating
-// in FP32 across all offsets.  Every block walks the offsets in the same
-// order, so the operators stream through L2 shared by the blocks of an XCD.
+// forms T_o (K x K) times the targets' source multipoles (K x 64) on
+// v_mfma_f32_16x16x32_bf16, accumulating in FP32 across its offsets.  Every
+// block walks the offsets in the same order, so the operators stream through L2
+// shared by the blocks of an XCD.
 //
 // Precision: every M2L operand x is split as hi = bf16(x), lo = bf16(x - hi)
 // (16 significant bits together) and a product is formed as
@@ -18,10 +18,12 @@
 // value; the multipoles are split once per evaluation (k_split_m).  M2M and
 // L2L use a three-way split (below).
 //
-// Operand layouts (checked on the device): for v_mfma_f32_32x32x16_bf16 lane l
-// holds A[l%32][8(l/32)+e] and B[8(l/32)+e][l%32], e = 0..7, and
-// C[8(r/4) + 4(l/32) + r%4][l%32], r = 0..15.  T_o is stored pre-swizzled in
-// that A order, so a wavefront loads a fragment with one 16-byte read per lane.
+// Operand layouts (checked on the device): for v_mfma_f32_16x16x32_bf16 lane l
+// holds A[l%16][8(l/16)+e] and B[8(l/16)+e][l%16], e = 0..7, and
+// C[4(l/16) + r][l%16], r = 0..3; for v_mfma_f32_32x32x16_bf16 (M2M, L2L)
+// A[l%32][8(l/32)+e], B[8(l/32)+e][l%32] and C[8(r/4) + 4(l/32) + r%4][l%32],
+// r = 0..15.  Operators are stored in that A order, so a wavefront loads a
+// fragment with one 16-byte read per lane.
 #include "gravity.hpp"
 
 namespace vg {
@@ -29,36 +31,31 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ constexpr int mt_of(int K) { return (K + 31) / 32; }
-// M2L row tiles: the odd counts 3 (p = 8) and 5 (p = 11) are padded to 4
-// and 6, so the kernel's 2 MT wavefronts spread evenly over the 4 SIMDs of a
-// CU (the padded rows are zero; p = 8: M2L 1.47 -> 1.38 ms and 29.4 -> 31.2
-// steps/s on the 4M Plummer input, p = 11: 3.84 -> 2.56 ms)
-__host__ __device__ constexpr int mt_m2l(int K) { return (mt_of(K) == 3 || mt_of(K) == 5) ? mt_of(K) + 1 : mt_of(K); }
 __host__ __device__ constexpr int ks_of(int K) { return (K + 15) / 16; }
 
 // FP64 operators (row-major K x K per offset) -> BF16 hi/lo A fragments of
-// the M2L blocks: frag[o][mt][h][ks][lane][e], so that any run of consecutive
-// m-tiles (hi and lo) is one contiguous range.  One block per (offset, m-tile):
-// the tile's 32 rows are read row by row into LDS (coalesced), then each thread
-// writes whole 8-coefficient fragment vectors.
+// the M2L: frag[o][16-row tile][32-column k-step][hi, lo][lane][8 columns], lane
+// 16 q + r holding row r, columns 8 q .. 8 q + 7 (zero past K).  One block per
+// (offset, row tile): the tile's rows are read into LDS (coalesced), then each
+// thread writes whole fragment words.
 __global__ __launch_bounds__(256) void k_split_ops(const int16_t *__restrict__ sel, const double *__restrict__ op64, int K, __bf16 *__restrict__ frag,
-                                                   int MT, int NKS) {
-    extern __shared__ double tile[];  // 32 rows x (16 NKS + 1)
-    const int o = sel[16 + blockIdx.x / MT] - 16, mt = blockIdx.x % MT;  // the M2L offsets of the walk only
-    const int kc = 16 * NKS, W = kc + 1;
+                                                   int NT, int KS) {
+    extern __shared__ double tile[];  // 16 rows x (32 KS + 1)
+    const int o = sel[16 + blockIdx.x / NT] - 16, rt = blockIdx.x % NT;  // the M2L offsets of the walk only
+    const int kc = 32 * KS, W = kc + 1;
     const double *src = op64 + static_cast<int64_t>(16 + o) * K * K;
-    for (int i = threadIdx.x; i < 32 * kc; i += 256) {
-        const int r = i / kc, col = i % kc, row = mt * 32 + r;
+    for (int i = threadIdx.x; i < 16 * kc; i += 256) {
+        const int r = i / kc, col = i % kc, row = rt * 16 + r;
         tile[r * W + col] = (row < K && col < K) ? src[static_cast<int64_t>(row) * K + col] : 0.0;
     }
     __syncthreads();
-    const int64_t base = (static_cast<int64_t>(o) * MT + mt) * 2 * NKS * 64;  // in 8-coefficient vectors
-    for (int v = threadIdx.x; v < 2 * NKS * 64; v += 256) {
-        const int h = v / (NKS * 64), ks = (v / 64) % NKS, l = v % 64;
-        const int r = l & 31, c0 = ks * 16 + (l >> 5) * 8;
+    const int64_t base = (static_cast<int64_t>(o) * NT + rt) * KS * 128;  // in 8-coefficient vectors
+    for (int v = threadIdx.x; v < KS * 128; v += 256) {
+        const int ks = v >> 7, h = (v >> 6) & 1, l = v & 63;
+        const int r = l & 15, c0 = ks * 32 + (l >> 4) * 8;
         bf16x8 out;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -70,338 +67,216 @@ __global__ __launch_bounds__(256) void k_split_ops(const int16_t *__restrict__ s
     }
 }
 
-// One block: 32*NT targets (children of octant qt of 32*NT parents) and NG
-// wavefronts per 32-row m-tile of the output.  Without KS each of them owns
-// NT/NG n-tiles of 32 targets over all k-steps; with KS (NG = 2) both own all
-// NT n-tiles, one the even and one the odd k-steps, and their sums are added
-// at the end, so every A fragment is loaded by one wavefront only.  Per offset
-// step:
-//   A (the wavefront's m-tile of T_o, hi and lo) streams from L2 straight
-//     into registers, a few k-steps ahead;
-//   B (the targets' source multipoles) sits in LDS as hi/lo MFMA fragments.
-// The k-steps of an offset are cut into two halves, and B is double-buffered
-// by half: while a half is multiplied from one buffer, the next half is
-// gathered into registers and stored into the other, so the only pause is one
-// barrier per half.  The B fragment of lane l is stored in slot
-// l ^ (k8 & 15), k8 = 2 ks + l / 32 (ks counted within the half), so that
-// both the row-wise stores and the fragment loads spread over the LDS banks.
-template <int P, int NT, int NG, bool KS>
-__global__ __launch_bounds__(64 * NG * mt_m2l((P + 1) * (P + 1))) void k_m2l_split(const int32_t *__restrict__ parents, int nparents,
-                                                                             const int32_t *__restrict__ child, const uint32_t *__restrict__ count,
-                                                                             const int32_t *__restrict__ nbr27, const uint4 *__restrict__ Ms,
-                                                                             float *__restrict__ L, const bf16x8 *__restrict__ ops, int ldk) {
-    constexpr int K = (P + 1) * (P + 1);
-    constexpr int MT = mt_m2l(K), NKS = ks_of(K);
-    constexpr int NTH = 64 * MT * NG;        // threads
-    constexpr int NW = KS ? NT : NT / NG;    // n-tiles per wavefront
-    static_assert(NT % NG == 0, "n-tiles must split evenly over the wavefronts of an m-tile");
-    static_assert(!KS || (NG == 2 && NKS >= 3), "the k-step split pairs two wavefronts per m-tile");
-    constexpr int TB = 32 * NT;              // targets per block
-    constexpr int TILE = 2 * NKS * 64;       // bf16x8 vectors of one m-tile of an operator (hi and lo)
-    constexpr int KH0 = KS ? 2 * ((NKS + 3) / 4) : (NKS + 1) / 2;  // k-steps of the first half (even with KS)
-    constexpr int NH = NKS > KH0 ? 2 : 1;     // halves per offset step
-    constexpr int CPT = (TB * 2 * KH0 + NTH - 1) / NTH;  // 8-coefficient chunks per thread and half
-    __shared__ bf16x8 sB[2][KH0][NT][2][64];  // [buffer][k-step in half][n-tile][hi/lo][lane]
-    __shared__ int16_t s_dn[189], s_qs[189], s_o[189];
-    __shared__ int32_t s_sb[27][TB];         // first child of each parent neighbour (-1: none)
-    __shared__ uint32_t s_live[7][TB];       // bit 8 dn + qs: that source cell holds particles
-    __shared__ float s_sgn[16 * NKS];        // D_qt: sign of each coefficient under this octant's mirror
-    __shared__ uint4 s_msk[2 * NKS];         // the same as BF16 sign-bit masks, 8 coefficients per entry
-    __shared__ uint8_t s_nl[189];            // KS: bit n set when some target of n-tile n has a source at that step
+// Shape of the split M2L at order P: 64 targets (four 16-target tiles) per
+// block, its NT 16-row tiles over WR wavefronts (RW each) and the target tiles
+// over WC.  128 targets, two by two wavefronts and three wavefronts for NT = 3
+// or 11 were slower (fewer blocks per CU, or operators read twice).
+template <int P>
+struct SplitShape {
+    static constexpr int K = (P + 1) * (P + 1), NT = (K + 15) / 16, KS = (K + 31) / 32;
+    static constexpr int TB = 64, WR = NT == 1 ? 1 : NT == 2 ? 2 : 4, WC = 4 / WR;
+    static constexpr int RW = (NT + WR - 1) / WR, NC = TB / 16 / WC, NW = WR * WC;
+    static constexpr int LD = 16 * ks_of(K);      // coefficients of a cell's row, hi or lo
+    static constexpr int CH = LD / 4;             // 16-byte words of a cell's hi and lo rows
+    static constexpr int SK = CH | 1;             // the same in LDS: an odd number, so reads have no bank conflicts
+    static constexpr int TPI = 64 / CH;           // targets a wavefront gathers with one load
+};
+
+// One block: 64 targets (children of octant qt of 64 parents).  Per walked
+// offset the block gathers the targets' source multipoles (hi and lo rows, one
+// 16-byte word per lane, with this octant's mirror signs) into LDS and
+// multiplies the operator by them, hi*hi + hi*lo + lo*hi; operator fragments come
+// straight from L2, each loaded by one wavefront where WC = 1, and the next offset's
+// multipoles are on their way during the products.  With nsplit > 1 the walked
+// offsets are cut into parts, one block each, with partial sums in part.
+//
+// Bound by the way to L2: at p = 12 a CU takes 26 B/clk of operators and
+// multipoles at 47 % of the matrix rate (64 B/clk is its port), so the
+// operators are read a k-step ahead (p < 10: four blocks per CU hide the rest;
+// two ahead cost a block and 10 to 15 %) or two (p >= 10: two blocks whatever the
+// depth; 1 to 3 % faster).  Wavefronts in their products go before the ones that
+// gather (s_setprio: -2 % at p = 12).  ms per evaluation, against 32x32x16
+// tiles over 32 or 64 targets staged by twice the wavefronts, uncut:
+//   Plummer N, p       2461, 4  16384, 8  262144, 8  1M, 9  4M, 8  4M, 10  4M, 12
+//   before                .254      .365       .451    .54   1.38    1.75    3.11
+//   here                  .026      .058       .095    .38   1.01    1.65    3.13
+// and 12.1 -> 11.8 at p = 12 on 16M bodies of two colliding spheres.
+template <int P>
+__global__ __launch_bounds__(64 * SplitShape<P>::NW, 2) void k_m2l_split(const int32_t *__restrict__ parents, int nparents,
+                                                                         const int32_t *__restrict__ child, const uint32_t *__restrict__ count,
+                                                                         const int32_t *__restrict__ nbr27, const uint4 *__restrict__ Ms,
+                                                                         float *__restrict__ L, const bf16x8 *__restrict__ ops, int nsplit,
+                                                                         float *__restrict__ part) {
+    using S = SplitShape<P>;
+    constexpr int TB = S::TB, NTH = 64 * S::NW;
+    constexpr int NG = (TB + S::NW * S::TPI - 1) / (S::NW * S::TPI);  // words a lane gathers
+    constexpr int PAD = 4 * S::KS > S::LD / 8 ? 4 * S::KS - S::LD / 8 : 0;  // words read past a row's end (times zero columns)
+    __shared__ uint4 sM[TB * S::SK + PAD];
+    __shared__ int32_t s_nc[27 * TB];  // first child of parent neighbour d of target t, or -1
+    __shared__ uint8_t s_nm[27 * TB];  // its non-empty children
+    __shared__ int32_t tgt[TB];
+    __shared__ int16_t s_o[189], s_dn[189], s_qs[189], s_live[189];
+    __shared__ int s_nlive, s_cnt[3], s_step[189];  // s_step: the walked offsets, operator | neighbour << 9 | octant << 14
+    static_assert(NTH >= 192, "m2l_live_steps");
     // XCD-aware placement: blocks go round-robin to the 8 XCDs, so XCD x takes
-    // the contiguous run of work items [x per, (x+1) per); the 8 octant blocks
-    // of a parent chunk, which read the same source multipoles and operators,
-    // run side by side on one XCD and share its L2.
+    // the contiguous run of work items [x W / 8, (x + 1) W / 8); the octant blocks
+    // of a parent chunk, which read the same multipoles, share its L2.
     const int nchunks = (nparents + TB - 1) / TB;
-    const int w = (blockIdx.x & 7) * nchunks + (blockIdx.x >> 3);
-    if (w >= 8 * nchunks) return;
-    const int chunk = w >> 3, qt = w & 7;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, so addresses built from it stay scalar
-    const int mt = wid % MT, n0 = KS ? 0 : (wid / MT) * NW;
-    const int kw = KS ? wid / MT : 0;  // KS: this wavefront takes the k-steps ks = kw mod 2
-    // Every block walks the 189 offsets e of octant 0 in one fixed order.  For
-    // octant qt the geometry is octant 0's mirrored in the axes where qt has a
-    // bit set (parent neighbour d -> mirror(d), source octant q -> q ^ qt), and
-    // the mirrored operator is D_qt T_e D_qt with D_qt diagonal +-1 (x -> -x:
-    // (-1)^m on cosine, -(-1)^m on sine coefficients; y -> -y: -1 on sine;
-    // z -> -z: (-1)^(n+m)).  So L = D_qt sum_e T_e (D_qt M): the signs go on the
-    // gathered multipoles and on the result, and all blocks share 189 operators.
+    const int per = nchunks * nsplit;
+    const int wi = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if (wi >= 8 * per) return;
+    const int sp = wi % nsplit, w = wi / nsplit, chunk = w >> 3, qt = w & 7;
+    const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, quad = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = (wv + static_cast<int>(blockIdx.x >> 3)) % S::WR, wc = wv / S::WR;  // the light wavefront changes its SIMD from block to block
     m2l_walk(tid, NTH, qt, s_o, s_dn, s_qs);
-    for (int k = tid; k < 16 * NKS; k += NTH) s_sgn[k] = static_cast<float>(m2l_mirror_sign(qt, k));
+    if (tid < TB) {
+        const int pi = chunk * TB + tid;
+        const int32_t p = pi < nparents ? parents[pi] : -1;
+        int32_t t = p >= 0 ? child[p] + qt : -1;
+        if (t >= 0 && count[t] == 0) t = -1;
+        tgt[tid] = t;
+        for (int k = S::CH; k < S::SK; ++k) sM[tid * S::SK + k] = make_uint4(0, 0, 0, 0);
+    }
+    for (int k = tid; k < PAD; k += NTH) sM[TB * S::SK + k] = make_uint4(0, 0, 0, 0);
     __syncthreads();
-    for (int k8 = tid; k8 < 2 * NKS; k8 += NTH) {
-        uint32_t w[4];
-        for (int i = 0; i < 4; ++i)
-            w[i] = (s_sgn[8 * k8 + 2 * i] < 0 ? 0x8000u : 0u) | (s_sgn[8 * k8 + 2 * i + 1] < 0 ? 0x80000000u : 0u);
-        s_msk[k8] = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-    for (int t = tid; t < TB; t += NTH) {
-        const int pi = chunk * TB + t;
-        int32_t P0 = pi < nparents ? parents[pi] : -1;
-        if (P0 >= 0 && count[child[P0] + qt] == 0) P0 = -1;
-        uint32_t live[7] = {0, 0, 0, 0, 0, 0, 0};
-        for (int dn = 0; dn < 27; ++dn) {
-            const int32_t sp = P0 >= 0 ? nbr27[27 * static_cast<int64_t>(P0) + dn] : -1;
-            const int32_t sb = sp >= 0 ? child[sp] : -1;
-            s_sb[dn][t] = sb;
-            if (sb >= 0)
-                for (int q = 0; q < 8; ++q)
-                    if (count[sb + q] > 0) live[(8 * dn + q) >> 5] |= 1u << ((8 * dn + q) & 31);
+    for (int i = tid; i < 27 * TB; i += NTH) {
+        const int d = i / TB, t = i % TB;
+        int32_t cb = -1;
+        uint32_t msk = 0;
+        if (tgt[t] >= 0) {
+            const int32_t p = nbr27[27 * static_cast<int64_t>(parents[chunk * TB + t]) + d];
+            cb = p >= 0 ? child[p] : -1;
+            if (cb >= 0)
+                for (int q = 0; q < 8; ++q) msk |= (count[cb + q] != 0 ? 1u : 0u) << q;
         }
-        for (int w = 0; w < 7; ++w) s_live[w][t] = live[w];
+        s_nc[i] = cb;
+        s_nm[i] = static_cast<uint8_t>(msk);
     }
     __syncthreads();
-    if constexpr (KS) {  // n-tiles without any source at a step skip its products (their B is zero)
-        for (int st = wid; st < 189; st += NTH / 64) {
-            const int bit = 8 * s_dn[st] + s_qs[st];
-            uint32_t m = 0;
-            for (int h = 0; h < NT / 2; ++h) {
-                const int t = 64 * h + lane;
-                const uint64_t b = __ballot((s_live[bit >> 5][t] >> (bit & 31)) & 1u);
-                m |= (b & 0xffffffffull ? 1u : 0u) << (2 * h);
-                m |= (b >> 32 ? 1u : 0u) << (2 * h + 1);
-            }
-            if (lane == 0) s_nl[st] = static_cast<uint8_t>(m);
-        }
-        __syncthreads();
+    m2l_live_steps(tid, s_live, &s_nlive, s_cnt, [&](int st) {
+        const int dn = s_dn[st], qs = s_qs[st];
+        int any = 0;
+        for (int t = 0; t < TB; ++t) any |= s_nm[dn * TB + t] >> qs;
+        return (any & 1) != 0;
+    });
+    // this lane gathers word ch of the targets (wv + NW u) TPI + sub, with its sign bits (negation commutes with the split)
+    const int sub = lane / S::CH, ch = lane % S::CH;
+    uint32_t sg[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int k = 8 * (ch % (S::LD / 8)) + 2 * e;
+        sg[e] = (k < S::K && m2l_mirror_sign(qt, k) < 0 ? 0x8000u : 0u) | (k + 1 < S::K && m2l_mirror_sign(qt, k + 1) < 0 ? 0x80000000u : 0u);
     }
-    // source cell of target t at step st (-1: none or empty); st is uniform
-    auto source_of = [&](int st, int t) -> int32_t {
-        const int dn = __builtin_amdgcn_readfirstlane(s_dn[st]), qs = __builtin_amdgcn_readfirstlane(s_qs[st]);
-        const int bit = 8 * dn + qs;
-        return ((s_live[bit >> 5][t] >> (bit & 31)) & 1u) ? s_sb[dn][t] + qs : -1;
-    };
-    // gather half h of step st's B operand into registers: chunk c -> target
-    // c / (2 kh), the 8 coefficients at k = 8 k8, k8 = 2 KH0 h + c % (2 kh), as
-    // BF16 hi and lo halves (Ms: per cell ldk hi values then ldk lo values, 16
-    // bytes per 8 coefficients)
-    uint4 gh[CPT], gl[CPT];
-    auto gather = [&](int st, int h) {
-        const int kh = h ? NKS - KH0 : KH0;
-#pragma unroll
-        for (int u = 0; u < CPT; ++u) {
-            const int c = tid + u * NTH;
-            const int t = c / (2 * kh), k8 = 2 * KH0 * h + c % (2 * kh);
-            const int32_t src_cell = (c < TB * 2 * kh) ? source_of(st, t) : -1;
-            if (src_cell >= 0) {
-                const uint4 *src = Ms + static_cast<int64_t>(src_cell) * (ldk / 4) + k8;  // ldk / 8 chunks of hi, then of lo
-                gh[u] = src[0];
-                gl[u] = src[ldk / 8];
-            } else {
-                gh[u] = make_uint4(0, 0, 0, 0);
-                gl[u] = make_uint4(0, 0, 0, 0);
-            }
-        }
-    };
-    // store into buffer bf as MFMA B fragments with this octant's signs
-    // (negation commutes with the split, so it is a flip of the sign bits):
-    // lane (k8l % 2) * 32 + t % 32 of n-tile t / 32, k-step k8l / 2 of the half
-    auto stash = [&](int bf, int h) {
-        const int kh = h ? NKS - KH0 : KH0;
-#pragma unroll
-        for (int u = 0; u < CPT; ++u) {
-            const int c = tid + u * NTH;
-            if (c >= TB * 2 * kh) continue;
-            const int t = c / (2 * kh), k8l = c % (2 * kh);
-            const uint4 m = s_msk[2 * KH0 * h + k8l];
-            const uint4 hv = make_uint4(gh[u].x ^ m.x, gh[u].y ^ m.y, gh[u].z ^ m.z, gh[u].w ^ m.w);
-            const uint4 lv = make_uint4(gl[u].x ^ m.x, gl[u].y ^ m.y, gl[u].z ^ m.z, gl[u].w ^ m.w);
-            const int ln = ((k8l & 1) * 32 + (t & 31)) ^ (k8l & 15);
-            sB[bf][k8l >> 1][t >> 5][0][ln] = __builtin_bit_cast(bf16x8, hv);  // typed stores: the loads below are bf16x8
-            sB[bf][k8l >> 1][t >> 5][1][ln] = __builtin_bit_cast(bf16x8, lv);
-        }
-    };
-    f32x16 acc[NW];
-#pragma unroll
-    for (int n = 0; n < NW; ++n)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[n][r] = 0.0f;
-    gather(0, 0);
-    stash(0, 0);
+    const int nlive = s_nlive;
+    if (tid < nlive) {
+        const int st = s_live[tid];
+        s_step[tid] = s_o[st] | s_dn[st] << 9 | s_qs[st] << 14;
+    }
     __syncthreads();
-    // A fragments of this wavefront's m-tile for operator o (uniform), flat k-step q
-    constexpr int TOT = 189 * NKS;
-    constexpr int PF = 3;  // A prefetch distance in k-steps
-    auto afrag = [&](int o, int ks, int h) -> bf16x8 {
-        const bf16x8 *base = ops + (static_cast<int64_t>(o) * MT + mt) * TILE + h * NKS * 64 + ks * 64;
-        return base[lane];
-    };
-    // B fragments of k-step ksl of buffer bf for this wavefront's n-tiles
-    // (slot = lane ^ ((2 ksl + lane / 32) % 16) = (lane ^ lane / 32) ^ (2 ksl % 16):
-    // one XOR with a constant on a per-lane byte offset)
-    uint32_t lb = (lane ^ (lane >> 5)) * 16u;
-    auto bfrag = [&](int bf, int ksl, bf16x8 *h, bf16x8 *l) {
-        const uint32_t off = lb ^ (((2u * ksl) & 14u) << 4);
-        const char *row = reinterpret_cast<const char *>(&sB[bf][ksl][n0][0][0]) + off;
+    const int lo = sp * nlive / nsplit, hi = (sp + 1) * nlive / nsplit;  // this block's walked offsets
+    f32x4 acc[S::RW][S::NC];
 #pragma unroll
-        for (int n = 0; n < NW; ++n) {
-            h[n] = *reinterpret_cast<const bf16x8 *>(row + (2 * n) * 1024);
-            l[n] = *reinterpret_cast<const bf16x8 *>(row + (2 * n + 1) * 1024);
+    for (int r = 0; r < S::RW; ++r)
+#pragma unroll
+        for (int n = 0; n < S::NC; ++n) acc[r][n] = f32x4{0, 0, 0, 0};
+    // fragments of k-step ks of this wavefront's row tiles wr, wr + WR, ... (a missing one repeats the last)
+    auto load_a = [&](int li, int ks, bf16x8 (*a)[2]) {
+        const bf16x8 *O = ops + static_cast<int64_t>(__builtin_amdgcn_readfirstlane(s_step[li]) & 511) * (S::NT * S::KS * 128) + ks * 128;
+#pragma unroll
+        for (int r = 0; r < S::RW; ++r) {
+            const bf16x8 *F = O + min(wr + S::WR * r, S::NT - 1) * (S::KS * 128);
+            a[r][0] = F[static_cast<unsigned>(lane)];
+            a[r][1] = F[64u + lane];
         }
     };
-    if constexpr (KS) {
-        // Wavefront position j of a step takes k-step ks = 2 j + kw (none when
-        // ks >= NKS); A of positions p + 1 .. p + PF is in flight.  B is read
-        // for the position itself.  Half h covers positions [h JH0, ...), the
-        // same for both wavefronts of an m-tile, so every wavefront meets the
-        // barriers at the same positions.
-        constexpr int NJ = (NKS + 1) / 2, JH0 = KH0 / 2;
-        constexpr int PFJ = 2;
-        constexpr int NSO = (PFJ + NJ - 1) / NJ + 1;  // steps the prefetch of one step reaches
-        // (positions without a k-step, and past the last step, load a valid
-        // fragment that is not used: no branch, so the ring needs no copies)
-        bf16x8 ah[PFJ], al[PFJ];
+    uint4 v[NG];
+    uint64_t dead = 0;  // bit u: the target of v[u] has no source here (TPI = 1, which reads row 0 for it)
+    static_assert(S::TPI > 1 || S::NW * NG == TB);
+    auto gather = [&](int li) {  // this lane's words of the multipoles of walked offset li
+        const int st = __builtin_amdgcn_readfirstlane(s_step[li]), dn = (st >> 9 & 31) * TB, qs = st >> 14;
+        if constexpr (S::TPI == 1) {  // a load takes one target, whose row lane u has looked up
+            const int t = wv + S::NW * (lane % NG);
+            const bool live = (s_nm[dn + t] >> qs) & 1;
+            const int cell = live ? s_nc[dn + t] + qs : 0;
+            dead = ~__ballot(live);
+            if (lane < S::CH) {
 #pragma unroll
-        for (int i = 0; i < PFJ; ++i) {
-            const int ks = min(2 * (i % NJ) + kw, NKS - 1);
-            const int o = __builtin_amdgcn_readfirstlane(s_o[i / NJ]);
-            ah[i] = afrag(o, ks, 0);
-            al[i] = afrag(o, ks, 1);
-        }
-        for (int st = 0; st < 189; ++st) {
-            int so[NSO];  // operators of steps st .. st + NSO - 1, scalar
-#pragma unroll
-            for (int i = 0; i < NSO; ++i) so[i] = __builtin_amdgcn_readfirstlane(st + i < 189 ? s_o[st + i] : 0);
-            asm volatile("" : "+v"(lb));  // recompute the B offsets per step rather than hold them all
-            const uint32_t nl = __builtin_amdgcn_readfirstlane(s_nl[st]);
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const int h = j < JH0 ? 0 : 1, jl = j - h * JH0, jh = h ? NJ - JH0 : JH0;
-                // with NKS odd the last k-step is shared: the even wavefront forms
-                // hi*hi + hi*lo, the odd one lo*hi, so neither waits for the other
-                constexpr bool SHARED_LAST = (NKS & 1) != 0;
-                const bool last = SHARED_LAST && j == NJ - 1;
-                const int ks = last ? NKS - 1 : 2 * j + kw, ksl = ks - h * KH0;
-                const bool active = ks < NKS;
-                const int bf = NH == 2 ? h : (st & 1);
-                const int nst = (NH == 2 && h == 0) ? st : st + 1, nhf = (NH == 2 && h == 0) ? 1 : 0;
-                const int nbf = NH == 2 ? nhf : ((st + 1) & 1);
-                const bool has_next = nst < 189;
-                const bf16x8 ch = ah[0], cl = al[0];
-#pragma unroll
-                for (int i = 0; i + 1 < PFJ; ++i) {
-                    ah[i] = ah[i + 1];
-                    al[i] = al[i + 1];
-                }
-                {
-                    const int jp = j + PFJ, kp = min(2 * (jp % NJ) + kw, NKS - 1);
-                    ah[PFJ - 1] = afrag(so[jp / NJ], kp, 0);
-                    al[PFJ - 1] = afrag(so[jp / NJ], kp, 1);
-                }
-                if (jl == 0 && has_next) gather(nst, nhf);
-                bf16x8 bh[NW], bl[NW];
-                if (active) bfrag(bf, ksl, bh, bl);
-                __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int n = 0; n < NW; ++n) {
-                    if (!((nl >> n) & 1u)) continue;
-                    if (!last || kw == 0) {
-                        acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, bh[n], acc[n], 0, 0, 0);
-                        acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, bl[n], acc[n], 0, 0, 0);
-                    }
-                    if (!last || kw == 1) acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cl, bh[n], acc[n], 0, 0, 0);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                if (jl + 1 == jh) {
-                    if (has_next) stash(nbf, nhf);
-                    __syncthreads();  // the next half is stored and this one is read
-                }
+                for (int u = 0; u < NG; ++u) v[u] = (Ms + static_cast<int64_t>(__builtin_amdgcn_readlane(cell, u)) * S::CH)[static_cast<unsigned>(lane)];
             }
+            return;
         }
-        // add the odd-k-step sums to the even ones through LDS (B is no longer needed)
-        static_assert(MT * NT * 16 * 64 * sizeof(float) <= sizeof(sB), "partial sums must fit in the B buffers");
-        float *red = reinterpret_cast<float *>(&sB[0][0][0][0][0]);
-        if (kw == 1)
 #pragma unroll
-            for (int n = 0; n < NW; ++n)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) red[((mt * NT + n) * 16 + r) * 64 + lane] = acc[n][r];
-        __syncthreads();
-        if (kw == 1) return;  // no barrier follows
-#pragma unroll
-        for (int n = 0; n < NW; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[n][r] += red[((mt * NT + n) * 16 + r) * 64 + lane];
-    } else {
-        // Software pipeline, kept in place by scheduling barriers: during k-step q
-        // the A fragments of q + 1 .. q + PF and the B fragments of q + 1 are in
-        // flight.  The next half is gathered at the first k-step of a half, after
-        // that k-step's A loads, and stored at the fourth (vector loads complete in
-        // issue order, so the A loads issued after the gather already wait for it
-        // there).
-        // operator of flat k-step q: step q / NKS, k-step q % NKS
-        auto op_of = [&](int q) -> int { return __builtin_amdgcn_readfirstlane(s_o[q / NKS]); };
-        bf16x8 ah[PF], al[PF];  // A of k-steps q .. q + PF - 1
-    #pragma unroll
-        for (int i = 0; i < PF; ++i) {
-            const int o = op_of(i);
-            ah[i] = afrag(o, i % NKS, 0);
-            al[i] = afrag(o, i % NKS, 1);
+        for (int u = 0; u < NG; ++u) {
+            v[u] = make_uint4(0, 0, 0, 0);
+            const int t = (wv + S::NW * u) * S::TPI + sub;
+            if (sub < S::TPI && t < TB && ((s_nm[dn + t] >> qs) & 1)) v[u] = Ms[static_cast<int64_t>(s_nc[dn + t] + qs) * S::CH + ch];
         }
-        bf16x8 bh[NW], bl[NW];
-        bfrag(0, 0, bh, bl);
-        for (int st = 0; st < 189; ++st) {
-            asm volatile("" : "+v"(lb));  // recompute the B offsets per step rather than hold them all
-    #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) {
-                const int h = ks < KH0 ? 0 : 1;             // half of this k-step
-                const int ksl = ks - h * KH0, kh = h ? NKS - KH0 : KH0;
-                const int bf = NH == 2 ? h : (st & 1);      // its buffer
-                const int nst = (NH == 2 && h == 0) ? st : st + 1, nhf = (NH == 2 && h == 0) ? 1 : 0;  // the next half
-                const int nbf = NH == 2 ? nhf : ((st + 1) & 1);
-                const bool has_next = nst < 189;
-                const int q = st * NKS + ks;
-                const bf16x8 ch = ah[0], cl = al[0];
-    #pragma unroll
-                for (int i = 0; i + 1 < PF; ++i) {
-                    ah[i] = ah[i + 1];
-                    al[i] = al[i + 1];
-                }
-                if (q + PF < TOT) {
-                    const int o = op_of(q + PF);
-                    ah[PF - 1] = afrag(o, (ks + PF) % NKS, 0);
-                    al[PF - 1] = afrag(o, (ks + PF) % NKS, 1);
-                }
-                if (ksl == 0 && has_next) gather(nst, nhf);
-                bf16x8 nh[NW], nl[NW];
-                if (ksl + 1 < kh) bfrag(bf, ksl + 1, nh, nl);
-                if (ksl == (kh - 1 < 3 ? kh - 1 : 3) && has_next) stash(nbf, nhf);
-                if (ksl + 1 == kh) {
-                    // this half's B is in registers and the next half is stored:
-                    // one barrier, then the first fragments of the next half
-                    __syncthreads();
-                    if (has_next) bfrag(nbf, 0, nh, nl);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-    #pragma unroll
-                for (int n = 0; n < NW; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, bh[n], acc[n], 0, 0, 0);
-    #pragma unroll
-                for (int n = 0; n < NW; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ch, bl[n], acc[n], 0, 0, 0);
-    #pragma unroll
-                for (int n = 0; n < NW; ++n) acc[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(cl, bh[n], acc[n], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
-    #pragma unroll
-                for (int n = 0; n < NW; ++n) {
-                    bh[n] = nh[n];
-                    bl[n] = nl[n];
-                }
-            }
-        }
+    };
+    const uint4 *Brow = sM + (wc * 16 * S::NC + col) * S::SK + quad;
+    constexpr int PF = P < 10 ? 1 : 2;  // k-steps of operator in flight (above)
+    bf16x8 an[PF][S::RW][2];
+    if (hi > lo) {
+#pragma unroll
+        for (int i = 0; i < PF; ++i) load_a(lo, i, an[i]);
+        gather(lo);
     }
-    // C[8(r/4) + 4(l/32) + r%4][l%32] of n-tile n -> row of this m-tile, target 32 n + l%32
+    for (int li = lo; li < hi; ++li) {
 #pragma unroll
-    for (int n = 0; n < NW; ++n) {
-        const int t = 32 * (n0 + n) + (lane & 31);
-        const int pi = chunk * TB + t;
-        const int32_t P0 = pi < nparents ? parents[pi] : -1;
-        if (P0 < 0) continue;
-        const int32_t tgt = child[P0] + qt;
-        if (count[tgt] == 0) continue;
+        for (int u = 0; u < NG; ++u) {
+            const int t = (wv + S::NW * u) * S::TPI + sub;
+            const uint32_t m = S::TPI == 1 && (dead >> u & 1) ? 0u : ~0u;
+            if (sub < S::TPI && t < TB) sM[t * S::SK + ch] = make_uint4((v[u].x ^ sg[0]) & m, (v[u].y ^ sg[1]) & m, (v[u].z ^ sg[2]) & m, (v[u].w ^ sg[3]) & m);
+        }
+        if (li + 1 < hi) gather(li + 1);  // on its way during the products
+        __syncthreads();  // the multipoles of this offset are in LDS
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int row = mt * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-            if (row < K) L[static_cast<int64_t>(tgt) * ldk + row] = acc[n][r] * s_sgn[row];
+        for (int ks = 0; ks < S::KS; ++ks) {
+            bf16x8 a[S::RW][2];
+#pragma unroll
+            for (int r = 0; r < S::RW; ++r) {
+                a[r][0] = an[0][r][0], a[r][1] = an[0][r][1];
+#pragma unroll
+                for (int i = 0; i + 1 < PF; ++i) an[i][r][0] = an[i + 1][r][0], an[i][r][1] = an[i + 1][r][1];
+            }
+            if (ks + PF < S::KS)
+                load_a(li, ks + PF, an[PF - 1]);
+            else if (li + 1 < hi)
+                load_a(li + 1, ks + PF - S::KS, an[PF - 1]);
+#pragma unroll
+            for (int n = 0; n < S::NC; ++n) {
+                const bf16x8 bh = __builtin_bit_cast(bf16x8, Brow[16 * n * S::SK + 4 * ks]);
+                const bf16x8 bl = __builtin_bit_cast(bf16x8, Brow[16 * n * S::SK + 4 * ks + S::LD / 8]);
+#pragma unroll
+                for (int r = 0; r < S::RW; ++r) {
+                    if (S::NT % S::WR != 0 && r == S::RW - 1 && wr + S::WR * r >= S::NT) continue;
+                    acc[r][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][0], bh, acc[r][n], 0, 0, 0);
+                    acc[r][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][0], bl, acc[r][n], 0, 0, 0);
+                    acc[r][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[r][1], bh, acc[r][n], 0, 0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_s_setprio(0);
+        __syncthreads();  // every wavefront has read the multipoles
+    }
+    // D: lane holds rows 4 quad .. 4 quad + 3 of a tile for target col
+#pragma unroll
+    for (int r = 0; r < S::RW; ++r) {
+        const int tile = wr + S::WR * r, r0 = 16 * tile + 4 * quad;
+        if (tile >= S::NT) continue;
+#pragma unroll
+        for (int n = 0; n < S::NC; ++n) {
+            const int ti = (wc * S::NC + n) * 16 + col;
+            const int32_t t = tgt[ti];
+            if (t < 0) continue;
+            f32x4 x = acc[r][n];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (r0 + e < S::K && m2l_mirror_sign(qt, r0 + e) < 0) x[e] = -x[e];
+            float *dst = nsplit == 1 ? L + static_cast<int64_t>(t) * S::LD
+                                     : part + (static_cast<int64_t>(sp) * 8 * nparents + static_cast<int64_t>(chunk * TB + ti) * 8 + qt) * S::LD;
+            *reinterpret_cast<f32x4 *>(dst + r0) = x;
         }
     }
 }
@@ -629,26 +504,26 @@ void launch_ml(Ctx &c, const int32_t *ids, int64_t n, bool m2m) {
 
 template <int P>
 void launch_split(Ctx &c, const int32_t *parents, int np) {
-    constexpr int K = (P + 1) * (P + 1);
-    constexpr int NT = 4, NG = 2;  // 128 targets, 12 wavefronts: 3 per SIMD
-    constexpr bool KS = ks_of(K) >= 3;
-    const unsigned grid = 8 * ceil_div(np, 32 * NT);  // one block per (parent chunk, child octant)
-    k_m2l_split<P, NT, NG, KS><<<grid, 64 * NG * mt_m2l(K), 0, c.stream>>>(parents, np, c.t.child, c.t.count, c.t.nbr27,
-                                                                     reinterpret_cast<const uint4 *>(c.msplit.p), c.L32,
-                                                                     reinterpret_cast<const bf16x8 *>(c.opsplit.p), c.ldk);
+    using S = SplitShape<P>;
+    if (c.ldk != S::LD) throw Error(1, "split M2L: the coefficient stride must be K rounded up to 16");
+    const unsigned grid = 8 * ceil_div(np, S::TB);  // one block per (parent chunk, child octant)
+    const int nsplit = m2l_parts(grid, c.ncu);
+    float *part = m2l_part_sums(c, np, nsplit);
+    k_m2l_split<P><<<grid * nsplit, 64 * S::NW, 0, c.stream>>>(parents, np, c.t.child, c.t.count, c.t.nbr27, reinterpret_cast<const uint4 *>(c.msplit.p),
+                                                             c.L32, reinterpret_cast<const bf16x8 *>(c.opsplit.p), nsplit, part);
     VG_LAUNCH_CHECK();
+    m2l_add_parts(c, parents, np, nsplit, part);
 }
 
 }  // namespace
 
 void m2l_split_operators(Ctx &c, int nvec) {
-    const int MT = mt_of(c.K), NKS = ks_of(c.K), MTL = mt_m2l(c.K);
+    const int MT = mt_of(c.K), NKS = ks_of(c.K), NT = ks_of(c.K), KS = mt_of(c.K);  // (16-row tiles, 32-column steps)
     const int64_t per = static_cast<int64_t>(MT) * NKS * 64;
-    c.opsplit.ensure(static_cast<size_t>(343 * 2 * static_cast<int64_t>(MTL) * NKS * 64 * 8));
+    c.opsplit.ensure(static_cast<size_t>(343) * NT * KS * 128 * 8);
     // split mode runs M2M, M2L and L2L from the fragments: no FP32 copies
     (void)nvec;
-    k_split_ops<<<189 * MTL, 256, 32 * (16 * NKS + 1) * sizeof(double), c.stream>>>(c.ops_sel, c.op64, c.K, reinterpret_cast<__bf16 *>(c.opsplit.p),
-                                                                                  MTL, NKS);
+    k_split_ops<<<189 * NT, 256, 16 * (32 * KS + 1) * sizeof(double), c.stream>>>(c.ops_sel, c.op64, c.K, reinterpret_cast<__bf16 *>(c.opsplit.p), NT, KS);
     c.opsplit_ml.ensure(static_cast<size_t>(16 * 3 * per * 8));
     k_split_ops_ml<<<ceil_div(16 * per, 256), 256, 0, c.stream>>>(c.op64, c.K, reinterpret_cast<__bf16 *>(c.opsplit_ml.p), MT, NKS);
     VG_LAUNCH_CHECK();
@@ -677,7 +552,6 @@ void fmm_m2l_split_list(Ctx &c, const int32_t *parents, int np) {
     if (np <= 0) return;
     const int64_t nc = c.t.ncells;
     c.msplit.ensure(static_cast<size_t>(nc) * 2 * c.ldk);
-    if (c.ldk % 16 != 0) throw Error(1, "split M2L: the coefficient stride must be a multiple of 16");
     k_split_m<<<ceil_div(nc, SPLIT_CELLS), 256, 0, c.stream>>>(reinterpret_cast<const float4 *>(c.M32.p), nc, c.ldk,
                                                              reinterpret_cast<uint2 *>(c.msplit.p));
     VG_LAUNCH_CHECK();
