@@ -323,16 +323,18 @@ int vipp_mlp_train(int32_t device, float *params, const float *x, const float *t
         net.par.ensure(NPAR);
         VG_HIP(hipMemcpyAsync(net.par.p, params, NPAR * sizeof(float), hipMemcpyHostToDevice, st.s));
         net.set_params(st.s, net.par);
-        vg::DevBuf<float> xd, td, wd, bx, bt, bw, gd;
+        vg::DevBuf<float> xd, td, wd, sse;
         vg::DevBuf<uint32_t> idx;
-        xd.ensure(n * IN), td.ensure(n * OUT), idx.ensure(n), gd.ensure(NPAR);
+        xd.ensure(n * IN), td.ensure(n * OUT), idx.ensure(n);
         const int64_t B = std::min<int64_t>(batch, n);
-        bx.ensure(B * IN), bt.ensure(B * OUT);
+        std::vector<float> terms(static_cast<size_t>(n / B * Net::loss_terms(B) + Net::loss_terms(n % B)));  // squared errors of an epoch's batches
+        std::vector<double> wsums;
+        sse.ensure(terms.size());
         VG_HIP(hipMemcpyAsync(xd.p, x, n * IN * sizeof(float), hipMemcpyHostToDevice, st.s));
         VG_HIP(hipMemcpyAsync(td.p, t, n * OUT * sizeof(float), hipMemcpyHostToDevice, st.s));
         if (w) {
             for (int64_t i = 0; i < n; ++i) need(std::isfinite(w[i]) && w[i] >= 0, VIPP_GRAV_E_INVALID, "sample weights must be finite and >= 0");
-            wd.ensure(n), bw.ensure(B);
+            wd.ensure(n);
             VG_HIP(hipMemcpyAsync(wd.p, w, n * sizeof(float), hipMemcpyHostToDevice, st.s));
         }
         std::vector<uint32_t> perm(static_cast<size_t>(n));
@@ -346,21 +348,32 @@ int vipp_mlp_train(int32_t device, float *params, const float *x, const float *t
             }
             VG_HIP(hipMemcpyAsync(idx.p, perm.data(), n * sizeof(uint32_t), hipMemcpyHostToDevice, st.s));
             const float lr_e = lr * (0.05f + 0.95f * 0.5f * (1.0f + std::cos(3.14159265358979f * static_cast<float>(e) / static_cast<float>(epochs))));
-            double sum = 0, wall = 0;
+            // the batches follow each other on the device; their losses come back once per epoch
+            wsums.clear();
+            int64_t nt = 0;
             for (int64_t off = 0; off < n; off += B) {
                 const int64_t nb = std::min<int64_t>(B, n - off);
-                gather_rows(st.s, xd, IN, idx.p + off, nb, bx);
-                gather_rows(st.s, td, OUT, idx.p + off, nb, bt);
                 double wsum = static_cast<double>(nb);
                 if (w) {
-                    gather_rows(st.s, wd, 1, idx.p + off, nb, bw);
                     wsum = 0;
                     for (int64_t i = 0; i < nb; ++i) wsum += w[perm[static_cast<size_t>(off + i)]];
-                    if (!(wsum > 0)) continue;  // a batch of zero-weight rows carries no gradient
                 }
-                sum += static_cast<double>(net.loss_grad(st.s, bx, bt, w ? bw.p : nullptr, wsum, nb, gd)) * wsum;
+                wsums.push_back(wsum);
+                if (!(wsum > 0)) continue;  // a batch of zero-weight rows carries no gradient
+                net.train_step(st.s, xd, td, w ? wd.p : nullptr, idx.p + off, wsum, nb, lr_e, ++step, sse.p + nt);
+                nt += Net::loss_terms(nb);
+            }
+            if (nt > 0) VG_HIP(hipMemcpyAsync(terms.data(), sse.p, nt * sizeof(float), hipMemcpyDeviceToHost, st.s));
+            VG_HIP(hipStreamSynchronize(st.s));  // perm and terms are free for the next epoch
+            double sum = 0, wall = 0;
+            nt = 0;
+            for (int64_t off = 0, k = 0; off < n; off += B, ++k) {
+                const double wsum = wsums[static_cast<size_t>(k)];
+                if (!(wsum > 0)) continue;
+                double s = 0;
+                for (int64_t i = Net::loss_terms(std::min<int64_t>(B, n - off)); i > 0; --i) s += terms[static_cast<size_t>(nt++)];
+                sum += static_cast<double>(static_cast<float>(s / (wsum * OUT))) * wsum;
                 wall += wsum;
-                net.adam_step(st.s, gd, lr_e, ++step);
             }
             if (epoch_loss) epoch_loss[e] = static_cast<float>(wall > 0 ? sum / wall : 0.0);
         }

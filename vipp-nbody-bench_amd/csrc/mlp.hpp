@@ -17,16 +17,22 @@ struct Net {
     DevBuf<_Float16> frag;    // FP16 weights in MFMA A-operand order
     // training state
     DevBuf<float> m, v;       // Adam moments
-    DevBuf<float> y, x16, z1, a1, z2, a2, dy, dz1, dz2, sse;
+    DevBuf<float> x16, a1, a2, dy, dz1, dz2;
 
     void set_params(hipStream_t st, const float *par_dev);  // copy (device) + pack
     void forward(hipStream_t st, const float *x, int64_t n, float *y) const;
     // (weighted) mean squared error and its gradient; w may be null (all 1), wsum = sum of w
     float loss_grad(hipStream_t st, const float *x, const float *t, const float *w, double wsum, int64_t n, float *grad);
-    void adam_step(hipStream_t st, const float *grad, float lr, int step);
-};
+    // One Adam step (number `step`, from 1) on the rows idx of x, t and w (w may be
+    // null, wsum is the sum of the weights).  sse gets the loss_terms(n) partial
+    // sums of the squared errors before the step, in stream order.
+    void train_step(hipStream_t st, const float *x, const float *t, const float *w, const uint32_t *idx, double wsum, int64_t n, float lr, int step,
+                    float *sse);
+    static int64_t loss_terms(int64_t n);
 
-void gather_rows(hipStream_t st, const float *src, int w, const uint32_t *idx, int64_t n, float *dst);
+  private:
+    void activations(hipStream_t st, const float *x, const float *t, const float *w, const uint32_t *idx, double wsum, int64_t n, float *sse);
+};
 
 }  // namespace mlp
 }  // namespace vg
