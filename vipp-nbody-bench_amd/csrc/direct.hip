@@ -21,12 +21,50 @@ namespace {
 
 constexpr int DT = 256;  // threads per block and sources per LDS tile
 
+// One source's terms as the reference forms them, for any distance.
+template <bool POT>
+__device__ inline void add_exact(double dx, double dy, double dz, double Gm, double m, double eps2, double *s) {
+    const double r2 = dx * dx + dy * dy + dz * dz + eps2;
+    const double r = sqrt(r2);
+    const double gm = Gm / (r2 * r);
+    s[0] += gm * dx, s[1] += gm * dy, s[2] += gm * dz;
+    if (POT) s[3] += m / r;
+}
+
+// The same from v_rsq_f64's y (2^-24 at worst): with e = 1 - r2 y^2,
+// r2^(-3/2) = y^3 (1 + 3/2 e + 15/8 e^2 + O(e^3)) and 1 / r = y (1 + e / 2 +
+// 3/8 e^2 + ..), e^3 below 2^-69.  A correctly rounded square root and quotient
+// take three times the instructions.  r2 = 0 and r2 = inf give NaN (see below).
+template <bool POT>
+__device__ inline void add_fast(double dx, double dy, double dz, double r2, double gm, double m, double *s) {
+    const double y = __builtin_amdgcn_rsq(r2);
+    const double yy = y * y;
+    const double e = fma(-r2, yy, 1.0);
+    const double c = (y * gm) * yy;
+    const double f = fma(c * e, fma(e, 1.875, 1.5), c);
+    s[0] = fma(f, dx, s[0]), s[1] = fma(f, dy, s[1]), s[2] = fma(f, dz, s[2]);
+    if (POT) s[3] = fma(m, fma(y * e, fma(e, 0.375, 0.5), y), s[3]);
+}
+
 // bad (may be null): set to 1 when a target index lies outside [0, n); such
-// a target is skipped (the host-side entry point checks indices beforehand)
+// a target is skipped (the host-side entry point checks indices beforehand).
+//
+// Bound by FP64 issue: 16 operations at 4.6 cycles and one v_rsq_f64 (16) for
+// 64 pairs.  4096 targets of 1M sources: 6.2 -> 2.9 ms, 65,536 of 100,000: 9.7 ->
+// 4.5 ms (sources through scalar loads instead of LDS: 0.3 ms more).  A target of
+// its own (solver_ref_naive.hpp:111-113) costs something only in the tiles that
+// hold one of the wavefront's targets.  By the reference's operations are formed
+// a sum that is not finite (a source at the target's place without softening,
+// distances whose square overflows) and, so that a caller may compare with the
+// formula to the last bit, the sums over up to EXACT_N sources, where a call is its
+// launches and copies (128 of 128: 56 us, against 45; 256 of 256: 78 against 58).
+constexpr int64_t EXACT_N = 128;
+template <bool POT>
 __global__ __launch_bounds__(DT) void k_direct(const double *__restrict__ x, const double *__restrict__ masses, double mass, int64_t n,
-                                               const int64_t *__restrict__ idx, int64_t nidx, int64_t slice, double G, double eps2, int potential,
+                                               const int64_t *__restrict__ idx, int64_t nidx, int64_t slice, double G, double eps2,
                                                double *__restrict__ part, double *__restrict__ bad) {
-    __shared__ double sx[DT], sy[DT], sz[DT], sm[DT];
+    __shared__ double2 sxy[DT], szg[DT];  // (x, y), (z, G m)
+    __shared__ double sm[POT ? DT : 1];
     const int64_t k = blockIdx.x * static_cast<int64_t>(DT) + threadIdx.x;
     const int64_t i0 = k < nidx ? idx[k] : -1;
     const bool live = k < nidx && i0 >= 0 && i0 < n;
@@ -35,36 +73,46 @@ __global__ __launch_bounds__(DT) void k_direct(const double *__restrict__ x, con
     const double xi = live ? x[3 * i] : 0, yi = live ? x[3 * i + 1] : 0, zi = live ? x[3 * i + 2] : 0;
     const int64_t j0 = blockIdx.y * slice;
     const int64_t j1 = j0 + slice < n ? j0 + slice : n;
-    double ax = 0, ay = 0, az = 0, pt = 0;
+    double s[4] = {0, 0, 0, 0};
     for (int64_t b = j0; b < j1; b += DT) {
         __syncthreads();
         const int64_t j = b + threadIdx.x;
         if (j < j1) {
-            sx[threadIdx.x] = x[3 * j];
-            sy[threadIdx.x] = x[3 * j + 1];
-            sz[threadIdx.x] = x[3 * j + 2];
-            sm[threadIdx.x] = masses ? masses[j] : mass;
+            const double m = masses ? masses[j] : mass;
+            sxy[threadIdx.x] = make_double2(x[3 * j], x[3 * j + 1]);
+            szg[threadIdx.x] = make_double2(x[3 * j + 2], G * m);
+            if (POT) sm[threadIdx.x] = m;
         }
         __syncthreads();
         const int nt = j1 - b < DT ? static_cast<int>(j1 - b) : DT;
-        for (int u = 0; u < nt; ++u) {
-            if (b + u == i) continue;  // solver_ref_naive.hpp:111-113
-            const double dx = sx[u] - xi, dy = sy[u] - yi, dz = sz[u] - zi;
-            const double r2 = dx * dx + dy * dy + dz * dz + eps2;
-            const double r = sqrt(r2);
-            const double gm = G * sm[u] / (r2 * r);
-            ax += gm * dx;
-            ay += gm * dy;
-            az += gm * dz;
-            if (potential) pt += sm[u] / r;
+        const int self = i >= b && i < b + nt ? static_cast<int>(i - b) : -1;
+        if (n <= EXACT_N) {
+            for (int u = 0; u < nt; ++u)
+                if (u != self) add_exact<POT>(sxy[u].x - xi, sxy[u].y - yi, szg[u].x - zi, szg[u].y, POT ? sm[u] : 0.0, eps2, s);
+        } else if (__ballot(self >= 0) == 0) {
+#pragma unroll 4
+            for (int u = 0; u < nt; ++u) {
+                const double dx = sxy[u].x - xi, dy = sxy[u].y - yi, dz = szg[u].x - zi;
+                add_fast<POT>(dx, dy, dz, fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2))), szg[u].y, POT ? sm[u] : 0.0, s);
+            }
+        } else {
+            for (int u = 0; u < nt; ++u) {
+                const double dx = sxy[u].x - xi, dy = sxy[u].y - yi, dz = szg[u].x - zi;
+                const double r2 = u == self ? 1.0 : fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));  // adds 0 dx = 0
+                add_fast<POT>(dx, dy, dz, r2, szg[u].y, POT && u != self ? sm[u] : 0.0, s);
+            }
         }
     }
     if (k >= nidx) return;
+    if (live && !(isfinite(s[0]) && isfinite(s[1]) && isfinite(s[2]) && isfinite(s[3]))) {
+        s[0] = s[1] = s[2] = s[3] = 0;
+        for (int64_t j = j0; j < j1; ++j) {
+            const double m = masses ? masses[j] : mass;
+            if (j != i) add_exact<POT>(x[3 * j] - xi, x[3 * j + 1] - yi, x[3 * j + 2] - zi, G * m, m, eps2, s);
+        }
+    }
     double *o = part + (static_cast<int64_t>(blockIdx.y) * nidx + k) * 4;
-    o[0] = live ? ax : 0.0;
-    o[1] = live ? ay : 0.0;
-    o[2] = live ? az : 0.0;
-    o[3] = live ? pt : 0.0;
+    for (int c = 0; c < 4; ++c) o[c] = live ? s[c] : 0.0;
 }
 
 __global__ __launch_bounds__(256) void k_direct_sum(const double *__restrict__ part, int64_t nidx, int S, double *__restrict__ a,
@@ -103,8 +151,8 @@ void launch_direct(Ctx &c, const int64_t *idx, int64_t nidx, double *part, int64
     const int64_t slice = ceil_div(c.n, S);
     S = ceil_div(c.n, slice);
     const dim3 grid(ceil_div(nidx, DT), static_cast<unsigned>(S));
-    k_direct<<<grid, DT, 0, c.stream>>>(c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.n, idx, nidx, slice, c.G, c.eps * c.eps, pot ? 1 : 0,
-                                        part, bad);
+    (pot ? k_direct<true> : k_direct<false>)<<<grid, DT, 0, c.stream>>>(c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.n, idx, nidx, slice, c.G,
+                                                                        c.eps * c.eps, part, bad);
     VG_LAUNCH_CHECK();
     k_direct_sum<<<ceil_div(nidx, 256), 256, 0, c.stream>>>(part, nidx, static_cast<int>(S), a, pot);
     VG_LAUNCH_CHECK();
