@@ -164,8 +164,7 @@ struct Ctx {
 
     // P2P work items
     DevBuf<uint32_t> p2p_scal, p2p_nchunk, p2p_cls, p2p_src, p2p_item_off, p2p_local, p2p_pre, p2p_btot;
-    DevBuf<uint32_t> p2p_ticket;  // per leaf: work items of a split leaf that have finished
-    DevBuf<int64_t> p2p_items;  // int2 (leaf index, chunk) or, in FP32, 32-byte records
+    DevBuf<char> p2p_items;  // 32-byte records
     DevBuf<float> p2p_part32;
     DevBuf<double> p2p_part64;
 

@@ -10,13 +10,9 @@
 //
 // Work items: a plan kernel counts each non-empty leaf's sources and cuts them
 // into even chunks, so leaves with long inherited lists spread over many
-// wavefronts or blocks; each (leaf, chunk) is one item.
-//  * FP64 (k_p2p): one 256-thread block per item, which flattens its ranges in
-//    LDS, streams the chunk's sources through LDS tiles and gives each lane
-//    T = 1..6 targets, in groups of 8 to 64 lanes, by leaf-size class (the
-//    fewest idle lanes).
-//  * FP32 (k_p2p_mc): one wavefront per item, squared distances on the matrix
-//    cores.
+// wavefronts; each (leaf, chunk) is one item, for one wavefront.
+//  * FP32 (k_p2p_mc): squared distances on the matrix cores.
+//  * FP64 (k_p2p_f64): pairs by differences.
 // A leaf with one chunk writes its result; split leaves write partial sums,
 // which are added in chunk order (deterministic).  With a nonzero softening the
 // i == j term is exactly zero (dx = dy = dz = 0), so it needs no branch;
@@ -26,18 +22,7 @@
 namespace vg {
 namespace {
 
-constexpr int P2P_THREADS = 256;
 constexpr int MAXE = 27 * (MAXD + 1);
-constexpr uint32_t P2P_CHUNK = 16384;  // sources per work item (at most; 8192 and 32768 measured slower on the 4M Plummer input)
-
-// Lane layout of a leaf with nt targets and T targets per lane: groups of
-// TPW lanes, the smallest TPW in {8, 16, 32, 64} with TPW T >= nt (0: none).
-__host__ __device__ inline int tpw_for(uint32_t nt, int T) {
-    for (int tp = 8; tp <= 64; tp *= 2)
-        if (static_cast<uint32_t>(tp * T) >= nt) return tp;
-    return 0;
-}
-constexpr int TMAX = 6;  // targets per lane of the largest regular class
 
 // Sources per work item of a leaf cut into nch: even, in whole groups of 64.
 __host__ __device__ inline uint32_t chunk_len(uint32_t total, uint32_t nch) { return ((total + nch - 1) / nch + 63) / 64 * 64; }
@@ -54,235 +39,14 @@ struct Vec4<double> {
 };
 
 __device__ inline float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
-// 1/sqrt(x) in FP64: the hardware estimate refined by two Newton steps
-// y <- y + y (1 - x y^2) / 2, each squaring the relative error, so the result
-// is within a few ulps of the correctly rounded value (x > 0; x = 0 gives NaN,
-// which the self-pair select replaces)
+// 1/sqrt(x) in FP64: with e = 1 - x y^2 of the hardware's estimate y (2^-24 at
+// worst), y (1 + e / 2 + 3/8 e^2) is off by its roundings and less than 2^-69
+// (x > 0; x = 0 gives NaN, which the self-pair select replaces)
 __device__ inline double rsq(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const double e = fma(-x, y * y, 1.0);
-        y = fma(y * e, 0.5, y);
-    }
-    return y;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x, y * y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
 }
-
-// Sources [src0, src1) of the leaf's flattened list against targets pt0 ..
-// pt0+nt-1.  out == nullptr: write the final G-scaled result to acc; else
-// write the raw partial sums to out[t].  UM (every particle has mass mu): the
-// pair terms leave the mass out and the sums are scaled by mu once.
-template <class R, bool SELF_GUARD, bool POT, bool UM, int T, class V4>
-__device__ __forceinline__ void p2p_leaf(V4 *tile, V4 *red, const uint32_t *ent_start, const uint32_t *ent_off, int E, uint32_t src0, uint32_t src1,
-                                         uint32_t nt, uint32_t pt0, const V4 *__restrict__ xs, R eps2, R G, R mu, V4 *__restrict__ acc,
-                                         V4 *__restrict__ out) {
-    constexpr int CH = sizeof(R) == 4 ? 1024 : 512;
-    const int tid = threadIdx.x;
-    const int TPW = tpw_for(nt, T);  // nt <= 64 T here
-    const int lane = tid & 63, wave = tid >> 6;
-    const int groups = 64 / TPW;
-    const int nsl = 4 * groups;
-    const int sl = wave * groups + lane / TPW;
-    const int ti = lane % TPW;
-    V4 xi[T];
-    R ax[T], ay[T], az[T], ph[T];
-#pragma unroll
-    for (int q = 0; q < T; ++q) {
-        const uint32_t t = ti + q * TPW;
-        xi[q] = t < nt ? xs[pt0 + t] : V4{R(1e30), R(1e30), R(1e30), R(0)};
-        ax[q] = ay[q] = az[q] = ph[q] = 0;
-    }
-    for (uint32_t c0 = src0; c0 < src1; c0 += CH) {
-        const uint32_t len = min(static_cast<uint32_t>(CH), src1 - c0);
-#pragma unroll
-        for (int u = 0; u < CH / P2P_THREADS; ++u) {
-            const uint32_t f = tid + u * P2P_THREADS;
-            const uint32_t g = c0 + min(f, len - 1);
-            int lo = 0;  // last e with ent_off[e] <= g (fixed trip count: E <= 1023)
-#pragma unroll
-            for (int step = 512; step > 0; step >>= 1)
-                if (lo + step <= E && ent_off[lo + step] <= g) lo += step;
-            if (f < len) tile[f] = xs[ent_start[lo] + (g - ent_off[lo])];
-        }
-        __syncthreads();
-        // slice sl takes the contiguous range [b0, b1) of this tile
-        const uint32_t per = (len + nsl - 1) / nsl;
-        const uint32_t b0 = min(len, sl * per), b1 = min(len, b0 + per);
-        uint32_t j = b0;
-        for (; j + 4 <= b1; j += 4) {
-            V4 sj[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) sj[u] = tile[j + u];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int q = 0; q < T; ++q) {
-                    const R dx = sj[u].x - xi[q].x, dy = sj[u].y - xi[q].y, dz = sj[u].z - xi[q].z;
-                    const R r2 = eps2 + dx * dx + dy * dy + dz * dz;
-                    R rinv = rsq(r2);
-                    if (SELF_GUARD) rinv = r2 > R(0) ? rinv : R(0);
-                    const R mr = UM ? rinv : sj[u].w * rinv;
-                    const R mr3 = mr * rinv * rinv;
-                    ax[q] += mr3 * dx;
-                    ay[q] += mr3 * dy;
-                    az[q] += mr3 * dz;
-                    if (POT) ph[q] += mr;
-                }
-        }
-        for (; j < b1; ++j) {
-            const V4 sj = tile[j];
-#pragma unroll
-            for (int q = 0; q < T; ++q) {
-                const R dx = sj.x - xi[q].x, dy = sj.y - xi[q].y, dz = sj.z - xi[q].z;
-                const R r2 = eps2 + dx * dx + dy * dy + dz * dz;
-                R rinv = rsq(r2);
-                if (SELF_GUARD) rinv = r2 > R(0) ? rinv : R(0);
-                const R mr = UM ? rinv : sj.w * rinv;
-                const R mr3 = mr * rinv * rinv;
-                ax[q] += mr3 * dx;
-                ay[q] += mr3 * dy;
-                az[q] += mr3 * dz;
-                if (POT) ph[q] += mr;
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int q = 0; q < T; ++q) red[q * P2P_THREADS + tid] = V4{ax[q], ay[q], az[q], ph[q]};
-    __syncthreads();
-    for (uint32_t t = tid; t < nt; t += P2P_THREADS) {
-        // target t lives in lane-slot (q, ti) of every slice
-        const int q = static_cast<int>(t / TPW), tl = static_cast<int>(t % TPW);
-        R sx = 0, sy = 0, sz = 0, sp = 0;
-        for (int s2 = 0; s2 < nsl; ++s2) {
-            const int owner = (s2 / groups) * 64 + (s2 % groups) * TPW + tl;
-            const V4 v = red[q * P2P_THREADS + owner];
-            sx += v.x;
-            sy += v.y;
-            sz += v.z;
-            sp += v.w;
-        }
-        if (UM) {
-            sx *= mu;
-            sy *= mu;
-            sz *= mu;
-            sp *= mu;
-        }
-        if (out) {
-            out[t] = V4{sx, sy, sz, sp};
-        } else {
-            if (POT && !SELF_GUARD) sp -= xs[pt0 + t].w * rsq(eps2);  // drop the m_i / eps self term
-            acc[pt0 + t] = V4{G * sx, G * sy, G * sz, sp};
-        }
-    }
-}
-
-// Lane layout: a wavefront holds 64/TPW groups of TPW lanes; the lanes of a
-// group take targets ti, ti+TPW, ... (up to TMAX per lane) and read the same
-// source at each step (an LDS broadcast).  The block's 4 x (64/TPW) groups
-// split every staged tile of sources.
-template <class R, bool SELF_GUARD, bool POT, bool UM, int T>
-__global__ __launch_bounds__(P2P_THREADS) void k_p2p(const int2 *__restrict__ items, const int32_t *__restrict__ leaves, const uint32_t *__restrict__ nchunk,
-                                                     const uint32_t *__restrict__ item_off, const int8_t *__restrict__ level,
-                                                     const uint32_t *__restrict__ start, const uint32_t *__restrict__ count, const int32_t *__restrict__ anc,
-                                                     const int32_t *__restrict__ ni, const int32_t *__restrict__ ni_cnt,
-                                                     const typename Vec4<R>::T *__restrict__ xs, R eps2, R G, R mu, typename Vec4<R>::T *__restrict__ acc,
-                                                     typename Vec4<R>::T *__restrict__ partial, uint32_t pstride, uint32_t *__restrict__ ticket) {
-    using V4 = typename Vec4<R>::T;
-    constexpr int CH = sizeof(R) == 4 ? 1024 : 512;
-    constexpr int TR = T <= TMAX ? T : 4;  // T = TMAX + 1: leaves in batches of 256 targets, 4 per lane
-    // source tiles while streaming, per-lane partial sums after (a barrier apart)
-    __shared__ V4 buf[CH > P2P_THREADS * TR ? CH : P2P_THREADS * TR];
-    V4 *tile = buf;
-    __shared__ uint32_t ent_start[MAXE];
-    __shared__ uint32_t ent_off[MAXE + 1];
-    __shared__ int32_t an[MAXD + 1];
-    __shared__ int32_t an_off[MAXD + 2];
-    V4 *red = buf;
-
-    const int2 item = items[blockIdx.x];  // (leaf index, chunk)
-    const int32_t c = leaves[item.x];
-    const int lev = level[c];
-    const uint32_t nt = count[c], pt0 = start[c];
-    const int tid = threadIdx.x;
-    if (tid <= lev) an[tid] = anc[static_cast<int64_t>(c) * (MAXD + 1) + tid];
-    __syncthreads();
-    if (tid < 64) {  // entry counts per ancestor, scanned by one wavefront
-        const int cntl = tid <= lev ? ni_cnt[an[tid]] : 0;
-        int incl = cntl;
-        for (int d = 1; d < 32; d <<= 1) {
-            const int o = __shfl_up(incl, d, 64);
-            if ((tid & 63) >= d) incl += o;
-        }
-        if (tid <= lev) an_off[tid] = incl - cntl;
-        if (tid == lev) an_off[lev + 1] = incl;
-    }
-    __syncthreads();
-    const int E = an_off[lev + 1];
-    for (int e = tid; e < E; e += P2P_THREADS) {
-        int l = 0;
-        while (an_off[l + 1] <= e) ++l;
-        const int32_t cell = ni[27 * static_cast<int64_t>(an[l]) + (e - an_off[l])];
-        ent_start[e] = start[cell];
-        ent_off[e + 1] = count[cell];
-    }
-    __syncthreads();
-    if (tid < 64) {  // prefix sum of the entry sizes
-        uint32_t carry = 0;
-        for (int b = 0; b < E; b += 64) {
-            const uint32_t v = (b + tid < E) ? ent_off[b + tid + 1] : 0u;
-            uint32_t incl = v;
-            for (int d = 1; d < 64; d <<= 1) {
-                const uint32_t o = __shfl_up(incl, d, 64);
-                if (tid >= d) incl += o;
-            }
-            if (b + tid < E) ent_off[b + tid + 1] = carry + incl;
-            carry += __shfl(incl, 63, 64);
-        }
-        if (tid == 0) ent_off[0] = 0;
-    }
-    __syncthreads();
-    const uint32_t total = ent_off[E];
-    const uint32_t per = chunk_len(total, nchunk[item.x]);
-    const uint32_t src0 = min(total, item.y * per), src1 = min(total, src0 + per);
-    V4 *out = nchunk[item.x] > 1 ? partial + static_cast<size_t>(item_off[item.x] + item.y) * pstride : nullptr;
-    if constexpr (T <= TMAX) {
-        p2p_leaf<R, SELF_GUARD, POT, UM, T>(tile, red, ent_start, ent_off, E, src0, src1, nt, pt0, xs, eps2, G, mu, acc, out);
-    } else {  // leaves above 64 TMAX points: batches of 256 targets, each streaming the sources again
-        for (uint32_t tb = 0; tb < nt; tb += 256) {
-            p2p_leaf<R, SELF_GUARD, POT, UM, 4>(tile, red, ent_start, ent_off, E, src0, src1, min(nt - tb, 256u), pt0 + tb, xs, eps2, G, mu, acc,
-                                                out ? out + tb : nullptr);
-            __syncthreads();
-        }
-    }
-    if (out) {
-        // A leaf split over several work items: the block that finishes last
-        // adds the partial sums in chunk order (the same order every run).
-        __shared__ uint32_t s_last;
-        const uint32_t nch = nchunk[item.x];
-        __threadfence();  // this block's partial sums are visible device-wide
-        __syncthreads();
-        if (tid == 0) s_last = atomicAdd(&ticket[item.x], 1u) == nch - 1 ? 1u : 0u;
-        __syncthreads();
-        if (s_last) {
-            __threadfence();  // and the other blocks' ones to this block
-            const V4 *pk = partial + static_cast<size_t>(item_off[item.x]) * pstride;
-            for (uint32_t t = tid; t < nt; t += P2P_THREADS) {
-                R sx = 0, sy = 0, sz = 0, sp = 0;
-                for (uint32_t q = 0; q < nch; ++q) {
-                    const V4 v = pk[static_cast<size_t>(q) * pstride + t];
-                    sx += v.x;
-                    sy += v.y;
-                    sz += v.z;
-                    sp += v.w;
-                }
-                if (POT && !SELF_GUARD) sp -= xs[pt0 + t].w * rsq(eps2);
-                acc[pt0 + t] = V4{G * sx, G * sy, G * sz, sp};
-            }
-        }
-    }
-}
-
 
 // ---- FP32: squared distances on the matrix cores -------------------------
 //
@@ -324,6 +88,11 @@ constexpr int mc_tiles(bool pot) { return pot ? 5 : 6; }
 // particles), less with few leaves, and at most 64 groups, one per lane of the
 // entry table.
 constexpr uint32_t MC_COST = 512, MC_MINCOST = 16;
+// FP64 items: 4 tiles at most (28 registers a tile, 6 spilled), and smaller ones with
+// fewer leaves than 64 per CU (16, 32 and 64: 198, 134 and 111 us at 16384 particles in leaves of
+// 18; least costs of 4, 8 and 16 alike).
+constexpr int F64_TILES = 4, F64_LEAVES = 64;
+constexpr uint32_t F64_MINCOST = 16;
 constexpr uint32_t MC_CHUNK = 64 * 64;
 // A leaf's targets go to items of at most mt tiles, evenly.
 __host__ __device__ inline uint32_t mc_batches(uint32_t nt, int mt) { return ((nt + 15) / 16 + mt - 1) / mt; }
@@ -363,12 +132,104 @@ struct alignas(32) McWork {
     uint32_t t0;
 };
 
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Where a work item's sources lie: lane g has, of the item's group of 64 sources g,
+// the entry of the first one and where entries begin in it.
+struct Sources {
+    uint32_t mlo, mhi;  // the begins, from the group's second source on
+    int rank;           // entry of the group's first source
+};
+__device__ __forceinline__ Sources lay_out_entries(const McWork &wk, int32_t *delta, uint64_t *mask, const uint32_t *__restrict__ start,
+                                                   const uint32_t *__restrict__ count, const int32_t *__restrict__ anc, const int32_t *__restrict__ ni,
+                                                   const int32_t *__restrict__ ni_cnt) {
+    const int lane = threadIdx.x, lev = wk.level;
+    const int32_t c = wk.cell;
+    Sources I;
+    mask[lane] = 0;
+    // the leaf's NI list: its ancestors' own entries, root first; lane l has ancestor l
+    const int32_t an = lane <= lev ? anc[static_cast<int64_t>(c) * (MAXD + 1) + lane] : 0;
+    const int an_cnt = lane <= lev ? ni_cnt[an] : 0;
+    int an_end = an_cnt;
+    for (int d = 1; d < 32; d <<= 1) {
+        const int o = __shfl_up(an_end, d, 64);
+        if (lane >= d) an_end += o;
+    }
+    const int E = __builtin_amdgcn_readlane(an_end, lev);
+    const uint64_t live = __ballot(an_cnt > 0);
+    auto entry = [&](int e, uint32_t &st, uint32_t &cn) {  // particle range of entry e
+        int l = 0;
+        for (uint64_t w = live; w; w &= w - 1) {  // the last ancestor with entries whose first one is <= e
+            const int k = __builtin_ctzll(w);
+            if (__builtin_amdgcn_readlane(an_end - an_cnt, k) <= e) l = k;
+        }
+        const int32_t a = __shfl(an, l, 64);
+        const int o = e - __shfl(an_end - an_cnt, l, 64);
+        st = cn = 0;
+        if (e < E) {
+            const int32_t cell = ni[27 * static_cast<int64_t>(a) + o];
+            st = start[cell];
+            cn = count[cell];
+        }
+    };
+    // the entries that reach into [src0, src1), empty ones dropped, and where they begin in it
+    const uint32_t src0 = wk.src0, src1 = src0 + wk.len;
+    wave_lds_sync();
+    uint32_t carry = 0, st, cn;
+    int kept = 0;
+    entry(lane, st, cn);
+    for (int e0 = 0; e0 < E && carry < src1; e0 += 64) {
+        uint32_t nst = 0, ncn = 0;
+        if (e0 + 64 < E) entry(e0 + 64 + lane, nst, ncn);  // on its way while this run is laid out
+        uint32_t incl = cn;
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        const uint32_t off = carry + incl - cn;
+        const bool in = cn > 0 && off + cn > src0 && off < src1;
+        const uint64_t bal = __ballot(in);
+        if (in) {
+            delta[kept + __popcll(bal & ((1ull << lane) - 1))] = static_cast<int32_t>(st - (off - src0));
+            const uint32_t o = max(off, src0) - src0;
+            atomicOr(reinterpret_cast<unsigned long long *>(&mask[o >> 6]), 1ull << (o & 63));
+        }
+        kept += __popcll(bal);
+        carry += __builtin_amdgcn_readlane(incl, 63);
+        st = nst, cn = ncn;
+    }
+    wave_lds_sync();
+    {  // lane g: the entry of group g's first source, and the later begins shifted so that mbcnt counts them
+        const uint64_t m = mask[lane];
+        const int own = __popcll(m);
+        int incl = own;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(incl, d, 64);
+            if (lane >= d) incl += o;
+        }
+        I.rank = incl - own + static_cast<int>(m & 1) - 1;
+        I.mlo = static_cast<uint32_t>(m >> 1);
+        I.mhi = static_cast<uint32_t>(m >> 33);
+    }
+    wave_lds_sync();
+    return I;
+}
+// Particle of source `lane` of group g (the last one again past len).
+__device__ __forceinline__ int32_t source_of(const Sources &S, const int32_t *delta, int g, uint32_t len) {
+    const uint32_t lo = __builtin_amdgcn_readlane(S.mlo, g), hi = __builtin_amdgcn_readlane(S.mhi, g);
+    const int e = __builtin_amdgcn_readlane(S.rank, g) + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+    return delta[e] + static_cast<int32_t>(min(64u * g + threadIdx.x, len - 1));
+}
+
 // What a wavefront knows of its work item.
 struct McItem {
     const float4 *xs;     // sorted particles (x, y, z relative to the root centre, m)
     uint32_t len;         // sources
-    uint32_t mlo, mhi;    // lane g: where entries begin in group g (from its second source on)
-    int rank;             // lane g: entry of group g's first source
+    Sources src;
     uint32_t pt0;         // first target
     int nt;               // targets
     float cell;           // half diagonal of the leaf
@@ -376,12 +237,6 @@ struct McItem {
     bool um;              // one mass: left out here, the sums are scaled once
     bool big;             // squared distances may leave the FP32 range
 };
-
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // The item's T tiles of 16 targets against its sources; emit(t, v) gets target
 // t's sums (force xyz, potential), in one lane.
@@ -436,11 +291,7 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
     const float *Qw = reinterpret_cast<const float *>(S.Q);
     const f4 zero = {0, 0, 0, 0};
     // far pass: groups of 64 sources, near tiles put aside
-    auto source = [&](int g) {  // this lane's source of group g
-        const uint32_t lo = __builtin_amdgcn_readlane(I.mlo, g), hi = __builtin_amdgcn_readlane(I.mhi, g);
-        const int e = __builtin_amdgcn_readlane(I.rank, g) + __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
-        return I.xs[S.delta[e] + static_cast<int32_t>(min(64u * g + lane, I.len - 1))];
-    };
+    auto source = [&](int g) { return I.xs[source_of(I.src, S.delta, g, I.len)]; };  // this lane's source of group g
     uint32_t mynear = 0;  // lane g: near tiles of group g
     float4 nx = source(0);
     for (int g = 0; g < ng; ++g) {
@@ -547,8 +398,8 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
     auto near_source = [&](int j) {  // this lane's source of the near tiles 4 j .. 4 j + 3
         const int n = 4 * j + quad;
         const int tl = S.near[min(n, nn - 1)], g = tl >> 2, pos = 16 * (tl & 3) + col;
-        const uint64_t m = static_cast<uint64_t>(static_cast<uint32_t>(__shfl(static_cast<int>(I.mhi), g, 64))) << 32 | static_cast<uint32_t>(__shfl(static_cast<int>(I.mlo), g, 64));
-        const int e = __shfl(I.rank, g, 64) + __popcll(m & ((1ull << pos) - 1));
+        const uint64_t m = static_cast<uint64_t>(static_cast<uint32_t>(__shfl(static_cast<int>(I.src.mhi), g, 64))) << 32 | static_cast<uint32_t>(__shfl(static_cast<int>(I.src.mlo), g, 64));
+        const int e = __shfl(I.src.rank, g, 64) + __popcll(m & ((1ull << pos) - 1));
         const uint32_t f = 64u * g + pos;
         float4 v = I.xs[S.delta[e] + static_cast<int32_t>(min(f, I.len - 1))];
         if (I.um) v.w = 1.0f;
@@ -611,78 +462,12 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
     __shared__ McLds S;
     const McWork wk = items[blockIdx.x];
     const int32_t c = wk.cell;
-    const int lev = wk.level, lane = threadIdx.x;
+    const int lane = threadIdx.x;
     McItem I;
     I.nt = static_cast<int>(wk.nt);
     I.pt0 = wk.pt0;
     I.len = wk.len;
-    uint64_t *mask = reinterpret_cast<uint64_t *>(S.Q);
-    mask[lane] = 0;
-    // the leaf's NI list: its ancestors' own entries, root first; lane l has ancestor l
-    const int32_t an = lane <= lev ? anc[static_cast<int64_t>(c) * (MAXD + 1) + lane] : 0;
-    const int an_cnt = lane <= lev ? ni_cnt[an] : 0;
-    int an_end = an_cnt;
-    for (int d = 1; d < 32; d <<= 1) {
-        const int o = __shfl_up(an_end, d, 64);
-        if (lane >= d) an_end += o;
-    }
-    const int E = __builtin_amdgcn_readlane(an_end, lev);
-    const uint64_t live = __ballot(an_cnt > 0);
-    auto entry = [&](int e, uint32_t &st, uint32_t &cn) {  // particle range of entry e
-        int l = 0;
-        for (uint64_t w = live; w; w &= w - 1) {  // the last ancestor with entries whose first one is <= e
-            const int k = __builtin_ctzll(w);
-            if (__builtin_amdgcn_readlane(an_end - an_cnt, k) <= e) l = k;
-        }
-        const int32_t a = __shfl(an, l, 64);
-        const int o = e - __shfl(an_end - an_cnt, l, 64);
-        st = cn = 0;
-        if (e < E) {
-            const int32_t cell = ni[27 * static_cast<int64_t>(a) + o];
-            st = start[cell];
-            cn = count[cell];
-        }
-    };
-    // the entries that reach into [src0, src1), empty ones dropped, and where they begin in it
-    const uint32_t src0 = wk.src0, src1 = src0 + wk.len;
-    wave_lds_sync();
-    uint32_t carry = 0, st, cn;
-    int kept = 0;
-    entry(lane, st, cn);
-    for (int e0 = 0; e0 < E && carry < src1; e0 += 64) {
-        uint32_t nst = 0, ncn = 0;
-        if (e0 + 64 < E) entry(e0 + 64 + lane, nst, ncn);  // on its way while this run is laid out
-        uint32_t incl = cn;
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t o = __shfl_up(incl, d, 64);
-            if (lane >= d) incl += o;
-        }
-        const uint32_t off = carry + incl - cn;
-        const bool in = cn > 0 && off + cn > src0 && off < src1;
-        const uint64_t bal = __ballot(in);
-        if (in) {
-            S.delta[kept + __popcll(bal & ((1ull << lane) - 1))] = static_cast<int32_t>(st - (off - src0));
-            const uint32_t o = max(off, src0) - src0;
-            atomicOr(reinterpret_cast<unsigned long long *>(&mask[o >> 6]), 1ull << (o & 63));
-        }
-        kept += __popcll(bal);
-        carry += __builtin_amdgcn_readlane(incl, 63);
-        st = nst, cn = ncn;
-    }
-    wave_lds_sync();
-    {  // lane g: the entry of group g's first source, and the later begins shifted so that mbcnt counts them
-        const uint64_t m = mask[lane];
-        const int own = __popcll(m);
-        int incl = own;
-        for (int d = 1; d < 64; d <<= 1) {
-            const int o = __shfl_up(incl, d, 64);
-            if (lane >= d) incl += o;
-        }
-        I.rank = incl - own + static_cast<int>(m & 1) - 1;
-        I.mlo = static_cast<uint32_t>(m >> 1);
-        I.mhi = static_cast<uint32_t>(m >> 33);
-    }
-    wave_lds_sync();
+    I.src = lay_out_entries(wk, S.delta, reinterpret_cast<uint64_t *>(S.Q), start, count, anc, ni, ni_cnt);
     I.xs = xs;
     const double lx = bmin[3ll * c], ly = bmin[3ll * c + 1], lz = bmin[3ll * c + 2], ux = bmax[3ll * c], uy = bmax[3ll * c + 1], uz = bmax[3ll * c + 2];
     const float wx = static_cast<float>(ux - lx), wy = static_cast<float>(uy - ly), wz = static_cast<float>(uz - lz);
@@ -722,37 +507,151 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
         mc_pass<MT, POT>(I, S, emit);
 }
 
+// ---- FP64 ----------------------------------------------------------------
+//
+// One wavefront per work item as above; pairs by differences, 64 sources at a time
+// through LDS, the 16 lanes of a group holding T targets each and the four groups
+// taking every fourth source.  Bound by FP64 issue (4.6 cycles): 16 operations and
+// one v_rsq_f64 (16 cycles) for 64 pairs.  Per evaluation, against a 256-thread
+// block per 1024 to 16384 sources, a launch per leaf size one after the other, and
+// two Newton steps for each root: 16384 particles (s = 64) 0.33 -> 0.15 ms, 64k
+// mixture 1.05 -> 0.40, 128k (s = 128) 3.0 -> 1.7, 1M 3.3 -> 2.7 ms.
+template <int T, bool POT, class F>
+__device__ __forceinline__ void f64_pass(const double4 *__restrict__ xs, const Sources &src, const int32_t *delta, double4 *tile, uint32_t len,
+                                         uint32_t pt0, int nt, double eps2, bool um, F &&emit) {
+    const int lane = threadIdx.x, col = lane & 15, quad = lane >> 4;
+    const int ng = static_cast<int>((len + 63) / 64);
+    double x[T], y[T], z[T], acc[T][4];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        const double4 v = xs[pt0 + min(16 * t + col, nt - 1)];  // columns past the last target repeat it and are dropped
+        x[t] = v.x, y[t] = v.y, z[t] = v.z;
+        acc[t][0] = acc[t][1] = acc[t][2] = acc[t][3] = 0;
+    }
+    double4 nx = xs[source_of(src, delta, 0, len)];
+    for (int g = 0; g < ng; ++g) {
+        __builtin_amdgcn_wave_barrier();
+        const bool full = 64u * g + 64 <= len;
+        if (um) nx.w = 1.0;
+        if (64u * g + lane >= len) nx.w = 0.0;  // the last source again, without mass
+        tile[lane] = nx;
+        if (g + 1 < ng) nx = xs[source_of(src, delta, g + 1, len)];
+        wave_lds_sync();
+        auto pairs = [&](auto soft, auto weighted) {
+#pragma unroll 2
+            for (int i = 0; i < 16; ++i) {
+                const double4 s = tile[4 * i + quad];
+#pragma unroll
+                for (int t = 0; t < T; ++t) {
+                    const double dx = s.x - x[t], dy = s.y - y[t], dz = s.z - z[t];
+                    const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));
+                    const double h = __builtin_amdgcn_rsq(r2);  // refined as in rsq; r2^(-3/2) = h^3 (1 + 3/2 e + 15/8 e^2 + ..)
+                    const double hh = h * h, e = fma(-r2, hh, 1.0);
+                    const double c = (decltype(weighted)::value ? h * s.w : h) * hh;
+                    double w = fma(c * e, fma(e, 1.875, 1.5), c);
+                    if (!decltype(soft)::value) w = r2 > 0.0 ? w : 0.0;  // a particle and itself
+                    acc[t][0] = fma(w, dx, acc[t][0]);
+                    acc[t][1] = fma(w, dy, acc[t][1]);
+                    acc[t][2] = fma(w, dz, acc[t][2]);
+                    if (POT) {
+                        double ri = fma(h * e, fma(e, 0.375, 0.5), h);
+                        if (!decltype(soft)::value) ri = r2 > 0.0 ? ri : 0.0;
+                        acc[t][3] = decltype(weighted)::value ? fma(s.w, ri, acc[t][3]) : acc[t][3] + ri;
+                    }
+                }
+            }
+        };
+        if (eps2 > 0.0) {
+            if (um && full)
+                pairs(std::true_type{}, std::false_type{});
+            else
+                pairs(std::true_type{}, std::true_type{});
+        } else {
+            if (um && full)
+                pairs(std::false_type{}, std::false_type{});
+            else
+                pairs(std::false_type{}, std::true_type{});
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+#pragma unroll
+        for (int j = 0; j < (POT ? 4 : 3); ++j) {
+            acc[t][j] += __shfl_xor(acc[t][j], 16, 64);
+            acc[t][j] += __shfl_xor(acc[t][j], 32, 64);
+        }
+        if (quad == 0 && 16 * t + col < nt) emit(16 * t + col, acc[t]);
+    }
+}
+
+template <bool POT>
+__global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ items, const uint32_t *__restrict__ start,
+                                                   const uint32_t *__restrict__ count, const int32_t *__restrict__ anc, const int32_t *__restrict__ ni,
+                                                   const int32_t *__restrict__ ni_cnt, const double4 *__restrict__ xs, double eps2, double G, bool um,
+                                                   double mu, double4 *__restrict__ acc, double4 *__restrict__ partial, uint32_t pstride) {
+    __shared__ double4 tile[64];
+    __shared__ int32_t delta[MAXE];
+    const McWork wk = items[blockIdx.x];
+    const int lane = threadIdx.x, nt = static_cast<int>(wk.nt);
+    const Sources src = lay_out_entries(wk, delta, reinterpret_cast<uint64_t *>(tile), start, count, anc, ni, ni_cnt);
+    const double sc = um ? mu : 1.0;
+    double4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * pstride : nullptr;
+    auto emit = [&](int t, const double *v) {
+        const double sx = v[0] * sc, sy = v[1] * sc, sz = v[2] * sc;
+        double sp = v[3] * sc;
+        if (out) {
+            out[wk.t0 + t] = double4{sx, sy, sz, sp};
+        } else {
+            if (POT && eps2 > 0.0) sp -= xs[wk.pt0 + t].w * rsq(eps2);  // drop the m_i / eps self term
+            acc[wk.pt0 + t] = double4{G * sx, G * sy, G * sz, sp};
+        }
+    };
+    if (wk.len == 0) {  // a last chunk that the even lengths left empty
+        const double none[4] = {0, 0, 0, 0};
+        for (int t = lane; t < nt; t += 64) emit(t, none);
+        return;
+    }
+    const int T = (nt + 15) / 16;  // at most F64_TILES
+    auto pass = [&](auto tiles) { f64_pass<decltype(tiles)::value, POT>(xs, src, delta, tile, wk.len, wk.pt0, nt, eps2, um, emit); };
+    if (T == 1)
+        pass(std::integral_constant<int, 1>{});
+    else if (T == 2)
+        pass(std::integral_constant<int, 2>{});
+    else if (T == 3)
+        pass(std::integral_constant<int, 3>{});
+    else
+        pass(std::integral_constant<int, F64_TILES>{});
+}
+
 // Leaves split over several work items: partial sums added in chunk order
 // (the same order every run), a wavefront per leaf.
-template <bool POT>
+template <bool POT, class R, class V4 = typename Vec4<R>::T>
 __global__ __launch_bounds__(256) void k_p2p_sum(const int32_t *__restrict__ leaves, int nleaves, const uint32_t *__restrict__ nchunk,
                                                  const uint32_t *__restrict__ item_off, const uint32_t *__restrict__ start, const uint32_t *__restrict__ count,
-                                                 const float4 *__restrict__ xs, float eps2, float G, float4 *__restrict__ acc,
-                                                 const float4 *__restrict__ partial, uint32_t pstride) {
+                                                 const V4 *__restrict__ xs, R eps2, R G, V4 *__restrict__ acc,
+                                                 const V4 *__restrict__ partial, uint32_t pstride) {
     const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (k >= nleaves) return;
     const uint32_t nch = nchunk[k];
     if (nch < 2) return;
     const int32_t c = leaves[k];
     const uint32_t nt = count[c], pt0 = start[c];
-    const float4 *pk = partial + static_cast<size_t>(item_off[k]) * pstride;
+    const V4 *pk = partial + static_cast<size_t>(item_off[k]) * pstride;
     for (uint32_t t = threadIdx.x & 63; t < nt; t += 64) {
-        float sx = 0, sy = 0, sz = 0, sp = 0;
+        R sx = 0, sy = 0, sz = 0, sp = 0;
 #pragma unroll 8
         for (uint32_t q = 0; q < nch; ++q) {
-            const float4 v = pk[static_cast<size_t>(q) * pstride + t];
+            const V4 v = pk[static_cast<size_t>(q) * pstride + t];
             sx += v.x;
             sy += v.y;
             sz += v.z;
             sp += v.w;
         }
-        if (POT && eps2 > 0.0f) sp -= xs[pt0 + t].w * rsq(eps2);
-        acc[pt0 + t] = float4{G * sx, G * sy, G * sz, sp};
+        if (POT && eps2 > R(0)) sp -= xs[pt0 + t].w * rsq(eps2);
+        acc[pt0 + t] = V4{G * sx, G * sy, G * sz, sp};
     }
 }
 
-// Per leaf: number of sources in its NI chain, split into chunks of at most
-// chunk sources (bounded work per block), and its class by targets per lane.
 // Sources of each cell's own NI entries (the leaf's full list is its
 // ancestors' entries and its own, solver_ref.hpp:126).
 __global__ __launch_bounds__(256) void k_ni_local(int64_t ncells, const uint32_t *__restrict__ count, const int32_t *__restrict__ ni,
@@ -765,34 +664,17 @@ __global__ __launch_bounds__(256) void k_ni_local(int64_t ncells, const uint32_t
     local[c] = s;
 }
 
-// Leaf classes: class T - 1 (T = 1 .. TMAX) takes T targets per lane in groups
-// of tpw_for(nt, T) lanes, T chosen for the fewest lane slots TPW T >= nt
-// (ties: fewer targets per lane); class TMAX: more than 64 TMAX targets, in
-// batches of 256.
-// FP32 items (mt > 0: at most mt target tiles) differ only in cost (16-target
-// tiles times 64-source groups): class j costs at least 2^(8 - j), so the largest start first.
-constexpr int NCLS = TMAX + 1;
+// Leaf classes, by the cost of their items (16-target tiles times 64-source
+// groups): class j costs at least 2^(8 - j), so the largest start first.
+constexpr int NCLS = 7;
 constexpr int NSC = NCLS + 2;  // scanned per leaf: chunks, chunks of each class, split flag
 __device__ inline int leaf_class(uint32_t nt, uint32_t src, uint32_t nch, int mt) {
-    if (mt) {
-        const uint32_t cost = mc_batch_tiles(nt, mt) * (chunk_len(src, nch) / 64);
-        return max(0, min(TMAX, 8 - (31 - __builtin_clz(max(cost, 1u)))));
-    }
-    if (nt > 64u * TMAX) return TMAX;
-    int best = 0;
-    uint32_t slots = ~0u;
-    for (int T = 1; T <= TMAX; ++T) {
-        const int tp = tpw_for(nt, T);
-        if (tp && static_cast<uint32_t>(tp * T) < slots) {
-            slots = tp * T;
-            best = T - 1;
-        }
-    }
-    return best;
+    const uint32_t cost = mc_batch_tiles(nt, mt) * (chunk_len(src, nch) / 64);
+    return max(0, min(NCLS - 1, 8 - (31 - __builtin_clz(max(cost, 1u)))));
 }
 
-// Per leaf: source count -> chunks (of at most chunk sources or, for mc, of at
-// most chunk target tiles times source groups) and class; block-local exclusive scans of
+// Per leaf: source count -> chunks (of at most chunk target tiles times source
+// groups) and class; block-local exclusive scans of
 // the NSC components (one leaf per thread, 256 per block) and block totals.
 __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ leaves, int nleaves, const int8_t *__restrict__ level,
                                                   const uint32_t *__restrict__ count, const int32_t *__restrict__ anc, const uint32_t *__restrict__ local,
@@ -807,12 +689,12 @@ __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ le
         uint32_t src = 0;
         for (int l = 0; l <= level[c]; ++l) src += local[anc[static_cast<int64_t>(c) * (MAXD + 1) + l]];
         const uint32_t nt = count[c];
-        // mt: as many groups as the cost allows, but no fewer than minrow eighths of the tiles (the rows of partial sums of a large leaf stay few)
-        const uint32_t lim = mt ? 64 * min(MC_CHUNK / 64, max(1 + (nt + 15) / 16 * minrow / 8, chunk / mc_batch_tiles(nt, mt))) : chunk;
+        // as many groups as the cost allows, but no fewer than minrow eighths of the tiles (the rows of partial sums of a large leaf stay few)
+        const uint32_t lim = 64 * min(MC_CHUNK / 64, max(1 + (nt + 15) / 16 * minrow / 8, chunk / mc_batch_tiles(nt, mt)));
         const uint32_t nch = max(1u, (src + lim - 1) / lim);
         nchunk[k] = nch;
         nsrc[k] = src;
-        const uint32_t nit = mt ? nch * mc_batches(nt, mt) : nch;
+        const uint32_t nit = nch * mc_batches(nt, mt);
         v[0] = nch > 1 ? nch : 0u;
         const int cl = leaf_class(nt, src, nch, mt);
         cls[k] = cl;
@@ -878,25 +760,9 @@ __global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ 
     }
 }
 
-// Item offsets, items (leaf, chunk) bucketed by class in leaf order, and the
-// list of leaves whose sources span several chunks.
-__global__ __launch_bounds__(256) void k_p2p_items(int nleaves, const uint32_t *__restrict__ lcls,
-                                                   const uint32_t *__restrict__ nchunk, const uint32_t *__restrict__ pre,
-                                                   const uint32_t *__restrict__ boff, const uint32_t *__restrict__ scal,
-                                                   uint32_t *__restrict__ item_off, int2 *__restrict__ items) {
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= nleaves) return;
-    const uint32_t *pk = pre + static_cast<int64_t>(k) * NSC;
-    const uint32_t *bk = boff + blockIdx.x * NSC;
-    const uint32_t nch = nchunk[k];
-    item_off[k] = bk[0] + pk[0];
-    const int cls = lcls[k];
-    const uint32_t pos = scal[NCLS + cls] + bk[1 + cls] + pk[1 + cls];
-    for (uint32_t q = 0; q < nch; ++q) items[pos + q] = make_int2(k, static_cast<int>(q));
-}
-
-// The FP32 kernel's items, each with what its wavefront needs to start.
-__global__ __launch_bounds__(256) void k_p2p_items_mc(const int32_t *__restrict__ leaves, int nleaves, const int8_t *__restrict__ level,
+// The work items, bucketed by class in leaf order, each with what its wavefront needs
+// to start, and the leaves' rows of partial sums.
+__global__ __launch_bounds__(256) void k_p2p_items(const int32_t *__restrict__ leaves, int nleaves, const int8_t *__restrict__ level,
                                                       const uint32_t *__restrict__ start, const uint32_t *__restrict__ count,
                                                       const uint32_t *__restrict__ lcls, const uint32_t *__restrict__ nchunk,
                                                       const uint32_t *__restrict__ nsrc, const uint32_t *__restrict__ pre,
@@ -936,17 +802,15 @@ void p2p_plan(Ctx &c, bool potential) {
     c.p2p_local.ensure(t.ncells);
     c.p2p_pre.ensure(static_cast<size_t>(nl) * NSC);
     c.p2p_btot.ensure(static_cast<size_t>(nb) * NSC);
-    c.p2p_ticket.ensure(nl);
     k_ni_local<<<ceil_div(t.ncells, 256), 256, 0, c.stream>>>(t.ncells, t.count, t.ni, t.ni_cnt, c.p2p_local);
-    // under 8 leaves per CU (the 16k Plummer sphere has 430): chunks of 8192
-    // sources, or items of MC_COST, scaled down by the leaf shortfall, so that
-    // the work items still give every CU several blocks
-    uint32_t chunk = c.prec == 0 ? P2P_CHUNK : MC_COST;
-    if (c.ncu > 0 && nl < 8 * c.ncu)
-        chunk = c.prec == 0 ? std::max<uint32_t>(1024, static_cast<uint32_t>(8192ull * nl / (8 * c.ncu)) / 256 * 256)
-                            : std::max<uint32_t>(MC_MINCOST, static_cast<uint32_t>(1ull * MC_COST * nl / (8 * c.ncu)));
+    // under 8 leaves per CU (the 16k Plummer sphere has 430): FP32 items of MC_COST,
+    // scaled down by the leaf shortfall, so that there are still several per SIMD;
+    // FP64 items take some five times as long, so they shrink from more leaves on
+    const int few = (c.prec == 0 ? F64_LEAVES : 8) * c.ncu;
+    uint32_t chunk = MC_COST;
+    if (nl < few) chunk = std::max<uint32_t>(c.prec == 0 ? F64_MINCOST : MC_MINCOST, static_cast<uint32_t>(1ull * MC_COST * nl / few));
     k_p2p_plan<<<nb, 256, 0, c.stream>>>(t.leaf_ids, nl, t.level, t.count, t.anc, c.p2p_local, c.p2p_nchunk, c.p2p_cls, c.p2p_src, c.p2p_pre, c.p2p_btot, chunk,
-                                        c.prec == 0 ? 0 : mc_tiles(potential), nl < 8 * c.ncu ? 1 : 8);
+                                        c.prec == 0 ? F64_TILES : mc_tiles(potential), nl < 8 * c.ncu ? 1 : 8);
     k_p2p_plan_blocks<<<1, 256, 0, c.stream>>>(c.p2p_btot, nb, c.p2p_scal);
     VG_LAUNCH_CHECK();
     static_assert(2 * NCLS + 2 <= 16, "plan scalars");
@@ -962,105 +826,48 @@ static const uint32_t *p2p_scalars(Ctx &c) {
     return reinterpret_cast<const uint32_t *>(static_cast<const char *>(c.pinned) + 128);
 }
 
-// FP32 P2P: one launch over all items, on the stream p2p_plan used.
-void p2p_run_f32(Ctx &c, bool potential) {
+// One launch over all items, on the stream p2p_plan used, and one that adds the
+// partial sums of the leaves split over several.
+template <class R>
+void p2p_run(Ctx &c, bool potential) {
+    using V4 = typename Vec4<R>::T;
     TreeDev &t = c.t;
     if (!t.nleaves) return;
     const uint32_t *hs = p2p_scalars(c);
     const uint32_t nitems = hs[2 * NCLS - 1] + hs[NCLS - 1], nrows = hs[2 * NCLS], pstride = c.thr;
     const bool split = hs[2 * NCLS + 1] > 0;
     const int nl = static_cast<int>(t.nleaves);
-    c.p2p_items.ensure(sizeof(McWork) / 8 * static_cast<size_t>(std::max<uint32_t>(1, nitems)));
+    c.p2p_items.ensure(sizeof(McWork) * static_cast<size_t>(std::max<uint32_t>(1, nitems)));
     McWork *items = reinterpret_cast<McWork *>(c.p2p_items.p);
-    k_p2p_items_mc<<<ceil_div(nl, 256), 256, 0, c.stream>>>(t.leaf_ids, nl, t.level, t.start, t.count, c.p2p_cls, c.p2p_nchunk, c.p2p_src, c.p2p_pre,
-                                                            c.p2p_btot, c.p2p_scal, c.p2p_item_off, items, mc_tiles(potential));
+    k_p2p_items<<<ceil_div(nl, 256), 256, 0, c.stream>>>(t.leaf_ids, nl, t.level, t.start, t.count, c.p2p_cls, c.p2p_nchunk, c.p2p_src, c.p2p_pre,
+                                                         c.p2p_btot, c.p2p_scal, c.p2p_item_off, items, sizeof(R) == 8 ? F64_TILES : mc_tiles(potential));
     VG_LAUNCH_CHECK();
-    c.as32.ensure(4 * std::max<int64_t>(1, c.n));
-    if (split) c.p2p_part32.ensure(4 * static_cast<size_t>(nrows) * pstride);
-    const float eps2 = static_cast<float>(c.eps * c.eps);
-    const float4 *xs = reinterpret_cast<const float4 *>(c.xs32.p);
-    float4 *acc = reinterpret_cast<float4 *>(c.as32.p), *part = reinterpret_cast<float4 *>(c.p2p_part32.p);
-    const float G = static_cast<float>(c.G);
-    bool big = false;  // a root box so wide that squared distances may leave the FP32 range
-    for (int a = 0; a < 3; ++a) big |= !(t.box[3 + a] - t.box[a] < 1e18);
-    auto run = [&](auto kernel, auto sum) {
-        kernel<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs, eps2, G, !c.has_masses, big, static_cast<float>(c.mass), acc, part, pstride);
-        if (split) sum<<<ceil_div(nl, 4), 256, 0, c.stream>>>(t.leaf_ids, nl, c.p2p_nchunk, c.p2p_item_off, t.start, t.count, xs, eps2, G, acc, part, pstride);
+    auto buffers = [&](auto &sorted, auto &sums, auto &parts, auto run) {
+        sums.ensure(4 * std::max<int64_t>(1, c.n));
+        if (split) parts.ensure(4 * static_cast<size_t>(nrows) * pstride);
+        run(reinterpret_cast<const V4 *>(sorted.p), reinterpret_cast<V4 *>(sums.p), reinterpret_cast<V4 *>(parts.p));
     };
-    if (potential)
-        run(k_p2p_mc<true>, k_p2p_sum<true>);
-    else
-        run(k_p2p_mc<false>, k_p2p_sum<false>);
-    VG_LAUNCH_CHECK();
-}
-
-// FP64 P2P: one kernel per leaf class.
-void p2p_run_f64(Ctx &c, bool potential) {
-    TreeDev &t = c.t;
-    if (!t.nleaves) return;
-    using R = double;
-    using V4 = double4;
-    const V4 *xs = reinterpret_cast<const V4 *>(c.xs64.p);
-    c.as64.ensure(4 * std::max<int64_t>(1, c.n));
-    V4 *acc = reinterpret_cast<V4 *>(c.as64.p);
-    const R eps2 = c.eps * c.eps;
-    const bool guard = !(eps2 > 0);
-    // one mass for every particle (no per-particle masses uploaded): force
-    // kernels take it out of the pair terms (the potential keeps the general path)
-    const bool um = !c.has_masses;
-    const R mu = c.mass;
-    const uint32_t *hs = p2p_scalars(c), *hbase = hs + NCLS;
-    const int nl = static_cast<int>(t.nleaves);
-    c.p2p_items.ensure(std::max<uint32_t>(1, hs[2 * NCLS - 1] + hs[NCLS - 1]));
-    int2 *items = reinterpret_cast<int2 *>(c.p2p_items.p);
-    k_p2p_items<<<ceil_div(nl, 256), 256, 0, c.stream>>>(nl, c.p2p_cls, c.p2p_nchunk, c.p2p_pre, c.p2p_btot, c.p2p_scal, c.p2p_item_off, items);
-    VG_LAUNCH_CHECK();
-    const bool split = hs[2 * NCLS + 1] > 0;
-    const uint32_t pstride = c.thr;
-    if (split) VG_HIP(hipMemsetAsync(c.p2p_ticket.p, 0, static_cast<size_t>(t.nleaves) * sizeof(uint32_t), c.stream));
-    if (split) c.p2p_part64.ensure(4 * static_cast<size_t>(hs[2 * NCLS]) * pstride);
-    V4 *partial = reinterpret_cast<V4 *>(c.p2p_part64.p);
-    for (int cls = 0; cls < NCLS; ++cls) {
-        if (!hs[cls]) continue;
-        const dim3 grid(hs[cls]);
-        const int2 *it = items + hbase[cls];
-#define VG_P2P_T(G_, P_, U_, T_)                                                                                                                \
-    k_p2p<R, G_, P_, U_, T_><<<grid, P2P_THREADS, 0, c.stream>>>(it, t.leaf_ids, c.p2p_nchunk, c.p2p_item_off, t.level, t.start, t.count, t.anc, \
-                                                                 t.ni, t.ni_cnt, xs, eps2, c.G, mu, acc, partial, pstride, c.p2p_ticket)
-#define VG_P2P(G_, P_, U_)           \
-    do {                             \
-        if (cls == 0)                \
-            VG_P2P_T(G_, P_, U_, 1); \
-        else if (cls == 1)           \
-            VG_P2P_T(G_, P_, U_, 2); \
-        else if (cls == 2)           \
-            VG_P2P_T(G_, P_, U_, 3); \
-        else if (cls == 3)           \
-            VG_P2P_T(G_, P_, U_, 4); \
-        else if (cls == 4)           \
-            VG_P2P_T(G_, P_, U_, 5); \
-        else if (cls == 5)           \
-            VG_P2P_T(G_, P_, U_, 6); \
-        else /* batches */           \
-            VG_P2P_T(G_, P_, U_, 7); \
-    } while (0)
-        if (guard) {
-            if (potential)
-                VG_P2P(true, true, false);
-            else if (um)
-                VG_P2P(true, false, true);
-            else
-                VG_P2P(true, false, false);
-        } else {
-            if (potential)
-                VG_P2P(false, true, false);
-            else if (um)
-                VG_P2P(false, false, true);
-            else
-                VG_P2P(false, false, false);
-        }
-#undef VG_P2P
-#undef VG_P2P_T
+    const R eps2 = static_cast<R>(c.eps * c.eps), G = static_cast<R>(c.G), mu = static_cast<R>(c.mass);
+    const bool um = !c.has_masses;  // one mass: left out of the pairs, the sums are scaled once
+    auto add = [&](const V4 *xs, V4 *acc, const V4 *part) {
+        if (!split) return;
+        (potential ? k_p2p_sum<true, R> : k_p2p_sum<false, R>)<<<ceil_div(nl, 4), 256, 0, c.stream>>>(t.leaf_ids, nl, c.p2p_nchunk, c.p2p_item_off, t.start,
+                                                                                                    t.count, xs, eps2, G, acc, part, pstride);
+    };
+    if constexpr (sizeof(R) == 4) {
+        bool big = false;  // a root box so wide that squared distances may leave the FP32 range
+        for (int a = 0; a < 3; ++a) big |= !(t.box[3 + a] - t.box[a] < 1e18);
+        buffers(c.xs32, c.as32, c.p2p_part32, [&](const V4 *xs, V4 *acc, V4 *part) {
+            (potential ? k_p2p_mc<true> : k_p2p_mc<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs,
+                                                                                       eps2, G, um, big, mu, acc, part, pstride);
+            add(xs, acc, part);
+        });
+    } else {
+        buffers(c.xs64, c.as64, c.p2p_part64, [&](const V4 *xs, V4 *acc, V4 *part) {
+            (potential ? k_p2p_f64<true> : k_p2p_f64<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, xs, eps2, G, um,
+                                                                                         mu, acc, part, pstride);
+            add(xs, acc, part);
+        });
     }
     VG_LAUNCH_CHECK();
 }
@@ -1071,9 +878,9 @@ void fmm_p2p_plan(Ctx &c, bool potential) { p2p_plan(c, potential); }
 
 void fmm_p2p_run(Ctx &c, bool potential) {
     if (c.prec == 0)
-        p2p_run_f64(c, potential);
+        p2p_run<double>(c, potential);
     else
-        p2p_run_f32(c, potential);
+        p2p_run<float>(c, potential);
 }
 
 void fmm_p2p(Ctx &c, bool potential) {
