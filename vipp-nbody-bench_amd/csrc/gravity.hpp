@@ -35,9 +35,12 @@ struct TreeDev {
     DevBuf<int32_t> grid;            // 3 per cell: integer position at its level (low side = 0)
     DevBuf<int32_t> anc;             // (MAXD+1) per cell: ancestor id at every level <= own level
     DevBuf<int32_t> int_ids;         // internal cells, level by level
+    DevBuf<uint32_t> int_start;      // their first positions
+    DevBuf<int32_t> int_parent;      // their parents, as indices into int_ids
     DevBuf<int32_t> leaf_ids;        // non-empty leaves
-    DevBuf<uint8_t> flags;           // scratch for compaction
-    DevBuf<uint32_t> lv;             // level table of a device-driven build
+    DevBuf<uint8_t> flags;           // non-empty leaves among the cells
+    DevBuf<uint32_t> leaf_cnt;       // per-block counts of these
+    DevBuf<uint32_t> lv;             // level table of the build
 
     // interaction lists (reference order, device ids)
     DevBuf<int32_t> nb, ni, ap;              // 27, 27, 189 slots per cell
@@ -131,7 +134,7 @@ struct Ctx {
     DevBuf<uint32_t> val[2];
     DevBuf<uint32_t> rs_hist;
     DevBuf<uint32_t> scal;      // small device scalars (counts, error flags)
-    DevBuf<uint32_t> cmp_cnt;   // per-block counts of the multi-block compaction
+    DevBuf<uint32_t> cmp_cnt;   // cells per level and block of the sorted codes
     DevBuf<uint32_t> perm;      // sorted position -> caller index
     // particles in sorted order
     DevBuf<double> xs64;        // 4 per particle: x, y, z, m
