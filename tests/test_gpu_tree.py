@@ -1,5 +1,6 @@
-"""Octree at the edges of its kernels: particle counts around the leaf threshold and
-around the 1024 (beyond 2^20 particles: 4096) sorted codes of a block, leaves counted in
+"""Octree at the edges of its kernels: particle counts around the leaf threshold,
+around the 1024 (beyond 2^20 particles: 4096) sorted codes of a block and around the sort's
+tiles (4096 codes; 64 tiles), leaves counted in
 one block and in many, on a first and on a second build in one context.  Bit for bit the
 oracle's tree and lists."""
 import numpy as np
@@ -25,8 +26,8 @@ def _points(n):
 
 
 # (threshold floor(sqrt(8) s): 2 at s = 1, 11 at 4, 181 at 64)
-@pytest.mark.parametrize("n,s", [(1, 1), (11, 4), (12, 4), (181, 64), (182, 64), (1023, 4), (1024, 4), (1025, 4), (2047, 64), (5000, 4), (40000, 2),
-                                 ((1 << 20) + 1025, 64)])
+@pytest.mark.parametrize("n,s", [(1, 1), (11, 4), (12, 4), (181, 64), (182, 64), (1023, 4), (1024, 4), (1025, 4), (2047, 64), (4096, 4), (4097, 4),
+                                 (5000, 4), (40000, 2), (64 * 4096, 64), (64 * 4096 + 1, 64), ((1 << 20) + 1025, 64)])
 def test_tree_at_the_edges(vg, orc, n, s):
     x = _points(n)
     rt, rl = orc.tree_and_lists(x, s)

