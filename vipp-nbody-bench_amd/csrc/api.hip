@@ -78,15 +78,14 @@ void join_p2p(Ctx &c) {
 
 // Untimed split-mode evaluations run the lists and P2P (VALU-bound, about
 // half the evaluation) on a second stream once the tree exists, so that the
-// operators and the upward pass (which need only the tree), and M2L
-// (MFMA-bound, after the lists), run beside them; L2P waits for P2P. The P2P
-// plan is enqueued with the lists and its item counts are read back while the
-// host enqueues the operators and the upward pass. The FP32 and FP64 modes,
+// operators (enqueued by tree_build) and the upward pass (which need only the
+// tree), and M2L (MFMA-bound, after the lists), run beside them; L2P waits for
+// P2P. The P2P plan is enqueued with the lists and its item counts are read back
+// while the host enqueues the upward pass. The FP32 and FP64 modes,
 // whose M2L is VALU-bound too, and timed evaluations keep one stream (the
 // events of a phase then bracket its own kernels only).
 static void evaluate_overlapped(Ctx &c, bool potential) {
-    VG_HIP(hipEventRecord(c.ev_fork, c.stream));
-    VG_HIP(hipStreamWaitEvent(c.stream2, c.ev_fork, 0));
+    VG_HIP(hipStreamWaitEvent(c.stream2, c.ev_tree, 0));  // not the operators behind the tree
     struct Swap {
         Ctx &c;
         explicit Swap(Ctx &c_) : c(c_) { std::swap(c.stream, c.stream2); }
@@ -102,7 +101,6 @@ static void evaluate_overlapped(Ctx &c, bool potential) {
             Swap on_stream2(c);
             fmm_p2p_plan(c, potential);
         }
-        operators_build(c);
         fmm_upward(c);  // enqueued while the P2P plan's item counts come back
         {
             Swap on_stream2(c);
@@ -129,23 +127,25 @@ void evaluate(Ctx &c, bool potential) {
     c.t.ref_valid = false;
     bool used[PH_COUNT] = {};
     if (!c.timing && c.stream2 && c.prec == 2) {
-        tree_build(c);
+        tree_build(c, true);
         evaluate_overlapped(c, potential);
         c.evaluated = true;
         return;
     }
     phase_begin(c, PH_TREE);
-    tree_build(c);
+    tree_build(c, !c.timing);
     phase_end(c, PH_TREE);
     used[PH_TREE] = true;
     phase_begin(c, PH_LISTS);
     lists_build(c);
     phase_end(c, PH_LISTS);
     used[PH_LISTS] = true;
-    phase_begin(c, PH_OPS);
-    operators_build(c);
-    phase_end(c, PH_OPS);
-    used[PH_OPS] = true;
+    if (c.timing) {
+        phase_begin(c, PH_OPS);
+        operators_build(c);
+        phase_end(c, PH_OPS);
+        used[PH_OPS] = true;
+    }
     phase_begin(c, PH_UP);
     fmm_upward(c);
     phase_end(c, PH_UP);
@@ -412,7 +412,7 @@ int vipp_grav_create(const vipp_grav_config *cfg, vipp_grav_ctx **out) {
             VG_HIP(hipDeviceGetAttribute(&c.ncu, hipDeviceAttributeMultiprocessorCount, c.device));
             VG_HIP(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
             VG_HIP(hipStreamCreateWithFlags(&c.stream2, hipStreamNonBlocking));
-            VG_HIP(hipEventCreateWithFlags(&c.ev_fork, hipEventDisableTiming));
+            VG_HIP(hipEventCreateWithFlags(&c.ev_tree, hipEventDisableTiming));
             VG_HIP(hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming));
             VG_HIP(hipEventCreateWithFlags(&c.ev_lists, hipEventDisableTiming));
             VG_HIP(hipEventCreateWithFlags(&c.ev_plan, hipEventDisableTiming));
@@ -444,7 +444,7 @@ int vipp_grav_destroy(vipp_grav_ctx *ctx) {
     });
     for (auto &e : ctx->c.ev)
         if (e) (void)hipEventDestroy(e);
-    if (ctx->c.ev_fork) (void)hipEventDestroy(ctx->c.ev_fork);
+    if (ctx->c.ev_tree) (void)hipEventDestroy(ctx->c.ev_tree);
     if (ctx->c.ev_join) (void)hipEventDestroy(ctx->c.ev_join);
     if (ctx->c.ev_lists) (void)hipEventDestroy(ctx->c.ev_lists);
     if (ctx->c.ev_plan) (void)hipEventDestroy(ctx->c.ev_plan);

@@ -66,10 +66,12 @@ constexpr int HSTRIDE = 2 * ((AL + 1) * (AL + 2) / 2) + 2;  // per offset: Y tab
 // (1, ry, rz): 0..7 M2M (child centre - parent centre of child octant o),
 // 8..15 L2L (their negatives), 16 + o M2L (source - target cell, o in base 7
 // holding (dx + 3, dy + 3, dz + 3)).
-__global__ __launch_bounds__(64) void k_harmonics(const int16_t *__restrict__ sel, int nvec, double ry, double rz, int lmax, double *__restrict__ out) {
+__global__ __launch_bounds__(64) void k_harmonics(const int16_t *__restrict__ sel, int nvec, const double *__restrict__ box, int lmax, double *__restrict__ out) {
     const int o = sel[blockIdx.x];  // the vectors any kernel reads (see operators_build)
     const int m = threadIdx.x;
     if (o >= nvec || m > lmax) return;
+    const double wx = box[3] - box[0], wy = box[4] - box[1], wz = box[5] - box[2];
+    const double ry = wx > 0 ? wy / wx : 1.0, rz = wx > 0 ? wz / wx : 1.0;
     double vx, vy, vz;
     if (o < 16) {
         const int q = o & 7;
@@ -1306,9 +1308,6 @@ void ops_selection(Ctx &c) {
 
 void operators_build(Ctx &c) {
     fmm_constants_init();
-    const TreeDev &t = c.t;
-    const double wx = t.box[3] - t.box[0], wy = t.box[4] - t.box[1], wz = t.box[5] - t.box[2];
-    const double ry = wx > 0 ? wy / wx : 1.0, rz = wx > 0 ? wz / wx : 1.0;
     // 8 M2M (child - parent), 8 L2L (parent - child) and 343 M2L (source -
     // target) offsets, formed on the device from the aspect ratio.  Only the
     // 189 M2L offsets of octant 0's walk are ever read (every octant uses them
@@ -1317,7 +1316,7 @@ void operators_build(Ctx &c) {
     const int nvec = 16 + 343;
     ops_selection(c);
     c.harm.ensure(static_cast<size_t>(nvec) * HSTRIDE);
-    k_harmonics<<<NOPS_USED, 64, 0, c.stream>>>(c.ops_sel, nvec, ry, rz, 2 * c.p, c.harm);
+    k_harmonics<<<NOPS_USED, 64, 0, c.stream>>>(c.ops_sel, nvec, c.box, 2 * c.p, c.harm);
     dim3 grid(NOPS_USED, ceil_div(c.K, OPS_ROWS));
     if (c.prec == 0) {
         c.op64.ensure(static_cast<size_t>(nvec) * c.K * c.K);

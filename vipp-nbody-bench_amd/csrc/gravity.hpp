@@ -106,7 +106,8 @@ struct Ctx {
     // M2L of the same evaluation (they share no buffer); M2L waits for the
     // lists (ev_lists), the scatter for P2P (join_p2p)
     hipStream_t stream2 = nullptr;
-    hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_lists = nullptr;
+    hipEvent_t ev_join = nullptr, ev_lists = nullptr;
+    hipEvent_t ev_tree = nullptr;  // the tree is built and its sizes are in the pinned words
     hipEvent_t ev_plan = nullptr;  // the P2P plan scalars are in the pinned words
     bool p2p_pending = false;
     // pinned host words for the scalars read back during an evaluation (tree
@@ -177,7 +178,7 @@ struct Ctx {
 };
 
 // phases (each launches on ctx.stream)
-void tree_build(Ctx &c);                 // AABB, codes, sort, cells, leaves, particle gather
+void tree_build(Ctx &c, bool operators); // AABB, codes, sort, cells, leaves, particle gather; with the operators enqueued before it waits
 void lists_build(Ctx &c);                // NB / NI / AP lists and the 27-neighbour table
 void ref_numbering(Ctx &c);              // reference cell ids (for export only)
 void operators_build(Ctx &c);            // M2M / L2L / M2L operators for the current root box

@@ -706,7 +706,10 @@ static void ensure_cells(TreeDev &t, int64_t ncell) {
     t.int_parent.ensure(ncell / 8 + 1);
 }
 
-void tree_build(Ctx &c) {
+// With operators, the operators (which need the root box alone) are enqueued
+// behind the tree before the host waits for its sizes: the device forms them while
+// the host wakes up and launches the lists.
+void tree_build(Ctx &c, bool operators) {
     hipStream_t st = c.stream;
     TreeDev &t = c.t;
     const int64_t n = c.n;
@@ -741,7 +744,10 @@ void tree_build(Ctx &c) {
     auto read_back = [&] {
         VG_HIP(hipMemcpyAsync(hbox, c.box, 7 * sizeof(double), hipMemcpyDeviceToHost, st));
         VG_HIP(hipMemcpyAsync(hlv, t.lv, LV_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        VG_HIP(hipStreamSynchronize(st));
+        VG_HIP(hipEventRecord(c.ev_tree, st));
+        if (operators) operators_build(c);
+        operators = false;
+        VG_HIP(hipEventSynchronize(c.ev_tree));
         if (hbox[6] != 0) throw Error(2, "non-finite particle coordinates");
     };
     // 2. path codes and a stable sort of the octants of levels 1..SH (bits below
@@ -819,6 +825,7 @@ void tree_build(Ctx &c) {
         k_leaf_sort<<<static_cast<unsigned>(t.nleaves), 256, c.thr * sizeof(uint32_t), st>>>(t.leaf_ids, t.start, t.count, v0, c.perm);
         k_gather<<<ceil_div(n, 256), 256, 0, st>>>(c.perm, n, c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.box, c.xs64, c.xs32);
         VG_LAUNCH_CHECK();
+        VG_HIP(hipEventRecord(c.ev_tree, st));
     }
     t.ref_valid = false;
 }
