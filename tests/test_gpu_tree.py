@@ -47,3 +47,17 @@ def test_first_tree_deeper_than_sixteen_levels(vg, orc):
             g.upload(x)
             assert_tree_equal(g.tree(), rt)
             assert_lists_equal(g.lists(), rl)
+
+
+# The lists are enqueued before the tree's size is known where twice the last tree's cells
+# are at most 2^18 (60,000 points: 114,000 cells), after it elsewhere (376,000 cells).
+@pytest.mark.parametrize("n", [60000, 200000])
+def test_lists_of_many_cells(vg, orc, n):
+    rng = np.random.default_rng(n)
+    with vg.Gravity(n, 1, 2, "f64", eps=1e-3) as g:
+        for _ in range(3):
+            x = rng.random((n, 3))
+            rt, rl = orc.tree_and_lists(x, 1)
+            g.upload(x)
+            assert_tree_equal(g.tree(), rt)
+            assert_lists_equal(g.lists(), rl)

@@ -85,18 +85,18 @@ void join_p2p(Ctx &c) {
 // whose M2L is VALU-bound too, and timed evaluations keep one stream (the
 // events of a phase then bracket its own kernels only).
 static void evaluate_overlapped(Ctx &c, bool potential) {
-    VG_HIP(hipStreamWaitEvent(c.stream2, c.ev_tree, 0));  // not the operators behind the tree
+    VG_HIP(hipStreamWaitEvent(c.stream2, c.lists_ahead ? c.ev_lists : c.ev_tree, 0));  // not the operators behind them
     struct Swap {
         Ctx &c;
         explicit Swap(Ctx &c_) : c(c_) { std::swap(c.stream, c.stream2); }
         ~Swap() { std::swap(c.stream, c.stream2); }
     };
     try {
-        {
+        if (!c.lists_ahead) {
             Swap on_stream2(c);
             lists_build(c);
+            VG_HIP(hipEventRecord(c.ev_lists, c.stream));
         }
-        VG_HIP(hipEventRecord(c.ev_lists, c.stream2));
         {
             Swap on_stream2(c);
             fmm_p2p_plan(c, potential);
@@ -137,7 +137,7 @@ void evaluate(Ctx &c, bool potential) {
     phase_end(c, PH_TREE);
     used[PH_TREE] = true;
     phase_begin(c, PH_LISTS);
-    lists_build(c);
+    if (!c.lists_ahead) lists_build(c);
     phase_end(c, PH_LISTS);
     used[PH_LISTS] = true;
     if (c.timing) {
@@ -232,9 +232,6 @@ HostLists host_lists(vg::Ctx &c) {
     h.nic = fetch(c, t.ni_cnt.p, nc);
     h.apc = fetch(c, t.ap_cnt.p, nc);
     VG_HIP(hipStreamSynchronize(c.stream));
-    uint32_t overflow = 0;
-    VG_HIP(hipMemcpy(&overflow, c.scal.p + 4, sizeof(uint32_t), hipMemcpyDeviceToHost));
-    if (overflow) throw vg::Error(VIPP_GRAV_E_DEVICE, "interaction list overflow");
     return h;
 }
 // full NI list of a cell: local entries of its ancestors, root first (solver_ref.hpp:126)

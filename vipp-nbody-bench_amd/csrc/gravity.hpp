@@ -37,6 +37,7 @@ struct TreeDev {
     DevBuf<int32_t> int_ids;         // internal cells, level by level
     DevBuf<uint32_t> int_start;      // their first positions
     DevBuf<int32_t> int_parent;      // their parents, as indices into int_ids
+    DevBuf<uint64_t> int_code;       // their path codes: the octants of their level's path, 3 bits each
     DevBuf<int32_t> leaf_ids;        // non-empty leaves
     DevBuf<uint8_t> flags;           // non-empty leaves among the cells
     DevBuf<uint32_t> leaf_cnt;       // per-block counts of these
@@ -110,6 +111,7 @@ struct Ctx {
     hipEvent_t ev_tree = nullptr;  // the tree is built and its sizes are in the pinned words
     hipEvent_t ev_plan = nullptr;  // the P2P plan scalars are in the pinned words
     bool p2p_pending = false;
+    bool lists_ahead = false;      // the lists were enqueued with the tree (ev_lists recorded)
     // pinned host words for the scalars read back during an evaluation (tree
     // level sizes, root box, P2P plan): a pinned copy returns sooner
     void *pinned = nullptr;
@@ -134,7 +136,6 @@ struct Ctx {
     DevBuf<uint64_t> key[2];
     DevBuf<uint32_t> val[2];
     DevBuf<uint32_t> rs_hist;
-    DevBuf<uint32_t> scal;      // small device scalars (counts, error flags)
     DevBuf<uint32_t> cmp_cnt;   // cells per level and block of the sorted codes
     DevBuf<uint32_t> perm;      // sorted position -> caller index
     // particles in sorted order
@@ -178,7 +179,7 @@ struct Ctx {
 };
 
 // phases (each launches on ctx.stream)
-void tree_build(Ctx &c, bool operators); // AABB, codes, sort, cells, leaves, particle gather; with the operators enqueued before it waits
+void tree_build(Ctx &c, bool ahead);     // AABB, codes, sort, cells, leaves, particle gather; ahead: operators and (lists_ahead) lists enqueued before it waits
 void lists_build(Ctx &c);                // NB / NI / AP lists and the 27-neighbour table
 void ref_numbering(Ctx &c);              // reference cell ids (for export only)
 void operators_build(Ctx &c);            // M2M / L2L / M2L operators for the current root box

@@ -177,13 +177,14 @@ __global__ __launch_bounds__(1024) void k_cells_scan(uint32_t *__restrict__ cnt,
     }
 }
 
-// The internal cells: id, first position and parent (as an internal cell), in order.
+// The internal cells: id, first position, parent (as an internal cell) and path code, in order.
 // A wavefront walks 64 R positions; lane d keeps the number of level d's cells that
 // start before the current 64, so a position's rank at each level gives the ids of
 // all its ancestors.
 __global__ __launch_bounds__(256) void k_cells_write(const uint64_t *__restrict__ key, int64_t n, uint32_t thr, int SH, int R,
                                                      const uint32_t *__restrict__ cnt, const uint32_t *__restrict__ lv, int64_t cap,
-                                                     int32_t *__restrict__ int_ids, uint32_t *__restrict__ int_start, int32_t *__restrict__ int_parent) {
+                                                     int32_t *__restrict__ int_ids, uint32_t *__restrict__ int_start, int32_t *__restrict__ int_parent,
+                                                     uint64_t *__restrict__ int_code) {
     __shared__ uint32_t s_cnt[4][MAXD + 1];
     if (!lv_cells(lv, SH, cap)) return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -210,6 +211,7 @@ __global__ __launch_bounds__(256) void k_cells_write(const uint64_t *__restrict_
                 int_ids[rank] = id;
                 int_start[rank] = static_cast<uint32_t>(i0 + 64 * r);
                 int_parent[rank] = up;
+                int_code[rank] = k >> (3 * (MAXD - d));
             }
             up = rank;
             id = 1 + 8 * rank + static_cast<int32_t>(k >> (3 * (MAXD - 1 - d)) & 7u);
@@ -507,104 +509,146 @@ __global__ __launch_bounds__(256) void k_gather(const uint32_t *__restrict__ per
 }
 
 // ---------------------------------------------------------------------------
-// Interaction lists, level by level (calc_link, solver_ref.hpp:115-162)
+// Interaction lists of all levels at once (calc_link, solver_ref.hpp:115-162)
 // ---------------------------------------------------------------------------
-__global__ void k_lists_root(const int32_t *__restrict__ child, int32_t *nb, int32_t *ni, int32_t *nb_cnt, int32_t *ni_cnt, int32_t *ap_cnt, int32_t *nbr27) {
-    if (threadIdx.x != 0) return;
-    for (int q = 0; q < 27; ++q) nbr27[q] = -1;
-    if (child[0] < 0) {  // solver_ref.hpp:149-150
-        ni[0] = 0;
-        ni_cnt[0] = 1;
-        nb_cnt[0] = 0;
-    } else {  // solver_ref.hpp:151-152
-        nb[0] = 0;
-        nb_cnt[0] = 1;
-        ni_cnt[0] = 0;
-        nbr27[13] = 0;
-    }
-    ap_cnt[0] = 0;
+// The NB list of an internal cell holds the internal cells of its level that
+// touch it or are itself: the parents of two such cells touch as well, and are
+// internal.  calc_link takes candidates in the order of the parent's NB list and
+// of their octants, and the root's list is the root, so every NB list is in the order
+// of the path codes.  So a cell's NB list needs no list of its parent: its 27
+// neighbour positions are looked up among its level's internal cells, which are in
+// the order of their path codes.  Bound by latency (a wavefront per cell: the
+// search's 5 to 17 dependent reads, then one of the candidates); one launch for
+// all levels, where a launch per level waited for the one before (and 64 candidates'
+// positions, read from memory, are now their octant and place): 500 particles 22 -> 10 us,
+// 1M at s = 64 56 to 107 -> 20.  Evaluation of 500 particles 191 -> 180 us, 16384 413 -> 380,
+// 64000 767 -> 729, 1M clustered 2.67 -> 2.55 ms.
+__device__ inline uint64_t spread3(uint32_t x) {  // bit i of 21 to bit 3 i
+    uint64_t v = x & 0x1fffffu;
+    v = (v | v << 32) & 0x1f00000000ffffull;
+    v = (v | v << 16) & 0x1f0000ff0000ffull;
+    v = (v | v << 8) & 0x100f00f00f00f00full;
+    v = (v | v << 4) & 0x10c30c30c30c30c3ull;
+    v = (v | v << 2) & 0x1249249249249249ull;
+    return v;
+}
+// Path code of a position at level d (octant bit a is set on the low side, octree.hpp:164-176).
+__device__ inline uint64_t path_code(int d, int x, int y, int z) {
+    const uint32_t m = (1u << d) - 1;
+    return spread3(~static_cast<uint32_t>(x) & m) | spread3(~static_cast<uint32_t>(y) & m) << 1 | spread3(~static_cast<uint32_t>(z) & m) << 2;
 }
 
-// Lists of the 8 children of one internal cell per wavefront (4 per block).
-// The siblings share their candidates: the children of the parent's NB
-// cells, taken in the order of solver_ref.hpp:129-147 (NB entry e, child
+// NB list of one internal cell and the NI and AP lists of its 8 children per wavefront
+// (4 per block).  The children share their candidates: the children of the
+// cell's NB cells, taken in the order of solver_ref.hpp:129-147 (NB entry e, child
 // offset q).  Lane l tests candidate 64 r + l of round r against all 8
-// siblings; each sibling's NB / NI / AP entries are appended in candidate
+// siblings; each sibling's NI / AP entries are appended in candidate
 // order through ballots and prefix popcounts, so the lists come out in the
-// reference's order.
-__global__ __launch_bounds__(256) void k_lists_level(const int32_t *__restrict__ pids, int np, const int32_t *__restrict__ child,
-                                                     const int32_t *__restrict__ grid, int32_t *__restrict__ nb, int32_t *__restrict__ ni,
-                                                     int32_t *__restrict__ ap, int32_t *__restrict__ nb_cnt, int32_t *__restrict__ ni_cnt,
-                                                     int32_t *__restrict__ ap_cnt, int32_t *__restrict__ nbr27, uint32_t *__restrict__ overflow) {
-    const int wv = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (wv >= np) return;  // whole wavefront
-    const unsigned lane = threadIdx.x & 63;
-    const uint64_t below = (1ull << lane) - 1;
-    const int32_t P = pids[wv];
-    const int32_t cb = child[P];
-    const int npn = nb_cnt[P];
-    for (int i = lane; i < 8 * 27; i += 64) nbr27[27 * static_cast<int64_t>(cb) + i] = -1;
-    int gx[8], gy[8], gz[8];
-    bool leaf[8];
-    int nbn[8], nin[8], apn[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        gx[t] = grid[3 * (cb + t)];
-        gy[t] = grid[3 * (cb + t) + 1];
-        gz[t] = grid[3 * (cb + t) + 2];
-        leaf[t] = child[cb + t] < 0;
-        nbn[t] = nin[t] = apn[t] = 0;
+// reference's order.  An entry needs no bound check: a cell has 27 positions
+// around it, and 8 x 27 candidates of which its 27 are not AP.
+__global__ __launch_bounds__(256) void k_lists(const uint32_t *__restrict__ lv, int SH, int64_t cap, const int32_t *__restrict__ int_ids,
+                                               const uint64_t *__restrict__ int_code, const int8_t *__restrict__ level, const int32_t *__restrict__ child,
+                                               const int32_t *__restrict__ grid, int32_t *__restrict__ nb, int32_t *__restrict__ ni, int32_t *__restrict__ ap,
+                                               int32_t *__restrict__ nb_cnt, int32_t *__restrict__ ni_cnt, int32_t *__restrict__ ap_cnt,
+                                               int32_t *__restrict__ nbr27) {
+    __shared__ int32_t s_r[4][28], s_o[4][28];
+    const int64_t nc = lv_cells(lv, SH, cap), nint = nc / 8;  // nc = 1 + 8 nint
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && nc > 0) {  // the root (solver_ref.hpp:149-152); with children, its NB list is its own wavefront's
+        ap_cnt[0] = 0;
+        ni_cnt[0] = nint ? 0 : 1;
+        if (nint == 0) {
+            ni[0] = 0;
+            nb_cnt[0] = 0;
+        }
     }
+    const int64_t r = blockIdx.x * 4ll + w;
+    if (r >= nint) return;  // whole wavefront
+    const int32_t P = int_ids[r], cb = static_cast<int32_t>(1 + 8 * r);
+    const int d = level[P];
+    const int px = grid[3 * P], py = grid[3 * P + 1], pz = grid[3 * P + 2];
+    bool leaf[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) leaf[t] = child[cb + t] < 0;
+    // lane l < 27: the internal cell at offset (l % 3 - 1, l / 3 % 3 - 1, l / 9 - 1), as an entry of int_ids, or -1
+    int32_t found = -1;
+    {
+        const int x = px + lane % 3 - 1, y = py + lane / 3 % 3 - 1, z = pz + lane / 9 - 1, side = 1 << d;
+        if (lane < 27 && x >= 0 && x < side && y >= 0 && y < side && z >= 0 && z < side) {
+            const uint64_t code = path_code(d, x, y, z);
+            uint32_t lo = lv[LV_I + d], hi = lv[LV_I + d + 1];  // the last cell whose code is not above
+            while (lo + 1 < hi) {
+                const uint32_t mid = (lo + hi) / 2;
+                if (int_code[mid] <= code)
+                    lo = mid;
+                else
+                    hi = mid;
+            }
+            if (int_code[lo] == code) found = static_cast<int32_t>(lo);
+        }
+    }
+    int at = 0;  // its place in the NB list
+    const int npn = __popcll(__ballot(found >= 0));
+    for (int l = 0; l < 27; ++l) {
+        const int32_t o = __builtin_amdgcn_readlane(found, l);
+        at += o >= 0 && o < found;
+    }
+    if (lane < 27) {
+        int32_t id = -1;
+        if (found >= 0) {
+            id = int_ids[found];
+            s_r[w][at] = found;
+            s_o[w][at] = lane;
+            nb[27 * static_cast<int64_t>(P) + at] = id;
+        }
+        nbr27[27 * static_cast<int64_t>(P) + lane] = id;
+    }
+    if (lane == 0) nb_cnt[P] = npn;
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const uint64_t below = (1ull << lane) - 1;
+    int nin[8], apn[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) nin[t] = apn[t] = 0;
     const int ncand = 8 * npn;
     for (int r0 = 0; r0 < ncand; r0 += 64) {
-        const int cand = r0 + static_cast<int>(lane);
+        const int cand = r0 + lane, q = lane & 7;
         const bool valid = cand < ncand;
         int32_t cc = 0;
-        int cx = 0, cy = 0, cz = 0;
+        int cx = 0, cy = 0, cz = 0;  // position relative to the first child position of P
         bool cint = false;
         if (valid) {
-            cc = child[nb[27 * static_cast<int64_t>(P) + cand / 8]] + cand % 8;
-            cx = grid[3 * cc];
-            cy = grid[3 * cc + 1];
-            cz = grid[3 * cc + 2];
+            const int o = s_o[w][cand / 8];
+            cc = 1 + 8 * s_r[w][cand / 8] + q;
+            cx = 2 * (o % 3 - 1) + 1 - (q & 1);
+            cy = 2 * (o / 3 % 3 - 1) + 1 - (q >> 1 & 1);
+            cz = 2 * (o / 9 - 1) + 1 - (q >> 2);
             cint = child[cc] >= 0;
         }
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
             const int32_t ct = cb + t;
-            const int dx = cx - gx[t], dy = cy - gy[t], dz = cz - gz[t];
+            const int dx = cx - (1 - (t & 1)), dy = cy - (1 - (t >> 1 & 1)), dz = cz - (1 - (t >> 2));
             const bool adj = dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1 && dz >= -1 && dz <= 1;  // fmm.hpp:475-493
-            const bool isnb = valid && adj && !leaf[t] && cint;
-            const bool isni = valid && adj && !isnb;
+            const bool isni = valid && adj && (leaf[t] || !cint);
             const bool isap = valid && !adj;
-            const uint64_t mnb = __ballot(isnb), mni = __ballot(isni), map = __ballot(isap);
-            if (isnb) {
-                const int k = nbn[t] + __popcll(mnb & below);
-                if (k < 27) nb[27 * static_cast<int64_t>(ct) + k] = cc;
-                nbr27[27 * static_cast<int64_t>(ct) + (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)] = cc;
-            }
-            if (isni) {
-                const int k = nin[t] + __popcll(mni & below);
-                if (k < 27) ni[27 * static_cast<int64_t>(ct) + k] = cc;
-            }
-            if (isap) {
-                const int k = apn[t] + __popcll(map & below);
-                if (k < 189) ap[189 * static_cast<int64_t>(ct) + k] = cc;
-            }
-            nbn[t] += __popcll(mnb);
+            const uint64_t mni = __ballot(isni), map = __ballot(isap);
+            if (isni) ni[27 * static_cast<int64_t>(ct) + nin[t] + __popcll(mni & below)] = cc;
+            if (isap) ap[189 * static_cast<int64_t>(ct) + apn[t] + __popcll(map & below)] = cc;
             nin[t] += __popcll(mni);
             apn[t] += __popcll(map);
         }
     }
     if (lane < 8) {
-        int a = 0, b = 0, d = 0;
+        int b = 0, e = 0;
+        bool lf = false;
 #pragma unroll
         for (int t = 0; t < 8; ++t)
-            if (lane == static_cast<unsigned>(t)) a = nbn[t], b = nin[t], d = apn[t];
-        if (a > 27 || b > 27 || d > 189) atomicOr(overflow, 1u);
-        nb_cnt[cb + lane] = min(a, 27);
-        ni_cnt[cb + lane] = min(b, 27);
-        ap_cnt[cb + lane] = min(d, 189);
+            if (lane == t) b = nin[t], e = apn[t], lf = leaf[t];
+        if (lf) nb_cnt[cb + lane] = 0;  // an internal child has its own wavefront
+        ni_cnt[cb + lane] = b;
+        ap_cnt[cb + lane] = e;
     }
 }
 
@@ -704,19 +748,36 @@ static void ensure_cells(TreeDev &t, int64_t ncell) {
     t.int_ids.ensure(ncell / 8 + 1);
     t.int_start.ensure(ncell / 8 + 1);
     t.int_parent.ensure(ncell / 8 + 1);
+    t.int_code.ensure(ncell / 8 + 1);
 }
 
-// With operators, the operators (which need the root box alone) are enqueued
-// behind the tree before the host waits for its sizes: the device forms them while
-// the host wakes up and launches the lists.
-void tree_build(Ctx &c, bool operators) {
+// The lists of a tree of at most cap cells, whose sizes the level table holds.
+static void lists_enqueue(Ctx &c, int SH, int64_t cap) {
+    TreeDev &t = c.t;
+    t.nb.ensure(27 * cap);
+    t.ni.ensure(27 * cap);
+    t.ap.ensure(189 * cap);
+    t.nb_cnt.ensure(cap);
+    t.ni_cnt.ensure(cap);
+    t.ap_cnt.ensure(cap);
+    t.nbr27.ensure(27 * cap);
+    k_lists<<<ceil_div(std::max<int64_t>(1, cap / 8), 4), 256, 0, c.stream>>>(t.lv, SH, cap, t.int_ids, t.int_code, t.level, t.child, t.grid, t.nb, t.ni,
+                                                                            t.ap, t.nb_cnt, t.ni_cnt, t.ap_cnt, t.nbr27);
+    VG_LAUNCH_CHECK();
+}
+
+// With ahead, the operators (which need the root box alone) and the lists of trees of
+// up to AHEAD_CELLS cells (room for the lists of twice the last tree's cells: at most
+// 283 MB) are enqueued behind the tree before the host waits for its sizes: the
+// device forms them while the host wakes up.
+constexpr int64_t AHEAD_CELLS = 1 << 18;
+void tree_build(Ctx &c, bool ahead) {
     hipStream_t st = c.stream;
     TreeDev &t = c.t;
     const int64_t n = c.n;
     // 1. root box
     //    (the RK4 stage that wrote x may have left its partial boxes)
     c.box.ensure(8);
-    c.scal.ensure(16);
     if (c.aabb_parts > 0) {
         k_aabb_final<<<1, 256, 0, st>>>(c.aabb_part, c.aabb_parts, c.box);
     } else {
@@ -741,15 +802,6 @@ void tree_build(Ctx &c, bool operators) {
     double *hbox = static_cast<double *>(c.pinned);                                     // 8 doubles
     uint32_t *hlv = reinterpret_cast<uint32_t *>(static_cast<char *>(c.pinned) + 512);  // LV_WORDS pinned host words
     static_assert(512 + 4 * LV_WORDS <= Ctx::PINNED_BYTES, "pinned words");
-    auto read_back = [&] {
-        VG_HIP(hipMemcpyAsync(hbox, c.box, 7 * sizeof(double), hipMemcpyDeviceToHost, st));
-        VG_HIP(hipMemcpyAsync(hlv, t.lv, LV_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-        VG_HIP(hipEventRecord(c.ev_tree, st));
-        if (operators) operators_build(c);
-        operators = false;
-        VG_HIP(hipEventSynchronize(c.ev_tree));
-        if (hbox[6] != 0) throw Error(2, "non-finite particle coordinates");
-    };
     // 2. path codes and a stable sort of the octants of levels 1..SH (bits below
     //    the deepest level do not matter: leaves are re-sorted by caller index): two
     //    levels beyond the previous tree's depth (consecutive evaluations differ
@@ -773,7 +825,7 @@ void tree_build(Ctx &c, bool operators) {
     };
     // 4. cells, the non-empty leaves, leaf order by caller index, particles in sorted order
     auto cells = [&] {
-        if (n > c.thr) k_cells_write<<<nb, 256, 0, st>>>(k0, n, c.thr, SH, R, c.cmp_cnt, t.lv, cap, t.int_ids, t.int_start, t.int_parent);
+        if (n > c.thr) k_cells_write<<<nb, 256, 0, st>>>(k0, n, c.thr, SH, R, c.cmp_cnt, t.lv, cap, t.int_ids, t.int_start, t.int_parent, t.int_code);
         k_cells_expand<<<ceil_div(cap, 256), 256, 0, st>>>(k0, n, c.thr, SH, t.lv, cap, t.int_ids, t.int_start, t.int_parent, c.box, t.start, t.count, t.child,
                                                            t.parent, t.octant, t.level, t.bmin, t.bmax, t.grid, t.anc, t.flags);
         if (cap <= LEAF_BLOCK) {
@@ -793,6 +845,21 @@ void tree_build(Ctx &c, bool operators) {
                 t.leaf_ids, t.lv, t.start, t.count, c.thr, v0, c.perm, c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.box, c.xs64, c.xs32);
         }
         VG_LAUNCH_CHECK();
+    };
+    bool operators = false;  // enqueued
+    auto read_back = [&] {
+        VG_HIP(hipMemcpyAsync(hbox, c.box, 7 * sizeof(double), hipMemcpyDeviceToHost, st));
+        VG_HIP(hipMemcpyAsync(hlv, t.lv, LV_WORDS * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+        VG_HIP(hipEventRecord(c.ev_tree, st));
+        c.lists_ahead = ahead && cap > 0 && cap <= AHEAD_CELLS;
+        if (c.lists_ahead) {
+            lists_enqueue(c, SH, cap);
+            VG_HIP(hipEventRecord(c.ev_lists, st));
+        }
+        if (ahead && !operators) operators_build(c);
+        operators = true;
+        VG_HIP(hipEventSynchronize(c.ev_tree));
+        if (hbox[6] != 0) throw Error(2, "non-finite particle coordinates");
     };
     for (;;) {
         sort_and_count();
@@ -830,27 +897,7 @@ void tree_build(Ctx &c, bool operators) {
     t.ref_valid = false;
 }
 
-void lists_build(Ctx &c) {
-    hipStream_t st = c.stream;
-    TreeDev &t = c.t;
-    const int64_t nc = t.ncells;
-    t.nb.ensure(27 * nc);
-    t.ni.ensure(27 * nc);
-    t.ap.ensure(189 * nc);
-    t.nb_cnt.ensure(nc);
-    t.ni_cnt.ensure(nc);
-    t.ap_cnt.ensure(nc);
-    t.nbr27.ensure(27 * nc);
-    VG_HIP(hipMemsetAsync(c.scal.p + 4, 0, sizeof(uint32_t), st));
-    k_lists_root<<<1, 64, 0, st>>>(t.child, t.nb, t.ni, t.nb_cnt, t.ni_cnt, t.ap_cnt, t.nbr27);
-    for (int d = 1; d <= t.depth; ++d) {  // children at level d of the internal cells of level d - 1
-        const int64_t a = t.int_off[d - 1], b = t.int_off[d];
-        if (b > a)
-            k_lists_level<<<ceil_div(b - a, 4), 256, 0, st>>>(t.int_ids.p + a, static_cast<int>(b - a), t.child, t.grid, t.nb, t.ni, t.ap, t.nb_cnt,
-                                                              t.ni_cnt, t.ap_cnt, t.nbr27, c.scal.p + 4);
-    }
-    VG_LAUNCH_CHECK();
-}
+void lists_build(Ctx &c) { lists_enqueue(c, MAXD, c.t.ncells); }
 
 void ref_numbering(Ctx &c) {
     hipStream_t st = c.stream;
