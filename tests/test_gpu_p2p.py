@@ -75,3 +75,21 @@ def test_p2p_f32_beyond_the_range_of_squared_distances(vg):
     ref = (w[..., None] * d).sum(1)
     assert np.isfinite(a).all()
     assert np.linalg.norm(a - ref) <= BOUND * np.linalg.norm(ref)
+
+
+# floor(sqrt(8) s) = 181 and 4242: leaves put in order by a wavefront each, and by a block each after the tree's sizes are known
+@pytest.mark.parametrize("s", [64, 1500])
+@pytest.mark.parametrize("mode", ["f64", "f32", "split"])
+def test_streams_equal_one_stream(vg, mode, s):
+    """Per-phase timing keeps one stream: the same results bit for bit, evaluation after evaluation."""
+    rng = np.random.default_rng(s)
+    n, runs = 12000, []
+    x = [rng.random((n, 3)) for _ in range(3)]
+    for timing in (False, True):
+        with vg.Gravity(n, s, 5, mode, eps=1e-3) as g:
+            g.set_timing(timing)
+            for y in x:
+                g.upload(y)
+                runs.append((g.accelerations(), g.energy()))
+    for a, b in zip(runs[:3], runs[3:]):
+        assert np.array_equal(a[0], b[0]) and a[1] == b[1]

@@ -892,7 +892,7 @@ void tree_build(Ctx &c, bool ahead) {
         k_leaf_sort<<<static_cast<unsigned>(t.nleaves), 256, c.thr * sizeof(uint32_t), st>>>(t.leaf_ids, t.start, t.count, v0, c.perm);
         k_gather<<<ceil_div(n, 256), 256, 0, st>>>(c.perm, n, c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.box, c.xs64, c.xs32);
         VG_LAUNCH_CHECK();
-        VG_HIP(hipEventRecord(c.ev_tree, st));
+        VG_HIP(hipEventRecord(c.lists_ahead ? c.ev_lists : c.ev_tree, st));  // what P2P waits for has these particles in order
     }
     t.ref_valid = false;
 }
