@@ -76,14 +76,16 @@ void join_p2p(Ctx &c) {
     c.p2p_pending = false;
 }
 
-// Untimed split-mode evaluations run the lists and P2P (VALU-bound, about
-// half the evaluation) on a second stream once the tree exists, so that the
-// operators (enqueued by tree_build) and the upward pass (which need only the
-// tree), and M2L (MFMA-bound, after the lists), run beside them; L2P waits for
-// P2P. The P2P plan is enqueued with the lists and its item counts are read back
-// while the host enqueues the upward pass. The FP32 and FP64 modes,
-// whose M2L is VALU-bound too, and timed evaluations keep one stream (the
-// events of a phase then bracket its own kernels only).
+// Untimed evaluations run the P2P (and the lists of large trees) on a second stream, so
+// that the upward pass, which needs only the tree, and M2L, which needs the lists,
+// run beside it; L2P waits for P2P.  P2P is bound by VALU issue and M2L by the
+// matrix cores (FP64: both by VALU issue), and on trees of up to a million particles neither
+// has work for every CU at all times.  One stream against two: FP32 64,000 particles
+// 2.91 -> 2.54 ms an RK4 step, 2^20 uniform 8.13 -> 7.93, 10^6 Plummer p = 12 17.4
+// -> 17.1, FP64 16384 1.52 -> 1.34, 500 alike.  The P2P plan is enqueued with the lists and
+// its item counts are read back while the host enqueues the upward pass.
+// Timed evaluations keep one stream (the events of a phase then bracket its own
+// kernels only).
 static void evaluate_overlapped(Ctx &c, bool potential) {
     VG_HIP(hipStreamWaitEvent(c.stream2, c.lists_ahead ? c.ev_lists : c.ev_tree, 0));  // not the operators behind them
     struct Swap {
@@ -126,26 +128,24 @@ void evaluate(Ctx &c, bool potential) {
     c.evaluated = false;
     c.t.ref_valid = false;
     bool used[PH_COUNT] = {};
-    if (!c.timing && c.stream2 && c.prec == 2) {
+    if (!c.timing) {
         tree_build(c, true);
         evaluate_overlapped(c, potential);
         c.evaluated = true;
         return;
     }
     phase_begin(c, PH_TREE);
-    tree_build(c, !c.timing);
+    tree_build(c, false);
     phase_end(c, PH_TREE);
     used[PH_TREE] = true;
     phase_begin(c, PH_LISTS);
-    if (!c.lists_ahead) lists_build(c);
+    lists_build(c);
     phase_end(c, PH_LISTS);
     used[PH_LISTS] = true;
-    if (c.timing) {
-        phase_begin(c, PH_OPS);
-        operators_build(c);
-        phase_end(c, PH_OPS);
-        used[PH_OPS] = true;
-    }
+    phase_begin(c, PH_OPS);
+    operators_build(c);
+    phase_end(c, PH_OPS);
+    used[PH_OPS] = true;
     phase_begin(c, PH_UP);
     fmm_upward(c);
     phase_end(c, PH_UP);

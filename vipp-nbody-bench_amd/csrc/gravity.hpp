@@ -103,9 +103,9 @@ struct Ctx {
     std::string err;
 
     hipStream_t stream = nullptr;
-    // split mode: the lists and P2P run on stream2 beside the upward pass and
+    // P2P (and the lists of large trees) run on stream2 beside the upward pass and
     // M2L of the same evaluation (they share no buffer); M2L waits for the
-    // lists (ev_lists), the scatter for P2P (join_p2p)
+    // lists (ev_lists), L2P for P2P (join_p2p)
     hipStream_t stream2 = nullptr;
     hipEvent_t ev_join = nullptr, ev_lists = nullptr;
     hipEvent_t ev_tree = nullptr;  // the tree is built and its sizes are in the pinned words
