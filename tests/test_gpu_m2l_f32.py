@@ -36,3 +36,39 @@ def test_f32_locals_match_f64(vg, p, n, s):
     a, b = L["f64"], L["f32"]
     scale = np.abs(a).max(axis=(1, 2), keepdims=True) + 1e-300
     assert (np.abs(a - b) / scale).max() < 2e-5
+
+
+# M2M and L2L on the matrix cores: 16 parents a tile on levels of few parents, two
+# tiles where a level has hundreds (leaves of 11 points); same bound for both expansions.
+@pytest.mark.parametrize("p", range(1, 13))
+@pytest.mark.parametrize("n,s", [(700, 40), (30011, 4)])
+def test_f32_expansions_match_f64(vg, p, n, s):
+    rng = np.random.default_rng(100 + p)
+    x = np.concatenate([0.05 * rng.standard_normal((n // 3, 3)), rng.random((n - n // 3, 3))])
+    m = rng.uniform(0.5, 1.5, n) / n
+    E = {}
+    for mode in ("f64", "f32"):
+        with vg.Gravity(n, s, p, mode, eps=1e-3) as g:
+            g.upload(x, None, m)
+            g.accelerations(copy=False)
+            E[mode] = g.expansions()
+    for a, b in zip(E["f64"][:2], E["f32"][:2]):
+        scale = np.abs(a).max(axis=(1, 2), keepdims=True) + 1e-300
+        assert (np.abs(a - b) / scale).max() < 2e-5
+
+
+def test_fallback_order_changes(vg):
+    """The closure's fallback order may change in a context: the operators' padding belongs to an order."""
+    import closure
+    rng = np.random.default_rng(4)
+    x = rng.random((20000, 3))
+    params = closure.init_params(1)
+
+    def forces(orders):
+        with vg.Gravity(len(x), 24, 4, "f32", eps=1e-3) as g:
+            g.upload(x)
+            for p in orders:
+                g.set_closure(params, bound=0.0, p_fallback=p)
+                a = g.accelerations()
+        return a
+    assert np.array_equal(forces([12, 8, 10]), forces([10]))

@@ -32,6 +32,7 @@ void swap_expansions(Ctx &c, ExpSet &e) {
     std::swap(c.p, e.p);
     std::swap(c.K, e.K);
     std::swap(c.ldk, e.ldk);
+    std::swap(c.frag_K, e.frag_K);
     c.harm.swap(e.harm);
     c.op64.swap(e.op64);
     c.op32.swap(e.op32);

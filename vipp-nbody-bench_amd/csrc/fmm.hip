@@ -154,10 +154,21 @@ struct OpFrag {
     }
 };
 
+// FP32 M2M and L2L operators, in the order in which k_ml_f32's lanes read them: fragments
+// as above, but lane 16 q + row holds the columns 4 i + q, i = 0 .. 3, so that the
+// products go through the columns in order.
+struct MlFrag {
+    int nt;
+    __host__ __device__ explicit MlFrag(int K) : nt((K + 15) / 16) {}
+    __host__ __device__ size_t size() const { return static_cast<size_t>(nt) * nt * 256; }
+    __host__ __device__ size_t at(int r, int c) const { return (static_cast<size_t>((r >> 4) * nt + (c >> 4)) * 64 + (c & 3) * 16 + (r & 15)) * 4 + (c & 15) / 4; }
+};
+
 // op block layout: [M2M 0..7][L2L 8..15][M2L 16..16+342], each K*K; M2L
-// blocks row-major [row][col] (or, with frag, OpFrag's order there), M2M and
-// L2L blocks column-major [col][row] (their kernels give each lane one output
-// row, so lanes then read consecutive words).
+// blocks row-major [row][col], M2M and L2L blocks column-major [col][row] (their
+// kernels give each lane one output row, so lanes then read consecutive words).
+// With frag (FP32): M2M and L2L blocks in op in MlFrag's order, M2L blocks in frag
+// in OpFrag's; what no column pair fills stays as it is there, zero.
 // One block per (operator, OPS_ROWS rows), 128 threads per row r; thread t of
 // a row takes the column pair (n, m >= 0) number t, i.e. the real-packed
 // columns of degree n, order m.
@@ -170,7 +181,8 @@ __global__ __launch_bounds__(128 * OPS_ROWS) void k_ops(const int16_t *__restric
     const int t = threadIdx.x & 127;
     const bool cmaj = blk < 16;
     const OpFrag fr(K);
-    const bool fragment = frag && !cmaj;  // every column is written below, the padding stays zero
+    const MlFrag ml(K);
+    const bool fragment = frag != nullptr;
     R *dst = cmaj ? op + static_cast<size_t>(blk) * K * K + r : op + (static_cast<size_t>(blk) * K + r) * K;
     const size_t cs = cmaj ? static_cast<size_t>(K) : 1;  // column stride
     if (r < K && !fragment)
@@ -227,7 +239,9 @@ __global__ __launch_bounds__(128 * OPS_ROWS) void k_ops(const int16_t *__restric
     }
     // the pair's real-packed columns (each written by this thread only)
     auto put = [&](int c, double v) {
-        if (fragment)
+        if (fragment && cmaj)
+            op[blk * ml.size() + ml.at(r, c)] = static_cast<R>(v);
+        else if (fragment)
             frag[(blk - 16) * fr.size() + fr.at(r, c)] = static_cast<R>(v);
         else
             dst[c * cs] = static_cast<R>(v);
@@ -376,22 +390,21 @@ __global__ __launch_bounds__(256) void k_p2m(const int32_t *__restrict__ leaves,
     for (int q = K + lane; q < ldk; q += 64) out[q] = R(0);
 }
 
-// M2M for the internal cells of one level (solver_ref.hpp:196-197).
-// M2M / L2L of one tree level, PB parents per block: every operator word read
+// FP64 M2M (solver_ref.hpp:196-197) and L2L of the internal cells of one tree level, PB parents per block: every operator word read
 // from L2 serves PB parents, and PB is chosen per level (pick_pb) so that the
 // launch still has enough blocks to fill the chip.  Operator blocks are
 // column-major, so the lanes (output rows) read consecutive words; the
 // staged expansions are [col][parent] so a lane reads its PB inputs as vectors.
-template <class R, int PB>
+template <int PB>
 __global__ __launch_bounds__(256) void k_m2m(const int32_t *__restrict__ ids, int nids, const int32_t *__restrict__ child,
-                                             const uint32_t *__restrict__ count, const R *__restrict__ op, int K, int ldk, R *__restrict__ M) {
-    __shared__ R cm[8 * MAXK][PB];  // [child q][col][parent]
+                                             const uint32_t *__restrict__ count, const double *__restrict__ op, int K, int ldk, double *__restrict__ M) {
+    __shared__ double cm[8 * MAXK][PB];  // [child q][col][parent]
     const int p0 = blockIdx.x * PB;
     const int np = min(PB, nids - p0);
     for (int i = threadIdx.x; i < PB * 8 * K; i += 256) {
         const int u = i % PB, qc = i / PB;  // qc = q K + col
         const int q = qc / K, col = qc % K;
-        R v = 0;
+        double v = 0;
         if (u < np) {
             const int32_t cb = child[ids[p0 + u]] + q;
             if (count[cb]) v = M[static_cast<size_t>(cb) * ldk + col];
@@ -403,13 +416,13 @@ __global__ __launch_bounds__(256) void k_m2m(const int32_t *__restrict__ ids, in
         int j = 0;
         while ((j + 1) * (j + 1) <= r) ++j;
         const int cend = (j + 1) * (j + 1);  // output degree j uses child degrees <= j
-        R acc[PB];
+        double acc[PB];
 #pragma unroll
         for (int u = 0; u < PB; ++u) acc[u] = 0;
         for (int q = 0; q < 8; ++q) {
-            const R *ocol = op + static_cast<size_t>(q) * K * K + r;
+            const double *ocol = op + static_cast<size_t>(q) * K * K + r;
             for (int col = 0; col < cend; ++col) {
-                const R a = ocol[static_cast<size_t>(col) * K];
+                const double a = ocol[static_cast<size_t>(col) * K];
 #pragma unroll
                 for (int u = 0; u < PB; ++u) acc[u] += a * cm[q * K + col][u];  // empty children are zero
             }
@@ -419,30 +432,30 @@ __global__ __launch_bounds__(256) void k_m2m(const int32_t *__restrict__ ids, in
             if (u < np) M[static_cast<size_t>(ids[p0 + u]) * ldk + r] = acc[u];
     }
     for (int i = K + threadIdx.x; i < ldk; i += 256)
-        for (int u = 0; u < np; ++u) M[static_cast<size_t>(ids[p0 + u]) * ldk + i] = R(0);
+        for (int u = 0; u < np; ++u) M[static_cast<size_t>(ids[p0 + u]) * ldk + i] = 0.0;
 }
 
-template <class R, int PB>
+template <int PB>
 __global__ __launch_bounds__(256) void k_l2l(const int32_t *__restrict__ ids, int nids, const int32_t *__restrict__ child,
-                                             const uint32_t *__restrict__ count, const R *__restrict__ op, int K, int ldk, R *__restrict__ L) {
-    __shared__ R pl[MAXK][PB];  // [col][parent]
+                                             const uint32_t *__restrict__ count, const double *__restrict__ op, int K, int ldk, double *__restrict__ L) {
+    __shared__ double pl[MAXK][PB];  // [col][parent]
     const int p0 = blockIdx.x * PB;
     const int np = min(PB, nids - p0);
     for (int i = threadIdx.x; i < PB * K; i += 256) {
         const int u = i % PB, col = i / PB;
-        pl[col][u] = u < np ? L[static_cast<size_t>(ids[p0 + u]) * ldk + col] : R(0);
+        pl[col][u] = u < np ? L[static_cast<size_t>(ids[p0 + u]) * ldk + col] : 0.0;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 8 * K; i += 256) {
         const int q = i / K, r = i % K;
-        const R *ocol = op + static_cast<size_t>(8 + q) * K * K + r;
+        const double *ocol = op + static_cast<size_t>(8 + q) * K * K + r;
         int j = 0;
         while ((j + 1) * (j + 1) <= r) ++j;
-        R acc[PB];
+        double acc[PB];
 #pragma unroll
         for (int u = 0; u < PB; ++u) acc[u] = 0;
         for (int col = j * j; col < K; ++col) {  // parent degrees >= j
-            const R a = ocol[static_cast<size_t>(col) * K];
+            const double a = ocol[static_cast<size_t>(col) * K];
 #pragma unroll
             for (int u = 0; u < PB; ++u) acc[u] += a * pl[col][u];
         }
@@ -825,6 +838,98 @@ __global__ __launch_bounds__(256, 2) void k_m2l_f32(const int32_t *__restrict__ 
     if constexpr (S::NT & 1) put(S::NT - 1, wr, sum[S::H][0]);
 }
 
+// ---------------------------------------------------------------------------
+// FP32 M2M (UP, solver_ref.hpp:196-197) and L2L (solver_ref.hpp:217-218) of one tree
+// level on v_mfma_f32_16x16x4.  A block takes one 16-row tile of 16 TN parents, a
+// wavefront each octant q: M2M multiplies child q's multipoles and the block adds the 8
+// products in octant order, L2L adds its product to child q's locals.  The operands of
+// four column groups at a time come from L2 straight into registers, without
+// LDS, and the column groups that the operator's triangle leaves empty are skipped
+// (M2M: degrees above the rows' last, L2L: below their first).  Products go
+// through the columns in order, so the sums are those of an FMA per column.
+// Most levels are small, and bound by the latency of one pass: a lane per operator row
+// with one column after the other (k_m2m_wide's form) took up to 43 us a level, where
+// this takes 6 to 13.  L2L per evaluation, then and now: 10^6 Plummer p = 12 301 -> 132 us,
+// 64,000 p = 8 50 -> 30, 2^20 uniform p = 8 62 -> 41; RK4 steps 17.1 -> 16.3, 2.49 -> 2.39 and
+// 7.92 -> 7.73 ms.
+// ---------------------------------------------------------------------------
+template <int P, int TN, bool UP>
+__global__ __launch_bounds__(512) void k_ml_f32(const int32_t *__restrict__ ids, int n, const int32_t *__restrict__ child,
+                                                const uint32_t *__restrict__ count, const f4 *__restrict__ op, float *__restrict__ X) {
+    using S = M2lShape<P>;
+    constexpr int NB = 4;  // column groups in flight
+    const int lane = threadIdx.x & 63, col = lane & 15, quad = lane >> 4;
+    const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rt = blockIdx.x % S::NT, p0 = blockIdx.x / S::NT * 16 * TN;
+    int32_t cell[TN], par[TN];  // child q (-1: empty or none) and parent of column 16 t + col
+    const float *src[TN];
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+        const int i = p0 + 16 * t + col;
+        par[t] = i < n ? ids[i] : -1;
+        cell[t] = par[t] >= 0 ? child[par[t]] + q : -1;
+        if (cell[t] >= 0 && count[cell[t]] == 0) cell[t] = -1;
+        const int32_t from = UP || cell[t] < 0 ? cell[t] : par[t];
+        src[t] = from >= 0 ? X + static_cast<size_t>(from) * S::LD : nullptr;
+    }
+    int g0 = 0, g1 = S::NT;  // column groups that hold something
+    {
+        const int r = UP ? min(16 * rt + 15, S::K - 1) : 16 * rt;
+        int j = 0;  // degree of row r
+        while ((j + 1) * (j + 1) <= r) ++j;
+        if (UP)
+            g1 = ((j + 1) * (j + 1) + 15) / 16;
+        else
+            g0 = j * j / 16;
+    }
+    const f4 *A = op + (static_cast<size_t>(UP ? q : 8 + q) * S::NT + rt) * S::NT * 64;
+    const f4 zero = {0, 0, 0, 0};
+    f4 acc[TN];
+#pragma unroll
+    for (int t = 0; t < TN; ++t) acc[t] = zero;
+    for (int g = g0; g < g1; g += NB) {
+        f4 a[NB], b[NB][TN];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+            a[u] = g + u < g1 ? A[(g + u) * 64 + lane] : zero;
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int k = 16 * (g + u) + 4 * i + quad;
+                    b[u][t][i] = g + u < g1 && src[t] && k < S::K ? src[t][k] : 0.0f;
+                }
+        }
+#pragma unroll
+        for (int u = 0; u < NB; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int t = 0; t < TN; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][i], b[u][t][i], acc[t], 0, 0, 0);
+    }
+    // lane: rows 16 rt + 4 quad .. + 3 of column 16 t + col
+    const int w = 4 * rt + quad;
+    if constexpr (UP) {
+        __shared__ f4 s_acc[8][TN][64];
+#pragma unroll
+        for (int t = 0; t < TN; ++t) s_acc[q][t][lane] = acc[t];
+        __syncthreads();
+        if (q < TN) {  // wavefront t adds the octants' products of its 16 parents
+            f4 sum = s_acc[0][q][lane];
+#pragma unroll
+            for (int o = 1; o < 8; ++o) sum += s_acc[o][q][lane];
+            const int i = p0 + 16 * q + col;
+            if (i < n && w < S::LD4) reinterpret_cast<f4 *>(X)[static_cast<size_t>(ids[i]) * S::LD4 + w] = sum;
+        }
+    } else {
+        if (w < S::LD4) {
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+                if (cell[t] >= 0) reinterpret_cast<f4 *>(X)[static_cast<size_t>(cell[t]) * S::LD4 + w] += acc[t];
+        }
+    }
+}
+
 // The nsplit partial sums of each non-empty M2L target into its local
 // expansion, in part order (one thread per target slot and coefficient).
 template <class R>
@@ -943,7 +1048,6 @@ template <>
 struct Bufs<double> {
     static double *M(Ctx &c) { return c.M64; }
     static double *L(Ctx &c) { return c.L64; }
-    static double *op(Ctx &c) { return c.op64; }
     static double *acc(Ctx &c) { return c.as64; }
     static void ensure(Ctx &c, size_t nc) {
         c.M64.ensure(nc * c.ldk + 16);
@@ -954,7 +1058,6 @@ template <>
 struct Bufs<float> {
     static float *M(Ctx &c) { return c.M32; }
     static float *L(Ctx &c) { return c.L32; }
-    static float *op(Ctx &c) { return c.op32; }
     static float *acc(Ctx &c) { return c.as32; }
     static void ensure(Ctx &c, size_t nc) {
         c.M32.ensure(nc * c.ldk + 16);
@@ -965,40 +1068,38 @@ struct Bufs<float> {
 // One parent per 1024-thread block, for the small levels near the root: the
 // (child q, row r) items are spread over the threads; M2M then adds the 8
 // children's partial rows through LDS.
-template <class R>
 __global__ __launch_bounds__(1024) void k_m2m_wide(const int32_t *__restrict__ ids, const int32_t *__restrict__ child, const uint32_t *__restrict__ count,
-                                                   const R *__restrict__ op, int K, int ldk, R *__restrict__ M) {
-    __shared__ R cm[8 * MAXK];
-    __shared__ R part[8 * MAXK];
+                                                   const double *__restrict__ op, int K, int ldk, double *__restrict__ M) {
+    __shared__ double cm[8 * MAXK];
+    __shared__ double part[8 * MAXK];
     const int32_t P = ids[blockIdx.x];
     const int32_t cb = child[P];
     for (int i = threadIdx.x; i < 8 * K; i += 1024) {
         const int q = i / K, col = i % K;
-        cm[i] = count[cb + q] ? M[static_cast<size_t>(cb + q) * ldk + col] : R(0);
+        cm[i] = count[cb + q] ? M[static_cast<size_t>(cb + q) * ldk + col] : double(0);
     }
     __syncthreads();
     for (int i = threadIdx.x; i < 8 * K; i += 1024) {
         const int q = i / K, r = i % K;
         int j = 0;
         while ((j + 1) * (j + 1) <= r) ++j;
-        const R *ocol = op + static_cast<size_t>(q) * K * K + r;
-        R sum = 0;
+        const double *ocol = op + static_cast<size_t>(q) * K * K + r;
+        double sum = 0;
         for (int col = 0; col < (j + 1) * (j + 1); ++col) sum += ocol[static_cast<size_t>(col) * K] * cm[q * K + col];
         part[i] = sum;
     }
     __syncthreads();
     for (int r = threadIdx.x; r < K; r += 1024) {
-        R sum = 0;
+        double sum = 0;
         for (int q = 0; q < 8; ++q) sum += part[q * K + r];  // children in order
         M[static_cast<size_t>(P) * ldk + r] = sum;
     }
-    for (int i = K + threadIdx.x; i < ldk; i += 1024) M[static_cast<size_t>(P) * ldk + i] = R(0);
+    for (int i = K + threadIdx.x; i < ldk; i += 1024) M[static_cast<size_t>(P) * ldk + i] = double(0);
 }
 
-template <class R>
 __global__ __launch_bounds__(1024) void k_l2l_wide(const int32_t *__restrict__ ids, const int32_t *__restrict__ child, const uint32_t *__restrict__ count,
-                                                   const R *__restrict__ op, int K, int ldk, R *__restrict__ L) {
-    __shared__ R pl[MAXK];
+                                                   const double *__restrict__ op, int K, int ldk, double *__restrict__ L) {
+    __shared__ double pl[MAXK];
     const int32_t P = ids[blockIdx.x];
     const int32_t cb = child[P];
     for (int i = threadIdx.x; i < K; i += 1024) pl[i] = L[static_cast<size_t>(P) * ldk + i];
@@ -1008,8 +1109,8 @@ __global__ __launch_bounds__(1024) void k_l2l_wide(const int32_t *__restrict__ i
         if (!count[cb + q]) continue;
         int j = 0;
         while ((j + 1) * (j + 1) <= r) ++j;
-        const R *ocol = op + static_cast<size_t>(8 + q) * K * K + r;
-        R sum = 0;
+        const double *ocol = op + static_cast<size_t>(8 + q) * K * K + r;
+        double sum = 0;
         for (int col = j * j; col < K; ++col) sum += ocol[static_cast<size_t>(col) * K] * pl[col];
         L[static_cast<size_t>(cb + q) * ldk + r] += sum;
     }
@@ -1021,46 +1122,66 @@ inline int pick_pb(int64_t nparents, int maxpb) {
     return pb;
 }
 
-template <class R>
-void m2m_level(Ctx &c, const int32_t *ids, int64_t n) {
+template <int P, bool UP>
+void ml_f32_launch(Ctx &c, const int32_t *ids, int n) {
+    using S = M2lShape<P>;
+    if (c.ldk != S::LD) throw Error(1, "FP32 M2M and L2L: the coefficient stride must be K rounded up to 4");
     const TreeDev &t = c.t;
-    if (sizeof(R) == 4 && c.prec == 2) {  // split mode: on the matrix cores
-        ml_split_level(c, ids, n, true);
-        return;
-    }
-    const int pb = pick_pb(n, 8);  // 8 children x PB staged expansions in LDS
-    if (n < 1024) {  // few parents: one wide block each
-        k_m2m_wide<R><<<static_cast<unsigned>(n), 1024, 0, c.stream>>>(ids, t.child, t.count, Bufs<R>::op(c), c.K, c.ldk, Bufs<R>::M(c));
-        return;
-    }
-#define VG_M2M(PB_) \
-    k_m2m<R, PB_><<<ceil_div(n, PB_), 256, 0, c.stream>>>(ids, static_cast<int>(n), t.child, t.count, Bufs<R>::op(c), c.K, c.ldk, Bufs<R>::M(c))
-    if (pb == 1) VG_M2M(1);
-    else if (pb == 2) VG_M2M(2);
-    else if (pb == 4) VG_M2M(4);
-    else VG_M2M(8);
-#undef VG_M2M
+    const f4 *op = reinterpret_cast<const f4 *>(c.op32.p);
+    float *X = UP ? c.M32.p : c.L32.p;
+    // two tiles of parents share an operator fragment where that leaves a block for every CU
+    if (ceil_div(n, 32) * S::NT >= c.ncu)
+        k_ml_f32<P, 2, UP><<<ceil_div(n, 32) * S::NT, 512, 0, c.stream>>>(ids, n, t.child, t.count, op, X);
+    else
+        k_ml_f32<P, 1, UP><<<ceil_div(n, 16) * S::NT, 512, 0, c.stream>>>(ids, n, t.child, t.count, op, X);
 }
 
-template <class R>
-void l2l_level(Ctx &c, const int32_t *ids, int64_t n) {
+template <bool UP>
+void ml_f32_level(Ctx &c, const int32_t *ids, int n) {
+    switch (c.p) {
+    case 1: ml_f32_launch<1, UP>(c, ids, n); break;
+    case 2: ml_f32_launch<2, UP>(c, ids, n); break;
+    case 3: ml_f32_launch<3, UP>(c, ids, n); break;
+    case 4: ml_f32_launch<4, UP>(c, ids, n); break;
+    case 5: ml_f32_launch<5, UP>(c, ids, n); break;
+    case 6: ml_f32_launch<6, UP>(c, ids, n); break;
+    case 7: ml_f32_launch<7, UP>(c, ids, n); break;
+    case 8: ml_f32_launch<8, UP>(c, ids, n); break;
+    case 9: ml_f32_launch<9, UP>(c, ids, n); break;
+    case 10: ml_f32_launch<10, UP>(c, ids, n); break;
+    case 11: ml_f32_launch<11, UP>(c, ids, n); break;
+    case 12: ml_f32_launch<12, UP>(c, ids, n); break;
+    default: throw Error(1, "M2M and L2L support 1 <= p <= 12");
+    }
+}
+
+// M2M (up) or L2L of the internal cells of one level
+void ml_level(Ctx &c, const int32_t *ids, int64_t n, bool up) {
     const TreeDev &t = c.t;
-    if (sizeof(R) == 4 && c.prec == 2) {
-        ml_split_level(c, ids, n, false);
+    if (c.prec == 2) {  // on the matrix cores, with split operands
+        ml_split_level(c, ids, n, up);
         return;
     }
-    const int pb = pick_pb(n, 16);
-    if (n < 1024) {
-        k_l2l_wide<R><<<static_cast<unsigned>(n), 1024, 0, c.stream>>>(ids, t.child, t.count, Bufs<R>::op(c), c.K, c.ldk, Bufs<R>::L(c));
+    if (c.prec == 1) {
+        up ? ml_f32_level<true>(c, ids, static_cast<int>(n)) : ml_f32_level<false>(c, ids, static_cast<int>(n));
         return;
     }
-#define VG_L2L(PB_) \
-    k_l2l<R, PB_><<<ceil_div(n, PB_), 256, 0, c.stream>>>(ids, static_cast<int>(n), t.child, t.count, Bufs<R>::op(c), c.K, c.ldk, Bufs<R>::L(c))
-    if (pb == 1) VG_L2L(1);
-    else if (pb == 2) VG_L2L(2);
-    else if (pb == 4) VG_L2L(4);
-    else if (pb == 8) VG_L2L(8);
+    if (n < 1024) {  // few parents: one wide block each
+        if (up)
+            k_m2m_wide<<<static_cast<unsigned>(n), 1024, 0, c.stream>>>(ids, t.child, t.count, c.op64, c.K, c.ldk, c.M64);
+        else
+            k_l2l_wide<<<static_cast<unsigned>(n), 1024, 0, c.stream>>>(ids, t.child, t.count, c.op64, c.K, c.ldk, c.L64);
+        return;
+    }
+#define VG_M2M(PB_) k_m2m<PB_><<<ceil_div(n, PB_), 256, 0, c.stream>>>(ids, static_cast<int>(n), t.child, t.count, c.op64, c.K, c.ldk, c.M64)
+#define VG_L2L(PB_) k_l2l<PB_><<<ceil_div(n, PB_), 256, 0, c.stream>>>(ids, static_cast<int>(n), t.child, t.count, c.op64, c.K, c.ldk, c.L64)
+    const int pb = pick_pb(n, up ? 8 : 16);  // M2M: 8 children x PB staged expansions in LDS
+    if (pb == 1) up ? VG_M2M(1) : VG_L2L(1);
+    else if (pb == 2) up ? VG_M2M(2) : VG_L2L(2);
+    else if (pb == 4) up ? VG_M2M(4) : VG_L2L(4);
+    else if (pb == 8) up ? VG_M2M(8) : VG_L2L(8);
     else VG_L2L(16);
+#undef VG_M2M
 #undef VG_L2L
 }
 
@@ -1092,7 +1213,7 @@ void upward_t(Ctx &c) {
     }
     for (int d = t.depth; d >= 2; --d) {
         const int64_t a = t.int_off[d], b = t.int_off[d + 1];
-        if (b > a) m2m_level<R>(c, t.int_ids.p + a, b - a);
+        if (b > a) ml_level(c, t.int_ids.p + a, b - a, true);
     }
     VG_LAUNCH_CHECK();
 }
@@ -1226,7 +1347,7 @@ void downward_t(Ctx &c) {
     TreeDev &t = c.t;
     for (int d = 2; d < t.depth; ++d) {  // parents at level d >= 2 feed children at level >= 3
         const int64_t a = t.int_off[d], b = t.int_off[d + 1];
-        if (b > a) l2l_level<R>(c, t.int_ids.p + a, b - a);
+        if (b > a) ml_level(c, t.int_ids.p + a, b - a, false);
     }
     join_p2p(c);  // L2P adds to the P2P accelerations
     bool fallback = false;
@@ -1324,14 +1445,15 @@ void operators_build(Ctx &c) {
     } else if (c.prec == 2) {
         c.op64.ensure(static_cast<size_t>(nvec) * c.K * c.K);
         k_ops<double><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op64, nullptr);
-        c.op32.ensure(static_cast<size_t>(nvec) * c.K * c.K);
         m2l_split_operators(c, nvec);
     } else {
-        c.op32.ensure(static_cast<size_t>(16) * c.K * c.K);
-        if (!c.opfrag.p) {
-            const size_t words = 343 * OpFrag(c.K).size();
+        if (c.frag_K != c.K) {  // the padding, once for each order (the closure's fallback order may change)
+            const size_t words = 343 * OpFrag(c.K).size(), words_ml = 16 * MlFrag(c.K).size();
             c.opfrag.ensure(words);
-            VG_HIP(hipMemsetAsync(c.opfrag.p, 0, words * sizeof(float), c.stream));  // the padding, once
+            c.op32.ensure(words_ml);
+            VG_HIP(hipMemsetAsync(c.opfrag.p, 0, words * sizeof(float), c.stream));
+            VG_HIP(hipMemsetAsync(c.op32.p, 0, words_ml * sizeof(float), c.stream));
+            c.frag_K = c.K;
         }
         k_ops<float><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op32, c.opfrag);
     }
@@ -1390,7 +1512,7 @@ void fmm_m2l_plain(Ctx &c) {
 }
 
 void l2l_list(Ctx &c, const int32_t *parents, int64_t np) {
-    if (np > 0) l2l_level<float>(c, parents, np);
+    if (np > 0) ml_level(c, parents, np, false);
     VG_LAUNCH_CHECK();
 }
 

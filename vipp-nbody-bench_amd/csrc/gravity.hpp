@@ -56,7 +56,7 @@ struct TreeDev {
 // the expansion order and everything sized by it; the closure's fallback keeps
 // a second set (order p_hi) and swaps it into the context while it runs
 struct ExpSet {
-    int p = 0, K = 0, ldk = 0;
+    int p = 0, K = 0, ldk = 0, frag_K = 0;
     DevBuf<double> harm, op64;
     DevBuf<float> op32, opfrag, M32, L32;
     DevBuf<uint16_t> opsplit, opsplit_ml, msplit;
@@ -151,9 +151,9 @@ struct Ctx {
     DevBuf<float> M32, L32;
     // translation operators
     DevBuf<double> harm;        // harmonic tables of the operator offsets
-    DevBuf<double> op64;        // M2M (8), L2L (8), M2L (343) blocks of K*K
-    DevBuf<float> op32;
-    DevBuf<float> opfrag;       // FP32 mode: M2L operators in the order the matrix cores' lanes read them
+    DevBuf<double> op64;        // M2M (8), L2L (8), M2L (343) blocks of K*K (FP64 and split modes)
+    DevBuf<float> op32, opfrag;  // FP32 mode: M2M and L2L, and M2L operators in the order the matrix cores' lanes read them
+    int frag_K = 0;             // the K whose padding in them is zero
     DevBuf<uint16_t> opsplit;   // M2L operators as BF16 hi/lo MFMA fragments
     DevBuf<uint16_t> opsplit_ml;  // the 8 M2M and 8 L2L operators, the same way
     DevBuf<float> ml_part;      // split M2M: the 8 octant products of one level before their sum
