@@ -118,8 +118,6 @@ static void evaluate_overlapped(Ctx &c, bool potential) {
     VG_HIP(hipStreamWaitEvent(c.stream, c.ev_lists, 0));  // M2L reads the parents' neighbour tables
     fmm_m2l(c);
     fmm_downward(c, potential);
-    join_p2p(c);
-    scatter_accel(c, potential);
 }
 
 void evaluate(Ctx &c, bool potential) {
@@ -161,7 +159,6 @@ void evaluate(Ctx &c, bool potential) {
     used[PH_M2L] = true;
     phase_begin(c, PH_DOWN);
     fmm_downward(c, potential);
-    scatter_accel(c, potential);
     phase_end(c, PH_DOWN);
     used[PH_DOWN] = true;
     collect_times(c, used);

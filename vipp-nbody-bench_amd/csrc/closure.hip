@@ -90,15 +90,15 @@ __global__ __launch_bounds__(256) void k_mark_chains(const int32_t *__restrict__
     for (int l = 0; l <= level[c]; ++l) need[anc[static_cast<int64_t>(c) * (MAXD + 1) + l]] = 1;
 }
 
-// ordered compaction of ids[i] with keep(ids[i]) (one block): out, and pos[i] =
-// number kept before i (pos[n] = total).  keep = need[ids[i]] or flag[i].
+// ordered compaction of ids[i] with need[ids[i]] (one block): out, and pos[i] =
+// number kept before i (pos[n] = total).
 __global__ __launch_bounds__(1024) void k_compact_keep(const int32_t *__restrict__ ids, int64_t n, const uint8_t *__restrict__ need,
-                                                       const uint8_t *__restrict__ flag, int32_t *__restrict__ out, uint32_t *__restrict__ pos) {
+                                                       int32_t *__restrict__ out, uint32_t *__restrict__ pos) {
     __shared__ uint32_t s[1024];
     uint32_t base = 0;
     for (int64_t b = 0; b < n; b += 1024) {
         const int64_t i = b + threadIdx.x;
-        const uint32_t k = i < n ? (need ? need[ids[i]] : flag[i]) : 0;
+        const uint32_t k = i < n ? need[ids[i]] : 0;
         s[threadIdx.x] = k;
         __syncthreads();
         for (int off = 1; off < 1024; off <<= 1) {  // inclusive Hillis-Steele scan
@@ -109,14 +109,14 @@ __global__ __launch_bounds__(1024) void k_compact_keep(const int32_t *__restrict
         }
         const uint32_t excl = s[threadIdx.x] - k;
         if (i < n) {
-            if (pos) pos[i] = base + excl;
+            pos[i] = base + excl;
             if (k) out[base + excl] = ids[i];
         }
         const uint32_t tot = s[1023];
         __syncthreads();
         base += tot;
     }
-    if (threadIdx.x == 0 && pos) pos[n] = base;
+    if (threadIdx.x == 0) pos[n] = base;
 }
 
 }  // namespace
@@ -168,10 +168,6 @@ bool closure_fallback_prepare(Ctx &c) {
     cl.nflag = nf;
     if (nf == 0) return false;
     const int64_t n = t.nleaves;
-    // flagged leaves, in leaf order
-    cl.fb_leaves.ensure(n);
-    k_compact_keep<<<1, 1024, 0, c.stream>>>(t.leaf_ids, n, nullptr, cl.flag, cl.fb_leaves, nullptr);
-    VG_LAUNCH_CHECK();
     // internal cells on their ancestor chains, level by level
     cl.need.ensure(t.ncells);
     VG_HIP(hipMemsetAsync(cl.need.p, 0, t.ncells, c.stream));
@@ -180,7 +176,7 @@ bool closure_fallback_prepare(Ctx &c) {
     const int64_t nint = t.int_off.back();
     cl.fb_int.ensure(std::max<int64_t>(1, nint));
     cl.fb_pos.ensure(nint + 1);
-    k_compact_keep<<<1, 1024, 0, c.stream>>>(t.int_ids, nint, cl.need, nullptr, cl.fb_int, cl.fb_pos);
+    k_compact_keep<<<1, 1024, 0, c.stream>>>(t.int_ids, nint, cl.need, cl.fb_int, cl.fb_pos);
     VG_LAUNCH_CHECK();
     std::vector<uint32_t> pos(static_cast<size_t>(nint + 1));
     VG_HIP(hipMemcpyAsync(pos.data(), cl.fb_pos.p, (nint + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream));
@@ -209,11 +205,11 @@ bool closure_fallback_prepare(Ctx &c) {
     return true;
 }
 
-void closure_fallback_l2p(Ctx &c) {
+void closure_fallback_l2p(Ctx &c, bool potential) {
     Closure &cl = c.cl;
     swap_expansions(c, cl.hi);
     try {
-        l2p_list(c, cl.fb_leaves, cl.nflag, nullptr);
+        l2p_flagged(c, potential, cl.flag);
     } catch (...) {
         swap_expansions(c, cl.hi);
         throw;

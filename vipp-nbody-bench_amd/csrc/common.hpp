@@ -72,6 +72,30 @@ struct DevBuf {
     operator T *() const { return p; }
 };
 
+// Four values of a particle in one 16- or 32-byte word.
+template <class R>
+struct QuadOf;
+template <>
+struct QuadOf<float> {
+    using T = float4;
+};
+template <>
+struct QuadOf<double> {
+    using T = double4;
+};
+template <class R>
+using Quad = typename QuadOf<R>::T;
+
+__device__ inline float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
+// 1/sqrt(x) in FP64: with e = 1 - x y^2 of the hardware's estimate y (2^-24 at
+// worst), y (1 + e / 2 + 3/8 e^2) is off by its roundings and less than 2^-69
+// (x > 0; x = 0 gives NaN, which the P2P's self-pair select replaces)
+__device__ inline double rsq(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x, y * y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
 // Real-packed index of a degree-n, order-m (m >= 0) coefficient: degree n owns
 // entries [n*n, (n+1)*(n+1)): Re(m=0), then (Re, Im) for m = 1..n.
 __host__ __device__ inline int kidx_re(int n, int m) { return m == 0 ? n * n : n * n + 2 * m - 1; }

@@ -78,7 +78,6 @@ struct Closure {
     // fallback
     ExpSet hi;                   // order-p_hi expansions and operators
     DevBuf<uint8_t> need;        // per cell: on the ancestor chain of a flagged leaf
-    DevBuf<int32_t> fb_leaves;   // flagged leaves
     DevBuf<int32_t> fb_int;      // needed internal cells, level by level
     DevBuf<uint32_t> fb_pos;     // compaction scratch
     std::vector<int64_t> fb_off; // fb_int offset of each level (depth + 2 entries)
@@ -188,9 +187,8 @@ void fmm_m2l(Ctx &c);                    // M2L (plain VALU or split MFMA by mod
 void fmm_p2p(Ctx &c, bool potential);    // near field into the sorted accelerations (plan, then run)
 void fmm_p2p_plan(Ctx &c, bool potential);  // P2P work items; the item counts are read back without waiting
 void fmm_p2p_run(Ctx &c, bool potential);  // waits for the item counts, then the P2P kernels
-void fmm_downward(Ctx &c, bool potential);  // L2L + L2P
+void fmm_downward(Ctx &c, bool potential);  // L2L, L2P and the way back to the caller's order
 void join_p2p(Ctx &c);                       // ctx.stream waits for a P2P launched on ctx.stream2
-void scatter_accel(Ctx &c, bool potential);  // sorted -> caller order
 void rk4_init(Ctx &c);
 void rk4_stage(Ctx &c, int stage, double dt);
 void count_work(Ctx &c);
@@ -199,7 +197,7 @@ double potential_energy(Ctx &c);
 void closure_inputs(Ctx &c, bool with_l25);  // network inputs of every non-empty leaf from the current L32
 void closure_apply(Ctx &c);                   // L~_25 += |L~_25| MLP(x) and fallback flags
 bool closure_fallback_prepare(Ctx &c);        // order-p_hi locals of the flagged leaves; false if none is flagged
-void closure_fallback_l2p(Ctx &c);            // order-p_hi L2P of the flagged leaves
+void closure_fallback_l2p(Ctx &c, bool potential);  // order-p_hi L2P of the flagged leaves
 void swap_expansions(Ctx &c, ExpSet &e);      // exchange the context's expansion set with e
 void m2l_list(Ctx &c, const int32_t *parents, int np);      // M2L of the children of the given internal cells
 int m2l_parts(unsigned grid, int ncu);        // parts of the walked offsets of an M2L grid
@@ -207,7 +205,7 @@ float *m2l_part_sums(Ctx &c, int np, int nsplit);  // their partial sums (FP32),
 void m2l_add_parts(Ctx &c, const int32_t *parents, int np, int nsplit, const float *part);
 void l2l_list(Ctx &c, const int32_t *parents, int64_t np);  // L2L into the children of the given internal cells (FP32)
 void ml_split_level(Ctx &c, const int32_t *ids, int64_t n, bool m2m);  // M2M (m2m) or L2L of one level on the matrix cores
-void l2p_list(Ctx &c, const int32_t *leaves, int64_t n, const uint8_t *skip);  // L2P of the given leaves (FP32)
+void l2p_flagged(Ctx &c, bool potential, const uint8_t *flag);  // L2P of the flagged leaves (FP32)
 void direct_subset(Ctx &c, const int64_t *idx, int64_t nidx, double *a, double *pot);  // FP64 O(N nidx) oracle forces
 // the same with idx, a and pot in device memory, its partial sums in the
 // library's static device scratch (no allocation); noalloc_init resolves that

@@ -14,7 +14,7 @@
 //  * FP32 (k_p2p_mc): squared distances on the matrix cores.
 //  * FP64 (k_p2p_f64): pairs by differences.
 // A leaf with one chunk writes its result; split leaves write partial sums,
-// which are added in chunk order (deterministic).  With a nonzero softening the
+// which L2P adds in chunk order (deterministic).  With a nonzero softening the
 // i == j term is exactly zero (dx = dy = dz = 0), so it needs no branch;
 // without softening a select removes it.
 #include "gravity.hpp"
@@ -26,27 +26,6 @@ constexpr int MAXE = 27 * (MAXD + 1);
 
 // Sources per work item of a leaf cut into nch: even, in whole groups of 64.
 __host__ __device__ inline uint32_t chunk_len(uint32_t total, uint32_t nch) { return ((total + nch - 1) / nch + 63) / 64 * 64; }
-
-template <class R>
-struct Vec4;
-template <>
-struct Vec4<float> {
-    using T = float4;
-};
-template <>
-struct Vec4<double> {
-    using T = double4;
-};
-
-__device__ inline float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
-// 1/sqrt(x) in FP64: with e = 1 - x y^2 of the hardware's estimate y (2^-24 at
-// worst), y (1 + e / 2 + 3/8 e^2) is off by its roundings and less than 2^-69
-// (x > 0; x = 0 gives NaN, which the self-pair select replaces)
-__device__ inline double rsq(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x, y * y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
-}
 
 // ---- FP32: squared distances on the matrix cores -------------------------
 //
@@ -623,35 +602,6 @@ __global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ it
         pass(std::integral_constant<int, F64_TILES>{});
 }
 
-// Leaves split over several work items: partial sums added in chunk order
-// (the same order every run), a wavefront per leaf.
-template <bool POT, class R, class V4 = typename Vec4<R>::T>
-__global__ __launch_bounds__(256) void k_p2p_sum(const int32_t *__restrict__ leaves, int nleaves, const uint32_t *__restrict__ nchunk,
-                                                 const uint32_t *__restrict__ item_off, const uint32_t *__restrict__ start, const uint32_t *__restrict__ count,
-                                                 const V4 *__restrict__ xs, R eps2, R G, V4 *__restrict__ acc,
-                                                 const V4 *__restrict__ partial, uint32_t pstride) {
-    const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (k >= nleaves) return;
-    const uint32_t nch = nchunk[k];
-    if (nch < 2) return;
-    const int32_t c = leaves[k];
-    const uint32_t nt = count[c], pt0 = start[c];
-    const V4 *pk = partial + static_cast<size_t>(item_off[k]) * pstride;
-    for (uint32_t t = threadIdx.x & 63; t < nt; t += 64) {
-        R sx = 0, sy = 0, sz = 0, sp = 0;
-#pragma unroll 8
-        for (uint32_t q = 0; q < nch; ++q) {
-            const V4 v = pk[static_cast<size_t>(q) * pstride + t];
-            sx += v.x;
-            sy += v.y;
-            sz += v.z;
-            sp += v.w;
-        }
-        if (POT && eps2 > R(0)) sp -= xs[pt0 + t].w * rsq(eps2);
-        acc[pt0 + t] = V4{G * sx, G * sy, G * sz, sp};
-    }
-}
-
 // Sources of each cell's own NI entries (the leaf's full list is its
 // ancestors' entries and its own, solver_ref.hpp:126).
 __global__ __launch_bounds__(256) void k_ni_local(int64_t ncells, const uint32_t *__restrict__ count, const int32_t *__restrict__ ni,
@@ -826,11 +776,11 @@ static const uint32_t *p2p_scalars(Ctx &c) {
     return reinterpret_cast<const uint32_t *>(static_cast<const char *>(c.pinned) + 128);
 }
 
-// One launch over all items, on the stream p2p_plan used, and one that adds the
-// partial sums of the leaves split over several.
+// One launch over all items, on the stream p2p_plan used; L2P adds the partial sums
+// of the leaves split over several.
 template <class R>
 void p2p_run(Ctx &c, bool potential) {
-    using V4 = typename Vec4<R>::T;
+    using V4 = Quad<R>;
     TreeDev &t = c.t;
     if (!t.nleaves) return;
     const uint32_t *hs = p2p_scalars(c);
@@ -849,24 +799,17 @@ void p2p_run(Ctx &c, bool potential) {
     };
     const R eps2 = static_cast<R>(c.eps * c.eps), G = static_cast<R>(c.G), mu = static_cast<R>(c.mass);
     const bool um = !c.has_masses;  // one mass: left out of the pairs, the sums are scaled once
-    auto add = [&](const V4 *xs, V4 *acc, const V4 *part) {
-        if (!split) return;
-        (potential ? k_p2p_sum<true, R> : k_p2p_sum<false, R>)<<<ceil_div(nl, 4), 256, 0, c.stream>>>(t.leaf_ids, nl, c.p2p_nchunk, c.p2p_item_off, t.start,
-                                                                                                    t.count, xs, eps2, G, acc, part, pstride);
-    };
     if constexpr (sizeof(R) == 4) {
         bool big = false;  // a root box so wide that squared distances may leave the FP32 range
         for (int a = 0; a < 3; ++a) big |= !(t.box[3 + a] - t.box[a] < 1e18);
         buffers(c.xs32, c.as32, c.p2p_part32, [&](const V4 *xs, V4 *acc, V4 *part) {
             (potential ? k_p2p_mc<true> : k_p2p_mc<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs,
                                                                                        eps2, G, um, big, mu, acc, part, pstride);
-            add(xs, acc, part);
         });
     } else {
         buffers(c.xs64, c.as64, c.p2p_part64, [&](const V4 *xs, V4 *acc, V4 *part) {
             (potential ? k_p2p_f64<true> : k_p2p_f64<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, xs, eps2, G, um,
                                                                                          mu, acc, part, pstride);
-            add(xs, acc, part);
         });
     }
     VG_LAUNCH_CHECK();

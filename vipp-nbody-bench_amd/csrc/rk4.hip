@@ -1,5 +1,4 @@
-// rk4.hip - FP64 classic RK4 on the caller-ordered state, the scatter of the
-// sorted forces back to caller order, energies and work counts.
+// rk4.hip - FP64 classic RK4 on the caller-ordered state, energies and work counts.
 //
 // The stage arithmetic is the reference's (solver_ref.hpp:36-104):
 //   x_out += (dt/6) v ; v_out += (dt/6) a      after the stage-0 force
@@ -67,18 +66,6 @@ __global__ __launch_bounds__(256) void k_rk4_stage(int64_t n3, double cw, double
         if (comp >= 3) comp -= 3;
     }
     aabb_block_store(lo, hi, bad, part + 7ll * blockIdx.x);
-}
-
-template <class R, class A>
-__global__ __launch_bounds__(256) void k_scatter(int64_t n, const uint32_t *__restrict__ perm, const R *__restrict__ acc4, A *__restrict__ a,
-                                                 double *__restrict__ pot) {
-    const int64_t k = blockIdx.x * 256ll + threadIdx.x;
-    if (k >= n) return;
-    const uint32_t i = perm[k];
-    a[3ll * i] = static_cast<A>(acc4[4 * k]);
-    a[3ll * i + 1] = static_cast<A>(acc4[4 * k + 1]);
-    a[3ll * i + 2] = static_cast<A>(acc4[4 * k + 2]);
-    if (pot) pot[i] = static_cast<double>(acc4[4 * k + 3]);
 }
 
 // FP64 block reduction of per-particle terms: kind 0 = m |v|^2, kind 1 = m * pot
@@ -156,20 +143,6 @@ void rk4_stage(Ctx &c, int stage, double dt) {
         k_rk4_stage<float><<<nb, 256, 0, c.stream>>>(n3, cw, h, last, c.acc32, c.x, c.v, c.x0, c.v0, c.xo, c.vo, c.aabb_part);
     VG_LAUNCH_CHECK();
     c.aabb_parts = nb;
-}
-
-void scatter_accel(Ctx &c, bool potential) {
-    const int64_t n = c.n;
-    if (potential) c.pot64.ensure(std::max<int64_t>(1, n));
-    double *pot = potential ? c.pot64.p : nullptr;
-    if (c.prec == 0) {
-        c.acc64.ensure(3 * std::max<int64_t>(1, n));
-        k_scatter<double, double><<<ceil_div(n, 256), 256, 0, c.stream>>>(n, c.perm, c.as64, c.acc64.p, pot);
-    } else {
-        c.acc32.ensure(3 * std::max<int64_t>(1, n));
-        k_scatter<float, float><<<ceil_div(n, 256), 256, 0, c.stream>>>(n, c.perm, c.as32, c.acc32.p, pot);
-    }
-    VG_LAUNCH_CHECK();
 }
 
 static double reduce_energy(Ctx &c, int kind) {
