@@ -45,6 +45,21 @@ void swap_expansions(Ctx &c, ExpSet &e) {
 }
 void fmm_constants_init();
 
+void wait_host_word(const uint32_t *word, uint32_t want, hipStream_t st) {
+    for (uint32_t spin = 1; __atomic_load_n(word, __ATOMIC_ACQUIRE) != want; ++spin) {
+        __builtin_ia32_pause();
+        if (spin % 16384) continue;
+        // a stream that has ended, or failed, without writing it never will
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();
+            continue;
+        }
+        VG_HIP(e);
+        if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != want) throw Error(VIPP_GRAV_E_DEVICE, "a kernel did not write its sizes");
+    }
+}
+
 void phase_begin(Ctx &c, Phase p) {
     if (c.timing) VG_HIP(hipEventRecord(c.ev[2 * p], c.stream));
 }
@@ -410,8 +425,8 @@ int vipp_grav_create(const vipp_grav_config *cfg, vipp_grav_ctx **out) {
             VG_HIP(hipEventCreateWithFlags(&c.ev_tree, hipEventDisableTiming));
             VG_HIP(hipEventCreateWithFlags(&c.ev_join, hipEventDisableTiming));
             VG_HIP(hipEventCreateWithFlags(&c.ev_lists, hipEventDisableTiming));
-            VG_HIP(hipEventCreateWithFlags(&c.ev_plan, hipEventDisableTiming));
-            VG_HIP(hipHostMalloc(&c.pinned, vg::Ctx::PINNED_BYTES, hipHostMallocDefault));
+            VG_HIP(hipHostMalloc(&c.pinned, vg::Ctx::PINNED_BYTES, hipHostMallocCoherent));
+            std::memset(c.pinned, 0, vg::Ctx::PINNED_BYTES);  // memory of an earlier context may hold the numbers wait_host_word waits for
             for (auto &e : c.ev) VG_HIP(hipEventCreate(&e));
             vg::fmm_constants_init();
             vg::noalloc_init(c.device);
@@ -442,7 +457,6 @@ int vipp_grav_destroy(vipp_grav_ctx *ctx) {
     if (ctx->c.ev_tree) (void)hipEventDestroy(ctx->c.ev_tree);
     if (ctx->c.ev_join) (void)hipEventDestroy(ctx->c.ev_join);
     if (ctx->c.ev_lists) (void)hipEventDestroy(ctx->c.ev_lists);
-    if (ctx->c.ev_plan) (void)hipEventDestroy(ctx->c.ev_plan);
     if (ctx->c.stream) (void)hipStreamDestroy(ctx->c.stream);
     if (ctx->c.stream2) (void)hipStreamDestroy(ctx->c.stream2);
     if (ctx->c.pinned) (void)hipHostFree(ctx->c.pinned);

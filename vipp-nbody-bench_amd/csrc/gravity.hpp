@@ -107,12 +107,12 @@ struct Ctx {
     // lists (ev_lists), L2P for P2P (join_p2p)
     hipStream_t stream2 = nullptr;
     hipEvent_t ev_join = nullptr, ev_lists = nullptr;
-    hipEvent_t ev_tree = nullptr;  // the tree is built and its sizes are in the pinned words
-    hipEvent_t ev_plan = nullptr;  // the P2P plan scalars are in the pinned words
+    hipEvent_t ev_tree = nullptr;  // the tree is built
+    uint32_t tree_seq = 0, plan_seq = 0;  // builds and P2P plans so far: the pinned words say whose they are
     bool p2p_pending = false;
     bool lists_ahead = false;      // the lists were enqueued with the tree (ev_lists recorded)
-    // pinned host words for the scalars read back during an evaluation (tree
-    // level sizes, root box, P2P plan): a pinned copy returns sooner
+    // pinned host words for what the host reads during an evaluation (tree
+    // level sizes, root box, P2P plan), written by the kernels themselves
     void *pinned = nullptr;
     static constexpr size_t PINNED_BYTES = 4096;
     bool timing = false;
@@ -212,6 +212,9 @@ void direct_subset(Ctx &c, const int64_t *idx, int64_t nidx, double *a, double *
 // scratch's address on a device (once per device, with the device current)
 void direct_subset_noalloc(Ctx &c, const int64_t *idx, int64_t nidx, double *a, double *pot);
 void noalloc_init(int device);
+
+// Waits until a kernel of the stream has written `want` to a pinned host word.
+void wait_host_word(const uint32_t *word, uint32_t want, hipStream_t st);
 
 void phase_begin(Ctx &c, Phase p);
 void phase_end(Ctx &c, Phase p);

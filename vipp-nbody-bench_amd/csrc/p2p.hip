@@ -677,7 +677,8 @@ __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ le
 // bases, the item total and the split-leaf total into scal:
 //   scal[0..NCLS) items per class, scal[NCLS..2 NCLS) class bases,
 //   scal[2 NCLS] rows of partial sums, scal[2 NCLS + 1] split leaves.
-__global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ btot, int nblocks, uint32_t *__restrict__ scal) {
+// host: the same in pinned host memory, then seq in its last word.
+__global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ btot, int nblocks, uint32_t *__restrict__ scal, uint32_t *host, uint32_t seq) {
     // exclusive scan of each component over the plan blocks, one wavefront per
     // component (wavefront-wide inclusive scans, carried across runs of 64)
     __shared__ uint32_t tot[NSC];
@@ -698,15 +699,19 @@ __global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ 
         if (lane == 0) tot[q] = carry;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {  // scal: [class items] [class bases] rows, split leaves
-        scal[2 * NCLS] = tot[0];
-        scal[2 * NCLS + 1] = tot[NSC - 1];
-        uint32_t base = 0;
-        for (int j = 0; j < NCLS; ++j) {
-            scal[j] = tot[1 + j];
-            scal[NCLS + j] = base;
-            base += tot[1 + j];
-        }
+    if (threadIdx.x < 2 * NCLS + 2) {  // scal: [class items] [class bases] rows, split leaves
+        const int j = threadIdx.x;
+        uint32_t v = 0;
+        if (j < NCLS)
+            v = tot[1 + j];
+        else if (j < 2 * NCLS)
+            for (int k = 0; k < j - NCLS; ++k) v += tot[1 + k];
+        else
+            v = tot[j == 2 * NCLS ? 0 : NSC - 1];
+        scal[j] = v;
+        host[j] = v;
+        __threadfence_system();
+        if (j == 0) __hip_atomic_store(host + 2 * NCLS + 2, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);  // behind this wavefront's stores
     }
 }
 
@@ -736,15 +741,14 @@ __global__ __launch_bounds__(256) void k_p2p_items(const int32_t *__restrict__ l
 }
 
 // Work items of the P2P: counts per leaf, then the plan scalars (items per
-// class) copied back to pinned host words, with ev_plan recorded after the
-// copy.  Nothing here waits, so the caller can enqueue other work before
+// class), written to pinned host words too.  Nothing here waits, so the caller can enqueue other work before
 // p2p_run needs the scalars.
 void p2p_plan(Ctx &c, bool potential) {
     TreeDev &t = c.t;
     if (!t.nleaves) return;
     const int nl = static_cast<int>(t.nleaves);
     const int nb = static_cast<int>(ceil_div(nl, 256));
-    c.p2p_scal.ensure(16);
+    c.p2p_scal.ensure(2 * NCLS + 2);
     c.p2p_nchunk.ensure(nl);
     c.p2p_cls.ensure(nl);
     c.p2p_src.ensure(nl);
@@ -761,19 +765,17 @@ void p2p_plan(Ctx &c, bool potential) {
     if (nl < few) chunk = std::max<uint32_t>(c.prec == 0 ? F64_MINCOST : MC_MINCOST, static_cast<uint32_t>(1ull * MC_COST * nl / few));
     k_p2p_plan<<<nb, 256, 0, c.stream>>>(t.leaf_ids, nl, t.level, t.count, t.anc, c.p2p_local, c.p2p_nchunk, c.p2p_cls, c.p2p_src, c.p2p_pre, c.p2p_btot, chunk,
                                         c.prec == 0 ? F64_TILES : mc_tiles(potential), nl < 8 * c.ncu ? 1 : 8);
-    k_p2p_plan_blocks<<<1, 256, 0, c.stream>>>(c.p2p_btot, nb, c.p2p_scal);
+    static_assert(2 * NCLS + 2 < 32, "plan scalars");
+    k_p2p_plan_blocks<<<1, 256, 0, c.stream>>>(c.p2p_btot, nb, c.p2p_scal, reinterpret_cast<uint32_t *>(static_cast<char *>(c.pinned) + 128), ++c.plan_seq);
     VG_LAUNCH_CHECK();
-    static_assert(2 * NCLS + 2 <= 16, "plan scalars");
-    uint32_t *hs = reinterpret_cast<uint32_t *>(static_cast<char *>(c.pinned) + 128);  // 16 pinned host words
-    VG_HIP(hipMemcpyAsync(hs, c.p2p_scal.p, 16 * sizeof(uint32_t), hipMemcpyDeviceToHost, c.stream));
-    VG_HIP(hipEventRecord(c.ev_plan, c.stream));
 }
 
 // The plan's scalars, waited for on the host: items per class, class bases,
 // rows of partial sums, split leaves.
 static const uint32_t *p2p_scalars(Ctx &c) {
-    VG_HIP(hipEventSynchronize(c.ev_plan));
-    return reinterpret_cast<const uint32_t *>(static_cast<const char *>(c.pinned) + 128);
+    const uint32_t *hs = reinterpret_cast<const uint32_t *>(static_cast<const char *>(c.pinned) + 128);
+    wait_host_word(hs + 2 * NCLS + 2, c.plan_seq, c.stream);
+    return hs;
 }
 
 // One launch over all items, on the stream p2p_plan used; L2P adds the partial sums
