@@ -513,9 +513,9 @@ int vipp_grav_step(vipp_grav_ctx *ctx, double dt, uint32_t nsteps) {
         // call only: outside it the caller may have written x (device_state)
         c.aabb_parts = 0;
         for (uint32_t s = 0; s < nsteps; ++s) {
-            vg::rk4_init(c);
+            int stage = 0;
             try {
-                for (int stage = 0; stage < 4; ++stage) {
+                for (; stage < 4; ++stage) {
                     vg::evaluate(c, false);
                     vg::phase_begin(c, vg::PH_RK4);
                     vg::rk4_stage(c, stage, dt);
@@ -530,10 +530,13 @@ int vipp_grav_step(vipp_grav_ctx *ctx, double dt, uint32_t nsteps) {
             } catch (...) {
                 // a stage state the tree cannot hold (E_INPUT, E_DEPTH): put back
                 // the state this step started from, so x and v hold the last
-                // completed step and the next query rebuilds from it
+                // completed step and the next query rebuilds from it (stage 0
+                // keeps it; before that x and v still hold it)
                 const size_t n3 = 3 * static_cast<size_t>(c.n);
-                (void)hipMemcpyAsync(c.x.p, c.x0.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, c.stream);
-                (void)hipMemcpyAsync(c.v.p, c.v0.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, c.stream);
+                if (stage > 0) {
+                    (void)hipMemcpyAsync(c.x.p, c.x0.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, c.stream);
+                    (void)hipMemcpyAsync(c.v.p, c.v0.p, n3 * sizeof(double), hipMemcpyDeviceToDevice, c.stream);
+                }
                 (void)hipStreamSynchronize(c.stream);
                 c.evaluated = false;
                 c.t.ref_valid = false;

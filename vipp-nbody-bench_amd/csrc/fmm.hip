@@ -944,6 +944,7 @@ __global__ __launch_bounds__(256) void k_m2l_sum(const int32_t *__restrict__ par
     if (count[t] == 0) return;
     const size_t stride = static_cast<size_t>(8) * nparents * ldk;
     R v = part[static_cast<size_t>(slot) * ldk + r];
+#pragma unroll 8
     for (int q = 1; q < nsplit; ++q) v += part[q * stride + static_cast<size_t>(slot) * ldk + r];
     Lx[static_cast<size_t>(t) * ldk + r] = v;
 }

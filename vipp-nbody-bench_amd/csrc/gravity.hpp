@@ -189,7 +189,6 @@ void fmm_p2p_plan(Ctx &c, bool potential);  // P2P work items; the item counts a
 void fmm_p2p_run(Ctx &c, bool potential);  // waits for the item counts, then the P2P kernels
 void fmm_downward(Ctx &c, bool potential);  // L2L, L2P and the way back to the caller's order
 void join_p2p(Ctx &c);                       // ctx.stream waits for a P2P launched on ctx.stream2
-void rk4_init(Ctx &c);
 void rk4_stage(Ctx &c, int stage, double dt);
 void count_work(Ctx &c);
 double kinetic_energy(Ctx &c);

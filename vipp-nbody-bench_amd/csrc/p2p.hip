@@ -602,18 +602,6 @@ __global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ it
         pass(std::integral_constant<int, F64_TILES>{});
 }
 
-// Sources of each cell's own NI entries (the leaf's full list is its
-// ancestors' entries and its own, solver_ref.hpp:126).
-__global__ __launch_bounds__(256) void k_ni_local(int64_t ncells, const uint32_t *__restrict__ count, const int32_t *__restrict__ ni,
-                                                  const int32_t *__restrict__ ni_cnt, uint32_t *__restrict__ local) {
-    const int64_t c = blockIdx.x * 256ll + threadIdx.x;
-    if (c >= ncells) return;
-    const int ne = ni_cnt[c];
-    uint32_t s = 0;
-    for (int e = 0; e < ne; ++e) s += count[ni[27 * c + e]];
-    local[c] = s;
-}
-
 // Leaf classes, by the cost of their items (16-target tiles times 64-source
 // groups): class j costs at least 2^(8 - j), so the largest start first.
 constexpr int NCLS = 7;
@@ -753,10 +741,8 @@ void p2p_plan(Ctx &c, bool potential) {
     c.p2p_cls.ensure(nl);
     c.p2p_src.ensure(nl);
     c.p2p_item_off.ensure(nl);
-    c.p2p_local.ensure(t.ncells);
     c.p2p_pre.ensure(static_cast<size_t>(nl) * NSC);
     c.p2p_btot.ensure(static_cast<size_t>(nb) * NSC);
-    k_ni_local<<<ceil_div(t.ncells, 256), 256, 0, c.stream>>>(t.ncells, t.count, t.ni, t.ni_cnt, c.p2p_local);
     // under 8 leaves per CU (the 16k Plummer sphere has 430): FP32 items of MC_COST,
     // scaled down by the leaf shortfall, so that there are still several per SIMD;
     // FP64 items take some five times as long, so they shrink from more leaves on

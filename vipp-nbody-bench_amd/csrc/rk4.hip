@@ -14,24 +14,15 @@
 namespace vg {
 namespace {
 
-__global__ __launch_bounds__(256) void k_rk4_init(int64_t n3, const double *__restrict__ x, const double *__restrict__ v, double *__restrict__ x0,
-                                                  double *__restrict__ v0, double *__restrict__ xo, double *__restrict__ vo) {
-    const int64_t i = blockIdx.x * 256ll + threadIdx.x;
-    if (i >= n3) return;
-    x0[i] = x[i];
-    xo[i] = x[i];
-    v0[i] = v[i];
-    vo[i] = v[i];
-}
-
-// accumulate with weight cw, then take the next Euler state with step h
-// (last stage: copy the accumulated state out instead).  Grid-stride over the
+// accumulate with weight cw, then take the next Euler state with step h (last
+// stage: copy the accumulated state out instead).  The first stage keeps the
+// state it finds as x0 and v0 and accumulates from it.  Grid-stride over the
 // 3n scalars; each block also leaves the partial bounding box of the positions
 // it wrote (7 doubles at part, the layout of k_aabb), so the next tree build
 // needs no pass of its own over x.
 template <class A>
-__global__ __launch_bounds__(256) void k_rk4_stage(int64_t n3, double cw, double h, int last, const A *__restrict__ a, double *__restrict__ x,
-                                                   double *__restrict__ v, const double *__restrict__ x0, const double *__restrict__ v0,
+__global__ __launch_bounds__(256) void k_rk4_stage(int64_t n3, double cw, double h, bool first, bool last, const A *__restrict__ a, double *__restrict__ x,
+                                                   double *__restrict__ v, double *__restrict__ x0, double *__restrict__ v0,
                                                    double *__restrict__ xo, double *__restrict__ vo, double *__restrict__ part) {
     double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
     double bad = 0;
@@ -41,9 +32,9 @@ __global__ __launch_bounds__(256) void k_rk4_stage(int64_t n3, double cw, double
     int comp = static_cast<int>(i % 3);
     for (; i < n3; i += stride) {
         const double ai = static_cast<double>(a[i]);
-        const double vi = v[i];
-        const double xon = xo[i] + cw * vi;
-        const double von = vo[i] + cw * ai;
+        const double vi = v[i], xi = first ? x[i] : 0.0;
+        const double xon = (first ? xi : xo[i]) + cw * vi;
+        const double von = (first ? vi : vo[i]) + cw * ai;
         double xn;
         if (last) {
             xn = xon;
@@ -51,8 +42,12 @@ __global__ __launch_bounds__(256) void k_rk4_stage(int64_t n3, double cw, double
         } else {
             xo[i] = xon;
             vo[i] = von;
-            xn = x0[i] + vi * h;
-            v[i] = v0[i] + ai * h;
+            if (first) {
+                x0[i] = xi;
+                v0[i] = vi;
+            }
+            xn = (first ? xi : x0[i]) + vi * h;
+            v[i] = (first ? vi : v0[i]) + ai * h;
         }
         x[i] = xn;
         if (!isfinite(xn)) bad = 1;
@@ -122,25 +117,19 @@ __global__ __launch_bounds__(256) void k_count(int64_t nc, const int8_t *__restr
 
 }  // namespace
 
-void rk4_init(Ctx &c) {
-    const int64_t n3 = 3 * c.n;
-    k_rk4_init<<<ceil_div(n3, 256), 256, 0, c.stream>>>(n3, c.x, c.v, c.x0, c.v0, c.xo, c.vo);
-    VG_LAUNCH_CHECK();
-}
-
 void rk4_stage(Ctx &c, int stage, double dt) {
     const int64_t n3 = 3 * c.n;
     // weights and Euler steps of solver_ref.hpp:58-99
     const double cw = (stage == 0 || stage == 3) ? dt / 6 : dt / 3;
     const double h = stage == 2 ? dt : dt / 2;
-    const int last = stage == 3;
+    const bool first = stage == 0, last = stage == 3;
     const int nb = static_cast<int>(std::min<int64_t>(1024, std::max<int64_t>(1, ceil_div(n3, 256))));
     c.aabb_part.ensure(7 * static_cast<size_t>(nb));
     c.aabb_parts = 0;
     if (c.prec == 0)
-        k_rk4_stage<double><<<nb, 256, 0, c.stream>>>(n3, cw, h, last, c.acc64, c.x, c.v, c.x0, c.v0, c.xo, c.vo, c.aabb_part);
+        k_rk4_stage<double><<<nb, 256, 0, c.stream>>>(n3, cw, h, first, last, c.acc64, c.x, c.v, c.x0, c.v0, c.xo, c.vo, c.aabb_part);
     else
-        k_rk4_stage<float><<<nb, 256, 0, c.stream>>>(n3, cw, h, last, c.acc32, c.x, c.v, c.x0, c.v0, c.xo, c.vo, c.aabb_part);
+        k_rk4_stage<float><<<nb, 256, 0, c.stream>>>(n3, cw, h, first, last, c.acc32, c.x, c.v, c.x0, c.v0, c.xo, c.vo, c.aabb_part);
     VG_LAUNCH_CHECK();
     c.aabb_parts = nb;
 }

@@ -564,7 +564,8 @@ __device__ inline uint64_t path_code(int d, int x, int y, int z) {
 }
 
 // NB list of one internal cell and the NI and AP lists of its 8 children per wavefront
-// (4 per block).  The children share their candidates: the children of the
+// (4 per block), and the number of particles in the NI cells of each (the P2P's sources).
+// The children share their candidates: the children of the
 // cell's NB cells, taken in the order of solver_ref.hpp:129-147 (NB entry e, child
 // offset q).  Lane l tests candidate 64 r + l of round r against all 8
 // siblings; each sibling's NI / AP entries are appended in candidate
@@ -575,13 +576,14 @@ __global__ __launch_bounds__(256) void k_lists(const uint32_t *__restrict__ lv, 
                                                const uint64_t *__restrict__ int_code, const int8_t *__restrict__ level, const int32_t *__restrict__ child,
                                                const int32_t *__restrict__ grid, int32_t *__restrict__ nb, int32_t *__restrict__ ni, int32_t *__restrict__ ap,
                                                int32_t *__restrict__ nb_cnt, int32_t *__restrict__ ni_cnt, int32_t *__restrict__ ap_cnt,
-                                               int32_t *__restrict__ nbr27) {
+                                               int32_t *__restrict__ nbr27, const uint32_t *__restrict__ count, uint32_t *__restrict__ local) {
     __shared__ int32_t s_r[4][28], s_o[4][28];
     const int64_t nc = lv_cells(lv, SH, cap), nint = nc / 8;  // nc = 1 + 8 nint
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (blockIdx.x == 0 && threadIdx.x == 0 && nc > 0) {  // the root (solver_ref.hpp:149-152); with children, its NB list is its own wavefront's
         ap_cnt[0] = 0;
         ni_cnt[0] = nint ? 0 : 1;
+        local[0] = nint ? 0 : count[0];
         if (nint == 0) {
             ni[0] = 0;
             nb_cnt[0] = 0;
@@ -634,8 +636,9 @@ __global__ __launch_bounds__(256) void k_lists(const uint32_t *__restrict__ lv, 
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const uint64_t below = (1ull << lane) - 1;
     int nin[8], apn[8];
+    uint32_t src[8];  // this lane's share of the particles in each child's NI cells
 #pragma unroll
-    for (int t = 0; t < 8; ++t) nin[t] = apn[t] = 0;
+    for (int t = 0; t < 8; ++t) nin[t] = apn[t] = 0, src[t] = 0;
     const int ncand = 8 * npn;
     for (int r0 = 0; r0 < ncand; r0 += 64) {
         const int cand = r0 + lane, q = lane & 7;
@@ -643,6 +646,7 @@ __global__ __launch_bounds__(256) void k_lists(const uint32_t *__restrict__ lv, 
         int32_t cc = 0;
         int cx = 0, cy = 0, cz = 0;  // position relative to the first child position of P
         bool cint = false;
+        uint32_t cn = 0;
         if (valid) {
             const int o = s_o[w][cand / 8];
             cc = 1 + 8 * s_r[w][cand / 8] + q;
@@ -650,6 +654,7 @@ __global__ __launch_bounds__(256) void k_lists(const uint32_t *__restrict__ lv, 
             cy = 2 * (o / 3 % 3 - 1) + 1 - (q >> 1 & 1);
             cz = 2 * (o / 9 - 1) + 1 - (q >> 2);
             cint = child[cc] >= 0;
+            cn = count[cc];
         }
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
@@ -663,17 +668,23 @@ __global__ __launch_bounds__(256) void k_lists(const uint32_t *__restrict__ lv, 
             if (isap) ap[189 * static_cast<int64_t>(ct) + apn[t] + __popcll(map & below)] = cc;
             nin[t] += __popcll(mni);
             apn[t] += __popcll(map);
+            src[t] += isni ? cn : 0u;
         }
     }
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+        for (int s = 32; s > 0; s >>= 1) src[t] += __shfl_xor(src[t], s, 64);
     if (lane < 8) {
         int b = 0, e = 0;
+        uint32_t n = 0;
         bool lf = false;
 #pragma unroll
         for (int t = 0; t < 8; ++t)
-            if (lane == t) b = nin[t], e = apn[t], lf = leaf[t];
+            if (lane == t) b = nin[t], e = apn[t], n = src[t], lf = leaf[t];
         if (lf) nb_cnt[cb + lane] = 0;  // an internal child has its own wavefront
         ni_cnt[cb + lane] = b;
         ap_cnt[cb + lane] = e;
+        local[cb + lane] = n;
     }
 }
 
@@ -786,8 +797,9 @@ static void lists_enqueue(Ctx &c, int SH, int64_t cap) {
     t.ni_cnt.ensure(cap);
     t.ap_cnt.ensure(cap);
     t.nbr27.ensure(27 * cap);
+    c.p2p_local.ensure(cap);
     k_lists<<<ceil_div(std::max<int64_t>(1, cap / 8), 4), 256, 0, c.stream>>>(t.lv, SH, cap, t.int_ids, t.int_code, t.level, t.child, t.grid, t.nb, t.ni,
-                                                                            t.ap, t.nb_cnt, t.ni_cnt, t.ap_cnt, t.nbr27);
+                                                                            t.ap, t.nb_cnt, t.ni_cnt, t.ap_cnt, t.nbr27, t.count, c.p2p_local);
     VG_LAUNCH_CHECK();
 }
 
