@@ -68,3 +68,32 @@ def test_coincident_and_far(vg):
     ra, rp, sa, sp = _reference(x[keep], near - (near > 300), np.full(n - 1, 1.0 / n), 1.0, 0.0)
     u = (n + 8) * 2.0 ** -53
     assert (abs(a[near] - ra) <= u * sa).all() and (abs(pot[near] - rp) <= u * sp).all()
+
+
+def test_direct_small_and_large_samples_in_one_context():
+    """Samples whose buffers the context keeps, and one of more than a million targets that it does not."""
+    import vipp_gravity as vg
+    rng = np.random.default_rng(12)
+    n = 3000
+    with vg.Gravity(n, 64, 4, "f64", eps=1e-3) as g:
+        g.upload(rng.random((n, 3)))
+        ref, pot = g.direct(np.arange(n), potential=True)
+        for k in (50, 1_100_000, 700):
+            idx = rng.integers(0, n, k)
+            a, b = g.direct(idx, potential=True)
+            # the sources are cut into other slices: sums of 3000 terms in another order
+            assert np.abs(a - ref[idx]).max() <= 1e-12 * np.abs(ref).max() and np.abs(b - pot[idx]).max() <= 1e-12 * pot.max()
+
+
+@pytest.mark.parametrize("n", [43690, 43691, 90001])
+def test_accelerations_through_the_staging_buffers(n):
+    """FP32 results come in pieces of 2^17 values: one, one and one value, and three."""
+    import vipp_gravity as vg
+    x = np.random.default_rng(n).random((n, 3))
+    a = {}
+    for mode in ("f64", "f32"):
+        with vg.Gravity(n, 64, 6, mode, eps=1e-2) as g:
+            g.upload(x)
+            a[mode] = g.accelerations()
+            assert np.array_equal(a[mode], g.accelerations())
+    assert np.abs(a["f32"] - a["f64"]).max() <= 1e-3 * np.abs(a["f64"]).max()

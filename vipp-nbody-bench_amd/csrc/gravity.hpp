@@ -114,7 +114,9 @@ struct Ctx {
     // pinned host words for what the host reads during an evaluation (tree
     // level sizes, root box, P2P plan), written by the kernels themselves
     void *pinned = nullptr;
-    static constexpr size_t PINNED_BYTES = 4096;
+    static constexpr size_t PINNED_BYTES = 12288, PINNED_ENERGY = 4096;  // from PINNED_ENERGY on: partial energies
+    float *stage = nullptr;  // two pinned buffers on the way of FP32 results to the host (fetch_widened)
+    hipEvent_t ev_stage[2] = {};
     bool timing = false;
     hipEvent_t ev[2 * PH_COUNT] = {};
     double phase_ms[PH_COUNT] = {};
@@ -172,6 +174,10 @@ struct Ctx {
     DevBuf<float> p2p_part32;
     DevBuf<double> p2p_part64;
 
+    // direct sums of a sample: kept where they are small (direct_subset)
+    DevBuf<int64_t> dir_idx;
+    DevBuf<double> dir_buf;
+
     double counts[8] = {};
 
     Closure cl;
@@ -191,8 +197,7 @@ void fmm_downward(Ctx &c, bool potential);  // L2L, L2P and the way back to the 
 void join_p2p(Ctx &c);                       // ctx.stream waits for a P2P launched on ctx.stream2
 void rk4_stage(Ctx &c, int stage, double dt);
 void count_work(Ctx &c);
-double kinetic_energy(Ctx &c);
-double potential_energy(Ctx &c);
+void energies(Ctx &c, double &kinetic, double &potential);  // of the state and of the potentials last formed
 void closure_inputs(Ctx &c, bool with_l25);  // network inputs of every non-empty leaf from the current L32
 void closure_apply(Ctx &c);                   // L~_25 += |L~_25| MLP(x) and fallback flags
 bool closure_fallback_prepare(Ctx &c);        // order-p_hi locals of the flagged leaves; false if none is flagged

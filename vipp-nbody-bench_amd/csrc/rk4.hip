@@ -63,14 +63,18 @@ __global__ __launch_bounds__(256) void k_rk4_stage(int64_t n3, double cw, double
     aabb_block_store(lo, hi, bad, part + 7ll * blockIdx.x);
 }
 
-// FP64 block reduction of per-particle terms: kind 0 = m |v|^2, kind 1 = m * pot
-__global__ __launch_bounds__(256) void k_energy(int64_t n, int kind, const double *__restrict__ v, const double *__restrict__ m, double mass,
-                                                const double *__restrict__ pot, double *__restrict__ part) {
+// FP64 block sums of m |v|^2 (the first half of the grid) and m pot (the second) into
+// pinned host memory: one launch and one wait, where two of each, a copy and a device
+// allocation took 56 us of the 995 that the energies of 256k particles took.
+constexpr int EN_BLOCKS = 256;
+__global__ __launch_bounds__(256) void k_energy(int64_t n, const double *__restrict__ v, const double *__restrict__ m, double mass,
+                                                const double *__restrict__ pot, double *part) {
     __shared__ double s[256];
+    const bool kinetic = blockIdx.x < EN_BLOCKS;
     double acc = 0;
-    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += static_cast<int64_t>(gridDim.x) * 256) {
+    for (int64_t i = blockIdx.x % EN_BLOCKS * 256ll + threadIdx.x; i < n; i += EN_BLOCKS * 256) {
         const double mi = m ? m[i] : mass;
-        if (kind == 0)
+        if (kinetic)
             acc += mi * (v[3 * i] * v[3 * i] + v[3 * i + 1] * v[3 * i + 1] + v[3 * i + 2] * v[3 * i + 2]);
         else
             acc += mi * pot[i];
@@ -134,23 +138,18 @@ void rk4_stage(Ctx &c, int stage, double dt) {
     c.aabb_parts = nb;
 }
 
-static double reduce_energy(Ctx &c, int kind) {
-    const int nb = 256;
-    DevBuf<double> part;
-    part.ensure(nb);
-    k_energy<<<nb, 256, 0, c.stream>>>(c.n, kind, c.v, c.has_masses ? c.m.p : nullptr, c.mass, c.pot64.p, part);
+void energies(Ctx &c, double &kinetic, double &potential) {
+    double *part = reinterpret_cast<double *>(static_cast<char *>(c.pinned) + Ctx::PINNED_ENERGY);
+    static_assert(Ctx::PINNED_ENERGY + 2 * EN_BLOCKS * sizeof(double) <= Ctx::PINNED_BYTES - 64, "pinned words");
+    k_energy<<<2 * EN_BLOCKS, 256, 0, c.stream>>>(c.n, c.v, c.has_masses ? c.m.p : nullptr, c.mass, c.pot64.p, part);
     VG_LAUNCH_CHECK();
-    std::vector<double> h(nb);
-    VG_HIP(hipMemcpyAsync(h.data(), part.p, nb * sizeof(double), hipMemcpyDeviceToHost, c.stream));
     VG_HIP(hipStreamSynchronize(c.stream));
-    double s = 0;
-    for (double q : h) s += q;  // fixed order: deterministic
-    return s;
+    double ke = 0, pe = 0;
+    for (int b = 0; b < EN_BLOCKS; ++b) ke += part[b];  // fixed order: deterministic
+    for (int b = 0; b < EN_BLOCKS; ++b) pe += part[EN_BLOCKS + b];
+    kinetic = 0.5 * ke;
+    potential = -0.5 * c.G * pe;
 }
-
-double kinetic_energy(Ctx &c) { return 0.5 * reduce_energy(c, 0); }
-
-double potential_energy(Ctx &c) { return -0.5 * c.G * reduce_energy(c, 1); }
 
 void count_work(Ctx &c) {
     TreeDev &t = c.t;
