@@ -96,6 +96,13 @@ __device__ inline double rsq(double x) {
     return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
+// x as two BF16 halves, hi = bf16(x) and lo = bf16(x - hi) (the split M2L's multipoles).
+__device__ __forceinline__ void split_m(float x, uint32_t &hi, uint32_t &lo) {
+    const __bf16 h = static_cast<__bf16>(x);
+    hi = __builtin_bit_cast(uint16_t, h);
+    lo = __builtin_bit_cast(uint16_t, static_cast<__bf16>(x - static_cast<float>(h)));
+}
+
 // Real-packed index of a degree-n, order-m (m >= 0) coefficient: degree n owns
 // entries [n*n, (n+1)*(n+1)): Re(m=0), then (Re, Im) for m = 1..n.
 __host__ __device__ inline int kidx_re(int n, int m) { return m == 0 ? n * n : n * n + 2 * m - 1; }

@@ -269,7 +269,7 @@ template <class R, int P>
 __global__ __launch_bounds__(256) void k_p2m(const int32_t *__restrict__ leaves, int nleaves, const int8_t *__restrict__ level,
                                              const uint32_t *__restrict__ start, const uint32_t *__restrict__ count, const double *__restrict__ bmin,
                                              const double *__restrict__ bmax, const double *__restrict__ xs64, double wx0, int K, int ldk,
-                                             R *__restrict__ M) {
+                                             R *__restrict__ M, uint16_t *__restrict__ Ms) {
     constexpr int p = P;       // the order is a template argument, so the recurrence unrolls fully
     constexpr int NS = P + 2;  // recurrence steps per lane
     __shared__ R red[4][64][2 * NS];
@@ -385,9 +385,19 @@ __global__ __launch_bounds__(256) void k_p2m(const int32_t *__restrict__ leaves,
         if (part == 1 && m == 0) continue;
         R sum = 0;
         for (int gg = 0; gg < G; ++gg) sum += red[w][gg * NM + oi][2 * ost + part];
-        out[part == 0 ? kidx_re(n, m) : kidx_im(n, m)] = sum;
+        const int at = part == 0 ? kidx_re(n, m) : kidx_im(n, m);
+        out[at] = sum;
+        if (Ms) {  // split mode: M2L's halves too
+            uint32_t h, l;
+            split_m(static_cast<float>(sum), h, l);
+            Ms[static_cast<size_t>(c) * 2 * ldk + at] = static_cast<uint16_t>(h);
+            Ms[static_cast<size_t>(c) * 2 * ldk + ldk + at] = static_cast<uint16_t>(l);
+        }
     }
-    for (int q = K + lane; q < ldk; q += 64) out[q] = R(0);
+    for (int q = K + lane; q < ldk; q += 64) {
+        out[q] = R(0);
+        if (Ms) Ms[static_cast<size_t>(c) * 2 * ldk + q] = Ms[static_cast<size_t>(c) * 2 * ldk + ldk + q] = 0;
+    }
 }
 
 // FP64 M2M (solver_ref.hpp:196-197) and L2L of the internal cells of one tree level, PB parents per block: every operator word read
@@ -1252,11 +1262,13 @@ template <class R>
 void upward_t(Ctx &c) {
     TreeDev &t = c.t;
     Bufs<R>::ensure(c, t.ncells);
+    if (c.prec == 2) c.msplit.ensure(static_cast<size_t>(t.ncells) * 2 * c.ldk);
+    uint16_t *ms = c.prec == 2 ? c.msplit.p : nullptr;
     const double wx0 = t.box[3] - t.box[0];
     if (t.nleaves) {
 #define VG_P2M(P_)                                                                                                                          \
     k_p2m<R, P_><<<ceil_div(t.nleaves, 4), 256, 0, c.stream>>>(t.leaf_ids, static_cast<int>(t.nleaves), t.level, t.start, t.count, t.bmin, \
-                                                               t.bmax, c.xs64, wx0, c.K, c.ldk, Bufs<R>::M(c))
+                                                               t.bmax, c.xs64, wx0, c.K, c.ldk, Bufs<R>::M(c), ms)
         switch (c.p) {
             case 1: VG_P2M(1); break;
             case 2: VG_P2M(2); break;

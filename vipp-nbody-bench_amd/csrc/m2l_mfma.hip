@@ -15,7 +15,7 @@
 // (16 significant bits together) and a product is formed as
 // hi*hi + hi*lo + lo*hi with FP32 accumulation; the dropped lo*lo term and the
 // split residuals are ~2^-18 of the product.  T_o is split from its FP64
-// value; the multipoles are split once per evaluation (k_split_m).  M2M and
+// value; the multipoles are split by the kernels that form them (P2M and M2M).  M2M and
 // L2L use a three-way split (below).
 //
 // Operand layouts (checked on the device): for v_mfma_f32_16x16x32_bf16 lane l
@@ -281,32 +281,6 @@ __global__ __launch_bounds__(64 * SplitShape<P>::NW, 2) void k_m2l_split(const i
     }
 }
 
-// M (FP32, row stride ldk, a multiple of 16) -> per cell ldk BF16 hi values
-// then ldk lo values.  A block takes SPLIT_CELLS cells, a thread 4
-// coefficients at a time (one 16-byte load, two 8-byte stores); the cell and
-// the position in it come from a 32-bit division of the block-local index.
-constexpr int SPLIT_CELLS = 32;
-__global__ __launch_bounds__(256) void k_split_m(const float4 *__restrict__ M, int64_t n, int ldk, uint2 *__restrict__ Ms) {
-    const uint32_t vpr = static_cast<uint32_t>(ldk) / 4;  // 4-coefficient vectors per cell
-    const int64_t c0 = static_cast<int64_t>(blockIdx.x) * SPLIT_CELLS;
-    const uint32_t nv = static_cast<uint32_t>(min<int64_t>(SPLIT_CELLS, n - c0)) * vpr;
-    for (uint32_t t = threadIdx.x; t < nv; t += 256) {
-        const uint32_t cl = t / vpr, k = t - cl * vpr;
-        const int64_t c = c0 + cl;
-        const float4 x = M[c * vpr + k];
-        const float v[4] = {x.x, x.y, x.z, x.w};
-        uint32_t h[4], l[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const __bf16 hb = static_cast<__bf16>(v[e]);
-            h[e] = __builtin_bit_cast(uint16_t, hb);
-            l[e] = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v[e] - static_cast<float>(hb)));
-        }
-        Ms[c * 2 * vpr + k] = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-        Ms[c * 2 * vpr + vpr + k] = make_uint2(l[0] | (l[1] << 16), l[2] | (l[3] << 16));
-    }
-}
-
 // ---------------------------------------------------------------------------
 // M2M and L2L of one tree level on the matrix cores.  Their work is small
 // (8 operators per level instead of 189 offsets), so they take a three-way
@@ -346,49 +320,38 @@ __global__ __launch_bounds__(256) void k_split_ops_ml(const double *__restrict__
     }
 }
 
-// Expansions of 32 cells (row stride ldk = 16 NKS; cells[t] < 0: zeros) ->
-// LDS as h/m/l B fragments of one n-tile, the M2L kernel's slot order.  Rows
-// K .. ldk-1 are read as zero whatever the buffer holds there (the locals'
-// padding is never written).
-template <int K, int NKS, int NTH>
-__device__ __forceinline__ void stage_split(bf16x8 (*sB)[3][64], const float *__restrict__ src, int ldk, const int32_t *cells) {
-    for (int c = threadIdx.x; c < 32 * 2 * NKS; c += NTH) {
-        const int t = c / (2 * NKS), k8 = c % (2 * NKS);
-        const int32_t cell = cells[t];
-        float4 a = make_float4(0, 0, 0, 0), b = a;
-        if (cell >= 0) {
-            const float4 *q = reinterpret_cast<const float4 *>(src + static_cast<int64_t>(cell) * ldk + 8 * k8);
-            a = q[0];
-            b = q[1];
+// One m-tile of T (fragment block fb) times the expansions src of the lanes' columns (row
+// stride 16 NKS; nullptr: zeros): the six products of the three-way split down to 2^-16
+// relative, smallest first.  Each lane splits the 8 coefficients that its operand
+// holds; those from K on are taken as zero whatever the buffer holds there (the
+// locals' padding is not defined).
+template <int K>
+__device__ __forceinline__ f32x16 ml_tile(const bf16x8 *__restrict__ fb, int mt, int lane, const float *__restrict__ src) {
+    constexpr int NKS = ks_of(K);
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    const bf16x8 *A = fb + static_cast<size_t>(mt * 3) * NKS * 64 + lane;
+    const int half = lane >> 5;
+#pragma unroll 4
+    for (int ks = 0; ks < NKS; ++ks) {
+        const bf16x8 ah = A[ks * 64], am = A[(NKS + ks) * 64], al = A[(2 * NKS + ks) * 64];
+        float4 x = make_float4(0, 0, 0, 0), y = x;
+        if (src) {
+            const float4 *w = reinterpret_cast<const float4 *>(src + 16 * ks + 8 * half);
+            x = w[0];
+            y = w[1];
         }
-        float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-        bf16x8 h, m, l;
+        const float v[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+        bf16x8 bh, bm, bl;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            if (8 * k8 + e >= K) v[e] = 0.0f;
-            __bf16 he, me, le;
-            split3(v[e], he, me, le);
-            h[e] = he;
-            m[e] = me;
-            l[e] = le;
+            __bf16 h, m, l;
+            split3(16 * ks + 8 * half + e < K ? v[e] : 0.0f, h, m, l);
+            bh[e] = h;
+            bm[e] = m;
+            bl[e] = l;
         }
-        const int ln = ((k8 & 1) * 32 + t) ^ (k8 & 15);
-        sB[k8 >> 1][0][ln] = h;
-        sB[k8 >> 1][1][ln] = m;
-        sB[k8 >> 1][2][ln] = l;
-    }
-}
-
-// acc += T (m-tile mt of fragment block fb) x B (LDS): the six products of
-// the three-way split down to 2^-16 relative, smallest first
-template <int NKS>
-__device__ __forceinline__ void mfma_split_tile(const bf16x8 *__restrict__ fb, int mt, int lane, bf16x8 (*sB)[3][64], f32x16 &acc) {
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) {
-        const bf16x8 ah = fb[(mt * 3) * NKS * 64 + ks * 64 + lane], am = fb[(mt * 3 + 1) * NKS * 64 + ks * 64 + lane],
-                     al = fb[(mt * 3 + 2) * NKS * 64 + ks * 64 + lane];
-        const int slot = lane ^ ((2 * ks + (lane >> 5)) & 15);
-        const bf16x8 bh = sB[ks][0][slot], bm = sB[ks][1][slot], bl = sB[ks][2][slot];
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bl, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, bm, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(al, bh, acc, 0, 0, 0);
@@ -396,95 +359,59 @@ __device__ __forceinline__ void mfma_split_tile(const bf16x8 *__restrict__ fb, i
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(am, bh, acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ah, bh, acc, 0, 0, 0);
     }
+    return acc;
 }
 
-// C of the wavefront's m-tile -> sO[t][row] (row stride OST, odd, so the 32
-// targets of one row fall in different banks)
-template <int OST>
-__device__ __forceinline__ void park_tile(float *sO, int mt, int lane, const f32x16 &acc) {
+// M2M (UP, solver_ref.hpp:196-197) and L2L (solver_ref.hpp:217-218) of one level: block =
+// (32 parents, one 32-row m-tile), a wavefront each octant q.  M2M: T_q M(child q), zero for
+// an empty child, summed in octant order through LDS into the parent's multipoles and
+// their halves for M2L.  L2L: L(child q) += T'_q L(parent) for every non-empty child.
+// Levels are small, and bound by launches and the latency of one pass; operands come from L2
+// straight into registers.  A block per octant, with the expansions split and the result
+// put together in LDS, needed a second kernel for the sum over the octants: M2M and L2L per
+// evaluation of 100k bodies p = 8 47 + 49 -> 37 + 41 us, L2L of 4M p = 12 226 -> 148, of 16M
+// 641 -> 383; a step of 4M 35.96 -> 35.64 ms, closure step of 1M 10.76 -> 10.58 (both with the
+// multipoles' halves written here and by P2M, not by a pass of their own).
+template <int P, bool UP>
+__global__ __launch_bounds__(512) void k_ml_split(const int32_t *__restrict__ ids, int n, const int32_t *__restrict__ child,
+                                                  const uint32_t *__restrict__ count, const bf16x8 *__restrict__ frag, float *__restrict__ X, int ldk,
+                                                  uint16_t *__restrict__ Ms) {
+    constexpr int K = (P + 1) * (P + 1), MT = mt_of(K), NKS = ks_of(K);
+    const int lane = threadIdx.x & 63, half = lane >> 5;
+    const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int mt = blockIdx.x % MT, i = static_cast<int>(blockIdx.x / MT) * 32 + (lane & 31);
+    const int32_t par = i < n ? ids[i] : -1;
+    int32_t cell = par >= 0 ? child[par] + q : -1;
+    if (cell >= 0 && count[cell] == 0) cell = -1;
+    const int32_t from = UP || cell < 0 ? cell : par;
+    const f32x16 acc = ml_tile<K>(frag + static_cast<size_t>(UP ? q : 8 + q) * MT * 3 * NKS * 64, mt, lane,
+                                  from >= 0 ? X + static_cast<size_t>(from) * ldk : nullptr);
+    // acc[4 g + e]: row 32 mt + 8 g + 4 half + e of column lane % 32
+    if constexpr (UP) {
+        __shared__ f32x4 s_acc[8][4][64];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) sO[(lane & 31) * OST + mt * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)] = acc[r];
-}
-
-// M2M (solver_ref.hpp:196-197), first pass: block = (32 parents, child
-// octant q) forms T_q M(child q) (zero for an empty child) into
-// part[q][parent][row], rows K .. ldk-1 zero (zero rows of the operators).
-template <int P>
-__global__ __launch_bounds__(64 * mt_of((P + 1) * (P + 1))) void k_m2m_split(const int32_t *__restrict__ ids, int n, const int32_t *__restrict__ child,
-                                                                          const uint32_t *__restrict__ count, const bf16x8 *__restrict__ frag,
-                                                                          const float *__restrict__ M, int ldk, float *__restrict__ part) {
-    constexpr int K = (P + 1) * (P + 1), MT = mt_of(K), NKS = ks_of(K), NTH = 64 * MT;
-    constexpr int OST = MT * 32 + 1;
-    __shared__ bf16x8 sB[NKS][3][64];
-    __shared__ float sO[32 * OST];
-    __shared__ int32_t s_cell[32];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int mt = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int q = blockIdx.x & 7, chunk = blockIdx.x >> 3;
-    if (tid < 32) {
-        const int32_t P0 = chunk * 32 + tid < n ? ids[chunk * 32 + tid] : -1;
-        const int32_t cq = P0 >= 0 ? child[P0] + q : -1;
-        s_cell[tid] = (cq >= 0 && count[cq] > 0) ? cq : -1;
-    }
-    __syncthreads();
-    stage_split<K, NKS, NTH>(sB, M, ldk, s_cell);
-    __syncthreads();
-    f32x16 acc;
+        for (int g = 0; g < 4; ++g) s_acc[q][g][lane] = f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+        __syncthreads();
+        const int row = 32 * mt + 8 * q + 4 * half;
+        if (q < 4 && par >= 0 && row < ldk) {  // wavefront g adds the octants' rows of group g
+            f32x4 sum = s_acc[0][q][lane];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    mfma_split_tile<NKS>(frag + static_cast<int64_t>(q) * MT * 3 * NKS * 64, mt, lane, sB, acc);
-    park_tile<OST>(sO, mt, lane, acc);
-    __syncthreads();
-    const int nt = min(32, n - chunk * 32);
-    for (int i = tid; i < nt * ldk; i += NTH) {
-        const int t = i / ldk, row = i % ldk;
-        part[(static_cast<int64_t>(q) * n + chunk * 32 + t) * ldk + row] = sO[t * OST + row];
-    }
-}
-
-// M2M, second pass: M(parent) = sum over q = 0..7 of part[q][parent], in that order
-__global__ __launch_bounds__(256) void k_m2m_sum(const int32_t *__restrict__ ids, int64_t n, int ldk, const float *__restrict__ part,
-                                                 float *__restrict__ M) {
-    const int64_t i = blockIdx.x * 256ll + threadIdx.x;
-    if (i >= n * ldk) return;
-    float s = 0.0f;
+            for (int o = 1; o < 8; ++o) sum += s_acc[o][q][lane];
+            *reinterpret_cast<f32x4 *>(X + static_cast<size_t>(par) * ldk + row) = sum;
+            uint32_t h[4], l[4];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) s += part[q * n * ldk + i];
-    M[static_cast<int64_t>(ids[i / ldk]) * ldk + i % ldk] = s;
-}
-
-// L2L (solver_ref.hpp:217-218): block = (32 parents, child octant q);
-// L(child q) += T'_q L(parent) for every non-empty child.
-template <int P>
-__global__ __launch_bounds__(64 * mt_of((P + 1) * (P + 1))) void k_l2l_split(const int32_t *__restrict__ ids, int n, const int32_t *__restrict__ child,
-                                                                          const uint32_t *__restrict__ count, const bf16x8 *__restrict__ frag,
-                                                                          float *__restrict__ L, int ldk) {
-    constexpr int K = (P + 1) * (P + 1), MT = mt_of(K), NKS = ks_of(K), NTH = 64 * MT;
-    constexpr int OST = MT * 32 + 1;
-    __shared__ bf16x8 sB[NKS][3][64];
-    __shared__ float sO[32 * OST];
-    __shared__ int32_t s_par[32], s_out[32];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int mt = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int q = blockIdx.x & 7, chunk = blockIdx.x >> 3;
-    if (tid < 32) {
-        const int32_t P0 = chunk * 32 + tid < n ? ids[chunk * 32 + tid] : -1;
-        const int32_t cq = P0 >= 0 ? child[P0] + q : -1;
-        s_par[tid] = P0;
-        s_out[tid] = (cq >= 0 && count[cq] > 0) ? cq : -1;
-    }
-    __syncthreads();
-    stage_split<K, NKS, NTH>(sB, L, ldk, s_par);
-    __syncthreads();
-    f32x16 acc;
+            for (int e = 0; e < 4; ++e) split_m(sum[e], h[e], l[e]);
+            uint16_t *m = Ms + static_cast<size_t>(par) * 2 * ldk + row;
+            *reinterpret_cast<uint2 *>(m) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+            *reinterpret_cast<uint2 *>(m + ldk) = make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16);
+        }
+    } else {
+        if (cell < 0) return;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
-    mfma_split_tile<NKS>(frag + static_cast<int64_t>(8 + q) * MT * 3 * NKS * 64, mt, lane, sB, acc);
-    park_tile<OST>(sO, mt, lane, acc);
-    __syncthreads();
-    for (int i = tid; i < 32 * K; i += NTH) {  // each child's row updated contiguously
-        const int t = i / K, row = i % K;
-        if (s_out[t] >= 0) L[static_cast<int64_t>(s_out[t]) * ldk + row] += sO[t * OST + row];
+        for (int g = 0; g < 4; ++g) {
+            const int row = 32 * mt + 8 * g + 4 * half;
+            if (row < ldk) *reinterpret_cast<f32x4 *>(X + static_cast<size_t>(cell) * ldk + row) += f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+        }
     }
 }
 
@@ -493,12 +420,11 @@ void launch_ml(Ctx &c, const int32_t *ids, int64_t n, bool m2m) {
     constexpr int K = (P + 1) * (P + 1);
     const unsigned grid = static_cast<unsigned>(ceil_div(n, 32));
     const bf16x8 *frag = reinterpret_cast<const bf16x8 *>(c.opsplit_ml.p);
-    if (m2m) {
-        c.ml_part.ensure(static_cast<size_t>(8 * n * c.ldk));
-        k_m2m_split<P><<<8 * grid, 64 * mt_of(K), 0, c.stream>>>(ids, static_cast<int>(n), c.t.child, c.t.count, frag, c.M32, c.ldk, c.ml_part);
-        k_m2m_sum<<<ceil_div(n * c.ldk, 256), 256, 0, c.stream>>>(ids, n, c.ldk, c.ml_part, c.M32);
-    } else
-        k_l2l_split<P><<<8 * grid, 64 * mt_of(K), 0, c.stream>>>(ids, static_cast<int>(n), c.t.child, c.t.count, frag, c.L32, c.ldk);
+    const int np = static_cast<int>(n);
+    if (m2m)
+        k_ml_split<P, true><<<grid * mt_of(K), 512, 0, c.stream>>>(ids, np, c.t.child, c.t.count, frag, c.M32, c.ldk, c.msplit);
+    else
+        k_ml_split<P, false><<<grid * mt_of(K), 512, 0, c.stream>>>(ids, np, c.t.child, c.t.count, frag, c.L32, c.ldk, nullptr);
     VG_LAUNCH_CHECK();
 }
 
@@ -550,11 +476,6 @@ void ml_split_level(Ctx &c, const int32_t *ids, int64_t n, bool m2m) {
 
 void fmm_m2l_split_list(Ctx &c, const int32_t *parents, int np) {
     if (np <= 0) return;
-    const int64_t nc = c.t.ncells;
-    c.msplit.ensure(static_cast<size_t>(nc) * 2 * c.ldk);
-    k_split_m<<<ceil_div(nc, SPLIT_CELLS), 256, 0, c.stream>>>(reinterpret_cast<const float4 *>(c.M32.p), nc, c.ldk,
-                                                             reinterpret_cast<uint2 *>(c.msplit.p));
-    VG_LAUNCH_CHECK();
     switch (c.p) {
         case 1: launch_split<1>(c, parents, np); break;
         case 2: launch_split<2>(c, parents, np); break;
