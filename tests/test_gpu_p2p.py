@@ -93,3 +93,39 @@ def test_streams_equal_one_stream(vg, mode, s):
                 runs.append((g.accelerations(), g.energy()))
     for a, b in zip(runs[:3], runs[3:]):
         assert np.array_equal(a[0], b[0]) and a[1] == b[1]
+
+
+# lengths times 2^l and masses times 2^k, as SI or cgs units have them, and G so that the
+# accelerations keep their size: r^-3, m x and the sums leave the FP32 range unless taken
+# in units of their own
+@pytest.mark.parametrize("l,k", [(0, 0), (37, 110), (53, 100), (53, 0), (60, 40), (0, 100), (0, -60)])
+@pytest.mark.parametrize("eps,masses", [(0.0, True), (1e-3, True), (1e-3, False)])
+def test_p2p_f32_units(vg, l, k, eps, masses):
+    n, s = 4100, 12
+    x = _points(n, "core", n) * 2.0 ** l
+    m = np.random.default_rng(1).uniform(0.5, 1.5, n) / n * 2.0 ** k if masses else None
+    r = {}
+    for mode in ("f64", "f32", "split"):
+        with vg.Gravity(n, s, 8, mode, eps=eps * 2.0 ** l, G=1.3 * 2.0 ** (2 * l - k), mass=2.0 ** k / n) as g:
+            g.upload(x, None, m)
+            r[mode] = g.accelerations(), g.energy()[1]
+    a = r["f64"][0]
+    for mode in ("f32", "split"):
+        b = r[mode][0]
+        assert np.linalg.norm(b - a) <= BOUND * np.linalg.norm(a), mode  # false for NaN
+        assert abs(r[mode][1] - r["f64"][1]) <= 5e-6 * abs(r["f64"][1]), mode
+
+
+def test_p2p_f32_softening_beyond_the_range(vg):
+    """A softening whose square FP32 does not hold: the near field vanishes, and the potential is the far field's."""
+    n = 2000
+    x = _points(n, "uniform", 2)
+    m = np.random.default_rng(2).uniform(0.5, 1.5, n) / n
+    for s in (16, 1000):
+        u = {}
+        for mode in ("f64", "f32"):
+            with vg.Gravity(n, s, 8, mode, eps=1e25) as g:
+                g.upload(x, None, m)
+                a, u[mode] = g.accelerations(), g.energy()[1]
+                assert np.isfinite(a).all() and (s < 1000 or (abs(a) < 1e-38).all())
+        assert abs(u["f32"] - u["f64"]) <= 5e-6 * abs(u["f64"])

@@ -96,6 +96,25 @@ __device__ inline double rsq(double x) {
     return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
+// The FP32 near field forms masses times positions and r^-3 by themselves, so it
+// takes positions in units of 2^length_shift and masses in units of 2^mass_shift, which
+// its last factors undo: powers of two, so no rounding changes, and 1 in ordinary
+// units.  Lengths to 2^40 need none (r^-3 above 2^-123, normal); a root box wider
+// than 2^64, whose squares FP32 does not hold, is shifted as one of 2^64, so that
+// clusters small beside it keep their range; a softening of any size is shifted in
+// full, since nothing counts beside it.  Masses to 2^60 need none (times 2^41: 2^101).
+__host__ __device__ inline int exponent_of(double v) {  // |v| < 2^e, at least half of that
+    return static_cast<int>(__builtin_bit_cast(uint64_t, v) >> 52 & 0x7ff) - 1022;
+}
+__host__ __device__ inline double pow2(int e) { return __builtin_bit_cast(double, static_cast<uint64_t>(1023 + e) << 52); }  // -1022 <= e <= 1023
+__host__ __device__ inline int length_shift(const double *box, double eps) {
+    int e = exponent_of(fmax(fmax(box[3] - box[0], box[4] - box[1]), box[5] - box[2]));
+    if (e > 64) e = 64;
+    if (exponent_of(eps) > e) e = exponent_of(eps);
+    return e > 40 ? e - 40 : 0;
+}
+inline int mass_shift(double largest) { return exponent_of(largest) > 60 ? exponent_of(largest) - 60 : 0; }
+
 // x as two BF16 halves, hi = bf16(x) and lo = bf16(x - hi) (the split M2L's multipoles).
 __device__ __forceinline__ void split_m(float x, uint32_t &hi, uint32_t &lo) {
     const __bf16 h = static_cast<__bf16>(x);

@@ -97,6 +97,7 @@ struct Ctx {
     int device = 0;
     int ncu = 0;  // compute units of the device
     bool has_masses = false;
+    int mshift = 0;  // mass_shift of the largest mass
     bool uploaded = false;
     bool evaluated = false;
     std::string err;
@@ -141,7 +142,7 @@ struct Ctx {
     DevBuf<uint32_t> perm;      // sorted position -> caller index
     // particles in sorted order
     DevBuf<double> xs64;        // 4 per particle: x, y, z, m
-    DevBuf<float> xs32;         // 4 per particle: x - root centre (FP32), m
+    DevBuf<float> xs32;         // 4 per particle: x - root centre (FP32) in units of 2^length_shift, m in units of 2^mshift
     DevBuf<double> as64;        // 4 per particle: accel xyz, potential
     DevBuf<float> as32;
 
@@ -196,6 +197,7 @@ void fmm_downward(Ctx &c, bool potential);  // L2L, L2P and the way back to the 
 void join_p2p(Ctx &c);                       // ctx.stream waits for a P2P launched on ctx.stream2
 void rk4_stage(Ctx &c, int stage, double dt);
 void count_work(Ctx &c);
+double largest_mass(Ctx &c);  // largest finite |m| of the uploaded masses
 void energies(Ctx &c, double &kinetic, double &potential);  // of the state and of the potentials last formed
 void closure_inputs(Ctx &c, bool with_l25);  // network inputs of every non-empty leaf from the current L32
 void closure_apply(Ctx &c);                   // L~_25 += |L~_25| MLP(x) and fallback flags
@@ -215,6 +217,13 @@ void direct_subset(Ctx &c, const int64_t *idx, int64_t nidx, double *a, double *
 // scratch's address on a device (once per device, with the device current)
 void direct_subset_noalloc(Ctx &c, const int64_t *idx, int64_t nidx, double *a, double *pot);
 void noalloc_init(int device);
+
+// The squared softening of the near field, for FP32 in the units of its lengths.
+template <class R>
+R p2p_eps2(const Ctx &c) {
+    const double e = sizeof(R) == 4 ? c.eps * pow2(-length_shift(c.t.box, c.eps)) : c.eps;
+    return static_cast<R>(e * e);
+}
 
 // Waits until a kernel of the stream has written `want` to a pinned host word.
 void wait_host_word(const uint32_t *word, uint32_t want, hipStream_t st);

@@ -48,6 +48,9 @@ __host__ __device__ inline uint32_t chunk_len(uint32_t total, uint32_t nch) { re
 // sizes in one launch: 0.85 -> 0.34 ms on a 100k Plummer sphere, 0.30 -> 0.10 ms
 // on 8,000 particles.
 //
+// Range: m x and r^-3 appear by themselves, so lengths and masses far from 1 (SI and
+// cgs units) come in units of their own (length_shift, mass_shift).
+//
 // Error: positions are taken relative to the centre of the targets' box (radius
 // R), so at distance d from the box the expansion loses (R + d)^2 / d^2 in the
 // relative accuracy of r^2.  Tiles of 16 sources that come nearer than R / 8 are
@@ -250,7 +253,7 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
         hx = 0.5f * (hi[0] - lo[0]), hy = 0.5f * (hi[1] - lo[1]), hz = 0.5f * (hi[2] - lo[2]);
         // sources up to near from the box are near; ns = 1 / (2 near), 0 where all are
         const float r = sqrtf(hx * hx + hy * hy + hz * hz);
-        const float nearest = fmaxf(r * MC_NEAR, I.cell * 0.0078125f);
+        const float nearest = fmaxf(fmaxf(r * MC_NEAR, I.cell * 0.0078125f), 0x1p-40f);  // r^-3 up to 2^120
         ns = r < 1e18f ? 0.5f / nearest : 0.0f;
         hx = -ns * (hx + I.cell * 1e-5f), hy = -ns * (hy + I.cell * 1e-5f), hz = -ns * (hz + I.cell * 1e-5f);
     }
@@ -436,8 +439,8 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
                                                        const uint32_t *__restrict__ count, const int32_t *__restrict__ anc,
                                                        const int32_t *__restrict__ ni, const int32_t *__restrict__ ni_cnt,
                                                        const double *__restrict__ bmin, const double *__restrict__ bmax, const float4 *__restrict__ xs,
-                                                       float eps2, float G, bool um, bool big, float mu, float4 *__restrict__ acc,
-                                                       float4 *__restrict__ partial, uint32_t pstride) {
+                                                       float eps2, float G, bool um, bool big, float fscale, float pscale, float mlen,
+                                                       float4 *__restrict__ acc, float4 *__restrict__ partial, uint32_t pstride, float unit) {
     __shared__ McLds S;
     const McWork wk = items[blockIdx.x];
     const int32_t c = wk.cell;
@@ -449,20 +452,19 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
     I.src = lay_out_entries(wk, S.delta, reinterpret_cast<uint64_t *>(S.Q), start, count, anc, ni, ni_cnt);
     I.xs = xs;
     const double lx = bmin[3ll * c], ly = bmin[3ll * c + 1], lz = bmin[3ll * c + 2], ux = bmax[3ll * c], uy = bmax[3ll * c + 1], uz = bmax[3ll * c + 2];
-    const float wx = static_cast<float>(ux - lx), wy = static_cast<float>(uy - ly), wz = static_cast<float>(uz - lz);
+    const float wx = static_cast<float>(ux - lx) * unit, wy = static_cast<float>(uy - ly) * unit, wz = static_cast<float>(uz - lz) * unit;
     I.cell = 0.5f * sqrtf(wx * wx + wy * wy + wz * wz);
     I.eps2 = eps2;
     I.um = um;
     I.big = big;
-    const float sc = um ? mu : 1.0f;
     float4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * pstride : nullptr;
     auto emit = [&](int t, const f4 &v) {
-        const float sx = v[0] * sc, sy = v[1] * sc, sz = v[2] * sc;
-        float sp = v[3] * sc;
+        const float sx = v[0] * fscale, sy = v[1] * fscale, sz = v[2] * fscale;
+        float sp = v[3] * pscale;
         if (out) {
             out[wk.t0 + t] = float4{sx, sy, sz, sp};
         } else {
-            if (POT && eps2 > 0.0f) sp -= xs[I.pt0 + t].w * rsq(eps2);  // drop the m_i / eps self term
+            if (POT && eps2 > 0.0f) sp -= xs[I.pt0 + t].w * rsq(eps2) * mlen;  // drop the m_i / eps self term
             acc[I.pt0 + t] = float4{G * sx, G * sy, G * sz, sp};
         }
     };
@@ -785,16 +787,22 @@ void p2p_run(Ctx &c, bool potential) {
         if (split) parts.ensure(4 * static_cast<size_t>(nrows) * pstride);
         run(reinterpret_cast<const V4 *>(sorted.p), reinterpret_cast<V4 *>(sums.p), reinterpret_cast<V4 *>(parts.p));
     };
-    const R eps2 = static_cast<R>(c.eps * c.eps), G = static_cast<R>(c.G), mu = static_cast<R>(c.mass);
+    const R G = static_cast<R>(c.G);
     const bool um = !c.has_masses;  // one mass: left out of the pairs, the sums are scaled once
     if constexpr (sizeof(R) == 4) {
-        bool big = false;  // a root box so wide that squared distances may leave the FP32 range
-        for (int a = 0; a < 3; ++a) big |= !(t.box[3 + a] - t.box[a] < 1e18);
+        // units of lengths and masses, and what takes sums of m x / r^3 and m / r out of them
+        const int ls = length_shift(t.box, c.eps);
+        const float eps2 = p2p_eps2<float>(c), unit = static_cast<float>(pow2(-ls)), mlen = static_cast<float>(std::ldexp(1.0, c.mshift - ls));
+        const float fscale = static_cast<float>(um ? std::ldexp(c.mass, -2 * ls) : std::ldexp(1.0, c.mshift - 2 * ls));
+        const float pscale = um ? static_cast<float>(std::ldexp(c.mass, -ls)) : mlen;
+        bool big = false;  // a root box so wide that squared distances may leave the FP32 range all the same
+        for (int a = 0; a < 3; ++a) big |= !((t.box[3 + a] - t.box[a]) * pow2(-ls) < 1e18);
         buffers(c.xs32, c.as32, c.p2p_part32, [&](const V4 *xs, V4 *acc, V4 *part) {
             (potential ? k_p2p_mc<true> : k_p2p_mc<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs,
-                                                                                       eps2, G, um, big, mu, acc, part, pstride);
+                                                                                       eps2, G, um, big, fscale, pscale, mlen, acc, part, pstride, unit);
         });
     } else {
+        const double eps2 = p2p_eps2<double>(c), mu = c.mass;
         buffers(c.xs64, c.as64, c.p2p_part64, [&](const V4 *xs, V4 *acc, V4 *part) {
             (potential ? k_p2p_f64<true> : k_p2p_f64<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, xs, eps2, G, um,
                                                                                          mu, acc, part, pstride);

@@ -63,6 +63,21 @@ __global__ __launch_bounds__(256) void k_rk4_stage(int64_t n3, double cw, double
     aabb_block_store(lo, hi, bad, part + 7ll * blockIdx.x);
 }
 
+// The largest finite |m| of each block's share, in pinned host memory.
+__global__ __launch_bounds__(256) void k_largest_mass(int64_t n, const double *__restrict__ m, double *part) {
+    __shared__ double s[256];
+    double v = 0;
+    for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += gridDim.x * 256ll)
+        if (isfinite(m[i])) v = fmax(v, fabs(m[i]));
+    s[threadIdx.x] = v;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if (threadIdx.x < static_cast<unsigned>(w)) s[threadIdx.x] = fmax(s[threadIdx.x], s[threadIdx.x + w]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) part[blockIdx.x] = s[0];
+}
+
 // FP64 block sums of m |v|^2 (the first half of the grid) and m pot (the second) into
 // pinned host memory: one launch and one wait, where two of each, a copy and a device
 // allocation took 56 us of the 995 that the energies of 256k particles took.
@@ -136,6 +151,14 @@ void rk4_stage(Ctx &c, int stage, double dt) {
         k_rk4_stage<float><<<nb, 256, 0, c.stream>>>(n3, cw, h, first, last, c.acc32, c.x, c.v, c.x0, c.v0, c.xo, c.vo, c.aabb_part);
     VG_LAUNCH_CHECK();
     c.aabb_parts = nb;
+}
+
+double largest_mass(Ctx &c) {
+    double *part = reinterpret_cast<double *>(static_cast<char *>(c.pinned) + Ctx::PINNED_ENERGY);
+    k_largest_mass<<<EN_BLOCKS, 256, 0, c.stream>>>(c.n, c.m, part);
+    VG_LAUNCH_CHECK();
+    VG_HIP(hipStreamSynchronize(c.stream));
+    return *std::max_element(part, part + EN_BLOCKS);
 }
 
 void energies(Ctx &c, double &kinetic, double &potential) {
