@@ -129,3 +129,30 @@ def test_p2p_f32_softening_beyond_the_range(vg):
                 a, u[mode] = g.accelerations(), g.energy()[1]
                 assert np.isfinite(a).all() and (s < 1000 or (abs(a) < 1e-38).all())
         assert abs(u["f32"] - u["f64"]) <= 5e-6 * abs(u["f64"])
+
+
+@pytest.mark.parametrize("gap", [0.11, 0.13, 0.16, 0.25, 0.42, 0.45, 0.6])
+def test_p2p_f32_single_pairs_of_a_large_leaf(vg, gap):
+    """One heavy source near a leaf as large as an octant of the root (R = 0.85), all other
+    masses negligible, so that each target's force is one pair's, on positions that
+    FP32 holds exactly.  By differences a pair is within 16 roundings (r^2 3, the root's
+    estimate 2, 3 x 3.5 for its cube, products 2.5); by the expansion, beyond R / 2,
+    within 2 (3/2 R)^2 / (R / 2)^2 = 18 of r^2, 27 of the force, and 12 more: 40."""
+    worst = 0.0
+    for seed in range(25):
+        rng = np.random.default_rng(seed)
+        t = -1 + 0.98 * rng.random((96, 3))
+        t[0], t[1] = -1, -0.02  # the leaf's corners
+        c = np.array([gap - 0.015, *(-0.02 - 0.5 * rng.random(2))]) + 0.004 * (rng.random((32, 3)) - 0.5)
+        x = np.round(np.concatenate([t, c, [[1.0, 1.0, 1.0]]]) * 2 ** 20) / 2 ** 20
+        h = 96 + rng.integers(32)
+        m = np.full(len(x), 2.0 ** -60)
+        m[h] = 1
+        with vg.Gravity(len(x), 40, 3, "f32", eps=0.0) as g:
+            g.upload(x, None, m)
+            a = g.accelerations()[:96]
+            assert g.counts()["cells"] == 9
+        d = x[h] - x[:96]
+        ref = d / ((d * d).sum(1) ** 1.5)[:, None]
+        worst = max(worst, (np.linalg.norm(a - ref, axis=1) / np.linalg.norm(ref, axis=1)).max())
+    assert worst <= 40 * 2.0 ** -24

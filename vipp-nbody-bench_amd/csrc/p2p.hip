@@ -52,15 +52,23 @@ __host__ __device__ inline uint32_t chunk_len(uint32_t total, uint32_t nch) { re
 // cgs units) come in units of their own (length_shift, mass_shift).
 //
 // Error: positions are taken relative to the centre of the targets' box (radius
-// R), so at distance d from the box the expansion loses (R + d)^2 / d^2 in the
-// relative accuracy of r^2.  Tiles of 16 sources that come nearer than R / 8 are
-// left to a second pass by differences, which also has the pairs of a particle
-// with itself: 15 % of the tiles on the 4M Plummer input (R / 16: 7 %, 3 % less
-// time, but 1 % larger median errors).  Against the FP64 mode at order 12 (2^18
-// particles) RMS and median force errors are what differences alone gave:
-// 4.27e-5 and 3.9e-7 (uniform), 1.63e-6 and 3.3e-7 (Plummer), 4.98e-5 and 5.3e-7
-// (mixture), most of it the rounding of positions relative to the root centre.
-constexpr float MC_NEAR = 1.0f / 8;
+// R), so at distance d from the box the expansion takes up to 1.5 (R + d)^2 / d^2
+// roundings (2^-24) of a pair's force, where differences of positions stored up to D
+// from the root centre lose 4 D / d and more to the rounding of these.  Tiles of 16
+// sources that come nearer than where the first is the second, (R + d)^2 = 3 D d, within
+// R / 8 to R / 2, are left to a second pass by differences, which also has the pairs of a
+// particle with itself: R / 8 for leaves small beside D (15 % of the tiles on the 4M
+// Plummer input), more for the large ones of shallow trees and of the root's middle.  With
+// R / 8 there too a pair was off by up to 107 roundings on positions that FP32 holds
+// exactly, now by 13 (differences: 7).  RMS, median and 99.99th percentile of the relative
+// force error against the FP64 mode at order 12, differences alone -> R / 8 everywhere -> this:
+//   2000 uniform, s = 200      6.3e-7 2.0e-7 1.32e-5   6.1e-7 1.3e-7 1.48e-5   5.7e-7 1.2e-7 1.32e-5
+//   8000 Plummer, s = 200      1.41e-6 1.34e-7 4.2e-5  1.42e-6 1.59e-7 4.2e-5  1.40e-6 1.32e-7 4.2e-5
+//   2^18 Plummer, s = 64       2.4e-6 3.4e-7 3.7e-5    2.4e-6 2.4e-7 3.7e-5    2.4e-6 2.4e-7 3.7e-5
+//   2^18 mixture, s = 64       1.8e-6 4.7e-7 4.7e-5    1.8e-6 3.8e-7 4.7e-5    1.8e-6 3.8e-7 4.7e-5
+// (the last two: position rounding).  R / 4 and R / 2 everywhere cost 3 and 7 % of a 4M
+// Plummer step, this rule nothing there and 0.7 to 1.4 % of one of 64,000 particles, s = 128.
+constexpr float MC_NEAR = 1.0f / 8, MC_NEAR_LARGE = 1.0f / 2;
 // 16-target tiles of an item at most: 8 registers a tile and 4 more in flight;
 // the potential's mass products take the registers of one (6 there: 0.71
 // against 0.66 ms at 2^18 particles)
@@ -253,7 +261,10 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
         hx = 0.5f * (hi[0] - lo[0]), hy = 0.5f * (hi[1] - lo[1]), hz = 0.5f * (hi[2] - lo[2]);
         // sources up to near from the box are near; ns = 1 / (2 near), 0 where all are
         const float r = sqrtf(hx * hx + hy * hy + hz * hz);
-        const float nearest = fmaxf(fmaxf(r * MC_NEAR, I.cell * 0.0078125f), 0x1p-40f);  // r^-3 up to 2^120
+        // (r + d)^2 = 3 D d at d = e - sqrt(e^2 - r^2), e = 3/2 D - r: r / 2 at e = 5/4 r
+        const float e = 1.5f * fmaxf(fmaxf(fabsf(cx) + hx, fabsf(cy) + hy), fabsf(cz) + hz) - r;
+        const float even = e > 1.25f * r ? fmaxf(MC_NEAR * r, e - sqrtf(e * e - r * r)) : MC_NEAR_LARGE * r;
+        const float nearest = fmaxf(fmaxf(even, I.cell * 0.0078125f), 0x1p-40f);  // r^-3 up to 2^120
         ns = r < 1e18f ? 0.5f / nearest : 0.0f;
         hx = -ns * (hx + I.cell * 1e-5f), hy = -ns * (hy + I.cell * 1e-5f), hz = -ns * (hz + I.cell * 1e-5f);
     }
