@@ -9,6 +9,8 @@ radius R, where the squared distance loses at most 2 (9/8 R)^2 / (R / 8)^2 ~ 160
 roundings of 2^-24, 1e-5, and the pair force 1.5 times that; sums over pairs of
 both signs of error stay below the single worst pair, and the FP32 expansions
 add 1e-6: 5e-5 of the force in the 2-norm leaves a factor of 3."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -156,3 +158,50 @@ def test_p2p_f32_single_pairs_of_a_large_leaf(vg, gap):
         ref = d / ((d * d).sum(1) ** 1.5)[:, None]
         worst = max(worst, (np.linalg.norm(a - ref, axis=1) / np.linalg.norm(ref, axis=1)).max())
     assert worst <= 40 * 2.0 ** -24
+
+
+def test_p2p_memory_of_large_leaves(vg):
+    """64 leaves of about 4096 particles with up to 27 x 4096 sources each, in FP64: partial sums of
+    at most 12 rows of 2^18 entries (101 MB, 134 where buffers grow in powers of two) beside
+    330 B a particle (173 MB for the same reason), and as much again for all else: 614 MB."""
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        f, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(total)) == 0
+        return f.value
+
+    n = 1 << 18
+    x = np.random.default_rng(9).random((n, 3))
+    with vg.Gravity(2000, 100, 4, "f64", eps=1e-3) as g:  # what the first context of a process takes
+        g.upload(x[:2000])
+        g.accelerations()
+    before = free()
+    with vg.Gravity(n, 5000, 4, "f64", eps=1e-3) as g:
+        g.upload(x)
+        g.accelerations()
+        used = before - free()
+        assert g.counts()["leaves"] == 64
+    assert used <= 614e6
+
+
+def test_p2p_items_in_pieces(vg):
+    """64 leaves of about 8192 particles, whose 65,000 to 220,000 sources go to 12 items each, in
+    pieces of 4096: accelerations against the direct sum, the two modes' energies against
+    each other.  Level-2 cells that do not touch are far enough apart for p = 12 to truncate
+    at 1e-5 of a force in the 2-norm; a piece left out or taken twice is 2 % of a leaf's
+    sources or more."""
+    n = 1 << 19
+    rng = np.random.default_rng(10)
+    x = rng.random((n, 3))
+    m = rng.uniform(0.5, 1.5, n) / n
+    idx = rng.choice(n, 2000, replace=False)
+    u = {}
+    for mode in ("f64", "f32"):
+        with vg.Gravity(n, 5000, 12, mode, eps=1e-3) as g:
+            g.upload(x, None, m)
+            a, u[mode] = g.accelerations(), g.energy()[1]
+            assert g.counts()["leaves"] == 64 and np.array_equal(a, g.accelerations())
+            ref = g.direct(idx)
+        assert np.linalg.norm(a[idx] - ref) <= 1e-4 * np.linalg.norm(ref), mode
+    assert abs(u["f32"] - u["f64"]) <= 5e-6 * abs(u["f64"])

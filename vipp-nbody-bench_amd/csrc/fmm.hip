@@ -978,8 +978,7 @@ template <class R>
 struct Near {
     const Quad<R> *acc;                 // sums of the leaves with one work item, times G
     const Quad<R> *part;                // rows of partial sums of the others
-    const uint32_t *nchunk, *item_off;  // per leaf: rows (1: none), first row
-    uint32_t pstride;
+    const uint32_t *nchunk, *item_off;  // per leaf: rows (1: none) of whole 16-particle tiles, first tile
     R eps2, unit, G;                    // eps2 in squares of 1 / unit (FP32: p2p_eps2)
     const uint32_t *perm;  // caller's index of a sorted particle
     R *a;                  // accelerations in the caller's order
@@ -1007,7 +1006,8 @@ __global__ __launch_bounds__(64) void k_l2p(const int32_t *__restrict__ leaves, 
         for (int i = threadIdx.x; i < K; i += 64) sl[i] = Lx[static_cast<size_t>(c) * ldk + i];
     __syncthreads();
     const uint32_t s = start[c], cnt = count[c], nch = near.nchunk[blockIdx.x];
-    const Quad<R> *part = near.part + static_cast<size_t>(nch > 1 ? near.item_off[blockIdx.x] : 0) * near.pstride;
+    const Quad<R> *part = near.part + static_cast<size_t>(nch > 1 ? near.item_off[blockIdx.x] : 0) * 16;
+    const uint32_t pstride = (cnt + 15) / 16 * 16;
     const double w = ldexp(wx0, -level[c]);
     const double iw = 1.0 / w;
     const double cx = (bmin[3 * c] + bmax[3 * c]) / 2, cy = (bmin[3 * c + 1] + bmax[3 * c + 1]) / 2, cz = (bmin[3 * c + 2] + bmax[3 * c + 2]) / 2;
@@ -1022,7 +1022,7 @@ __global__ __launch_bounds__(64) void k_l2p(const int32_t *__restrict__ leaves, 
             v.x = v.y = v.z = v.w = 0;
 #pragma unroll 8
             for (uint32_t q = 0; q < nch; ++q) {
-                const Quad<R> u = part[static_cast<size_t>(q) * near.pstride + i];
+                const Quad<R> u = part[static_cast<size_t>(q) * pstride + i];
                 v.x += u.x;
                 v.y += u.y;
                 v.z += u.z;
@@ -1111,7 +1111,7 @@ Near<R> near_of(Ctx &c, const DevBuf<R> &acc, const DevBuf<R> &part, DevBuf<R> &
     const size_t n = static_cast<size_t>(std::max<int64_t>(1, c.n));
     a.ensure(3 * n);
     if (potential) c.pot64.ensure(n);
-    return {reinterpret_cast<const Quad<R> *>(acc.p), reinterpret_cast<const Quad<R> *>(part.p), c.p2p_nchunk, c.p2p_item_off, c.thr,
+    return {reinterpret_cast<const Quad<R> *>(acc.p), reinterpret_cast<const Quad<R> *>(part.p), c.p2p_nchunk, c.p2p_item_off,
             p2p_eps2<R>(c), static_cast<R>(sizeof(R) == 4 ? pow2(-length_shift(c.t.box, c.eps)) : 1.0), static_cast<R>(c.G), c.perm, a.p, potential ? c.pot64.p : nullptr};
 }
 

@@ -13,10 +13,10 @@
 // wavefronts; each (leaf, chunk) is one item, for one wavefront.
 //  * FP32 (k_p2p_mc): squared distances on the matrix cores.
 //  * FP64 (k_p2p_f64): pairs by differences.
-// A leaf with one chunk writes its result; split leaves write partial sums,
-// which L2P adds in chunk order (deterministic).  With a nonzero softening the
-// i == j term is exactly zero (dx = dy = dz = 0), so it needs no branch;
-// without softening a select removes it.
+// A leaf with one chunk writes its result; split leaves write partial sums, a row of
+// whole 16-target tiles for each chunk, which L2P adds in chunk order
+// (deterministic).  With a nonzero softening the i == j term is exactly zero (dx =
+// dy = dz = 0), so it needs no branch; without softening a select removes it.
 #include "gravity.hpp"
 
 namespace vg {
@@ -84,6 +84,15 @@ constexpr uint32_t MC_COST = 512, MC_MINCOST = 16;
 constexpr int F64_TILES = 4, F64_LEAVES = 64;
 constexpr uint32_t F64_MINCOST = 16;
 constexpr uint32_t MC_CHUNK = 64 * 64;
+// Rows of partial sums of a leaf at most: 12, or as many as keep all particles' rows
+// within 3 2^20 entries (48 MB, FP64 96), or one for 16 sources of each particle (leaves of
+// few particles with long lists; of up to 4096 particles).  Where an item then has more
+// than MC_CHUNK sources (leaves of thousands of particles), as many launches as that takes
+// add to its row.  A context's memory in GB with rows as long as the largest leaf for every
+// 512 to 4096 sources, and with these: FP64, 2^19 Plummer particles with s = 2000, 34.5 ->
+// 0.46; 2^20 uniform, s = 5000, 17.6 -> 0.92, FP32 4.6 -> 0.62; evaluations 59 -> 56, 28.2 -> 27.7
+// and 11.3 -> 11.6 ms (the last with the wider near pass above).
+constexpr uint32_t PART_ROWS = 12, PART_ENTRIES = 3u << 20, PART_MAXLEAF = 4096;
 // A leaf's targets go to items of at most mt tiles, evenly.
 __host__ __device__ inline uint32_t mc_batches(uint32_t nt, int mt) { return ((nt + 15) / 16 + mt - 1) / mt; }
 __host__ __device__ inline uint32_t mc_batch_tiles(uint32_t nt, int mt) { return ((nt + 15) / 16 + mc_batches(nt, mt) - 1) / mc_batches(nt, mt); }
@@ -118,9 +127,18 @@ struct alignas(32) McWork {
     int32_t cell, level;  // the leaf
     uint32_t pt0, nt;     // its targets: particles pt0 .. pt0 + nt - 1, of the leaf's from t0 on
     uint32_t src0, len;   // its share of the leaf's sources
-    uint32_t out;         // row of partial sums of this share, ~0: the only share
+    uint32_t out;         // first tile of this share's row of partial sums, ~0: the only share
     uint32_t t0;
 };
+
+// The piece of the item that a launch takes: MC_CHUNK of its sources; false if there is none.
+__device__ __forceinline__ bool take_piece(McWork &wk, uint32_t piece) {
+    const uint32_t at = piece * MC_CHUNK;
+    if (piece && at >= wk.len) return false;
+    wk.src0 += at;
+    wk.len = min(MC_CHUNK, wk.len - at);
+    return true;
+}
 
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
@@ -451,9 +469,10 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
                                                        const int32_t *__restrict__ ni, const int32_t *__restrict__ ni_cnt,
                                                        const double *__restrict__ bmin, const double *__restrict__ bmax, const float4 *__restrict__ xs,
                                                        float eps2, float G, bool um, bool big, float fscale, float pscale, float mlen,
-                                                       float4 *__restrict__ acc, float4 *__restrict__ partial, uint32_t pstride, float unit) {
+                                                       float4 *__restrict__ acc, float4 *__restrict__ partial, float unit, uint32_t piece) {
     __shared__ McLds S;
-    const McWork wk = items[blockIdx.x];
+    McWork wk = items[blockIdx.x];
+    if (!take_piece(wk, piece)) return;
     const int32_t c = wk.cell;
     const int lane = threadIdx.x;
     McItem I;
@@ -468,18 +487,23 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
     I.eps2 = eps2;
     I.um = um;
     I.big = big;
-    float4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * pstride : nullptr;
+    float4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * 16 : nullptr;
     auto emit = [&](int t, const f4 &v) {
         const float sx = v[0] * fscale, sy = v[1] * fscale, sz = v[2] * fscale;
         float sp = v[3] * pscale;
         if (out) {
-            out[wk.t0 + t] = float4{sx, sy, sz, sp};
+            float4 o = float4{sx, sy, sz, sp};
+            if (piece) {
+                const float4 u = out[wk.t0 + t];
+                o.x += u.x, o.y += u.y, o.z += u.z, o.w += u.w;
+            }
+            out[wk.t0 + t] = o;
         } else {
             if (POT && eps2 > 0.0f) sp -= xs[I.pt0 + t].w * rsq(eps2) * mlen;  // drop the m_i / eps self term
             acc[I.pt0 + t] = float4{G * sx, G * sy, G * sz, sp};
         }
     };
-    if (I.len == 0) {  // a last chunk that the even lengths left empty
+    if (wk.len == 0) {  // a last chunk that the even lengths left empty
         for (int t = lane; t < I.nt; t += 64) emit(t, f4{0, 0, 0, 0});
         return;
     }
@@ -580,19 +604,25 @@ template <bool POT>
 __global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ items, const uint32_t *__restrict__ start,
                                                    const uint32_t *__restrict__ count, const int32_t *__restrict__ anc, const int32_t *__restrict__ ni,
                                                    const int32_t *__restrict__ ni_cnt, const double4 *__restrict__ xs, double eps2, double G, bool um,
-                                                   double mu, double4 *__restrict__ acc, double4 *__restrict__ partial, uint32_t pstride) {
+                                                   double mu, double4 *__restrict__ acc, double4 *__restrict__ partial, uint32_t piece) {
     __shared__ double4 tile[64];
     __shared__ int32_t delta[MAXE];
-    const McWork wk = items[blockIdx.x];
+    McWork wk = items[blockIdx.x];
+    if (!take_piece(wk, piece)) return;
     const int lane = threadIdx.x, nt = static_cast<int>(wk.nt);
-    const Sources src = lay_out_entries(wk, delta, reinterpret_cast<uint64_t *>(tile), start, count, anc, ni, ni_cnt);
     const double sc = um ? mu : 1.0;
-    double4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * pstride : nullptr;
+    double4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * 16 : nullptr;
+    const Sources src = lay_out_entries(wk, delta, reinterpret_cast<uint64_t *>(tile), start, count, anc, ni, ni_cnt);
     auto emit = [&](int t, const double *v) {
         const double sx = v[0] * sc, sy = v[1] * sc, sz = v[2] * sc;
         double sp = v[3] * sc;
         if (out) {
-            out[wk.t0 + t] = double4{sx, sy, sz, sp};
+            double4 o = double4{sx, sy, sz, sp};
+            if (piece) {
+                const double4 u = out[wk.t0 + t];
+                o.x += u.x, o.y += u.y, o.z += u.z, o.w += u.w;
+            }
+            out[wk.t0 + t] = o;
         } else {
             if (POT && eps2 > 0.0) sp -= xs[wk.pt0 + t].w * rsq(eps2);  // drop the m_i / eps self term
             acc[wk.pt0 + t] = double4{G * sx, G * sy, G * sz, sp};
@@ -618,7 +648,8 @@ __global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ it
 // Leaf classes, by the cost of their items (16-target tiles times 64-source
 // groups): class j costs at least 2^(8 - j), so the largest start first.
 constexpr int NCLS = 7;
-constexpr int NSC = NCLS + 2;  // scanned per leaf: chunks, chunks of each class, split flag
+constexpr int NSC = NCLS + 2;  // scanned per leaf: tiles of partial sums, items of each class, split flag
+constexpr int NBT = NSC + 1;   // words of a plan block: their totals, and the most pieces of an item
 __device__ inline int leaf_class(uint32_t nt, uint32_t src, uint32_t nch, int mt) {
     const uint32_t cost = mc_batch_tiles(nt, mt) * (chunk_len(src, nch) / 64);
     return max(0, min(NCLS - 1, 8 - (31 - __builtin_clz(max(cost, 1u)))));
@@ -630,9 +661,12 @@ __device__ inline int leaf_class(uint32_t nt, uint32_t src, uint32_t nch, int mt
 __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ leaves, int nleaves, const int8_t *__restrict__ level,
                                                   const uint32_t *__restrict__ count, const int32_t *__restrict__ anc, const uint32_t *__restrict__ local,
                                                   uint32_t *__restrict__ nchunk, uint32_t *__restrict__ cls, uint32_t *__restrict__ nsrc, uint32_t *__restrict__ pre,
-                                                  uint32_t *__restrict__ btot, uint32_t chunk, int mt, uint32_t minrow) {
-    __shared__ uint32_t wtot[4][NSC];
+                                                  uint32_t *__restrict__ btot, uint32_t chunk, int mt, uint32_t minrow,
+                                                  uint32_t maxrows) {
+    __shared__ uint32_t wtot[4][NSC], s_pieces;
     const int k = blockIdx.x * 256 + threadIdx.x;
+    if (threadIdx.x == 0) s_pieces = 1;
+    __syncthreads();
     const unsigned lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     uint32_t v[NSC] = {};
     if (k < nleaves) {
@@ -642,16 +676,17 @@ __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ le
         const uint32_t nt = count[c];
         // as many groups as the cost allows, but no fewer than minrow eighths of the tiles (the rows of partial sums of a large leaf stay few)
         const uint32_t lim = 64 * min(MC_CHUNK / 64, max(1 + (nt + 15) / 16 * minrow / 8, chunk / mc_batch_tiles(nt, mt)));
-        const uint32_t nch = max(1u, (src + lim - 1) / lim);
+        const uint32_t nch = min(max(maxrows, src / (16 * min(nt, PART_MAXLEAF)) + 1), max(1u, (src + lim - 1) / lim));
         nchunk[k] = nch;
         nsrc[k] = src;
         const uint32_t nit = nch * mc_batches(nt, mt);
-        v[0] = nch > 1 ? nch : 0u;
+        v[0] = nch > 1 ? nch * ((nt + 15) / 16) : 0u;
         const int cl = leaf_class(nt, src, nch, mt);
         cls[k] = cl;
 #pragma unroll
         for (int q = 0; q < NCLS; ++q) v[1 + q] = q == cl ? nit : 0u;
         v[NSC - 1] = nch > 1 ? 1u : 0u;
+        if (chunk_len(src, nch) > MC_CHUNK) atomicMax(&s_pieces, (chunk_len(src, nch) + MC_CHUNK - 1) / MC_CHUNK);
     }
     uint32_t inc[NSC];
 #pragma unroll
@@ -670,37 +705,43 @@ __global__ __launch_bounds__(256) void k_p2p_plan(const int32_t *__restrict__ le
         uint32_t base = 0;
         for (unsigned u = 0; u < w; ++u) base += wtot[u][q];
         if (k < nleaves) pre[static_cast<int64_t>(k) * NSC + q] = base + inc[q] - v[q];
-        if (threadIdx.x == 255) btot[blockIdx.x * NSC + q] = base + inc[q];
+        if (threadIdx.x == 255) btot[blockIdx.x * NBT + q] = base + inc[q];
     }
+    if (threadIdx.x == 255) btot[blockIdx.x * NBT + NSC] = s_pieces;
 }
 
 // One block: exclusive scan of the block totals; writes the class counts and
 // bases, the item total and the split-leaf total into scal:
 //   scal[0..NCLS) items per class, scal[NCLS..2 NCLS) class bases,
-//   scal[2 NCLS] rows of partial sums, scal[2 NCLS + 1] split leaves.
+//   scal[2 NCLS] tiles of partial sums, scal[2 NCLS + 1] split leaves, scal[2 NCLS + 2] the
+//   most pieces of an item.
 // host: the same in pinned host memory, then seq in its last word.
 __global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ btot, int nblocks, uint32_t *__restrict__ scal, uint32_t *host, uint32_t seq) {
     // exclusive scan of each component over the plan blocks, one wavefront per
     // component (wavefront-wide inclusive scans, carried across runs of 64)
-    __shared__ uint32_t tot[NSC];
+    __shared__ uint32_t tot[NSC], s_pieces;
     const unsigned lane = threadIdx.x & 63;
     for (int q = threadIdx.x >> 6; q < NSC; q += 4) {
         uint32_t carry = 0;
         for (int b0 = 0; b0 < nblocks; b0 += 64) {
             const int b = b0 + static_cast<int>(lane);
-            const uint32_t v = b < nblocks ? btot[b * NSC + q] : 0u;
+            const uint32_t v = b < nblocks ? btot[b * NBT + q] : 0u;
             uint32_t x = v;
             for (int d = 1; d < 64; d <<= 1) {
                 const uint32_t o = __shfl_up(x, d, 64);
                 if (lane >= static_cast<unsigned>(d)) x += o;
             }
-            if (b < nblocks) btot[b * NSC + q] = carry + x - v;
+            if (b < nblocks) btot[b * NBT + q] = carry + x - v;
             carry += __shfl(x, 63, 64);
         }
         if (lane == 0) tot[q] = carry;
     }
+    if (threadIdx.x == 0) s_pieces = 1;
     __syncthreads();
-    if (threadIdx.x < 2 * NCLS + 2) {  // scal: [class items] [class bases] rows, split leaves
+    for (int b = threadIdx.x; b < nblocks; b += 256)
+        if (btot[b * NBT + NSC] > 1) atomicMax(&s_pieces, btot[b * NBT + NSC]);
+    __syncthreads();
+    if (threadIdx.x < 2 * NCLS + 3) {  // scal: [class items] [class bases] tiles, split leaves, pieces
         const int j = threadIdx.x;
         uint32_t v = 0;
         if (j < NCLS)
@@ -708,16 +749,16 @@ __global__ __launch_bounds__(256) void k_p2p_plan_blocks(uint32_t *__restrict__ 
         else if (j < 2 * NCLS)
             for (int k = 0; k < j - NCLS; ++k) v += tot[1 + k];
         else
-            v = tot[j == 2 * NCLS ? 0 : NSC - 1];
+            v = j == 2 * NCLS ? tot[0] : j == 2 * NCLS + 1 ? tot[NSC - 1] : s_pieces;
         scal[j] = v;
         host[j] = v;
         __threadfence_system();
-        if (j == 0) __hip_atomic_store(host + 2 * NCLS + 2, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);  // behind this wavefront's stores
+        if (j == 0) __hip_atomic_store(host + 2 * NCLS + 3, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);  // behind this wavefront's stores
     }
 }
 
 // The work items, bucketed by class in leaf order, each with what its wavefront needs
-// to start, and the leaves' rows of partial sums.
+// to start, and where the leaves' partial sums begin.
 __global__ __launch_bounds__(256) void k_p2p_items(const int32_t *__restrict__ leaves, int nleaves, const int8_t *__restrict__ level,
                                                       const uint32_t *__restrict__ start, const uint32_t *__restrict__ count,
                                                       const uint32_t *__restrict__ lcls, const uint32_t *__restrict__ nchunk,
@@ -727,7 +768,7 @@ __global__ __launch_bounds__(256) void k_p2p_items(const int32_t *__restrict__ l
     const int k = blockIdx.x * 256 + threadIdx.x;
     if (k >= nleaves) return;
     const uint32_t *pk = pre + static_cast<int64_t>(k) * NSC;
-    const uint32_t *bk = boff + blockIdx.x * NSC;
+    const uint32_t *bk = boff + blockIdx.x * NBT;
     const uint32_t nch = nchunk[k], off = bk[0] + pk[0], src = nsrc[k], per = chunk_len(src, nch);
     item_off[k] = off;
     const int cls = lcls[k];
@@ -737,7 +778,7 @@ __global__ __launch_bounds__(256) void k_p2p_items(const int32_t *__restrict__ l
     for (uint32_t t0 = 0; t0 < nt; t0 += bt)
         for (uint32_t q = 0; q < nch; ++q) {
             const uint32_t s0 = min(src, q * per);
-            *it++ = McWork{c, level[c], pt0 + t0, min(bt, nt - t0), s0, min(src, s0 + per) - s0, nch > 1 ? off + q : ~0u, t0};
+            *it++ = McWork{c, level[c], pt0 + t0, min(bt, nt - t0), s0, min(src, s0 + per) - s0, nch > 1 ? off + q * ((nt + 15) / 16) : ~0u, t0};
         }
 }
 
@@ -749,13 +790,13 @@ void p2p_plan(Ctx &c, bool potential) {
     if (!t.nleaves) return;
     const int nl = static_cast<int>(t.nleaves);
     const int nb = static_cast<int>(ceil_div(nl, 256));
-    c.p2p_scal.ensure(2 * NCLS + 2);
+    c.p2p_scal.ensure(2 * NCLS + 3);
     c.p2p_nchunk.ensure(nl);
     c.p2p_cls.ensure(nl);
     c.p2p_src.ensure(nl);
     c.p2p_item_off.ensure(nl);
     c.p2p_pre.ensure(static_cast<size_t>(nl) * NSC);
-    c.p2p_btot.ensure(static_cast<size_t>(nb) * NSC);
+    c.p2p_btot.ensure(static_cast<size_t>(nb) * NBT);
     // under 8 leaves per CU (the 16k Plummer sphere has 430): FP32 items of MC_COST,
     // scaled down by the leaf shortfall, so that there are still several per SIMD;
     // FP64 items take some five times as long, so they shrink from more leaves on
@@ -763,29 +804,30 @@ void p2p_plan(Ctx &c, bool potential) {
     uint32_t chunk = MC_COST;
     if (nl < few) chunk = std::max<uint32_t>(c.prec == 0 ? F64_MINCOST : MC_MINCOST, static_cast<uint32_t>(1ull * MC_COST * nl / few));
     k_p2p_plan<<<nb, 256, 0, c.stream>>>(t.leaf_ids, nl, t.level, t.count, t.anc, c.p2p_local, c.p2p_nchunk, c.p2p_cls, c.p2p_src, c.p2p_pre, c.p2p_btot, chunk,
-                                        c.prec == 0 ? F64_TILES : mc_tiles(potential), nl < 8 * c.ncu ? 1 : 8);
-    static_assert(2 * NCLS + 2 < 32, "plan scalars");
+                                        c.prec == 0 ? F64_TILES : mc_tiles(potential), nl < 8 * c.ncu ? 1 : 8,
+                                        std::max<uint32_t>(PART_ROWS, static_cast<uint32_t>(PART_ENTRIES / c.n)));
+    static_assert(2 * NCLS + 3 < 32, "plan scalars");
     k_p2p_plan_blocks<<<1, 256, 0, c.stream>>>(c.p2p_btot, nb, c.p2p_scal, reinterpret_cast<uint32_t *>(static_cast<char *>(c.pinned) + 128), ++c.plan_seq);
     VG_LAUNCH_CHECK();
 }
 
 // The plan's scalars, waited for on the host: items per class, class bases,
-// rows of partial sums, split leaves.
+// tiles of partial sums, split leaves, pieces.
 static const uint32_t *p2p_scalars(Ctx &c) {
     const uint32_t *hs = reinterpret_cast<const uint32_t *>(static_cast<const char *>(c.pinned) + 128);
-    wait_host_word(hs + 2 * NCLS + 2, c.plan_seq, c.stream);
+    wait_host_word(hs + 2 * NCLS + 3, c.plan_seq, c.stream);
     return hs;
 }
 
-// One launch over all items, on the stream p2p_plan used; L2P adds the partial sums
-// of the leaves split over several.
+// One launch over all items (one for each piece of the longest), on the stream
+// p2p_plan used; L2P adds the partial sums of the leaves split over several.
 template <class R>
 void p2p_run(Ctx &c, bool potential) {
     using V4 = Quad<R>;
     TreeDev &t = c.t;
     if (!t.nleaves) return;
     const uint32_t *hs = p2p_scalars(c);
-    const uint32_t nitems = hs[2 * NCLS - 1] + hs[NCLS - 1], nrows = hs[2 * NCLS], pstride = c.thr;
+    const uint32_t nitems = hs[2 * NCLS - 1] + hs[NCLS - 1], ntiles = hs[2 * NCLS], pieces = hs[2 * NCLS + 2];
     const bool split = hs[2 * NCLS + 1] > 0;
     const int nl = static_cast<int>(t.nleaves);
     c.p2p_items.ensure(sizeof(McWork) * static_cast<size_t>(std::max<uint32_t>(1, nitems)));
@@ -795,7 +837,7 @@ void p2p_run(Ctx &c, bool potential) {
     VG_LAUNCH_CHECK();
     auto buffers = [&](auto &sorted, auto &sums, auto &parts, auto run) {
         sums.ensure(4 * std::max<int64_t>(1, c.n));
-        if (split) parts.ensure(4 * static_cast<size_t>(nrows) * pstride);
+        if (split) parts.ensure(4 * 16 * static_cast<size_t>(ntiles));
         run(reinterpret_cast<const V4 *>(sorted.p), reinterpret_cast<V4 *>(sums.p), reinterpret_cast<V4 *>(parts.p));
     };
     const R G = static_cast<R>(c.G);
@@ -809,14 +851,16 @@ void p2p_run(Ctx &c, bool potential) {
         bool big = false;  // a root box so wide that squared distances may leave the FP32 range all the same
         for (int a = 0; a < 3; ++a) big |= !((t.box[3 + a] - t.box[a]) * pow2(-ls) < 1e18);
         buffers(c.xs32, c.as32, c.p2p_part32, [&](const V4 *xs, V4 *acc, V4 *part) {
-            (potential ? k_p2p_mc<true> : k_p2p_mc<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs,
-                                                                                       eps2, G, um, big, fscale, pscale, mlen, acc, part, pstride, unit);
+            for (uint32_t p = 0; p < pieces; ++p)
+                (potential ? k_p2p_mc<true> : k_p2p_mc<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs,
+                                                                                       eps2, G, um, big, fscale, pscale, mlen, acc, part, unit, p);
         });
     } else {
         const double eps2 = p2p_eps2<double>(c), mu = c.mass;
         buffers(c.xs64, c.as64, c.p2p_part64, [&](const V4 *xs, V4 *acc, V4 *part) {
-            (potential ? k_p2p_f64<true> : k_p2p_f64<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, xs, eps2, G, um,
-                                                                                         mu, acc, part, pstride);
+            for (uint32_t p = 0; p < pieces; ++p)
+                (potential ? k_p2p_f64<true> : k_p2p_f64<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, xs, eps2, G, um,
+                                                                                         mu, acc, part, p);
         });
     }
     VG_LAUNCH_CHECK();
