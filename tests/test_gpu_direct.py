@@ -5,6 +5,8 @@ in extended precision.
 
 Bound: a sum of n terms in FP64, each within 8 roundings of its exact value: n + 8
 roundings of 2^-53 of the sum of the terms' magnitudes."""
+import time
+
 import numpy as np
 import pytest
 
@@ -97,3 +99,29 @@ def test_accelerations_through_the_staging_buffers(n):
             a[mode] = g.accelerations()
             assert np.array_equal(a[mode], g.accelerations())
     assert np.abs(a["f32"] - a["f64"]).max() <= 1e-3 * np.abs(a["f64"]).max()
+
+
+@pytest.mark.parametrize("potential", [False, True])
+def test_coincident_pair_costs_its_tile_only(vg, potential):
+    """256 targets, 2^18 sources in slices of 4096 (16 tiles): a sum that is not finite is formed again over
+    its tile, at three times the cost of the fast form, one tile in 16 a slice.  Half the call again
+    is room for the clock; a slice walked by one thread took three times the call."""
+    n = 1 << 18
+    x = np.random.default_rng(5).random((n, 3))
+    idx = np.arange(256)
+    best = []
+    for pair in (False, True):
+        if pair:
+            x[n - 100] = x[7]
+        with vg.Gravity(n, 64, 4, "f64", eps=0.0) as g:
+            g.upload(x)
+            g.direct(idx, potential=potential)
+            t = []
+            for _ in range(30):
+                t0 = time.perf_counter()
+                a = g.direct(idx, potential=potential)
+                t.append(time.perf_counter() - t0)
+            best.append(min(t))
+            a = a[0] if potential else a
+            assert np.isnan(a[7]).all() == pair and np.isfinite(np.delete(a, 7, 0)).all()
+    assert best[1] <= 1.5 * best[0]

@@ -53,11 +53,14 @@ __device__ inline void add_fast(double dx, double dy, double dz, double r2, doub
 // 64 pairs.  4096 targets of 1M sources: 6.2 -> 2.9 ms, 65,536 of 100,000: 9.7 ->
 // 4.5 ms (sources through scalar loads instead of LDS: 0.3 ms more).  A target of
 // its own (solver_ref_naive.hpp:111-113) costs something only in the tiles that
-// hold one of the wavefront's targets.  By the reference's operations are formed
-// a sum that is not finite (a source at the target's place without softening,
-// distances whose square overflows) and, so that a caller may compare with the
-// formula to the last bit, the sums over up to EXACT_N sources, where a call is its
-// launches and copies (128 of 128: 56 us, against 45; 256 of 256: 78 against 58).
+// hold one of the wavefront's targets.  By the reference's operations are formed a
+// tile's sum that is not finite (a source at the target's place without softening,
+// distances whose square overflows; one such pair, 256 targets of 2^18 sources: 0.37 ->
+// 0.39 ms, 1.17 with its thread walking the slice again) and the sums over up to
+// EXACT_N sources: callers, the tests among them, compare the forces of tiny systems with
+// the formula component by component at 1e-13, and where terms cancel any other
+// rounding shows (4.7e-13 at 64 sources).  A call is its launches and copies there (128 of
+// 128: 50 us, against 42; 256 of 256: 78 against 51).
 constexpr int64_t EXACT_N = 128;
 template <bool POT>
 __global__ __launch_bounds__(DT) void k_direct(const double *__restrict__ x, const double *__restrict__ masses, double mass, int64_t n,
@@ -86,31 +89,32 @@ __global__ __launch_bounds__(DT) void k_direct(const double *__restrict__ x, con
         __syncthreads();
         const int nt = j1 - b < DT ? static_cast<int>(j1 - b) : DT;
         const int self = i >= b && i < b + nt ? static_cast<int>(i - b) : -1;
-        if (n <= EXACT_N) {
-            for (int u = 0; u < nt; ++u)
-                if (u != self) add_exact<POT>(sxy[u].x - xi, sxy[u].y - yi, szg[u].x - zi, szg[u].y, POT ? sm[u] : 0.0, eps2, s);
-        } else if (__ballot(self >= 0) == 0) {
+        double t[4] = {0, 0, 0, 0};  // the tile's sums
+        bool exact = n <= EXACT_N;
+        if (!exact) {
+            if (__ballot(self >= 0) == 0) {
 #pragma unroll 4
-            for (int u = 0; u < nt; ++u) {
-                const double dx = sxy[u].x - xi, dy = sxy[u].y - yi, dz = szg[u].x - zi;
-                add_fast<POT>(dx, dy, dz, fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2))), szg[u].y, POT ? sm[u] : 0.0, s);
+                for (int u = 0; u < nt; ++u) {
+                    const double dx = sxy[u].x - xi, dy = sxy[u].y - yi, dz = szg[u].x - zi;
+                    add_fast<POT>(dx, dy, dz, fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2))), szg[u].y, POT ? sm[u] : 0.0, t);
+                }
+            } else {
+                for (int u = 0; u < nt; ++u) {
+                    const double dx = sxy[u].x - xi, dy = sxy[u].y - yi, dz = szg[u].x - zi;
+                    const double r2 = u == self ? 1.0 : fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));  // adds 0 dx = 0
+                    add_fast<POT>(dx, dy, dz, r2, szg[u].y, POT && u != self ? sm[u] : 0.0, t);
+                }
             }
-        } else {
-            for (int u = 0; u < nt; ++u) {
-                const double dx = sxy[u].x - xi, dy = sxy[u].y - yi, dz = szg[u].x - zi;
-                const double r2 = u == self ? 1.0 : fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));  // adds 0 dx = 0
-                add_fast<POT>(dx, dy, dz, r2, szg[u].y, POT && u != self ? sm[u] : 0.0, s);
-            }
+            exact = live && !(isfinite(t[0]) && isfinite(t[1]) && isfinite(t[2]) && isfinite(t[3]));
         }
+        if (exact) {
+            t[0] = t[1] = t[2] = t[3] = 0;
+            for (int u = 0; u < nt; ++u)
+                if (u != self) add_exact<POT>(sxy[u].x - xi, sxy[u].y - yi, szg[u].x - zi, szg[u].y, POT ? sm[u] : 0.0, eps2, t);
+        }
+        for (int c = 0; c < 4; ++c) s[c] += t[c];
     }
     if (k >= nidx) return;
-    if (live && !(isfinite(s[0]) && isfinite(s[1]) && isfinite(s[2]) && isfinite(s[3]))) {
-        s[0] = s[1] = s[2] = s[3] = 0;
-        for (int64_t j = j0; j < j1; ++j) {
-            const double m = masses ? masses[j] : mass;
-            if (j != i) add_exact<POT>(x[3 * j] - xi, x[3 * j + 1] - yi, x[3 * j + 2] - zi, G * m, m, eps2, s);
-        }
-    }
     double *o = part + (static_cast<int64_t>(blockIdx.y) * nidx + k) * 4;
     for (int c = 0; c < 4; ++c) o[c] = live ? s[c] : 0.0;
 }
