@@ -32,10 +32,8 @@ namespace {
 constexpr int AL = 2 * MAXP;        // A_n^m needed up to n = 2p
 constexpr int AW = 2 * AL + 1;
 __constant__ double cA[(AL + 1) * AW];
-// R recurrences: diag[m], sub[m], r1[n][m], r2[n][m]
-__constant__ double cDiag[MAXP + 1], cSub[MAXP + 1], cR1[(MAXP + 1) * (MAXP + 1)], cR2[(MAXP + 1) * (MAXP + 1)];
-// ladder coefficients of the gradient: dz[n][m] = sqrt((n+m)(n-m)), am[n][m] = sqrt((n+m)(n+m-1)), bm[n][m] = sqrt((n-m)(n-m-1))
-__constant__ double cLz[(MAXP + 2) * (MAXP + 2)], cLa[(MAXP + 2) * (MAXP + 2)], cLb[(MAXP + 2) * (MAXP + 2)];
+// R recurrences of P2M: diag[m], r1[n][m], r2[n][m]
+__constant__ double cDiag[MAXP + 1], cR1[(MAXP + 1) * (MAXP + 1)], cR2[(MAXP + 1) * (MAXP + 1)];
 
 struct dc {
     double re, im;
@@ -964,8 +962,9 @@ __global__ __launch_bounds__(256) void k_m2l_sum(const int32_t *__restrict__ par
 // potential, d/dz and (d/dx - i d/dy) directly, so no table is stored.
 // ---------------------------------------------------------------------------
 // Recurrence and ladder coefficients as functions of (n, m): with p a template
-// parameter and the loops unrolled they fold to immediates (the same values
-// as the __constant__ tables, which serve the kernels with a runtime order).
+// parameter and the loops unrolled they fold to immediates (P2M, whose lanes have
+// different orders m, reads the first three from the __constant__ tables).  The last
+// three are the gradient's ladder.
 __device__ __forceinline__ double k_diag(int m) { return -sqrt((2.0 * m - 1) / (2.0 * m)); }
 __device__ __forceinline__ double k_r1(int n, int m) { return (2.0 * n - 1) / sqrt(static_cast<double>(n - m) * (n + m)); }
 __device__ __forceinline__ double k_r2(int n, int m) { return sqrt(static_cast<double>(n + m - 1) * (n - m - 1) / (static_cast<double>(n - m) * (n + m))); }
@@ -1443,7 +1442,7 @@ void downward_t(Ctx &c, bool potential) {
 
 }  // namespace
 
-void m2l_split_operators(Ctx &c, int nvec);
+void m2l_split_operators(Ctx &c);
 
 // The tables live in each device's constant memory: upload them once per
 // device (the caller has made the context's device current).
@@ -1464,30 +1463,17 @@ void fmm_constants_init() {
             for (int i = 1; i <= n - am; ++i) d *= i;
             A[n * AW + AL + m] = (n % 2 == 0 ? 1.0 : -1.0) / d;  // fmm.hpp:201-221
         }
-    std::vector<double> diag(MAXP + 1, 0), sub(MAXP + 1, 0), r1((MAXP + 1) * (MAXP + 1), 0), r2((MAXP + 1) * (MAXP + 1), 0);
+    std::vector<double> diag(MAXP + 1, 0), r1((MAXP + 1) * (MAXP + 1), 0), r2((MAXP + 1) * (MAXP + 1), 0);
     for (int m = 1; m <= MAXP; ++m) diag[m] = -std::sqrt((2.0 * m - 1) / (2.0 * m));
-    for (int m = 0; m <= MAXP; ++m) sub[m] = std::sqrt(2.0 * m + 1);
     for (int n = 1; n <= MAXP; ++n)
         for (int m = 0; m < n; ++m) {
             r1[n * (MAXP + 1) + m] = (2.0 * n - 1) / std::sqrt(static_cast<double>(n - m) * (n + m));
             r2[n * (MAXP + 1) + m] = std::sqrt(static_cast<double>(n + m - 1) * (n - m - 1) / (static_cast<double>(n - m) * (n + m)));
         }
-    const int LW = MAXP + 2;
-    std::vector<double> lz(LW * LW, 0), la(LW * LW, 0), lb(LW * LW, 0);
-    for (int l = 0; l < LW; ++l)
-        for (int m = 0; m < LW; ++m) {
-            lz[l * LW + m] = (m <= l) ? std::sqrt(static_cast<double>(l + m) * (l - m)) : 0.0;
-            la[l * LW + m] = (m <= l) ? std::sqrt(static_cast<double>(l + m) * (l + m - 1)) : 0.0;
-            lb[l * LW + m] = (m + 1 <= l) ? std::sqrt(static_cast<double>(l - m) * (l - m - 1)) : 0.0;
-        }
     VG_HIP(hipMemcpyToSymbol(HIP_SYMBOL(cA), A.data(), A.size() * sizeof(double)));
     VG_HIP(hipMemcpyToSymbol(HIP_SYMBOL(cDiag), diag.data(), diag.size() * sizeof(double)));
-    VG_HIP(hipMemcpyToSymbol(HIP_SYMBOL(cSub), sub.data(), sub.size() * sizeof(double)));
     VG_HIP(hipMemcpyToSymbol(HIP_SYMBOL(cR1), r1.data(), r1.size() * sizeof(double)));
     VG_HIP(hipMemcpyToSymbol(HIP_SYMBOL(cR2), r2.data(), r2.size() * sizeof(double)));
-    VG_HIP(hipMemcpyToSymbol(HIP_SYMBOL(cLz), lz.data(), lz.size() * sizeof(double)));
-    VG_HIP(hipMemcpyToSymbol(HIP_SYMBOL(cLa), la.data(), la.size() * sizeof(double)));
-    VG_HIP(hipMemcpyToSymbol(HIP_SYMBOL(cLb), lb.data(), lb.size() * sizeof(double)));
     if (done.size() <= static_cast<size_t>(dev)) done.resize(static_cast<size_t>(dev) + 1, false);
     done[static_cast<size_t>(dev)] = true;
 }
@@ -1523,7 +1509,7 @@ void operators_build(Ctx &c) {
     } else if (c.prec == 2) {
         c.op64.ensure(static_cast<size_t>(nvec) * c.K * c.K);
         k_ops<double><<<grid, 128 * OPS_ROWS, 0, c.stream>>>(c.ops_sel, c.harm, c.p, c.K, c.op64, nullptr);
-        m2l_split_operators(c, nvec);
+        m2l_split_operators(c);
     } else {
         if (c.frag_K != c.K) {  // the padding, once for each order (the closure's fallback order may change)
             const size_t words = 343 * OpFrag(c.K).size(), words_ml = 16 * MlFrag(c.K).size();

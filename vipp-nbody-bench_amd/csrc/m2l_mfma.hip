@@ -443,12 +443,11 @@ void launch_split(Ctx &c, const int32_t *parents, int np) {
 
 }  // namespace
 
-void m2l_split_operators(Ctx &c, int nvec) {
+void m2l_split_operators(Ctx &c) {
     const int MT = mt_of(c.K), NKS = ks_of(c.K), NT = ks_of(c.K), KS = mt_of(c.K);  // (16-row tiles, 32-column steps)
     const int64_t per = static_cast<int64_t>(MT) * NKS * 64;
     c.opsplit.ensure(static_cast<size_t>(343) * NT * KS * 128 * 8);
     // split mode runs M2M, M2L and L2L from the fragments: no FP32 copies
-    (void)nvec;
     k_split_ops<<<189 * NT, 256, 16 * (32 * KS + 1) * sizeof(double), c.stream>>>(c.ops_sel, c.op64, c.K, reinterpret_cast<__bf16 *>(c.opsplit.p), NT, KS);
     c.opsplit_ml.ensure(static_cast<size_t>(16 * 3 * per * 8));
     k_split_ops_ml<<<ceil_div(16 * per, 256), 256, 0, c.stream>>>(c.op64, c.K, reinterpret_cast<__bf16 *>(c.opsplit_ml.p), MT, NKS);
