@@ -195,8 +195,8 @@ def main():
         "ms_per_step": ms_per_step, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
         "dtype": {"split": "bf16-split+f32+f64", "f32": "f32+f64", "f64": "f64"}[mode], "data": "synthetic",
         "config": {"workload": args.workload, "n": n, "s": w["s"], "p": p, "eps": w["eps"], "dt": w["dt"],
-                   "m2l": {"f32": "fp32 VALU", "split": "bf16 hi/lo split on MFMA (3 products), fp32 accumulate", "f64": "fp64"}[mode],
-                   "m2m_l2l": {"f32": "fp32 VALU", "split": "bf16 three-way split on MFMA (6 products), fp32 accumulate", "f64": "fp64"}[mode],
+                   "m2l": {"f32": "fp32 on MFMA", "split": "bf16 hi/lo split on MFMA (3 products), fp32 accumulate", "f64": "fp64"}[mode],
+                   "m2m_l2l": {"f32": "fp32 on MFMA", "split": "bf16 three-way split on MFMA (6 products), fp32 accumulate", "f64": "fp64"}[mode],
                    "p2p": "fp64" if mode == "f64" else "fp32", "p2m_l2p": "fp64" if mode == "f64" else "fp32",
                    "state": "fp64", "parallelism": "1 GPU"},
         "roofline": roofline,
@@ -344,7 +344,7 @@ def config_line(vgm, workloads, name):
 
 
 def plain_reference(vgm, x, v, masses, w, n, steps, value, err_ref=None):
-    """The plain GPU FMM (FP32 P2P, FP32 M2L on the vector units, same p) on the
+    """The plain GPU FMM (FP32 P2P, FP32 M2L on the FP32 matrix cores, same p) on the
     same input and step count: the comparison the headline metric asks for."""
     idx, d = err_ref if err_ref is not None else (None, None)
     out, _ = timed_run(vgm, x, v, masses, w, "f32", w["p"], steps, err_idx=idx, d=d)

@@ -40,7 +40,7 @@ struct Vector;
 
 enum class GpuPrecision : uint32_t {
     f64 = VIPP_GRAV_F64,          // FP64 everywhere
-    f32 = VIPP_GRAV_F32,          // FP32 P2P and M2L on the vector units, FP64 state
+    f32 = VIPP_GRAV_F32,          // FP32 P2P and expansions, FP64 state
     split = VIPP_GRAV_F32_SPLIT,  // FP32 P2P, BF16 hi/lo M2L on MFMA, FP64 state
 };
 

@@ -189,7 +189,7 @@ void lists_build(Ctx &c);                // NB / NI / AP lists and the 27-neighb
 void ref_numbering(Ctx &c);              // reference cell ids (for export only)
 void operators_build(Ctx &c);            // M2M / L2L / M2L operators for the current root box
 void fmm_upward(Ctx &c);                 // P2M + M2M
-void fmm_m2l(Ctx &c);                    // M2L (plain VALU or split MFMA by mode)
+void fmm_m2l(Ctx &c);                    // M2L (FP64 on VALU, FP32 and split on the matrix cores)
 void fmm_p2p(Ctx &c, bool potential);    // near field into the sorted accelerations (plan, then run)
 void fmm_p2p_plan(Ctx &c, bool potential);  // P2P work items; the item counts are read back without waiting
 void fmm_p2p_run(Ctx &c, bool potential);  // waits for the item counts, then the P2P kernels
