@@ -118,6 +118,22 @@ def test_p2p_f32_units(vg, l, k, eps, masses):
         assert abs(r[mode][1] - r["f64"][1]) <= 5e-6 * abs(r["f64"][1]), mode
 
 
+@pytest.mark.parametrize("k,eps,masses", [(88, 1e-3, True), (0, 1e-7, False)])
+def test_p2p_f32_small_softening_in_a_wide_box(vg, k, eps, masses):
+    """The pair of a particle with itself forms m / eps^3, which FP32 holds in the caller's
+    units (2^106 and 2^70) and has to in those of a box 2^63 wide too."""
+    n, s, l = 4100, 12, 60
+    x = _points(n, "core", n) * 2.0 ** l
+    m = np.random.default_rng(1).uniform(0.5, 1.5, n) / n * 2.0 ** k if masses else None
+    a = {}
+    for mode in ("f64", "f32", "split"):
+        with vg.Gravity(n, s, 8, mode, eps=eps, G=1.3 * 2.0 ** (2 * l - k), mass=2.0 ** k / n) as g:
+            g.upload(x, None, m)
+            a[mode] = g.accelerations()
+    for mode in ("f32", "split"):
+        assert np.linalg.norm(a[mode] - a["f64"]) <= BOUND * np.linalg.norm(a["f64"]), mode  # false for NaN
+
+
 def test_p2p_f32_softening_beyond_the_range(vg):
     """A softening whose square FP32 does not hold: the near field vanishes, and the potential is the far field's."""
     n = 2000

@@ -437,7 +437,6 @@ int vipp_grav_create(const vipp_grav_config *cfg, vipp_grav_ctx **out) {
             c.eps = cfg->epsilon;
             c.G = cfg->G;
             c.mass = cfg->mass;
-            c.mshift = vg::mass_shift(c.mass);
             c.flags = cfg->flags;
             c.device = cfg->device;
             VG_HIP(hipSetDevice(c.device));
@@ -509,7 +508,7 @@ int vipp_grav_upload(vipp_grav_ctx *ctx, const double *x, const double *v, const
             c.m.ensure(static_cast<size_t>(c.n));
             VG_HIP(hipMemcpyAsync(c.m.p, masses, c.n * sizeof(double), hipMemcpyHostToDevice, c.stream));
         }
-        c.mshift = vg::mass_shift(masses ? vg::largest_mass(c) : c.mass);
+        c.mmax = masses ? vg::largest_mass(c) : 1.0;
         VG_HIP(hipStreamSynchronize(c.stream));
         c.uploaded = true;
         c.evaluated = false;

@@ -102,7 +102,10 @@ __device__ inline double rsq(double x) {
 // units.  Lengths to 2^40 need none (r^-3 above 2^-123, normal); a root box wider
 // than 2^64, whose squares FP32 does not hold, is shifted as one of 2^64, so that
 // clusters small beside it keep their range; a softening of any size is shifted in
-// full, since nothing counts beside it.  Masses to 2^60 need none (times 2^41: 2^101).
+// full, since nothing counts beside it.  Masses to 2^40 need none, larger ones are taken
+// to 2^40 (times 2^41: 2^81); and where shorter lengths would make m / eps^3, which the pair
+// of a particle with itself forms and multiplies by 0, leave the range, masses are
+// shifted by up to three times as much, so that it is no larger than in the caller's units.
 __host__ __device__ inline int exponent_of(double v) {  // |v| < 2^e, at least half of that
     return static_cast<int>(__builtin_bit_cast(uint64_t, v) >> 52 & 0x7ff) - 1022;
 }
@@ -113,7 +116,16 @@ __host__ __device__ inline int length_shift(const double *box, double eps) {
     if (exponent_of(eps) > e) e = exponent_of(eps);
     return e > 40 ? e - 40 : 0;
 }
-inline int mass_shift(double largest) { return exponent_of(largest) > 60 ? exponent_of(largest) - 60 : 0; }
+__host__ __device__ inline int mass_shift(int length, double largest, double eps) {
+    const int em = exponent_of(largest);
+    int b = em > 40 ? em - 40 : 0;
+    if (eps != 0) {
+        const int self = em + 3 * (length + 1 - exponent_of(eps)) - 126, most = 3 * length;  // m / eps^3 below 2^126
+        const int need = self < most ? self : most;
+        if (need > b) b = need;
+    }
+    return b;
+}
 
 // x as two BF16 halves, hi = bf16(x) and lo = bf16(x - hi) (the split M2L's multipoles).
 __device__ __forceinline__ void split_m(float x, uint32_t &hi, uint32_t &lo) {

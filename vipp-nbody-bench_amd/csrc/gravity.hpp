@@ -97,7 +97,7 @@ struct Ctx {
     int device = 0;
     int ncu = 0;  // compute units of the device
     bool has_masses = false;
-    int mshift = 0;  // mass_shift of the largest mass
+    double mmax = 1;  // the largest mass; 1 without a mass array, whose pairs leave it out (mass_shift)
     bool uploaded = false;
     bool evaluated = false;
     std::string err;
@@ -142,7 +142,7 @@ struct Ctx {
     DevBuf<uint32_t> perm;      // sorted position -> caller index
     // particles in sorted order
     DevBuf<double> xs64;        // 4 per particle: x, y, z, m
-    DevBuf<float> xs32;         // 4 per particle: x - root centre (FP32) in units of 2^length_shift, m in units of 2^mshift
+    DevBuf<float> xs32;         // 4 per particle: x - root centre (FP32) in units of 2^length_shift, m in units of 2^mass_shift
     DevBuf<double> as64;        // 4 per particle: accel xyz, potential
     DevBuf<float> as32;
 
@@ -218,12 +218,21 @@ void direct_subset(Ctx &c, const int64_t *idx, int64_t nidx, double *a, double *
 void direct_subset_noalloc(Ctx &c, const int64_t *idx, int64_t nidx, double *a, double *pot);
 void noalloc_init(int device);
 
-// The squared softening of the near field, for FP32 in the units of its lengths.
-template <class R>
-R p2p_eps2(const Ctx &c) {
-    const double e = sizeof(R) == 4 ? c.eps * pow2(-length_shift(c.t.box, c.eps)) : c.eps;
-    return static_cast<R>(e * e);
-}
+// The units of the near field: FP32 ones of its own (length_shift, mass_shift), FP64 the
+// caller's.
+struct PairUnits {
+    int length = 0, mass = 0;
+    template <class R>
+    static PairUnits of(const Ctx &c) {
+        PairUnits u;
+        if (sizeof(R) == 4) {
+            u.length = length_shift(c.t.box, c.eps);
+            u.mass = mass_shift(u.length, c.mmax, c.eps);
+        }
+        return u;
+    }
+    double eps2(const Ctx &c) const { return c.eps * pow2(-length) * (c.eps * pow2(-length)); }
+};
 
 // Waits until a kernel of the stream has written `want` to a pinned host word.
 void wait_host_word(const uint32_t *word, uint32_t want, hipStream_t st);

@@ -242,7 +242,8 @@ struct McItem {
     int nt;               // targets
     float cell;           // half diagonal of the leaf
     float eps2;
-    bool um;              // one mass: left out here, the sums are scaled once
+    bool um;              // one mass: m1 here, the sums are scaled once
+    float m1;             // a power of two, 1 in ordinary units
     bool big;             // squared distances may leave the FP32 range
 };
 
@@ -307,7 +308,7 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
     float4 nx = source(0);
     for (int g = 0; g < ng; ++g) {
         float x = nx.x - cx, y = nx.y - cy, z = nx.z - cz;
-        float m = I.um ? 1.0f : nx.w;
+        float m = I.um ? I.m1 : nx.w;
         if (g + 1 < ng)
             nx = source(g + 1);
         else if (64u * g + lane >= I.len)  // the last source again, without mass
@@ -413,7 +414,7 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
         const int e = __shfl(I.src.rank, g, 64) + __popcll(m & ((1ull << pos) - 1));
         const uint32_t f = 64u * g + pos;
         float4 v = I.xs[S.delta[e] + static_cast<int32_t>(min(f, I.len - 1))];
-        if (I.um) v.w = 1.0f;
+        if (I.um) v.w = I.m1;
         if (n >= nn || f >= I.len) v.w = 0.0f;
         return v;
     };
@@ -468,7 +469,7 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
                                                        const uint32_t *__restrict__ count, const int32_t *__restrict__ anc,
                                                        const int32_t *__restrict__ ni, const int32_t *__restrict__ ni_cnt,
                                                        const double *__restrict__ bmin, const double *__restrict__ bmax, const float4 *__restrict__ xs,
-                                                       float eps2, float G, bool um, bool big, float fscale, float pscale, float mlen,
+                                                       float eps2, float G, bool um, float m1, bool big, float fscale, float pscale, float mlen,
                                                        float4 *__restrict__ acc, float4 *__restrict__ partial, float unit, uint32_t piece) {
     __shared__ McLds S;
     McWork wk = items[blockIdx.x];
@@ -486,6 +487,7 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
     I.cell = 0.5f * sqrtf(wx * wx + wy * wy + wz * wz);
     I.eps2 = eps2;
     I.um = um;
+    I.m1 = m1;
     I.big = big;
     float4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * 16 : nullptr;
     auto emit = [&](int t, const f4 &v) {
@@ -843,20 +845,22 @@ void p2p_run(Ctx &c, bool potential) {
     const R G = static_cast<R>(c.G);
     const bool um = !c.has_masses;  // one mass: left out of the pairs, the sums are scaled once
     if constexpr (sizeof(R) == 4) {
-        // units of lengths and masses, and what takes sums of m x / r^3 and m / r out of them
-        const int ls = length_shift(t.box, c.eps);
-        const float eps2 = p2p_eps2<float>(c), unit = static_cast<float>(pow2(-ls)), mlen = static_cast<float>(std::ldexp(1.0, c.mshift - ls));
-        const float fscale = static_cast<float>(um ? std::ldexp(c.mass, -2 * ls) : std::ldexp(1.0, c.mshift - 2 * ls));
-        const float pscale = um ? static_cast<float>(std::ldexp(c.mass, -ls)) : mlen;
+        // the units, and what takes sums of m x / r^3 and m / r out of them
+        const PairUnits u = PairUnits::of<float>(c);
+        const int ls = u.length;
+        const double m = um ? c.mass : 1.0;
+        const float eps2 = static_cast<float>(u.eps2(c)), unit = static_cast<float>(pow2(-ls)), mlen = static_cast<float>(std::ldexp(1.0, u.mass - ls));
+        const float fscale = static_cast<float>(std::ldexp(m, u.mass - 2 * ls)), pscale = static_cast<float>(std::ldexp(m, u.mass - ls));
+        const float m1 = static_cast<float>(pow2(-u.mass));
         bool big = false;  // a root box so wide that squared distances may leave the FP32 range all the same
         for (int a = 0; a < 3; ++a) big |= !((t.box[3 + a] - t.box[a]) * pow2(-ls) < 1e18);
         buffers(c.xs32, c.as32, c.p2p_part32, [&](const V4 *xs, V4 *acc, V4 *part) {
             for (uint32_t p = 0; p < pieces; ++p)
                 (potential ? k_p2p_mc<true> : k_p2p_mc<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs,
-                                                                                       eps2, G, um, big, fscale, pscale, mlen, acc, part, unit, p);
+                                                                                       eps2, G, um, m1, big, fscale, pscale, mlen, acc, part, unit, p);
         });
     } else {
-        const double eps2 = p2p_eps2<double>(c), mu = c.mass;
+        const double eps2 = PairUnits::of<double>(c).eps2(c), mu = c.mass;
         buffers(c.xs64, c.as64, c.p2p_part64, [&](const V4 *xs, V4 *acc, V4 *part) {
             for (uint32_t p = 0; p < pieces; ++p)
                 (potential ? k_p2p_f64<true> : k_p2p_f64<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, xs, eps2, G, um,

@@ -453,14 +453,15 @@ __global__ __launch_bounds__(64 * LS_WAVES) void k_leaf_sort_w(const int32_t *__
                                                                const uint32_t *__restrict__ start, const uint32_t *__restrict__ count, uint32_t thr,
                                                                const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
                                                                const double *__restrict__ x, const double *__restrict__ m, double mass,
-                                                               const double *__restrict__ box, double eps, double munit, double *__restrict__ xs64,
+                                                               const double *__restrict__ box, double eps, double mmax, double *__restrict__ xs64,
                                                                float *__restrict__ xs32) {
     extern __shared__ uint32_t sv[];
     const uint32_t nl = lv[LV_NLEAF];  // 0 when the build did not complete
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     uint32_t *sw = sv + w * thr;
     const double cx = (box[0] + box[3]) / 2, cy = (box[1] + box[4]) / 2, cz = (box[2] + box[5]) / 2;
-    const double unit = pow2(-length_shift(box, eps));
+    const int ls = length_shift(box, eps);
+    const double unit = pow2(-ls), munit = pow2(-mass_shift(ls, mmax, eps));
     auto put = [&](uint32_t k, uint32_t i, double px, double py, double pz, double mi) {
         out[k] = i;
         xs64[4ll * k] = px;
@@ -519,7 +520,7 @@ __global__ __launch_bounds__(64 * LS_WAVES) void k_leaf_sort_w(const int32_t *__
 }
 
 __global__ __launch_bounds__(256) void k_gather(const uint32_t *__restrict__ perm, int64_t n, const double *__restrict__ x, const double *__restrict__ m,
-                                                double mass, const double *__restrict__ box, double eps, double munit, double *__restrict__ xs64,
+                                                double mass, const double *__restrict__ box, double eps, double mmax, double *__restrict__ xs64,
                                                 float *__restrict__ xs32) {
     const int64_t k = blockIdx.x * 256ll + threadIdx.x;
     if (k >= n) return;
@@ -531,7 +532,8 @@ __global__ __launch_bounds__(256) void k_gather(const uint32_t *__restrict__ per
     xs64[4 * k + 2] = pz;
     xs64[4 * k + 3] = mi;
     const double cx = (box[0] + box[3]) / 2, cy = (box[1] + box[4]) / 2, cz = (box[2] + box[5]) / 2;
-    const double unit = pow2(-length_shift(box, eps));
+    const int ls = length_shift(box, eps);
+    const double unit = pow2(-ls), munit = pow2(-mass_shift(ls, mmax, eps));
     xs32[4 * k] = static_cast<float>((px - cx) * unit);
     xs32[4 * k + 1] = static_cast<float>((py - cy) * unit);
     xs32[4 * k + 2] = static_cast<float>((pz - cz) * unit);
@@ -885,7 +887,7 @@ void tree_build(Ctx &c, bool ahead) {
             // count changes little; the blocks loop over any excess)
             const int64_t leaves = t.nleaves > 0 ? std::max<int64_t>(1024, t.nleaves + t.nleaves / 4) : cap;
             k_leaf_sort_w<<<ceil_div(std::min(cap, leaves), LS_WAVES), 64 * LS_WAVES, LS_WAVES * c.thr * sizeof(uint32_t), st>>>(
-                t.leaf_ids, t.lv, t.start, t.count, c.thr, v0, c.perm, c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.box, c.eps, pow2(-c.mshift), c.xs64,
+                t.leaf_ids, t.lv, t.start, t.count, c.thr, v0, c.perm, c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.box, c.eps, c.mmax, c.xs64,
                 c.xs32);
         }
         VG_LAUNCH_CHECK();
@@ -935,7 +937,7 @@ void tree_build(Ctx &c, bool ahead) {
     t.nleaves = hlv[LV_NLEAF];
     if (t.nleaves && c.thr > LS_MAXTHR) {
         k_leaf_sort<<<static_cast<unsigned>(t.nleaves), 256, c.thr * sizeof(uint32_t), st>>>(t.leaf_ids, t.start, t.count, v0, c.perm);
-        k_gather<<<ceil_div(n, 256), 256, 0, st>>>(c.perm, n, c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.box, c.eps, pow2(-c.mshift), c.xs64, c.xs32);
+        k_gather<<<ceil_div(n, 256), 256, 0, st>>>(c.perm, n, c.x, c.has_masses ? c.m.p : nullptr, c.mass, c.box, c.eps, c.mmax, c.xs64, c.xs32);
         VG_LAUNCH_CHECK();
         VG_HIP(hipEventRecord(c.lists_ahead ? c.ev_lists : c.ev_tree, st));  // what P2P waits for has these particles in order
     }
