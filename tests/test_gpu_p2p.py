@@ -221,3 +221,23 @@ def test_p2p_items_in_pieces(vg):
             ref = g.direct(idx)
         assert np.linalg.norm(a[idx] - ref) <= 1e-4 * np.linalg.norm(ref), mode
     assert abs(u["f32"] - u["f64"]) <= 5e-6 * abs(u["f64"])
+
+
+@pytest.mark.parametrize("mode", ["f64", "f32", "split"])
+@pytest.mark.parametrize("n", [3, 17, 50, 700])
+@pytest.mark.parametrize("masses", [False, True])
+def test_potential_without_the_particle_itself(vg, mode, n, masses):
+    """Softening far below the distances, m_i / eps far above the potential: the energy of one leaf
+    against the sum over pairs.  Terms of one sign, each within 8 roundings, and their sums:
+    n + 8 roundings of 2^-24 or 2^-53."""
+    rng = np.random.default_rng(n)
+    x = np.round(rng.random((n, 3)) * 2 ** 18) / 2 ** 18
+    m = rng.uniform(0.5, 1.5, n) / n if masses else np.full(n, 1.0 / n)
+    with vg.Gravity(n, 1500, 3, mode, eps=1e-5) as g:
+        g.upload(x, None, m if masses else None)
+        u = g.energy()[1]
+    ref = np.longdouble(0)
+    for i in range(n):
+        d = (np.delete(x, i, 0) - x[i]).astype(np.longdouble)
+        ref -= m[i] / 2 * (np.delete(m, i) / np.sqrt((d * d).sum(1) + np.longdouble(1e-5) ** 2)).sum()
+    assert abs(u - ref) <= (n + 8) * 2.0 ** (-53 if mode == "f64" else -24) * abs(ref)

@@ -87,14 +87,6 @@ template <class R>
 using Quad = typename QuadOf<R>::T;
 
 __device__ inline float rsq(float x) { return __builtin_amdgcn_rsqf(x); }
-// 1/sqrt(x) in FP64: with e = 1 - x y^2 of the hardware's estimate y (2^-24 at
-// worst), y (1 + e / 2 + 3/8 e^2) is off by its roundings and less than 2^-69
-// (x > 0; x = 0 gives NaN, which the P2P's self-pair select replaces)
-__device__ inline double rsq(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x, y * y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
-}
 
 // The FP32 near field forms masses times positions and r^-3 by themselves, so it
 // takes positions in units of 2^length_shift and masses in units of 2^mass_shift, which

@@ -978,7 +978,7 @@ struct Near {
     const Quad<R> *acc;                 // sums of the leaves with one work item, times G
     const Quad<R> *part;                // rows of partial sums of the others
     const uint32_t *nchunk, *item_off;  // per leaf: rows (1: none) of whole 16-particle tiles, first tile
-    R eps2, unit, G;                    // eps2 in squares of 1 / unit (PairUnits)
+    R G;
     const uint32_t *perm;  // caller's index of a sorted particle
     R *a;                  // accelerations in the caller's order
     double *pot;           // potentials, or nullptr
@@ -1027,7 +1027,6 @@ __global__ __launch_bounds__(64) void k_l2p(const int32_t *__restrict__ leaves, 
                 v.z += u.z;
                 v.w += u.w;
             }
-            if (POT && near.eps2 > R(0)) v.w -= static_cast<R>(xm.w) * (rsq(near.eps2) * near.unit);  // drop the m_i / eps self term
             v.x *= near.G, v.y *= near.G, v.z *= near.G;
         }
         auto store = [&] {
@@ -1111,7 +1110,7 @@ Near<R> near_of(Ctx &c, const DevBuf<R> &acc, const DevBuf<R> &part, DevBuf<R> &
     a.ensure(3 * n);
     if (potential) c.pot64.ensure(n);
     return {reinterpret_cast<const Quad<R> *>(acc.p), reinterpret_cast<const Quad<R> *>(part.p), c.p2p_nchunk, c.p2p_item_off,
-            static_cast<R>(PairUnits::of<R>(c).eps2(c)), static_cast<R>(pow2(-PairUnits::of<R>(c).length)), static_cast<R>(c.G), c.perm, a.p, potential ? c.pot64.p : nullptr};
+            static_cast<R>(c.G), c.perm, a.p, potential ? c.pot64.p : nullptr};
 }
 
 template <class R>

@@ -15,8 +15,12 @@
 //  * FP64 (k_p2p_f64): pairs by differences.
 // A leaf with one chunk writes its result; split leaves write partial sums, a row of
 // whole 16-target tiles for each chunk, which L2P adds in chunk order
-// (deterministic).  With a nonzero softening the i == j term is exactly zero (dx =
-// dy = dz = 0), so it needs no branch; without softening a select removes it.
+// (deterministic).  With a nonzero softening the i == j force is exactly zero (dx = dy
+// = dz = 0), so it needs no branch; without softening a select removes it.  The i == j
+// potential m_i / eps is left out by the particle's index, in the few groups of sources
+// that hold targets: subtracted afterwards, it leaves the rounding of sums as large as
+// itself (FP32, eps = 1e-4, energy of 17 particles: 8e-6 off, now 1.2e-8; of 120 with one
+// mass: 1.1e-6, now 4.5e-8).
 #include "gravity.hpp"
 
 namespace vg {
@@ -119,7 +123,7 @@ struct McLds {
     float4 Q[64];          // m (x, y, z, 1) of the staged sources; (x, y, z, m) in the near pass; while the entries are laid out, their masks
     int32_t delta[MAXE];   // per entry of the item: particle index minus position in the item
     uint16_t near[64 * 4]; // 16-source tiles left to the near pass
-    float4 M[16];          // masses of the staged sources (for the potential)
+    float4 M[16];          // for the potential: masses of the staged sources; in the near pass, their indices
 };
 
 // A work item as the plan leaves it.
@@ -407,13 +411,15 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
             if (mynear >> k & 1) S.near[at++] = static_cast<uint16_t>(4 * lane + k);
         wave_lds_sync();
     }
+    int ni = 0;  // particle index of nx
     auto near_source = [&](int j) {  // this lane's source of the near tiles 4 j .. 4 j + 3
         const int n = 4 * j + quad;
         const int tl = S.near[min(n, nn - 1)], g = tl >> 2, pos = 16 * (tl & 3) + col;
         const uint64_t m = static_cast<uint64_t>(static_cast<uint32_t>(__shfl(static_cast<int>(I.src.mhi), g, 64))) << 32 | static_cast<uint32_t>(__shfl(static_cast<int>(I.src.mlo), g, 64));
         const int e = __shfl(I.src.rank, g, 64) + __popcll(m & ((1ull << pos) - 1));
         const uint32_t f = 64u * g + pos;
-        float4 v = I.xs[S.delta[e] + static_cast<int32_t>(min(f, I.len - 1))];
+        ni = S.delta[e] + static_cast<int32_t>(min(f, I.len - 1));
+        float4 v = I.xs[ni];
         if (I.um) v.w = I.m1;
         if (n >= nn || f >= I.len) v.w = 0.0f;
         return v;
@@ -422,15 +428,19 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
     for (int j = 0; 4 * j < nn; ++j) {
         __builtin_amdgcn_wave_barrier();
         S.Q[lane] = nx;
+        const int who = ni - static_cast<int>(I.pt0);  // the target that it is
+        if (POT) reinterpret_cast<int *>(S.M)[lane] = who;
+        const bool own = POT && __ballot(who >= 0 && who < I.nt) != 0;  // the few tiles that hold targets
         if (4 * j + 4 < nn) nx = near_source(j + 1);
         wave_lds_sync();
         const int kn = min(4, nn - 4 * j);
-        auto pairs = [&](auto soft) {
+        auto pairs = [&](auto soft, auto own) {
 #pragma unroll 1
             for (int k = 0; k < kn; ++k) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float4 s = S.Q[16 * k + 4 * quad + i];
+                    const int self = decltype(own)::value ? reinterpret_cast<const int *>(S.M)[16 * k + 4 * quad + i] - col : 0;
 #pragma unroll
                     for (int t = 0; t < T; ++t) {
                         const float dx = s.x - xt[t], dy = s.y - yt[t], dz = s.z - zt[t];
@@ -441,15 +451,17 @@ __device__ __forceinline__ void mc_pass(const McItem &I, McLds &S, F &&emit) {
                         acc[t][0] += w * dx;
                         acc[t][1] += w * dy;
                         acc[t][2] += w * dz;
-                        if (POT) acc[t][3] += mr;
+                        if (POT) acc[t][3] += decltype(own)::value && self == 16 * t ? 0.0f : mr;
                     }
                 }
             }
         };
-        if (I.eps2 > 0.0f)
-            pairs(std::true_type{});
+        if (!(I.eps2 > 0.0f))
+            pairs(std::false_type{}, std::false_type{});
+        else if (POT && own)
+            pairs(std::true_type{}, std::bool_constant<POT>{});
         else
-            pairs(std::false_type{});
+            pairs(std::true_type{}, std::false_type{});
     }
     // the four lane groups hold the sums over their own source rows
 #pragma unroll
@@ -469,7 +481,7 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
                                                        const uint32_t *__restrict__ count, const int32_t *__restrict__ anc,
                                                        const int32_t *__restrict__ ni, const int32_t *__restrict__ ni_cnt,
                                                        const double *__restrict__ bmin, const double *__restrict__ bmax, const float4 *__restrict__ xs,
-                                                       float eps2, float G, bool um, float m1, bool big, float fscale, float pscale, float mlen,
+                                                       float eps2, float G, bool um, float m1, bool big, float fscale, float pscale,
                                                        float4 *__restrict__ acc, float4 *__restrict__ partial, float unit, uint32_t piece) {
     __shared__ McLds S;
     McWork wk = items[blockIdx.x];
@@ -491,8 +503,7 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
     I.big = big;
     float4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * 16 : nullptr;
     auto emit = [&](int t, const f4 &v) {
-        const float sx = v[0] * fscale, sy = v[1] * fscale, sz = v[2] * fscale;
-        float sp = v[3] * pscale;
+        const float sx = v[0] * fscale, sy = v[1] * fscale, sz = v[2] * fscale, sp = v[3] * pscale;
         if (out) {
             float4 o = float4{sx, sy, sz, sp};
             if (piece) {
@@ -501,7 +512,6 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
             }
             out[wk.t0 + t] = o;
         } else {
-            if (POT && eps2 > 0.0f) sp -= xs[I.pt0 + t].w * rsq(eps2) * mlen;  // drop the m_i / eps self term
             acc[I.pt0 + t] = float4{G * sx, G * sy, G * sz, sp};
         }
     };
@@ -535,7 +545,7 @@ __global__ __launch_bounds__(64, 4) void k_p2p_mc(const McWork *__restrict__ ite
 // two Newton steps for each root: 16384 particles (s = 64) 0.33 -> 0.15 ms, 64k
 // mixture 1.05 -> 0.40, 128k (s = 128) 3.0 -> 1.7, 1M 3.3 -> 2.7 ms.
 template <int T, bool POT, class F>
-__device__ __forceinline__ void f64_pass(const double4 *__restrict__ xs, const Sources &src, const int32_t *delta, double4 *tile, uint32_t len,
+__device__ __forceinline__ void f64_pass(const double4 *__restrict__ xs, const Sources &src, const int32_t *delta, double4 *tile, int *who, uint32_t len,
                                          uint32_t pt0, int nt, double eps2, bool um, F &&emit) {
     const int lane = threadIdx.x, col = lane & 15, quad = lane >> 4;
     const int ng = static_cast<int>((len + 63) / 64);
@@ -546,24 +556,32 @@ __device__ __forceinline__ void f64_pass(const double4 *__restrict__ xs, const S
         x[t] = v.x, y[t] = v.y, z[t] = v.z;
         acc[t][0] = acc[t][1] = acc[t][2] = acc[t][3] = 0;
     }
-    double4 nx = xs[source_of(src, delta, 0, len)];
+    int ni = source_of(src, delta, 0, len);  // particle index of nx
+    double4 nx = xs[ni];
     for (int g = 0; g < ng; ++g) {
         __builtin_amdgcn_wave_barrier();
         const bool full = 64u * g + 64 <= len;
         if (um) nx.w = 1.0;
         if (64u * g + lane >= len) nx.w = 0.0;  // the last source again, without mass
         tile[lane] = nx;
-        if (g + 1 < ng) nx = xs[source_of(src, delta, g + 1, len)];
+        const int me = ni - static_cast<int>(pt0);  // the target that it is
+        if (POT) who[lane] = me;
+        const bool own = POT && __ballot(me >= 0 && me < nt) != 0;  // the few groups that hold targets
+        if (g + 1 < ng) {
+            ni = source_of(src, delta, g + 1, len);
+            nx = xs[ni];
+        }
         wave_lds_sync();
-        auto pairs = [&](auto soft, auto weighted) {
+        auto pairs = [&](auto soft, auto weighted, auto own) {
 #pragma unroll 2
             for (int i = 0; i < 16; ++i) {
                 const double4 s = tile[4 * i + quad];
+                const int self = decltype(own)::value ? who[4 * i + quad] - col : 0;
 #pragma unroll
                 for (int t = 0; t < T; ++t) {
                     const double dx = s.x - x[t], dy = s.y - y[t], dz = s.z - z[t];
                     const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));
-                    const double h = __builtin_amdgcn_rsq(r2);  // refined as in rsq; r2^(-3/2) = h^3 (1 + 3/2 e + 15/8 e^2 + ..)
+                    const double h = __builtin_amdgcn_rsq(r2);  // 2^-24 at worst; r2^(-3/2) = h^3 (1 + 3/2 e + 15/8 e^2 + ..), e^3 below 2^-69
                     const double hh = h * h, e = fma(-r2, hh, 1.0);
                     const double c = (decltype(weighted)::value ? h * s.w : h) * hh;
                     double w = fma(c * e, fma(e, 1.875, 1.5), c);
@@ -574,21 +592,24 @@ __device__ __forceinline__ void f64_pass(const double4 *__restrict__ xs, const S
                     if (POT) {
                         double ri = fma(h * e, fma(e, 0.375, 0.5), h);
                         if (!decltype(soft)::value) ri = r2 > 0.0 ? ri : 0.0;
+                        if (decltype(own)::value) ri = self == 16 * t ? 0.0 : ri;
                         acc[t][3] = decltype(weighted)::value ? fma(s.w, ri, acc[t][3]) : acc[t][3] + ri;
                     }
                 }
             }
         };
         if (eps2 > 0.0) {
-            if (um && full)
-                pairs(std::true_type{}, std::false_type{});
+            if (POT && own)
+                pairs(std::true_type{}, std::true_type{}, std::bool_constant<POT>{});
+            else if (um && full)
+                pairs(std::true_type{}, std::false_type{}, std::false_type{});
             else
-                pairs(std::true_type{}, std::true_type{});
+                pairs(std::true_type{}, std::true_type{}, std::false_type{});
         } else {
             if (um && full)
-                pairs(std::false_type{}, std::false_type{});
+                pairs(std::false_type{}, std::false_type{}, std::false_type{});
             else
-                pairs(std::false_type{}, std::true_type{});
+                pairs(std::false_type{}, std::true_type{}, std::false_type{});
         }
     }
 #pragma unroll
@@ -608,7 +629,7 @@ __global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ it
                                                    const int32_t *__restrict__ ni_cnt, const double4 *__restrict__ xs, double eps2, double G, bool um,
                                                    double mu, double4 *__restrict__ acc, double4 *__restrict__ partial, uint32_t piece) {
     __shared__ double4 tile[64];
-    __shared__ int32_t delta[MAXE];
+    __shared__ int32_t delta[MAXE], who[POT ? 64 : 1];
     McWork wk = items[blockIdx.x];
     if (!take_piece(wk, piece)) return;
     const int lane = threadIdx.x, nt = static_cast<int>(wk.nt);
@@ -616,8 +637,7 @@ __global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ it
     double4 *out = wk.out != ~0u ? partial + static_cast<size_t>(wk.out) * 16 : nullptr;
     const Sources src = lay_out_entries(wk, delta, reinterpret_cast<uint64_t *>(tile), start, count, anc, ni, ni_cnt);
     auto emit = [&](int t, const double *v) {
-        const double sx = v[0] * sc, sy = v[1] * sc, sz = v[2] * sc;
-        double sp = v[3] * sc;
+        const double sx = v[0] * sc, sy = v[1] * sc, sz = v[2] * sc, sp = v[3] * sc;
         if (out) {
             double4 o = double4{sx, sy, sz, sp};
             if (piece) {
@@ -626,7 +646,6 @@ __global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ it
             }
             out[wk.t0 + t] = o;
         } else {
-            if (POT && eps2 > 0.0) sp -= xs[wk.pt0 + t].w * rsq(eps2);  // drop the m_i / eps self term
             acc[wk.pt0 + t] = double4{G * sx, G * sy, G * sz, sp};
         }
     };
@@ -636,7 +655,7 @@ __global__ __launch_bounds__(64, 4) void k_p2p_f64(const McWork *__restrict__ it
         return;
     }
     const int T = (nt + 15) / 16;  // at most F64_TILES
-    auto pass = [&](auto tiles) { f64_pass<decltype(tiles)::value, POT>(xs, src, delta, tile, wk.len, wk.pt0, nt, eps2, um, emit); };
+    auto pass = [&](auto tiles) { f64_pass<decltype(tiles)::value, POT>(xs, src, delta, tile, who, wk.len, wk.pt0, nt, eps2, um, emit); };
     if (T == 1)
         pass(std::integral_constant<int, 1>{});
     else if (T == 2)
@@ -849,7 +868,7 @@ void p2p_run(Ctx &c, bool potential) {
         const PairUnits u = PairUnits::of<float>(c);
         const int ls = u.length;
         const double m = um ? c.mass : 1.0;
-        const float eps2 = static_cast<float>(u.eps2(c)), unit = static_cast<float>(pow2(-ls)), mlen = static_cast<float>(std::ldexp(1.0, u.mass - ls));
+        const float eps2 = static_cast<float>(u.eps2(c)), unit = static_cast<float>(pow2(-ls));
         const float fscale = static_cast<float>(std::ldexp(m, u.mass - 2 * ls)), pscale = static_cast<float>(std::ldexp(m, u.mass - ls));
         const float m1 = static_cast<float>(pow2(-u.mass));
         bool big = false;  // a root box so wide that squared distances may leave the FP32 range all the same
@@ -857,7 +876,7 @@ void p2p_run(Ctx &c, bool potential) {
         buffers(c.xs32, c.as32, c.p2p_part32, [&](const V4 *xs, V4 *acc, V4 *part) {
             for (uint32_t p = 0; p < pieces; ++p)
                 (potential ? k_p2p_mc<true> : k_p2p_mc<false>)<<<nitems, 64, 0, c.stream>>>(items, t.start, t.count, t.anc, t.ni, t.ni_cnt, t.bmin, t.bmax, xs,
-                                                                                       eps2, G, um, m1, big, fscale, pscale, mlen, acc, part, unit, p);
+                                                                                       eps2, G, um, m1, big, fscale, pscale, acc, part, unit, p);
         });
     } else {
         const double eps2 = PairUnits::of<double>(c).eps2(c), mu = c.mass;
